@@ -1,0 +1,67 @@
+"""The weight-streaming bf16 kernels (few rows per expert, csrc/moe_stream.h) at the sizes where they can go wrong:
+live rows around the 4-row, 32-row, 64-row and 128-row edges, blocks of one expert that take several passes, one slab
+and more slabs than stages, the short-contraction down kernel (H = 128, 256) and the general one, tiles of one
+and of two units of weight rows."""
+import pytest
+import torch
+
+from helpers import BF16_GATE, rel_clamp
+from oracle import moe_oracle as O
+from test_gpu_bf16 import _inputs
+from test_gpu_mxfp8 import _routing_by_counts
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 4, 5, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129]
+
+
+@pytest.mark.parametrize("K,N,E,split", [
+    (128, 256, 40, True),     # one slab up, H = 128 down
+    (384, 512, 40, False),    # three slabs, H = 256 down
+    (640, 768, 40, True),     # H = 384: general down kernel, three slabs
+    (3072, 256, 40, True),    # more slabs than stages
+    (512, 1024, 64, False),   # jobs of two units of weight rows in both kernels
+])
+def test_stream_kernels_at_row_edges(K, N, E, split, device):
+    import prime_moe
+    counts = EDGES + [0] * (E - len(EDGES))
+    ids, wts = _routing_by_counts(counts, 2, device, seed=K)
+    T = ids.shape[0]
+    assert 2 * T <= 32 * E  # the rule of the dispatch
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    outs = []
+    for _ in range(2):
+        torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+        out = torch.zeros((T, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, 2, 128, 64, 4, 2, 1, 1, split)
+        outs.append(out)
+    torch.cuda.synchronize()
+    got = outs[0].float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+def test_stream_kernels_with_dropped_rows_and_blocks(device):
+    """Holes in a block (tokens beyond M), a block without an expert, a misaligned end of the schedule."""
+    import prime_moe
+    T, K, E, N, top_k = 24, 256, 6, 512, 2
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=3)
+    ids = torch.randint(0, E, (T, top_k), device=device, generator=g, dtype=torch.int32)
+    wts = torch.softmax(torch.randn((T, top_k), device=device, generator=g), -1)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    keep = 17
+    e_bad = e.clone()
+    e_bad[1] = E + 3
+    w_ref = wts.clone()
+    w_ref[ids == int(e[1])] = 0.0
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), w_ref.cpu())[:keep]
+    for length in (s.numel(), int(n[0]) - 100):  # (the cut rows are padding of the last block)
+        assert bool((s[length:int(n[0])] < 0).all())
+        out = torch.empty((keep, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_bf16(x[:keep].contiguous(), w1, w2, s[:length].contiguous(), e_bad, n, wts, out, top_k,
+                                 128, 64, 4, 2, 1, 1, True)
+        torch.cuda.synchronize()
+        got = out.float().cpu()
+        assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
