@@ -20,6 +20,7 @@
 
 #include "moe_pipeline.h"
 #include "moe_ring.h"
+#include "moe_stream_mx.h"
 
 namespace pmoe {
 
@@ -42,9 +43,23 @@ struct Job {
     bool w_once;  // no other row tile of this expert: nobody else reads the weight rows of this job
 };
 
-// Workgroup id -> job: one load from the work list, which the prologue lays out by workgroup id (see
-// emit_work); entries of workgroups without work are -1.
+// Workgroup id -> job.  With a work list: one load from it, which the prologue lays out by workgroup id (see
+// emit_work); entries of workgroups without work are -1.  Without one (few rows per expert, see use_direct): every
+// live block is a row tile of its own, its jobs are consecutive workgroups.
 __device__ __forceinline__ bool resolve_job(const MoeArgs &a, Job &j) {
+    if (a.work == nullptr) {
+        const int n_jobs = (a.n_wtiles + a.per_job - 1) / a.per_job;
+        j.first = (int)blockIdx.x / n_jobs;
+        if (j.first >= min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks)) return false;
+        j.e = a.expert_ids[j.first];
+        if (j.e < 0 || j.e >= a.E) return false;
+        j.nb = 1;
+        j.wt = ((int)blockIdx.x - j.first * n_jobs) * a.per_job;
+        j.n_sub = min(a.per_job, a.n_wtiles - j.wt);
+        j.w_once = (j.first == 0 || a.expert_ids[j.first - 1] != j.e) &&
+                   (j.first + 1 >= a.n_blocks || a.expert_ids[j.first + 1] != j.e);
+        return true;
+    }
     const int4 w = a.work[blockIdx.x];
     if (w.x < 0) return false;
     j.first = w.x & 0x0fffffff;
@@ -242,14 +257,15 @@ __device__ __forceinline__ void store_act_tile(const MoeArgs &a, const char *til
 // tile row `row` (0..255: block 0, then block 1) in `tok_base`; weight rows: the tile's two 128-row
 // halves start at w_base[0/1] with `w_pitch` bytes per row.  Scales (mxfp8): `tok_sc_off(row)` /
 // `w_sc_off(row)` are the byte offsets of the row's first 4-scale dword; the dword of the next 128-wide
-// K tile lies 512 bytes on in both (blocked weight scales, tiled token-side scales).  Only the live 32-row
+// K tile lies 512 bytes on in the blocked weight scales, tok_sc_step in the token side's (512 if they are tiled,
+// 4 in a row-major matrix).  Only the live 32-row
 // fragments of the two blocks (ntf0, ntf1 of them) are copied; they are packed one after the other in
 // the stage (see ring::Layout).
 template <int DT, int RB, typename TokOff, typename TokScOff, typename WScOff>
 __device__ __forceinline__ void setup_ring_loader(ring::Loader<RB> &ld, const ring::Layout &lay, int tid,
                                                   uint32_t w_pitch, int ntf0, int ntf1, const RowInfo<2> &ri,
                                                   bool w_once, TokOff tok_row_off,
-                                                  const uint8_t *tok_sc_base, TokScOff tok_sc_off,
+                                                  const uint8_t *tok_sc_base, uint32_t tok_sc_step, TokScOff tok_sc_off,
                                                   const uint8_t *w_sc_base, WScOff w_sc_off) {
     using L = ring::Loader<RB>;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -292,7 +308,7 @@ __device__ __forceinline__ void setup_ring_loader(ring::Loader<RB> &ld, const ri
             const int row = c < 32 * ntf0 ? c : kBlockRows + c - 32 * ntf0;
             ld.sc_base = reinterpret_cast<const char *>(tok_sc_base);
             ld.sc_off = tok_sc_off(row);
-            ld.sc_step = 512u;
+            ld.sc_step = tok_sc_step;
             ld.sc_dst = lay.scale_off + 64 * wave * 4;
         }
     }
@@ -344,8 +360,12 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, R
     setup_ring_loader<DT, RB>(
         ld, lay, tid, row_bytes, ntf0, ntf1, ri, job.w_once,
         [&](int row) { return (uint32_t)max(ri.tok[row], 0) * row_bytes; },
-        reinterpret_cast<const uint8_t *>(a.xs_tiled + (int64_t)first * kt128 * kBlockRows),
-        [&](int row) { return (uint32_t)(((row >> 7) * kt128 * kBlockRows + (row & 127)) * 4); },
+        a.work != nullptr ? reinterpret_cast<const uint8_t *>(a.xs_tiled + (int64_t)first * kt128 * kBlockRows) : a.x_scales,
+        a.work != nullptr ? 512u : 4u,
+        [&](int row) {
+            return a.work != nullptr ? (uint32_t)(((row >> 7) * kt128 * kBlockRows + (row & 127)) * 4)
+                                     : (uint32_t)(max(ri.tok[row], 0) * kb);
+        },
         a.w1_scales + (int64_t)e * N * kb,
         [&](int row) { return (uint32_t)blocked_scale_off((row < 128 ? h0 : H + h0 - 128) + row, 0, K >> 7); });
 
@@ -407,6 +427,7 @@ __global__ __launch_bounds__(512) void moe_up_kernel(MoeArgs a) {
     using L = SplitLds<DT>;
     __shared__ __attribute__((aligned(1024))) char lds[L::kTotal];
     RowInfo<2> &ri = *reinterpret_cast<RowInfo<2> *>(lds + L::kRowInfoOff);
+    if (a.work == nullptr) stream::invert(a, 512);  // (no prologue did)
     Job j;
     if (!resolve_job(a, j)) return;
     const int ntf = load_row_info<2>(a, j.first, j.nb, ri);
@@ -453,7 +474,7 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
     set_weights(k0);
     setup_ring_loader<DT, RB>(
         ld, lay, tid, row_bytes, ntf0, ntf1, ri, job.w_once, [&](int row) { return (uint32_t)row * row_bytes; },
-        reinterpret_cast<const uint8_t *>(a.act_scales + (int64_t)first * ht128 * kBlockRows),
+        reinterpret_cast<const uint8_t *>(a.act_scales + (int64_t)first * ht128 * kBlockRows), 512u,
         [&](int row) { return (uint32_t)(((row >> 7) * ht128 * kBlockRows + (row & 127)) * 4); },
         a.w2_scales + (int64_t)e * K * hb,
         [&](int row) { return (uint32_t)blocked_scale_off(min(k0 + row, K - 1), 0, ht128); });
@@ -672,6 +693,21 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
     }
 }
 
+// Weight-streaming kernels (moe_stream_mx.h).  n_tiles: weight tiles per block (0: the up kernel only inverts).
+template <bool UP>
+__global__ __launch_bounds__(512, 4) void moe_stream_kernel_mx(MoeArgs a, int n_tiles) {
+    __shared__ __attribute__((aligned(1024))) stream::Shared sh;
+    stream::for_each_job<UP>(a, n_tiles, [&](int blk, int e, int tile, int id) { stream::mx_run_job<UP>(a, sh, blk, e, tile, id); });
+}
+
+// Down GEMM for H = RB without a prologue (see stream::for_each_turn).
+template <int RB>
+__global__ __launch_bounds__(256, 2) void moe_stream_down_short_kernel_mx(MoeArgs a) {
+    __shared__ __attribute__((aligned(1024))) char bufs[4][stream::ShortDownMx<RB>::kBytes];
+    stream::ShortDownMx<RB> eng(a, bufs[__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)]);
+    stream::for_each_turn(a, a.K / stream::ShortDownMx<RB>::kTurnCols, eng);
+}
+
 // out[t] = bf16(sum over the token's top_k pairs p, in pair order, of w[p] * y[p]) (ACCUMULATE: added to
 // what `out` holds).  A pair counts if inv[p] is a row of the schedule that really holds p in a block with
 // an expert; otherwise the schedule dropped it, nobody wrote y[p], and it contributes nothing.  A pair id
@@ -862,10 +898,70 @@ struct SchedBuffers {
     int4 *work_down;
 };
 
+// Blocks with work that the host can expect: an expert each, and no more than there are pairs.
+static int64_t expected_blocks(const MoeArgs &a) {
+    return std::min<int64_t>(a.n_blocks, std::min<int64_t>(a.E, (int64_t)a.M * a.top_k));
+}
+// Few rows per expert: blocks hardly ever share an expert, so there is nothing to pair and no schedule to build, and
+// consecutive workgroups on consecutive weight tiles read one narrow window of the weights.  Whole op with / without
+// the prologue and its work lists (256 experts of K 7168 x N 4096, top 8): 290 / 304 us at 5 tokens, 1824 / 1835 at 512
+// (16 rows per expert), 1938 / 1922 at 1024; skewed (Zipf) 931 / 951 at 64, 1751 / 1880 at 512.  With few up jobs for
+// the chip the streaming up kernel pays longer: 37 experts of K 4096 x N 256, top 9: 53 / 71 us at 128 tokens, 58 / 94
+// at 256 (62 rows per expert).
+static bool use_direct(const MoeArgs &a) {
+    const int64_t rows = expected_blocks(a) * (a.H / 128) < resident_grid() / 2 ? 64 : 24;
+    return (int64_t)a.M * a.top_k <= rows * a.E;
+}
+
+static int launch_direct_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
+    const int mask = g_phase_mask, n_cus = resident_grid();
+    const int64_t blocks = expected_blocks(a);
+    auto launch_stream = [&](auto kernel, int n_tiles) {
+        const int grid = (int)std::min<int64_t>((int64_t)a.n_blocks * std::max(n_tiles, 1), 2 * n_cus);
+        if (grid > 0) hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, s, a, n_tiles);
+    };
+    auto launch_ring = [&](auto kernel, bool down, int n_wt) {
+        MoeArgs d = a;
+        d.work = nullptr;
+        d.n_wtiles = n_wt;
+        d.per_job = tiles_per_workgroup(down, (int)blocks, n_wt);
+        const int grid = a.n_blocks * ((n_wt + d.per_job - 1) / d.per_job);
+        if (grid > 0) hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, s, d);
+    };
+    const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
+    if (mask & PMOE_PHASE_UP) {
+        // narrow jobs while wide tiles do not give every CU one (us at 128 / 256 / 640 / 1024 wide jobs, stream against
+        // ring, whole op: 75.5 / 81.7, 130 / 129, 291 / 290, 419 / 406)
+        if (blocks * n_wt_up < n_cus) launch_stream(moe_stream_kernel_mx<true>, a.H / 32);
+        else launch_ring(moe_up_kernel<DT_FP8>, false, n_wt_up);
+    } else if (mask & PMOE_PHASE_PROLOGUE) {
+        launch_stream(moe_stream_kernel_mx<true>, 0);
+    }
+    if (mask & PMOE_PHASE_DOWN) {
+        if (a.H <= 256) {
+            // (257 experts of K 7168, H 256: 250 against 282 us at 128 tokens; 37 of K 4096, H 128: 23 / 29 at 8)
+            const int grid = (int)std::min<int64_t>((int64_t)a.n_blocks * (a.K / 128), 2 * n_cus);
+            if (grid > 0) {
+                if (a.H == 128) hipLaunchKernelGGL(moe_stream_down_short_kernel_mx<128>, dim3(grid), dim3(256), 0, s, a);
+                else hipLaunchKernelGGL(moe_stream_down_short_kernel_mx<256>, dim3(grid), dim3(256), 0, s, a);
+            }
+        } else if (blocks * n_wt_down < 5 * n_cus && (int64_t)a.M * a.top_k <= 4 * blocks) {
+            // (256 experts, K 7168, H 2048, stream against ring, whole op: 71.6 / 75.5 us at 1 token, 126 / 130 at 2,
+            // 288 / 291 at 5, 408 / 406 at 8; 32 experts with 8 rows each, K 2048, H 1024: 45.0 / 44.6)
+            launch_stream(moe_stream_kernel_mx<false>, a.K / 64);
+        } else {
+            launch_ring(moe_down_kernel<DT_FP8>, true, n_wt_down);
+        }
+    }
+    if (mask & PMOE_PHASE_FINALIZE) launch_finalize(a, out, split, n_wt_down, s);
+    return check_launch("fused_moe_mxfp8 launch");
+}
+
 static int launch_mxfp8_pipeline(MoeArgs a, const SchedBuffers &sb, void *out, int split, hipStream_t s) {
     constexpr int DT = DT_FP8;
     const int mask = g_phase_mask;
     a.n_blocks = (a.sorted_num + kBlockRows - 1) / kBlockRows;
+    if (use_direct(a)) return launch_direct_pipeline(a, out, split, s);
     a.n_wtiles = a.H / 128;
     const int n_wt_down = (a.K + kWRows - 1) / kWRows;
     const int per_up = tiles_per_workgroup(false, a.n_blocks, a.n_wtiles);

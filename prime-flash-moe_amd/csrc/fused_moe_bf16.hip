@@ -561,60 +561,19 @@ __global__ __launch_bounds__(512) void moe_down_kernel_bf16(MoeArgs a) {
     }
 }
 
-// Weight-streaming kernels (moe_stream.h).  The up kernel also inverts the sorted order for finalize (see the
-// prologue above, which this path does without).  n_tiles: weight tiles per block (0: only invert).
+// Weight-streaming kernels (moe_stream.h).  n_tiles: weight tiles per block (0: the up kernel only inverts).
 template <bool UP, int U>
 __global__ __launch_bounds__(512, 4) void moe_stream_kernel(MoeArgs a, int n_tiles) {
     __shared__ __attribute__((aligned(1024))) stream::Shared sh;
-    const int tid = threadIdx.x, grid = (int)gridDim.x;
-    // sorted id (threads 0 .. 127) and expert of a job's block, fetched under the job before; for the first job
-    // without waiting for the length of the schedule
-    auto fetch = [&](int j, int &id, int &e) {
-        id = e = -1;
-        const int blk = n_tiles > 0 ? j / n_tiles : a.n_blocks;
-        if (blk < a.n_blocks) {
-            const int s = blk * kBlockRows + tid;
-            if (tid < kBlockRows && s < a.sorted_num) id = a.sorted_ids[s];
-            e = a.expert_ids[blk];
-        }
-    };
-    int id, e;
-    fetch((int)blockIdx.x, id, e);
-    const int ntpp = a.ntpp[0];
-    const int n_jobs = min((ntpp + kBlockRows - 1) / kBlockRows, a.n_blocks) * n_tiles;
-    if (UP) {
-        const int n_rows = min(ntpp, a.sorted_num), n_pairs = a.M * a.top_k;
-        for (int s = (int)blockIdx.x * 512 + tid; s < n_rows; s += grid * 512) {
-            const int p = a.sorted_ids[s], es = a.expert_ids[s >> 7];
-            if (p >= 0 && p < n_pairs && es >= 0 && es < a.E) a.inv[p] = s;
-        }
-    }
-    for (int j = (int)blockIdx.x; j < n_jobs; j += grid) {
-        const int blk = j / n_tiles;
-        int next_id, next_e;
-        fetch(j + grid, next_id, next_e);
-        if (e >= 0 && e < a.E) stream::run_job<UP, U>(a, sh, blk, __builtin_amdgcn_readfirstlane(e), j - blk * n_tiles, id);
-        id = next_id;
-        e = next_e;
-    }
+    stream::for_each_job<UP>(a, n_tiles, [&](int blk, int e, int tile, int id) { stream::run_job<UP, U>(a, sh, blk, e, tile, id); });
 }
 
-// Down GEMM of the streaming path for H = RB / 2 (see stream::down_short): jobs of `chunk` groups of four units (128
-// output columns, one unit per wave) of a live block.
+// Down GEMM of the streaming path for H = RB / 2 (see stream::for_each_turn).
 template <int RB>
-__global__ __launch_bounds__(256, RB == 256 ? 4 : 2) void moe_stream_down_short_kernel(MoeArgs a, int chunk) {
-    __shared__ __attribute__((aligned(1024))) char bufs[4][stream::Unit<RB>::kBytes];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
-    const int n_groups = a.K / 128;
-    const int n_chunks = (n_groups + chunk - 1) / chunk;
-    for (int j = (int)blockIdx.x; j < n_live * n_chunks; j += (int)gridDim.x) {
-        const int blk = j / n_chunks, first = (j - blk * n_chunks) * chunk, last = min(n_groups, first + chunk);
-        const int e = __builtin_amdgcn_readfirstlane(a.expert_ids[blk]);
-        const int s0 = blk * kBlockRows + lane;
-        const int id0 = s0 < a.sorted_num ? a.sorted_ids[s0] : -1, id1 = s0 + 64 < a.sorted_num ? a.sorted_ids[s0 + 64] : -1;
-        if (e >= 0 && e < a.E) stream::down_short<RB>(a, bufs[wave], blk, e, id0, id1, 4 * first + wave, 4, 4 * last);
-    }
+__global__ __launch_bounds__(256, RB == 256 ? 4 : 2) void moe_stream_down_short_kernel(MoeArgs a) {
+    __shared__ __attribute__((aligned(1024))) char bufs[4][stream::ShortDown<RB>::kBytes];
+    stream::ShortDown<RB> eng(a, bufs[__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)]);
+    stream::for_each_turn(a, a.K / 32, eng);
 }
 
 // ------------------------------------------------------------------------------------------ host
@@ -623,7 +582,13 @@ __global__ __launch_bounds__(256, RB == 256 ? 4 : 2) void moe_stream_down_short_
 // stream against tall tiles, us (graph replays): 8 large experts (K 4096, N 28672, top 2) 117 / 300 at 1 token, 424 /
 // 567 at 32, 487 / 570 at 128 (32 rows per expert), 576 / 573 at 192; 128 small experts (K 2048, N 1536, top 8) 24 /
 // 45 at 1 token, 163 / 232 at 64, 251 / 264 at 384, 285 / 282 at 512 (32 rows per expert), 343 / 293 at 768.
-static bool use_stream(const MoeArgs &a) { return (int64_t)a.M * a.top_k <= 32 * (int64_t)a.E; }
+// With few jobs of tall tiles and no deep mode to share them it pays longer (37 experts, K 4096, N 256, top 9: 74 / 121
+// at 256 tokens, 62 rows per expert).
+static bool use_stream(const MoeArgs &a) {
+    const int64_t tall_jobs = std::min<int64_t>(a.n_blocks, a.E) * (a.H / 128);
+    const int64_t rows = tall_jobs < resident_grid() / 2 && !a.deep_ok ? 64 : 32;
+    return (int64_t)a.M * a.top_k <= rows * a.E;
+}
 
 static int launch_stream_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
     const int mask = phase_mask();
@@ -639,13 +604,9 @@ static int launch_stream_pipeline(MoeArgs a, void *out, int split, hipStream_t s
     if (mask & PMOE_PHASE_UP) launch(moe_stream_kernel<true, 1>, moe_stream_kernel<true, 2>, a.H / 16);
     else if (mask & PMOE_PHASE_PROLOGUE) launch(moe_stream_kernel<true, 1>, moe_stream_kernel<true, 2>, 0);
     if ((mask & PMOE_PHASE_DOWN) && a.H <= 256 && a.n_blocks > 0) {
-        // two groups a turn: the workgroups then read one narrow window of W2 that moves through it, which the HBM
-        // channels serve evenly (257 experts, K 7168, H 256: 158 us; 4 groups 160, 14 groups 188, every workgroup
-        // its own 2 MB 239; the general kernel 219)
-        const int chunk = 2;
         const int grid = (int)std::min<int64_t>((int64_t)a.n_blocks * (a.K / 128), (a.H == 128 ? 4 : 2) * resident_grid());
-        if (a.H == 128) hipLaunchKernelGGL(moe_stream_down_short_kernel<256>, dim3(grid), dim3(256), 0, s, a, chunk);
-        else hipLaunchKernelGGL(moe_stream_down_short_kernel<512>, dim3(grid), dim3(256), 0, s, a, chunk);
+        if (a.H == 128) hipLaunchKernelGGL(moe_stream_down_short_kernel<256>, dim3(grid), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(moe_stream_down_short_kernel<512>, dim3(grid), dim3(256), 0, s, a);
     } else if (mask & PMOE_PHASE_DOWN) {
         launch(moe_stream_kernel<false, 1>, moe_stream_kernel<false, 2>, a.K / 32);
     }

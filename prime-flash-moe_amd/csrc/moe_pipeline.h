@@ -116,7 +116,8 @@ struct MoeArgs {
     uint32_t *act_scales; // scales of the activation (written by the up kernel's epilogue)
     char *y;              // (M * top_k, K) bf16, by pair id: down-projected rows, before the routing weights
     int32_t *inv;         // (M * top_k): sorted row of each pair id (validated against sorted_ids when read)
-    const int4 *work;     // mxfp8: this kernel's work list, one entry per workgroup
+    const int4 *work;     // mxfp8: this kernel's work list, one entry per workgroup; null: jobs by arithmetic (Job)
+    int per_job;          // mxfp8 without a work list: weight tiles per job
     // bf16 (tall tiles): the schedule, see TallPlan
     TallPlan *plan;
     int4 *tiles;          // row tiles of this kernel (the up kernel's or the down kernel's cut)

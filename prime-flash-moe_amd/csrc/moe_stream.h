@@ -21,6 +21,8 @@
 // there; 8 of 128 experts of K 2048 x N 1536, one row each: up 21.4 -> 13.9, down 11.9 -> 7.9 us.  A flattened variant
 // (the next job's first stages requested before the partial sums are added up) ran equal or 6 % slower.
 #pragma once
+#include <type_traits>
+
 #include "moe_ring.h"
 
 namespace pmoe {
@@ -225,90 +227,182 @@ __device__ __forceinline__ void run_job(const MoeArgs &a, Shared &sh, int blk, i
     __syncthreads();  // the table may be written again
 }
 
-// ---- Down GEMM with a short contraction (RB = 2 H = 256 or 512 bytes per row).
-//
-// A unit of 32 weight rows is then only 8 or 16 contiguous KB, and starting and ending a job for every one or two of
-// them (a latency each, and eight partial sums to add) costs more than its stream.  Here every wave works alone:
-// the token fragment sits in registers for the whole contraction, a unit is copied into the wave's own LDS, read into
-// registers at once, and the next unit's copy runs under the matrix instructions, the store and, above all, the other
-// waves.  No barrier, nothing to add up.
-template <int RB>
-struct Unit {
-    static constexpr int kSteps = RB / 32;            // 16-wide sub-steps of the contraction
-    static constexpr int kChunks = RB / 16;           // 16-byte chunks of a row
-    static constexpr int kRowsPerCopy = 1024 / RB;
-    static constexpr int kCopies = 32 / kRowsPerCopy;
-    static constexpr int kBytes = 32 * RB;
-};
-
-// Units first, first + step, ... < last of block `blk` (expert e); id0 / id1 = sorted ids of rows lane / lane + 64.
-// LDS: chunk c of row r in slot c ^ (r & 15) (16 consecutive rows cover the 64 banks once).
-template <int RB>
-__device__ __forceinline__ void down_short(const MoeArgs &a, char *buf, int blk, int e, int id0, int id1, int first,
-                                           int step, int last) {
-    using G = Unit<RB>;
-    const int lane = threadIdx.x & 63, half = lane >> 5, r = lane & 31;
-    const unsigned n_pairs = (unsigned)(a.M * a.top_k);
-    const uint64_t m0 = __ballot((unsigned)id0 < n_pairs), m1 = __ballot((unsigned)id1 < n_pairs);
-    const int n_rows = m1 ? 128 - __builtin_clzll(m1) : m0 ? 64 - __builtin_clzll(m0) : 0;
-    if (n_rows == 0 || first >= last) return;
-    // copy i moves rows kRowsPerCopy i ..: this lane's is row kRowsPerCopy i + sub, slot lane % kChunks
-    const int sub = lane / G::kChunks;
-    const uint32_t lane_off = (uint32_t)sub * RB + (uint32_t)((lane % G::kChunks) ^ sub) * 16u;
-    const bool once = n_rows <= 32;
-    const char *w_exp = a.w2 + (int64_t)e * a.K * RB;
-    auto issue = [&](int u) {
-        const char *w = ring::uniform_ptr(w_exp + (int64_t)u * G::kBytes);
-#pragma unroll
-        for (int i = 0; i < G::kCopies; ++i) {
-            const uint32_t off = (lane_off ^ (uint32_t)(((i * G::kRowsPerCopy) & 15) << 4)) + i * 1024u;
-            if (once) ring::copy16_once(w, off, buf + i * 1024);
-            else ring::copy16(w, off, buf + i * 1024);
-        }
-    };
-    const char *rd = buf + r * RB;
-
-    for (int t = 0; t * 32 < n_rows; ++t) {
-        issue(first);
-        const int p = __shfl(t < 2 ? id0 : id1, 32 * (t & 1) + r, 64);
-        const bool live = (unsigned)p < n_pairs;
-        bf16x8 b[G::kSteps];
-        const char *tok = a.act + ((int64_t)blk * kBlockRows + 32 * t + r) * RB + half * 16;
-#pragma unroll
-        for (int j = 0; j < G::kSteps; ++j) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) b[j][i] = (__bf16)0.f;
-            if (live) b[j] = *reinterpret_cast<const bf16x8 *>(tok + j * 32);
-        }
-        char *dst = a.y + ((int64_t)(live ? p : 0) * a.K + 4 * half) * 2;
-        for (int u = first; u < last; u += step) {
-            asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // the unit has landed
-            bf16x8 w[G::kSteps];
-#pragma unroll
-            for (int j = 0; j < G::kSteps; ++j)
-                w[j] = *reinterpret_cast<const bf16x8 *>(rd + (((2 * j + half) ^ (r & 15)) << 4));
-            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // it is in registers: the buffer may be filled again
-            if (u + step < last) issue(u + step);
-            f32x16 acc[2];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
-#pragma unroll
-            for (int j = 0; j < G::kSteps; ++j) acc[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j], b[j], acc[j & 1], 0, 0, 0);
-            if (live) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float v[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = acc[0][4 * q + i] + acc[1][4 * q + i];
-                    uint2 pk;
-                    pk.x = pack2_bf16(v[0], v[1]);
-                    pk.y = pack2_bf16(v[2], v[3]);
-                    *reinterpret_cast<uint2 *>(dst + (32 * u + 8 * q) * 2) = pk;
-                }
-            }
-        }
+// Inverts the sorted order for finalize: inv[pair id] = sorted row (entries of pairs that are not in the schedule keep
+// what the buffer held; the reader validates them).  All workgroups of the grid, `threads` threads each.
+__device__ __forceinline__ void invert(const MoeArgs &a, int threads) {
+    const int n_rows = min(a.ntpp[0], a.sorted_num), n_pairs = a.M * a.top_k;
+    for (int s = (int)blockIdx.x * threads + (int)threadIdx.x; s < n_rows; s += (int)gridDim.x * threads) {
+        const int p = a.sorted_ids[s], es = a.expert_ids[s >> 7];
+        if (p >= 0 && p < n_pairs && es >= 0 && es < a.E) a.inv[p] = s;
     }
 }
+
+// The jobs of this workgroup: job(block, expert, weight tile, sorted id of this thread's row).  The up kernel also
+// inverts the sorted order.
+template <bool UP, typename Job>
+__device__ __forceinline__ void for_each_job(const MoeArgs &a, int n_tiles, Job job) {
+    const int tid = threadIdx.x, grid = (int)gridDim.x;
+    // sorted id (threads 0 .. 127) and expert of a job's block, fetched under the job before; for the first job
+    // without waiting for the length of the schedule
+    auto fetch = [&](int j, int &id, int &e) {
+        id = e = -1;
+        const int blk = n_tiles > 0 ? j / n_tiles : a.n_blocks;
+        if (blk < a.n_blocks) {
+            const int s = blk * kBlockRows + tid;
+            if (tid < kBlockRows && s < a.sorted_num) id = a.sorted_ids[s];
+            e = a.expert_ids[blk];
+        }
+    };
+    int id, e;
+    fetch((int)blockIdx.x, id, e);
+    const int ntpp = a.ntpp[0];
+    const int n_jobs = min((ntpp + kBlockRows - 1) / kBlockRows, a.n_blocks) * n_tiles;
+    if (UP) invert(a, 512);
+    for (int j = (int)blockIdx.x; j < n_jobs; j += grid) {
+        const int blk = j / n_tiles;
+        int next_id, next_e;
+        fetch(j + grid, next_id, next_e);
+        if (e >= 0 && e < a.E) job(blk, __builtin_amdgcn_readfirstlane(e), j - blk * n_tiles, id);
+        id = next_id;
+        e = next_e;
+    }
+}
+
+// ---- Down GEMM with a short contraction (at most 512 bytes per weight row).
+//
+// A unit of 32 weight rows is then only a few contiguous KB, and starting and ending a job for every one or two of
+// them (a latency each, and eight partial sums to add) costs more than its stream.  Here every wave works alone: it
+// copies a turn (up to 16 KB of one expert's rows) into its own LDS, reads it into registers at once, and runs the
+// block's token fragments past it; the next turn's copy and its first token fragment are under way meanwhile.  No
+// barrier, nothing to add up, and no weight row is read twice.  A workgroup's four waves take neighbouring turns, and
+// neighbouring workgroups neighbouring jobs: what the chip reads at one time is one narrow window that moves through
+// W2, which the HBM channels serve evenly (257 experts, K 7168, H 256 in bf16: 158 us; with 14 turns in a row per wave
+// 188, with 28 of its own per wave 239; the general kernel 219).
+//
+// Engine: request() starts the copy of a turn, request_tokens() the loads of the block's first token fragment (`pair`:
+// pair id of the lane's row of it), wait() makes both land in registers, compute() does the work of the turn.
+template <typename Engine>
+__device__ __forceinline__ void for_each_turn(const MoeArgs &a, int n_turns, Engine &eng) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
+    const int n_jobs = (n_turns + 3) / 4, total = n_live * n_jobs;
+    const unsigned n_pairs = (unsigned)(a.M * a.top_k);
+    struct Job {
+        int blk, turn, e, id0, id1, n_rows;
+    };
+    // job j of this wave; its sorted ids (rows lane and lane + 64) and expert
+    auto fetch = [&](int j, Job &job) {
+        job.n_rows = -1;
+        job.e = job.id0 = job.id1 = -1;
+        job.blk = job.turn = 0;
+        if (j < total) {
+            job.blk = j / n_jobs;
+            job.turn = (j - job.blk * n_jobs) * 4 + wave;
+            const int s0 = job.blk * kBlockRows + lane;
+            if (s0 < a.sorted_num) job.id0 = a.sorted_ids[s0];
+            if (s0 + 64 < a.sorted_num) job.id1 = a.sorted_ids[s0 + 64];
+            job.e = a.expert_ids[job.blk];
+        }
+    };
+    auto count = [&](Job &job) {  // n_rows = 0: nothing to do
+        const bool ok = job.turn < n_turns && (unsigned)__builtin_amdgcn_readfirstlane(job.e) < (unsigned)a.E;
+        const uint64_t m0 = __ballot((unsigned)job.id0 < n_pairs), m1 = __ballot((unsigned)job.id1 < n_pairs);
+        job.n_rows = !ok ? 0 : m1 ? 128 - __builtin_clzll(m1) : m0 ? 64 - __builtin_clzll(m0) : 0;
+    };
+    int j = (int)blockIdx.x;
+    Job cur, next;
+    fetch(j, cur);
+    count(cur);
+    auto request = [&](const Job &job) {
+        if (job.n_rows > 0) eng.request(__builtin_amdgcn_readfirstlane(job.e), job.turn);
+    };
+    auto request_tokens = [&](const Job &job) {
+        if (job.n_rows > 0) eng.request_tokens(job.blk, __shfl(job.id0, lane & 31, 64));
+    };
+    request(cur);
+    request_tokens(cur);
+    for (; j < total; j += (int)gridDim.x) {
+        fetch(j + (int)gridDim.x, next);
+        if (cur.n_rows > 0) eng.wait();
+        count(next);
+        request(next);
+        if (cur.n_rows > 0) eng.compute(cur.blk, cur.turn, cur.id0, cur.id1, cur.n_rows);
+        request_tokens(next);
+        cur = next;
+    }
+}
+
+// bf16, RB = 2 H = 256 or 512 bytes per row; a turn is one unit of 32 weight rows (output columns).
+// LDS: chunk c of row r in slot c ^ (r & 15) (16 consecutive rows cover the 64 banks once).
+template <int RB>
+struct ShortDown {
+    static constexpr int kSteps = RB / 32;   // 16-wide sub-steps of the contraction
+    static constexpr int kChunks = RB / 16;  // 16-byte chunks of a row
+    static constexpr int kRowsPerCopy = 1024 / RB;
+    static constexpr int kBytes = 32 * RB;
+    static constexpr int kTurnCols = 32;
+
+    const MoeArgs &a;
+    char *buf;
+    bf16x8 w[kSteps], b[kSteps] = {};  // the turn's rows, a token fragment
+
+    __device__ __forceinline__ ShortDown(const MoeArgs &args, char *lds) : a(args), buf(lds) {}
+    // Token fragment from row row0 on.  Rows without a pair are not loaded: their lanes keep what they hold, which only
+    // reaches output rows nobody stores (loading them too: 216 us instead of 158 with 3 rows in 32).
+    __device__ __forceinline__ void load_tokens(bf16x8 (&dst)[kSteps], int blk, int row0, int pair) const {
+        const int lane = threadIdx.x & 63;
+        if ((unsigned)pair >= (unsigned)(a.M * a.top_k)) return;
+        const char *tok = a.act + ((int64_t)blk * kBlockRows + row0 + (lane & 31)) * RB + (lane >> 5) * 16;
+#pragma unroll
+        for (int j = 0; j < kSteps; ++j) dst[j] = *reinterpret_cast<const bf16x8 *>(tok + j * 32);
+    }
+    __device__ __forceinline__ void request(int e, int turn) {
+        const int lane = threadIdx.x & 63, sub = lane / kChunks;
+        const uint32_t lane_off = (uint32_t)sub * RB + (uint32_t)((lane % kChunks) ^ sub) * 16u;
+        const char *src = ring::uniform_ptr(a.w2 + ((int64_t)e * a.K + turn * 32) * RB);
+#pragma unroll
+        for (int i = 0; i < 32 / kRowsPerCopy; ++i)
+            ring::copy16_once(src, (lane_off ^ (uint32_t)(((i * kRowsPerCopy) & 15) << 4)) + i * 1024u, buf + i * 1024);
+    }
+    __device__ __forceinline__ void request_tokens(int blk, int pair) { load_tokens(b, blk, 0, pair); }
+    __device__ __forceinline__ void wait() {
+        const int lane = threadIdx.x & 63, r = lane & 31, half = lane >> 5;
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // the turn has landed
+#pragma unroll
+        for (int j = 0; j < kSteps; ++j) {
+            // (taken over here: the compiler's wait for them, placed behind the next copies, would wait for those too)
+            asm volatile("" : "+v"(b[j]));
+            w[j] = *reinterpret_cast<const bf16x8 *>(buf + r * RB + (((2 * j + half) ^ (r & 15)) << 4));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // it is in registers: the buffer may be filled again
+    }
+    __device__ __forceinline__ void compute(int blk, int turn, int id0, int id1, int n_rows) {
+        const int lane = threadIdx.x & 63, r = lane & 31, half = lane >> 5;
+        int p = __shfl(id0, r, 64);
+        for (int row0 = 0;;) {
+            f32x16 acc;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+            for (int j = 0; j < kSteps; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j], b[j], acc, 0, 0, 0);
+            asm volatile("" : "+v"(acc));  // (kept out of the branch: every lane takes part)
+            if ((unsigned)p < (unsigned)(a.M * a.top_k)) {
+                char *dst = a.y + ((int64_t)p * a.K + 32 * turn + 4 * half) * 2;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    uint2 pk;
+                    pk.x = pack2_bf16(acc[4 * q], acc[4 * q + 1]);
+                    pk.y = pack2_bf16(acc[4 * q + 2], acc[4 * q + 3]);
+                    *reinterpret_cast<uint2 *>(dst + 16 * q) = pk;
+                }
+            }
+            row0 += 32;
+            if (row0 >= n_rows) break;
+            p = __shfl(row0 < 64 ? id0 : id1, (row0 & 32) + r, 64);
+            load_tokens(b, blk, row0, p);
+        }
+    }
+};
 
 }  // namespace stream
 }  // namespace pmoe

@@ -1,14 +1,15 @@
-"""The weight-streaming bf16 kernels (few rows per expert, csrc/moe_stream.h) at the sizes where they can go wrong:
+"""The weight-streaming kernels (few rows per expert, csrc/moe_stream.h and moe_stream_mx.h) at the sizes where they can go wrong:
 live rows around the 4-row, 32-row, 64-row and 128-row edges, blocks of one expert that take several passes, one slab
-and more slabs than stages, the short-contraction down kernel (H = 128, 256) and the general one, tiles of one
-and of two units of weight rows."""
+and more slabs than stages, the short-contraction down kernels (H = 128, 256) and the general ones, tiles of one
+and of two units of weight rows, and the mxfp8 ring kernels without a work list."""
 import pytest
 import torch
 
-from helpers import BF16_GATE, rel_clamp
+from helpers import (BF16_GATE, MX_COS_GATE, MX_FLIP_DELTA, MX_RELL2_GATE, cosine, mx_elementwise_gates, rel_clamp,
+                     rel_l2)
 from oracle import moe_oracle as O
 from test_gpu_bf16 import _inputs
-from test_gpu_mxfp8 import _routing_by_counts
+from test_gpu_mxfp8 import _quantised_inputs, _routing_by_counts
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +66,39 @@ def test_stream_kernels_with_dropped_rows_and_blocks(device):
         torch.cuda.synchronize()
         got = out.float().cpu()
         assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
+SPARSE = [129, 65, 64, 33, 32, 5] + [1] * 60
+
+
+@pytest.mark.parametrize("K,N,E,counts,split", [
+    (256, 256, 40, EDGES, True),       # streaming up kernel with one slab, H = 128 down
+    (512, 512, 40, EDGES, False),      # H = 256 down
+    (2304, 512, 40, EDGES, True),      # more slabs than stages, a last group of turns that is not full
+    (256, 2048, 40, EDGES, False),     # ring kernels without a work list
+    (256, 768, 256, SPARSE, True),     # general streaming down kernel, H = 384: the last slab has one half
+    (1024, 512 + 256, 256, SPARSE, False),
+])
+def test_mx_kernels_without_a_schedule_at_row_edges(K, N, E, counts, split, device):
+    import prime_moe
+    counts = counts + [0] * (E - len(counts))
+    counts[-1] += sum(counts) % 2
+    ids, wts = _routing_by_counts(counts, 2, device, seed=K)
+    T = ids.shape[0]
+    g, a, deq = _quantised_inputs(T, K, E, N, device, seed=N)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    outs = []
+    for _ in range(2):
+        torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+        out = torch.zeros((T, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_mxfp8(a["x"], a["x_scales"], a["w1"], a["w1_scales"], a["w2"], a["w2_scales"], *sched, wts,
+                                  out, 2, 128, 64, 4, 2, 1, split)
+        outs.append(out)
+    torch.cuda.synchronize()
+    ref, bound = O.fused_moe_dense(deq["x"], deq["w1"], deq["w2"], ids.cpu(), wts.cpu(), act_mx=True,
+                                   flip_delta=MX_FLIP_DELTA)
+    got = outs[0].float().cpu()
+    assert torch.isfinite(got).all()
+    assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
+    mx_elementwise_gates(got, ref, bound)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
