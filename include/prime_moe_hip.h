@@ -54,12 +54,14 @@ int pmoe_moe_align(const int32_t *topk_ids, int32_t *sorted_token_ids, int32_t *
 
 /*
  * The same sort with scratch memory from the caller, which lets it spread over many
- * workgroups (three launches) when n is large; no counterpart in the reference, whose
- * kernel is one thread block for any n.  The query returns 0 for sizes the single
- * workgroup of pmoe_moe_align handles (then `workspace` may be null); with a null or too
- * small workspace the call falls back to that single workgroup.  Same output, bit for bit.
+ * workgroups (two launches) when n is large; no counterpart in the reference, whose
+ * kernel is one thread block for any n.  The first query returns the least scratch that
+ * does so (0 for n <= 16384), the second what spreads it as far as it pays (0 for
+ * n <= 8192); where a query returns 0 `workspace` may be null, and with a null or too small
+ * workspace the call falls back to a single workgroup.  Same output, bit for bit.
  */
 size_t pmoe_moe_align_workspace_bytes(int n, int num_experts);
+size_t pmoe_moe_align_workspace_bytes_fast(int n, int num_experts);
 int pmoe_moe_align_ws(const int32_t *topk_ids, int32_t *sorted_token_ids, int32_t *expert_ids,
                       int32_t *num_tokens_post_padded, int n, int num_experts, int block_m,
                       int pad_to, int max_padded, int max_blocks, void *workspace,

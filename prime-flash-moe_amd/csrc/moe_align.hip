@@ -2,313 +2,20 @@
 //
 // Semantics follow the reference kernel (prime_moe/csrc/kernels/fused_moe_bf16_kernel.cu:853-907)
 // except that the within-expert order is made unique (ascending pair id) instead of being
-// left to an atomic race.  One workgroup, wave64:
-//   1. each wave histograms a contiguous slice of the ids into its own LDS row,
-//   2. per expert, the per-wave counts become exclusive per-wave bases; the padded
-//      per-expert totals are prefix-summed by one wave with a shuffle scan,
-//   3. each wave walks its slice again 64 ids at a time; lanes holding the same
-//      expert find each other with one ballot per id bit, the lane's rank inside
-//      that group is a popcount of the lower lanes, and the destination is
-//      offs[e] + base[wave][e] + rank.
+// left to an atomic race.  Up to kSingleMaxIds ids one workgroup does it (align_sort.h): ranks inside the waves,
+// per-expert counts of the waves -> bases, padded totals -> prefix, scatter.  More ids spread over workgroups.
 // All arithmetic is int32 and the output is a pure function of the input.
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 
+#include "align_sort.h"
 #include "pmoe_common.h"
 
-namespace {
+namespace pmoe {
+using align::kMaxExperts;
 
-constexpr int kMaxExperts = 1024;
-
-template <int NW>
-__global__ __launch_bounds__(NW * 64) void moe_align_kernel(
-    const int32_t *__restrict__ topk_ids, int32_t *__restrict__ sorted_token_ids,
-    int32_t *__restrict__ expert_ids, int32_t *__restrict__ num_tokens_post_padded, int n,
-    int num_experts, int block_m, int pad_to, int max_padded, int max_blocks, int id_bits) {
-    extern __shared__ int32_t smem[];
-    int32_t *offs = smem;                          // [E+1] exclusive prefix of padded counts
-    int32_t *padc = smem + (num_experts + 1);      // [E]   padded count per expert
-    int32_t *wbase = smem + (2 * num_experts + 1);  // [NW][E] per-wave counts, then running bases
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    constexpr int NT = NW * 64;
-    const int E = num_experts;
-
-    for (int i = tid; i < NW * E; i += NT) wbase[i] = 0;
-    __syncthreads();
-
-    // contiguous slice per wave, a multiple of 64 ids so groups never straddle waves
-    const int per_wave = (n + NT - 1) / NT * 64;
-    const int beg = wave * per_wave;
-    const int end = min(n, beg + per_wave);
-    int32_t *mine = wbase + wave * E;
-    for (int i = beg + lane; i < end; i += 64) {
-        int e = topk_ids[i];
-        if (e >= 0 && e < E) atomicAdd(mine + e, 1);
-    }
-    __syncthreads();
-
-    // per expert: counts of the waves -> exclusive bases; padded total of the expert
-    for (int e = tid; e < E; e += NT) {
-        int run = 0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            int c = wbase[w * E + e];
-            wbase[w * E + e] = run;
-            run += c;
-        }
-        padc[e] = (run + pad_to - 1) / pad_to * pad_to;
-    }
-    __syncthreads();
-
-    // exclusive prefix over experts by wave 0: serial inside a lane's chunk, shuffle scan across
-    if (wave == 0) {
-        const int chunk = (E + 63) >> 6;
-        const int b = lane * chunk;
-        int local = 0;
-        for (int j = 0; j < chunk; ++j)
-            if (b + j < E) local += padc[b + j];
-        int incl = local;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            int v = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += v;
-        }
-        int run = incl - local;
-        for (int j = 0; j < chunk; ++j)
-            if (b + j < E) {
-                offs[b + j] = run;
-                run += padc[b + j];
-            }
-        if (lane == 63) offs[E] = incl;  // lane 63's inclusive sum is the grand total
-    }
-    __syncthreads();
-    const int total = offs[E];
-    if (tid == 0) num_tokens_post_padded[0] = total;
-
-    for (int i = tid; i < max_padded; i += NT) sorted_token_ids[i] = -1;
-    for (int j = tid; j < max_blocks; j += NT) {
-        const int row = j * block_m;
-        int owner = E - 1;
-        if (row < total) {
-            int lo = 0, hi = E - 1;
-            while (lo < hi) {
-                int mid = (lo + hi + 1) >> 1;
-                if (offs[mid] <= row) lo = mid;
-                else hi = mid - 1;
-            }
-            owner = lo;
-        }
-        expert_ids[j] = owner;
-    }
-    __syncthreads();  // the -1 fill is complete before any pair id lands on top of it
-
-    for (int i0 = beg; i0 < end; i0 += 64) {
-        const int i = i0 + lane;
-        int e = (i < end) ? topk_ids[i] : -1;
-        const bool valid = e >= 0 && e < E;
-        unsigned long long peers = __ballot(valid);
-        for (int b = 0; b < id_bits; ++b) {
-            const bool bit = (e >> b) & 1;
-            const unsigned long long set = __ballot(bit);
-            peers &= bit ? set : ~set;
-        }
-        if (valid) {
-            const int rank = __popcll(peers & ((1ull << lane) - 1ull));
-            const int cnt = __popcll(peers);
-            const int base = mine[e];
-            sorted_token_ids[offs[e] + base + rank] = i;
-            if (rank == cnt - 1) mine[e] = base + cnt;  // one writer per group, after all reads
-        }
-    }
-}
-
-// ---- many ids: the same sort spread over workgroups, three launches.
-//   count:   workgroup g histograms ids [g S, (g+1) S) -> counts[g][e]
-//   scan:    one workgroup turns counts[.][e] into exclusive bases over the workgroups, writes the
-//            per-expert totals cnt[e], the padded exclusive prefix offs[0..E], the total and expert_ids
-//   scatter: workgroup g sorts its slice as the single-workgroup kernel does (per-wave histogram,
-//            ballot ranks) and writes pair id i to offs[e] + counts[g][e] + base of its wave + rank;
-//            it also writes -1 to the padding slots of its share of the output (a slot is padding if
-//            it lies at or behind cnt[e] inside its expert's padded range, or behind the total), so
-//            no slot is written twice and no order between workgroups is needed.
-// Slices are contiguous and ascending in g, waves inside a slice likewise: the order inside an expert is
-// ascending pair id, bit for bit what the single workgroup produces.
-constexpr int kSliceIds = 8192;       // ids per workgroup
-constexpr int kSingleMaxIds = 16384;  // up to here one workgroup is faster than three launches
-
-struct AlignScratch {
-    int32_t *counts;  // [G][E]
-    int32_t *offs;    // [E + 1]
-    int32_t *cnt;     // [E]
-};
-
-__global__ __launch_bounds__(1024) void align_count_kernel(const int32_t *__restrict__ topk_ids, int n, int E,
-                                                           int32_t *__restrict__ counts) {
-    extern __shared__ int32_t smem[];
-    const int tid = threadIdx.x, g = blockIdx.x;
-    for (int e = tid; e < E; e += 1024) smem[e] = 0;
-    __syncthreads();
-    const int beg = g * kSliceIds, end = min(n, beg + kSliceIds);
-    for (int i = beg + tid; i < end; i += 1024) {
-        const int e = topk_ids[i];
-        if (e >= 0 && e < E) atomicAdd(smem + e, 1);
-    }
-    __syncthreads();
-    for (int e = tid; e < E; e += 1024) counts[g * E + e] = smem[e];
-}
-
-__global__ __launch_bounds__(1024) void align_scan_kernel(AlignScratch sc, int G, int E, int block_m, int pad_to,
-                                                          int max_blocks, int32_t *__restrict__ expert_ids,
-                                                          int32_t *__restrict__ num_tokens_post_padded) {
-    extern __shared__ int32_t smem[];
-    int32_t *offs = smem;            // [E + 1]
-    int32_t *padc = smem + (E + 1);  // [E]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int e = tid; e < E; e += 1024) {
-        int run = 0;
-        for (int g = 0; g < G; ++g) {
-            const int c = sc.counts[g * E + e];
-            sc.counts[g * E + e] = run;
-            run += c;
-        }
-        sc.cnt[e] = run;
-        padc[e] = (run + pad_to - 1) / pad_to * pad_to;
-    }
-    __syncthreads();
-    if (wave == 0) {  // exclusive prefix over experts, as in the single-workgroup kernel
-        const int chunk = (E + 63) >> 6;
-        const int b = lane * chunk;
-        int local = 0;
-        for (int j = 0; j < chunk; ++j)
-            if (b + j < E) local += padc[b + j];
-        int incl = local;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            int v = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += v;
-        }
-        int run = incl - local;
-        for (int j = 0; j < chunk; ++j)
-            if (b + j < E) {
-                offs[b + j] = run;
-                run += padc[b + j];
-            }
-        if (lane == 63) offs[E] = incl;
-    }
-    __syncthreads();
-    const int total = offs[E];
-    if (tid == 0) num_tokens_post_padded[0] = total;
-    for (int e = tid; e <= E; e += 1024) sc.offs[e] = offs[e];
-    for (int j = tid; j < max_blocks; j += 1024) {
-        const int row = j * block_m;
-        int owner = E - 1;
-        if (row < total) {
-            int lo = 0, hi = E - 1;
-            while (lo < hi) {
-                int mid = (lo + hi + 1) >> 1;
-                if (offs[mid] <= row) lo = mid;
-                else hi = mid - 1;
-            }
-            owner = lo;
-        }
-        expert_ids[j] = owner;
-    }
-}
-
-template <int NW>
-__global__ __launch_bounds__(NW * 64) void align_scatter_kernel(const int32_t *__restrict__ topk_ids,
-                                                                int32_t *__restrict__ sorted_token_ids,
-                                                                AlignScratch sc, int n, int E, int max_padded,
-                                                                int id_bits) {
-    extern __shared__ int32_t smem[];
-    int32_t *offs = smem;                  // [E + 1]
-    int32_t *cnt = smem + (E + 1);         // [E]
-    int32_t *wbase = smem + (2 * E + 1);   // [NW][E] per-wave counts, then running bases
-    constexpr int NT = NW * 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = blockIdx.x, G = gridDim.x;
-    for (int e = tid; e <= E; e += NT) offs[e] = sc.offs[e];
-    for (int e = tid; e < E; e += NT) cnt[e] = sc.cnt[e];
-    for (int i = tid; i < NW * E; i += NT) wbase[i] = 0;
-    __syncthreads();
-
-    // this workgroup's share of the -1 fill
-    {
-        const int total = offs[E];
-        const int per = (max_padded + G - 1) / G;
-        const int pend = min(max_padded, (g + 1) * per);
-        for (int pos = g * per + tid; pos < pend; pos += NT) {
-            bool pad = pos >= total;
-            if (!pad) {
-                int lo = 0, hi = E - 1;
-                while (lo < hi) {
-                    int mid = (lo + hi + 1) >> 1;
-                    if (offs[mid] <= pos) lo = mid;
-                    else hi = mid - 1;
-                }
-                pad = pos - offs[lo] >= cnt[lo];
-            }
-            if (pad) sorted_token_ids[pos] = -1;
-        }
-    }
-
-    // the slice, one contiguous run of a multiple of 64 ids per wave
-    const int sbeg = g * kSliceIds, send = min(n, sbeg + kSliceIds);
-    constexpr int per_wave = kSliceIds / NW;
-    const int beg = sbeg + wave * per_wave;
-    const int end = min(send, beg + per_wave);
-    int32_t *mine = wbase + wave * E;
-    for (int i = beg + lane; i < end; i += 64) {
-        const int e = topk_ids[i];
-        if (e >= 0 && e < E) atomicAdd(mine + e, 1);
-    }
-    __syncthreads();
-    for (int e = tid; e < E; e += NT) {
-        int run = offs[e] + sc.counts[g * E + e];  // first slot of this workgroup's ids of expert e
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const int c = wbase[w * E + e];
-            wbase[w * E + e] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    for (int i0 = beg; i0 < end; i0 += 64) {
-        const int i = i0 + lane;
-        const int e = (i < end) ? topk_ids[i] : -1;
-        const bool valid = e >= 0 && e < E;
-        unsigned long long peers = __ballot(valid);
-        for (int b = 0; b < id_bits; ++b) {
-            const bool bit = (e >> b) & 1;
-            const unsigned long long set = __ballot(bit);
-            peers &= bit ? set : ~set;
-        }
-        if (valid) {
-            const int rank = __popcll(peers & ((1ull << lane) - 1ull));
-            const int c = __popcll(peers);
-            const int base = mine[e];
-            sorted_token_ids[base + rank] = i;
-            if (rank == c - 1) mine[e] = base + c;  // one writer per group, after all reads
-        }
-    }
-}
-
-
-// Scratch of the entry point that allocates nothing (pmoe_moe_align_static): counts[G][E], offs[E + 1],
-// cnt[E] of the multi-workgroup sort for up to kStaticMaxIds ids and kMaxExperts experts, 520 KB held by
-// every device the library runs on until the process ends.  In host code this name is only a handle for
-// hipGetSymbolAddress; kernels get the address that call returns.
-constexpr int kStaticMaxIds = PMOE_ALIGN_STATIC_MAX_IDS;
-constexpr size_t kStaticWords = (size_t)(kStaticMaxIds / kSliceIds) * kMaxExperts + 2 * kMaxExperts + 1;
-static __device__ __align__(256) int32_t scratch[kStaticWords];
-
-int id_bits_for(int num_experts) {
-    int id_bits = 1;
-    while ((1 << id_bits) < num_experts) ++id_bits;
-    return id_bits;
-}
-
-int validate(const int32_t *topk_ids, const int32_t *sorted_token_ids, const int32_t *expert_ids,
+int moe_align_validate(const int32_t *topk_ids, const int32_t *sorted_token_ids, const int32_t *expert_ids,
              const int32_t *num_tokens_post_padded, int n, int num_experts, int block_m, int pad_to, int max_padded,
              int max_blocks) {
     PMOE_REQUIRE(num_experts > 0 && block_m > 0 && pad_to > 0, "moe_align: block_m, bpc and num_experts must be positive");
@@ -323,53 +30,224 @@ int validate(const int32_t *topk_ids, const int32_t *sorted_token_ids, const int
     return PMOE_OK;
 }
 
-// One workgroup sorts everything.
-int launch_single(const int32_t *topk_ids, int32_t *sorted_token_ids, int32_t *expert_ids,
-                  int32_t *num_tokens_post_padded, int n, int num_experts, int block_m, int pad_to, int max_padded,
-                  int max_blocks, hipStream_t s) {
-    const int id_bits = id_bits_for(num_experts);
-    if (num_experts <= 512) {
-        constexpr int NW = 16;
-        const size_t smem = sizeof(int32_t) * (size_t)(2 * num_experts + 1 + NW * num_experts);
-        hipLaunchKernelGGL(moe_align_kernel<NW>, dim3(1), dim3(NW * 64), smem, s, topk_ids, sorted_token_ids,
-                           expert_ids, num_tokens_post_padded, n, num_experts, block_m, pad_to, max_padded,
-                           max_blocks, id_bits);
-    } else {
-        constexpr int NW = 8;
-        const size_t smem = sizeof(int32_t) * (size_t)(2 * num_experts + 1 + NW * num_experts);
-        hipLaunchKernelGGL(moe_align_kernel<NW>, dim3(1), dim3(NW * 64), smem, s, topk_ids, sorted_token_ids,
-                           expert_ids, num_tokens_post_padded, n, num_experts, block_m, pad_to, max_padded,
-                           max_blocks, id_bits);
+}  // namespace pmoe
+
+namespace {
+
+using namespace pmoe::align;
+
+// One workgroup, n <= NW * 64 * PER (8192 ids of 8 experts: 11.5 -> 6 us against loading and ranking 64 ids at a time).
+template <int NW, int PER>
+__global__ __launch_bounds__(NW * 64) void moe_align_kernel(const int32_t *__restrict__ topk_ids, Outputs o, int n, int E,
+                                                            int id_bits) {
+    extern __shared__ int32_t smem[];
+    int id[PER];
+    load_ids<NW, PER>(id, topk_ids, 0, n);
+    sort_in_workgroup<NW, PER>(id, o, E, id_bits, smem);
+}
+
+// ---- many ids: the same sort spread over workgroups, two launches.
+//   count:   workgroup g counts ids [g S, (g + 1) S) per expert -> counts[g][e]
+//   scatter: every workgroup sums counts[.][e] itself (all slices: totals and the padded prefix; the slices before
+//            its own: its bases), ranks its slice as above and writes pair id i to offs[e] + base + rank; it also
+//            writes its share of the padding slots (those at or behind an expert's count, and past the total) and of
+//            expert_ids.  No slot is written twice and no order between workgroups is needed.
+// Slices are contiguous and ascending in g, waves inside a slice likewise: the order inside an expert is
+// ascending pair id, bit for bit what the single workgroup produces.
+// Ranking is what a slice costs (ballots, a few hundred instructions per 64 ids of a wave), so slices are as small as
+// the scratch allows, from 1024 ids on, up to 64 of them: 65536 ids of 128 experts take 20 us in 8 slices.
+constexpr int kMinSliceIds = 1024, kMaxSliceIds = 8192;
+constexpr int kFewIds = 8192;         // up to here one workgroup is as fast (8192 ids: 8.7 us; 16384: 19.6)
+constexpr int kSingleMaxIds = 16384;  // up to here the small scratch of pmoe_moe_align_workspace_bytes is nothing
+
+int slice_ids(int n) {
+    int s = kMinSliceIds;
+    while (s < kMaxSliceIds && (int64_t)s * 64 < n) s *= 2;
+    return s;
+}
+int n_slices(int n, int slice) { return (int)(((int64_t)n + slice - 1) / slice); }
+
+template <int NW, int PER>
+__global__ __launch_bounds__(NW * 64) void align_count_kernel(const int32_t *__restrict__ topk_ids, int n, int E, int id_bits,
+                                                              int32_t *__restrict__ counts) {
+    extern __shared__ int32_t smem[];  // [NW][E]
+    constexpr int NT = NW * 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = blockIdx.x;
+    int id[PER], ord[PER];
+    load_ids<NW, PER>(id, topk_ids, (int64_t)g * NT * PER, n);
+    for (int i = tid; i < NW * E; i += NT) smem[i] = 0;
+    __syncthreads();
+    rank_ids<PER>(id, ord, smem + wave * E, E, id_bits, lane);
+    __syncthreads();
+    for (int e = tid; e < E; e += NT) {
+        int c = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) c += smem[w * E + e];
+        counts[(size_t)g * E + e] = c;
     }
+}
+
+template <int NW, int PER>
+__global__ __launch_bounds__(NW * 64) void align_scatter_kernel(const int32_t *__restrict__ topk_ids, const int32_t *__restrict__ counts,
+                                                                Outputs o, int n, int E, int id_bits) {
+    extern __shared__ int32_t smem[];
+    constexpr int NT = NW * 64;
+    int32_t *offs = smem, *padc = smem + E + 1, *table = smem + 2 * E + 1;  // table: [NW][E]
+    int32_t *tot = table + NW * E, *before = tot + E;                       // all ids of e; those in earlier slices
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = blockIdx.x, G = gridDim.x;
+    int id[PER], ord[PER];
+    load_ids<NW, PER>(id, topk_ids, (int64_t)g * NT * PER, n);
+    for (int i = tid; i < (NW + 2) * E; i += NT) table[i] = 0;
+    __syncthreads();
+    {
+        // thread (part, e) sums every parts-th slice
+        const int bits = 32 - __builtin_clz(max(E - 1, 1)), pitch = 1 << bits, parts = max(1, NT >> bits);
+        for (int i = tid; i < pitch * parts; i += NT) {
+            const int e = i & (pitch - 1), part = i >> bits;
+            if (e >= E) continue;
+            int all = 0, mine = 0;
+#pragma unroll 8
+            for (int s = part; s < G; s += parts) {
+                const int c = counts[(size_t)s * E + e];
+                all += c;
+                mine += s < g ? c : 0;
+            }
+            atomicAdd(tot + e, all);
+            atomicAdd(before + e, mine);
+        }
+    }
+    rank_ids<PER>(id, ord, table + wave * E, E, id_bits, lane);
+    __syncthreads();
+    for (int e = tid; e < E; e += NT) {
+        int run = before[e];
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const int c = table[w * E + e];
+            table[w * E + e] = run;
+            run += c;
+        }
+        padc[e] = (tot[e] + o.pad_to - 1) / o.pad_to * o.pad_to;
+    }
+    __syncthreads();
+    scan_experts(padc, offs, E);
+    __syncthreads();
+    const int total = offs[E];
+    if (g == 0 && tid == 0) o.num_tokens_post_padded[0] = total;
+    for (int j = g * NT + tid; j < o.max_blocks; j += G * NT) o.expert_ids[j] = owner_of(offs, E, j * o.block_m);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = id[i];
+        if ((unsigned)e < (unsigned)E)
+            o.sorted_token_ids[offs[e] + table[wave * E + e] + ord[i]] = (g * NW * PER + wave * PER + i) * 64 + lane;
+    }
+    // padding: an expert's by one wave, the slots past the total by everybody
+    for (int e = g * NW + wave; e < E; e += G * NW)
+        for (int pos = offs[e] + tot[e] + lane; pos < offs[e + 1]; pos += 64) o.sorted_token_ids[pos] = -1;
+    for (int64_t pos = (int64_t)total + g * NT + tid; pos < o.max_padded; pos += (int64_t)G * NT) o.sorted_token_ids[pos] = -1;
+}
+
+// Any number of ids by one workgroup, for callers without scratch memory: a pass that counts, then the sort run by
+// run with the experts' bases carried on.
+template <int NW>
+__global__ __launch_bounds__(NW * 64) void align_runs_kernel(const int32_t *__restrict__ topk_ids, Outputs o, int n, int E, int id_bits) {
+    extern __shared__ int32_t smem[];
+    constexpr int NT = NW * 64, PER = 16, RUN = NT * PER;
+    int32_t *offs = smem, *padc = smem + E + 1, *table = smem + 2 * E + 1, *base = table + NW * E;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    fill_minus_one(o, NT);
+    for (int i = tid; i < (NW + 1) * E; i += NT) table[i] = 0;
+    __syncthreads();
+    int id[PER], ord[PER];
+    for (int64_t r = 0; r < n; r += RUN) {
+        load_ids<NW, PER>(id, topk_ids, r, n);
+        rank_ids<PER>(id, ord, table + wave * E, E, id_bits, lane);
+    }
+    __syncthreads();
+    for (int e = tid; e < E; e += NT) {
+        int c = 0;
+        for (int w = 0; w < NW; ++w) c += table[w * E + e];
+        padc[e] = (c + o.pad_to - 1) / o.pad_to * o.pad_to;
+    }
+    __syncthreads();
+    scan_experts(padc, offs, E);
+    __syncthreads();
+    if (tid == 0) o.num_tokens_post_padded[0] = offs[E];
+    for (int j = tid; j < o.max_blocks; j += NT) o.expert_ids[j] = owner_of(offs, E, j * o.block_m);
+    for (int64_t r = 0; r < n; r += RUN) {
+        load_ids<NW, PER>(id, topk_ids, r, n);
+        for (int i = tid; i < NW * E; i += NT) table[i] = 0;
+        __syncthreads();
+        rank_ids<PER>(id, ord, table + wave * E, E, id_bits, lane);
+        __syncthreads();
+        for (int e = tid; e < E; e += NT) {
+            int run = base[e];
+            for (int w = 0; w < NW; ++w) {
+                const int c = table[w * E + e];
+                table[w * E + e] = run;
+                run += c;
+            }
+            base[e] = run;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int e = id[i];
+            if ((unsigned)e < (unsigned)E)
+                o.sorted_token_ids[offs[e] + table[wave * E + e] + ord[i]] = (int)r + (wave * PER + i) * 64 + lane;
+        }
+        __syncthreads();
+    }
+}
+
+// Scratch of the entry point that allocates nothing (pmoe_moe_align_static): counts[G][E] (and 2 E + 1 words more)
+// of the multi-workgroup sort for up to kStaticMaxIds ids and kMaxExperts experts, 520 KB held by
+// every device the library runs on until the process ends.  In host code this name is only a handle for
+// hipGetSymbolAddress; kernels get the address that call returns.
+constexpr int kStaticMaxIds = PMOE_ALIGN_STATIC_MAX_IDS;
+constexpr size_t kStaticWords = (size_t)(kStaticMaxIds / kMaxSliceIds) * kMaxExperts + 2 * kMaxExperts + 1;
+static __device__ __align__(256) int32_t scratch[kStaticWords];
+
+// One workgroup sorts everything.  (16 waves; 8 above 512 experts, whose tables would not fit the LDS otherwise.)
+int launch_single(const int32_t *topk_ids, const Outputs &o, int n, int E, hipStream_t s) {
+    const int id_bits = id_bits_for(E);
+    auto launch = [&](auto nw) {
+        constexpr int NW = decltype(nw)::value;
+        const size_t smem = sizeof(int32_t) * (size_t)sort_words(NW, E);
+        const int per = (n + NW * 64 - 1) / (NW * 64);
+        auto go = [&](auto kernel, size_t bytes) { hipLaunchKernelGGL(kernel, dim3(1), dim3(NW * 64), bytes, s, topk_ids, o, n, E, id_bits); };
+        if (per <= 1) go(moe_align_kernel<NW, 1>, smem);
+        else if (per <= 2) go(moe_align_kernel<NW, 2>, smem);
+        else if (per <= 4) go(moe_align_kernel<NW, 4>, smem);
+        else if (per <= 8) go(moe_align_kernel<NW, 8>, smem);
+        else if (per <= 16) go(moe_align_kernel<NW, 16>, smem);
+        else go(align_runs_kernel<NW>, smem + sizeof(int32_t) * E);
+    };
+    if (E <= 512) launch(std::integral_constant<int, 16>{});
+    else launch(std::integral_constant<int, 8>{});
     return pmoe::check_launch("moe_align launch");
 }
 
-// The three launches of the multi-workgroup sort; `words` holds G * E + 2 E + 1 int32 of device scratch,
-// every one of which is written before it is read.
-int launch_multi(const int32_t *topk_ids, int32_t *sorted_token_ids, int32_t *expert_ids,
-                 int32_t *num_tokens_post_padded, int n, int num_experts, int block_m, int pad_to, int max_padded,
-                 int max_blocks, int32_t *words, hipStream_t s) {
-    const int id_bits = id_bits_for(num_experts);
-    const int G = (n + kSliceIds - 1) / kSliceIds;
-    AlignScratch sc;
-    sc.counts = words;
-    sc.offs = sc.counts + (size_t)G * num_experts;
-    sc.cnt = sc.offs + num_experts + 1;
-    hipLaunchKernelGGL(align_count_kernel, dim3(G), dim3(1024), sizeof(int32_t) * num_experts, s, topk_ids, n,
-                       num_experts, sc.counts);
-    hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(1024), sizeof(int32_t) * (2 * num_experts + 1), s, sc, G,
-                       num_experts, block_m, pad_to, max_blocks, expert_ids, num_tokens_post_padded);
-    if (num_experts <= 512) {
-        constexpr int NW = 16;
-        hipLaunchKernelGGL(align_scatter_kernel<NW>, dim3(G), dim3(NW * 64),
-                           sizeof(int32_t) * (size_t)(2 * num_experts + 1 + NW * num_experts), s, topk_ids,
-                           sorted_token_ids, sc, n, num_experts, max_padded, id_bits);
-    } else {
-        constexpr int NW = 8;
-        hipLaunchKernelGGL(align_scatter_kernel<NW>, dim3(G), dim3(NW * 64),
-                           sizeof(int32_t) * (size_t)(2 * num_experts + 1 + NW * num_experts), s, topk_ids,
-                           sorted_token_ids, sc, n, num_experts, max_padded, id_bits);
-    }
+// The two launches of the multi-workgroup sort in slices of `slice` ids; `words` holds n_slices * E int32 of device
+// scratch, every one of which is written before it is read.
+int launch_multi(const int32_t *topk_ids, const Outputs &o, int n, int E, int slice, int32_t *words, hipStream_t s) {
+    const int id_bits = id_bits_for(E);
+    const int G = n_slices(n, slice);
+    auto launch = [&](auto nw, auto p) {
+        constexpr int NW = decltype(nw)::value, PER = decltype(p)::value;
+        hipLaunchKernelGGL((align_count_kernel<NW, PER>), dim3(G), dim3(NW * 64), sizeof(int32_t) * (size_t)NW * E, s, topk_ids, n, E,
+                           id_bits, words);
+        hipLaunchKernelGGL((align_scatter_kernel<NW, PER>), dim3(G), dim3(NW * 64), sizeof(int32_t) * (size_t)(sort_words(NW, E) + 2 * E), s,
+                           topk_ids, words, o, n, E, id_bits);
+    };
+    auto with_per = [&](auto nw) {
+        constexpr int NW = decltype(nw)::value;
+        if (slice <= 1024) launch(nw, std::integral_constant<int, 1024 / (NW * 64)>{});
+        else if (slice <= 2048) launch(nw, std::integral_constant<int, 2048 / (NW * 64)>{});
+        else if (slice <= 4096) launch(nw, std::integral_constant<int, 4096 / (NW * 64)>{});
+        else launch(nw, std::integral_constant<int, 8192 / (NW * 64)>{});
+    };
+    if (E <= 512) with_per(std::integral_constant<int, 16>{});
+    else with_per(std::integral_constant<int, 8>{});
     return pmoe::check_launch("moe_align launch");
 }
 
@@ -407,8 +285,14 @@ int static_scratch(const void *data, int32_t **out) {
 
 extern "C" size_t pmoe_moe_align_workspace_bytes(int n, int num_experts) {
     if (n <= kSingleMaxIds || num_experts <= 0 || num_experts > kMaxExperts) return 0;
-    const size_t G = ((size_t)n + kSliceIds - 1) / kSliceIds;
+    const size_t G = (size_t)n_slices(n, kMaxSliceIds);
     return sizeof(int32_t) * (G * (size_t)num_experts + 2 * (size_t)num_experts + 1);
+}
+
+extern "C" size_t pmoe_moe_align_workspace_bytes_fast(int n, int num_experts) {
+    if (n <= kFewIds || num_experts <= 0 || num_experts > kMaxExperts) return 0;
+    return std::max(sizeof(int32_t) * (size_t)n_slices(n, slice_ids(n)) * (size_t)num_experts,
+                    pmoe_moe_align_workspace_bytes(n, num_experts));
 }
 
 extern "C" int pmoe_moe_align(const int32_t *topk_ids, int32_t *sorted_token_ids,
@@ -423,33 +307,37 @@ extern "C" int pmoe_moe_align_ws(const int32_t *topk_ids, int32_t *sorted_token_
                                  int32_t *num_tokens_post_padded, int n, int num_experts, int block_m, int pad_to,
                                  int max_padded, int max_blocks, void *workspace, size_t workspace_bytes,
                                  void *stream) {
-    if (int rc = validate(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
+    if (int rc = pmoe::moe_align_validate(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
                           pad_to, max_padded, max_blocks))
         return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const size_t ws_need = pmoe_moe_align_workspace_bytes(n, num_experts);
-    if (ws_need > 0 && workspace != nullptr && workspace_bytes >= ws_need) {
-        PMOE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3) == 0, "moe_align: workspace must be 4-byte aligned");
-        return launch_multi(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
-                            pad_to, max_padded, max_blocks, static_cast<int32_t *>(workspace), s);
+    const Outputs o{sorted_token_ids, expert_ids, num_tokens_post_padded, block_m, pad_to, max_padded, max_blocks};
+    if (n > kFewIds && workspace != nullptr) {
+        // the finest slices whose counts fit the scratch
+        for (int slice = slice_ids(n); slice <= kMaxSliceIds; slice *= 2)
+            if (sizeof(int32_t) * (size_t)n_slices(n, slice) * num_experts <= workspace_bytes) {
+                PMOE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3) == 0, "moe_align: workspace must be 4-byte aligned");
+                return launch_multi(topk_ids, o, n, num_experts, slice, static_cast<int32_t *>(workspace), s);
+            }
     }
-    return launch_single(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
-                         pad_to, max_padded, max_blocks, s);
+    return launch_single(topk_ids, o, n, num_experts, s);
 }
 
 extern "C" int pmoe_moe_align_static(const int32_t *topk_ids, int32_t *sorted_token_ids, int32_t *expert_ids,
                                      int32_t *num_tokens_post_padded, int n, int num_experts, int block_m,
                                      int pad_to, int max_padded, int max_blocks, void *stream) {
-    if (int rc = validate(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
+    if (int rc = pmoe::moe_align_validate(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
                           pad_to, max_padded, max_blocks))
         return rc;
     PMOE_REQUIRE(n <= kStaticMaxIds, "moe_align_static: at most %d ids fit the built-in scratch, got %d", kStaticMaxIds, n);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const Outputs o{sorted_token_ids, expert_ids, num_tokens_post_padded, block_m, pad_to, max_padded, max_blocks};
     if (n <= kSingleMaxIds)  // one workgroup sorts these in its LDS: no device scratch involved
-        return launch_single(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
-                             pad_to, max_padded, max_blocks, s);
+        return launch_single(topk_ids, o, n, num_experts, s);
     int32_t *words = nullptr;
     if (int rc = static_scratch(topk_ids, &words)) return rc;
-    return launch_multi(topk_ids, sorted_token_ids, expert_ids, num_tokens_post_padded, n, num_experts, block_m,
-                        pad_to, max_padded, max_blocks, words, s);
+    // the finest slices whose counts fit the array
+    int slice = slice_ids(n);
+    while (slice < kMaxSliceIds && (size_t)n_slices(n, slice) * num_experts > kStaticWords) slice *= 2;
+    return launch_multi(topk_ids, o, n, num_experts, slice, words, s);
 }

@@ -109,7 +109,7 @@ struct Schedule {
           expert_ids(empty({sz.max_blocks}, at::kInt, dev)),
           num_tokens_post_padded(empty({1}, at::kInt, dev)) {
         // many ids: scratch for the multi-workgroup sort (0 bytes when one workgroup does it)
-        ws_bytes = pmoe_moe_align_workspace_bytes((int)n, (int)num_experts);
+        ws_bytes = pmoe_moe_align_workspace_bytes_fast((int)n, (int)num_experts);
         if (ws_bytes > 0) ws = workspace(ws_bytes, dev);
     }
     void *ws_ptr() const { return ws_bytes > 0 ? ws.data_ptr() : nullptr; }

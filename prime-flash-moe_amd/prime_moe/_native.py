@@ -21,6 +21,7 @@ SIGNATURES = {
     "pmoe_last_error": (ctypes.c_char_p, []),
     "pmoe_moe_align": (_c_int, [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p]),
     "pmoe_moe_align_workspace_bytes": (_c_size_t, [_c_int] * 2),
+    "pmoe_moe_align_workspace_bytes_fast": (_c_size_t, [_c_int] * 2),
     "pmoe_moe_align_ws": (_c_int, [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p, _c_size_t, _c_void_p]),
     "pmoe_moe_align_static": (_c_int, [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p]),
     "pmoe_fused_moe_bf16_workspace_bytes": (_c_size_t, [_c_int] * 7),

@@ -1,0 +1,47 @@
+"""moe_align at the edges of its launch shapes (one workgroup, slices of 1024 .. 8192 ids), the scratch sizes that choose
+between them, and the router's one-kernel form: bit-exact against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as O
+from test_gpu_route import _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,E", [(8192, 8), (8193, 37), (9000, 700), (65536, 128), (65537, 128), (131073, 600), (262145, 5)])
+def test_align_at_slice_edges_with_every_scratch(n, E, device):
+    import prime_moe
+    from prime_moe import _native
+    lib = _native.load()
+    ids = np.random.default_rng(n).integers(-1, E, size=n).astype(np.int32)
+    ids[: n // 3] = E // 2  # a hot expert
+    keep = np.flatnonzero(ids >= 0)
+    s_c, e_c, t_c = O.moe_align_fast(ids[keep], E, 128, 1)
+    pad_to, max_padded, max_blocks = prime_moe.align_sizes(n, E, 128, 1)
+    s_w = np.full(max_padded, -1, dtype=np.int32)
+    s_w[: s_c.size] = np.where(s_c >= 0, keep[np.maximum(s_c, 0)], -1)
+    e_w = np.full(max_blocks, E - 1, dtype=np.int32)
+    e_w[: e_c.size] = e_c
+    dev_ids = torch.from_numpy(ids).to(device)
+    small, fast = lib.pmoe_moe_align_workspace_bytes(n, E), lib.pmoe_moe_align_workspace_bytes_fast(n, E)
+    assert fast >= small and (fast > 0) == (n > 8192)
+    for nbytes in sorted({0, 4, small, (small + fast) // 2, fast}):
+        s = torch.full((max_padded,), 0x5a5a5a5a, dtype=torch.int32, device=device)
+        e = torch.full((max_blocks,), 0x5a5a5a5a, dtype=torch.int32, device=device)
+        t = torch.full((1,), 0x5a5a5a5a, dtype=torch.int32, device=device)
+        ws = torch.full((max(nbytes, 4),), 0x5a, dtype=torch.uint8, device=device)
+        _native.check(lib.pmoe_moe_align_ws(dev_ids.data_ptr(), s.data_ptr(), e.data_ptr(), t.data_ptr(), n, E, 128, pad_to,
+                                            max_padded, max_blocks, ws.data_ptr() if nbytes else None, nbytes,
+                                            torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        for got, want in zip((s, e, t), (s_w, e_w, t_c)):
+            np.testing.assert_array_equal(got.cpu().numpy(), want, err_msg=f"{nbytes} bytes of scratch")
+
+
+@pytest.mark.parametrize("T,E,k", [(16, 512, 32), (17, 512, 8), (8, 513, 32), (9, 1024, 4), (16, 64, 32), (2, 33, 32)])
+def test_route_around_the_one_kernel_form(T, E, k, device):
+    g = torch.Generator(device=device).manual_seed(T + E + k)
+    _check(torch.randn((T, E), generator=g, device=device), k, bias=torch.randn((E,), generator=g, device=device))
+    _check(torch.randint(-2, 3, (T, E), generator=g, device=device).to(torch.bfloat16), k, block_m=32, bpc=2)
