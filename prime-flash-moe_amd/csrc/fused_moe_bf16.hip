@@ -289,17 +289,79 @@ __device__ __forceinline__ float4 *partial_block(const MoeArgs &a, int part, int
 
 // The queue of an XCD: its workgroups (workgroup w is number w / 8 of XCD w mod 8) start with the slot of their own
 // number and take further slots from the XCD's counter, which the prologue sets to the number of workgroups
-// per XCD.  Thread 0 asks for the next slot when the K loop of a tile ends (`ask`), so that the answer arrives
-// under the epilogue (asked earlier, a busy workgroup would hold a job that an idle one could run); `pass`
-// hands it to every thread through `word`, a word of LDS that nothing else uses at that moment.
+// per XCD.  Thread 0 asks for the next slot before the last slab but one of a tile (asked much earlier, a busy
+// workgroup would hold a job that an idle one could run); `pass` hands it to every thread.
 __device__ __forceinline__ int ask_slot(int *counter) { return threadIdx.x == 0 ? atomicAdd(counter, 1) : 0; }
-__device__ __forceinline__ int pass_slot(int asked, int *word) {
-    __syncthreads();  // whatever used the LDS before is done
+__device__ __forceinline__ int pass_slot(int asked, char *lds) {
+    int *word = reinterpret_cast<int *>(lds + tall::kWordOff);
     if (threadIdx.x == 0) *word = asked;
     __syncthreads();
-    const int pos = *word;
-    __syncthreads();  // everybody has read the word: the LDS is free again
-    return __builtin_amdgcn_readfirstlane(pos);
+    return __builtin_amdgcn_readfirstlane(*word);
+}
+
+// One job of a resident kernel.
+struct Work {
+    int state;  // 1: a job; 0: the slot is empty; -1: the queue has ended
+    int pos, tile, part, parts, wt;
+    int e, f0, fg;                  // expert, first token fragment, pairs of fragments (from the row tile)
+    int slab0, n_slabs, deep_part;  // its share of the contraction; deep_part < 0: not shared
+};
+__device__ __forceinline__ Work slot_work(int pos, int n_wt, const KernelPlan &kp) {
+    Work w;
+    TallJob j;
+    w.pos = pos;
+    w.state = resolve_tall_job(8 * pos + (int)(blockIdx.x & 7), n_wt, kp, j);
+    w.tile = j.tile;
+    w.part = j.part;
+    w.parts = j.parts;
+    w.wt = j.wt;
+    return w;
+}
+// Completes a job with its row tile's entry `tl`.
+__device__ __forceinline__ void tile_work(Work &w, const int4 &tl, const KernelPlan &kp, int n_slabs) {
+    w.f0 = __builtin_amdgcn_readfirstlane(tl.x);
+    w.fg = __builtin_amdgcn_readfirstlane(tl.y);
+    w.e = __builtin_amdgcn_readfirstlane(tl.z);
+    w.slab0 = 0;
+    w.n_slabs = n_slabs;
+    w.deep_part = -1;
+    if (kp.deep) {
+        w.slab0 = w.part * n_slabs / w.parts;
+        w.n_slabs = (w.part + 1) * n_slabs / w.parts - w.slab0;
+        w.deep_part = w.part;
+    } else if (w.parts > 1) {
+        w.fg = row_split(w.f0, w.fg, w.part, w.parts);
+        if (w.fg == 0) w.state = 0;
+    }
+}
+// Workgroups that run side by side start their K walks at different slabs.
+__device__ __forceinline__ int k_start(const Work &w) { return (w.pos & 7) % w.n_slabs; }
+
+// Hand-over from tile to tile.  A workgroup fills the LDS of its CU, so nothing else runs while a tile is set up,
+// waits for its first slab and stores its results.  The next job is therefore looked up, and the copies of its first
+// slabs are issued, under the epilogue of the current one, whose waves transpose through a few KB of their own
+// (no barriers) behind the stages that are being filled.  The lookup is a chain (slot -> row tile entry -> row
+// ids of the gather -> copies) whose links are spread over the first fragments of the epilogue:
+//   epilogue(q): fragment q of the wave's FG;  link(0) .. link(kLinks - 1): the links, in order.
+template <int FG, int kLinks, typename Epilogue, typename Link>
+__device__ __forceinline__ void epilogue_with_links(Epilogue epilogue, Link link) {
+    link(0);
+#pragma unroll
+    for (int t = 0; t < FG; ++t) {
+        epilogue(t);
+        PMOE_TALL_FENCE();
+        if (t + 1 < kLinks) link(t + 1);
+    }
+#pragma unroll
+    for (int l = FG + 1; l < kLinks; ++l) link(l);
+}
+
+// LDS written by some lanes of a wave is read by others of the same wave: LDS operations of a wave are executed in
+// order, only the compiler has to keep them so.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Up kernel tile: token fragments f0 .. f0 + 2 FG - 1 x activation columns [128 wt, 128 wt + 128) of expert e,
@@ -307,111 +369,140 @@ __device__ __forceinline__ int pass_slot(int asked, int *word) {
 // rows; wave v of a group owns gate/up rows 32v..32v+31, so gate and up of one activation element sit in the
 // same lane and register: SwiGLU in registers, the 2H-wide tensor never leaves the chip.
 // deep_part >= 0: the contraction is shared (deep mode); the fp32 sums go to up_partials instead.
+// `pre`: the first slabs are on their way (tok_ahead: the offsets of their token rows); `next` returns the
+// job after this one, with `pre` and tok_ahead for it.
+struct UpTile {
+    const char *x, *w_gate, *w_up;
+    uint32_t row_bytes;
+};
+__device__ __forceinline__ UpTile up_operands(const MoeArgs &a, const Work &w) {
+    UpTile u;
+    u.row_bytes = (uint32_t)a.K * 2u;
+    u.x = a.x + w.slab0 * tall::kRB;
+    u.w_gate = a.w1 + ((int64_t)w.e * a.N + w.wt * 128) * a.K * 2 + w.slab0 * tall::kRB;
+    u.w_up = u.w_gate + (int64_t)a.H * a.K * 2;
+    return u;
+}
+// Byte offset in x of the token of sorted row `s`; dead rows read token 0.
+__device__ __forceinline__ uint32_t gather_off(const MoeArgs &a, int64_t s, uint32_t row_bytes) {
+    const int p = s < a.sorted_num ? a.sorted_ids[s] : -1;
+    return ((uint32_t)p < (uint32_t)(a.M * a.top_k) ? (uint32_t)p / (uint32_t)a.top_k : 0u) * row_bytes;
+}
 template <int FG>
-__device__ __forceinline__ int up_tile_tall(const MoeArgs &a, int e, int f0, int wt, int slab0, int n_slabs,
-                                            int deep_part, int pos, int *counter, char *lds) {
+__device__ __forceinline__ void up_tile_tall(const MoeArgs &a, const KernelPlan &kp, const Work &w, int *counter, char *lds,
+                                             bool &pre, uint32_t (&tok_ahead)[tall::kMaxFrags / 2], Work &next) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, w4 = wave & 3;
-    const int K = a.K, H = a.H, N = a.N;
-    const int h0 = wt * 128;
-    const int64_t row0 = (int64_t)f0 * 32;
-    const uint32_t row_bytes = (uint32_t)K * 2u;
-    const uint32_t n_pairs = (uint32_t)(a.M * a.top_k);
-    const char *w_gate = a.w1 + ((int64_t)e * N + h0) * K * 2 + slab0 * tall::kRB;
+    const int H = a.H;
+    const int h0 = w.wt * 128;
+    const int64_t row0 = (int64_t)w.f0 * 32;
+    const UpTile u = up_operands(a, w);
     tall::Loader<FG, true> ld;
-    ld.setup(tid, a.x + slab0 * tall::kRB, w_gate, w_gate + (int64_t)H * K * 2, row_bytes, row_bytes, [&](int row) {
-        const int64_t s = row0 + row;
-        const int p = s < a.sorted_num ? a.sorted_ids[s] : -1;
-        const uint32_t tok = (uint32_t)p < n_pairs ? (uint32_t)p / (uint32_t)a.top_k : 0u;  // dead rows read token 0
-        return tok * row_bytes;
-    });
+    ld.setup(tid, u.x, u.w_gate, u.w_up, u.row_bytes, u.row_bytes,
+             [&](int row) { return gather_off(a, row0 + row, u.row_bytes); }, pre ? tok_ahead : nullptr);
     const int wrow[2] = {32 * w4, 128 + 32 * w4};
     f32x16 acc[2][FG];
     zero_acc<FG>(acc);
-    const int start = (pos & 7) % n_slabs;  // workgroups that run side by side start their K walks at different slabs
-    tall::main_loop<FG>(acc, ld, lds, n_slabs, wrow, grp * FG, lane, start);
-    const int asked = ask_slot(counter);
+    int asked = 0;
+    tall::main_loop<FG>(acc, ld, lds, w.n_slabs, wrow, grp * FG, lane, k_start(w), pre, [&] { asked = ask_slot(counter); },
+                        [] {});
 
-    const int r = lane & 31, half = lane >> 5;
-    if (deep_part >= 0) {
+    int lane_e = lane;
+    asm volatile("" : "+v"(lane_e));
+    const int r = lane_e & 31, half = lane_e >> 5;
+    char *scratch = lds + tall::kScratchOff + wave * tall::kScratchBytes;
+    constexpr int kPitch = 80;  // 32 activation columns + 16 B pad
+    int4 tl = make_int4(0, 0, 0, 0);
+    pre = false;
+    epilogue_with_links<FG, 3>(
+        [&](int t) {
+            if (w.deep_part >= 0) {
+                float4 *dst = partial_block(a, w.deep_part, w.f0 + grp * FG + t, w.wt);
 #pragma unroll
-        for (int t = 0; t < FG; ++t) {
-            float4 *dst = partial_block(a, deep_part, f0 + grp * FG + t, wt);
+                for (int f = 0; f < 2; ++f)
 #pragma unroll
-            for (int f = 0; f < 2; ++f)
+                    for (int q = 0; q < 4; ++q)
+                        dst[((f * 4 + q) * 4 + w4) * 64 + lane_e] =
+                            make_float4(acc[f][t][4 * q], acc[f][t][4 * q + 1], acc[f][t][4 * q + 2], acc[f][t][4 * q + 3]);
+                return;
+            }
+            // register i of lane_e l = activation column 32 w4 + 8(i/4) + 4(l/32) + i%4 of token row 32 t + l%32
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    dst[((f * 4 + q) * 4 + w4) * 64 + lane] =
-                        make_float4(acc[f][t][4 * q], acc[f][t][4 * q + 1], acc[f][t][4 * q + 2], acc[f][t][4 * q + 3]);
+            for (int g = 0; g < 4; ++g) {
+                uint2 pk;
+                pk.x = pack2_bf16(swiglu(acc[0][t][4 * g], acc[1][t][4 * g]), swiglu(acc[0][t][4 * g + 1], acc[1][t][4 * g + 1]));
+                pk.y = pack2_bf16(swiglu(acc[0][t][4 * g + 2], acc[1][t][4 * g + 2]),
+                                  swiglu(acc[0][t][4 * g + 3], acc[1][t][4 * g + 3]));
+                *reinterpret_cast<uint2 *>(scratch + r * kPitch + 16 * g + 8 * half) = pk;
+            }
+            wave_lds_order();
+            // 64 bytes of a row by 4 lanes, to the activation rows (by sorted row)
+            char *dst = a.act + ((row0 + (grp * FG + t) * 32) * H + h0 + 32 * w4) * 2 + (lane_e & 3) * 16;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = (lane_e >> 2) + 16 * i;
+                const uint4 v = *reinterpret_cast<const uint4 *>(scratch + row * kPitch + (lane_e & 3) * 16);
+                *reinterpret_cast<uint4 *>(dst + (int64_t)row * H * 2) = v;
+            }
+            wave_lds_order();
+        },
+        [&](int link) {
+            if (link == 0) {
+                next = slot_work(pass_slot(asked, lds), a.n_wtiles, kp);
+                if (next.state > 0) tl = a.tiles[next.tile];
+            } else if (link == 1) {
+                if (next.state > 0) tile_work(next, tl, kp, a.K * 2 / tall::kRB);
+                if (next.state > 0) {
+                    const int row = 8 * wave + (lane_e >> 3);
+                    const uint32_t chunk = (uint32_t)((lane_e & 7) ^ ((row >> 1) & 7)) * 16u;
+#pragma unroll
+                    for (int q = 0; q < tall::kMaxFrags / 2; ++q)
+                        if (q < next.fg) tok_ahead[q] = gather_off(a, (int64_t)next.f0 * 32 + row + 64 * q, u.row_bytes) + chunk;
+                    pre = true;
+                }
+            } else if (next.state > 0) {
+                const UpTile n = up_operands(a, next);
+                tall::pre_issue<true>(next.fg, lds, wave, lane_e, n.x, n.w_gate, n.w_up, n.row_bytes, n.row_bytes, tok_ahead,
+                                      next.n_slabs, k_start(next));
+            }
+        });
+}
+
+// The walk of a resident kernel over its queue; tile<FG>() runs a tile and finds the next job.
+template <typename Run>
+__device__ __forceinline__ void walk_queue(const KernelPlan &kp, const int4 *tiles, int n_wt, int n_slabs, int *counter,
+                                           char *lds, Run run) {
+    Work w = slot_work((int)(blockIdx.x >> 3), n_wt, kp);
+    if (w.state > 0) tile_work(w, tiles[w.tile], kp, n_slabs);
+    while (w.state >= 0) {
+        if (w.state == 0) {
+            __syncthreads();  // the word may still be read
+            w = slot_work(pass_slot(ask_slot(counter), lds), n_wt, kp);
+            if (w.state > 0) tile_work(w, tiles[w.tile], kp, n_slabs);
+            continue;
         }
-        return asked;
+        Work next;
+        run(w, next);
+        w = next;
     }
-    // register i of lane l = activation column 32 w4 + 8(i/4) + 4(l/32) + i%4 of token row 32 t + l%32
-    char *tile = lds + grp * (32 * FG * kActPitchBf16);
-#pragma unroll
-    for (int t = 0; t < FG; ++t) {
-        const int row = 32 * t + r;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int hl = 32 * w4 + 8 * g + 4 * half;  // tile-local activation column
-            uint2 pk;
-            pk.x = pack2_bf16(swiglu(acc[0][t][4 * g], acc[1][t][4 * g]), swiglu(acc[0][t][4 * g + 1], acc[1][t][4 * g + 1]));
-            pk.y = pack2_bf16(swiglu(acc[0][t][4 * g + 2], acc[1][t][4 * g + 2]),
-                              swiglu(acc[0][t][4 * g + 3], acc[1][t][4 * g + 3]));
-            *reinterpret_cast<uint2 *>(tile + row * kActPitchBf16 + hl * 2) = pk;
-        }
-    }
-    __syncthreads();
-    // coalesced copy of the group's 32 FG x 128 tile to the activation rows (by sorted row)
-    const int gt = tid & 255, c = gt & 15;
-    const int64_t grow0 = row0 + grp * 32 * FG;
-#pragma unroll
-    for (int i = 0; i < 2 * FG; ++i) {
-        const int row = (gt >> 4) + 16 * i;
-        const uint4 v = *reinterpret_cast<const uint4 *>(tile + row * kActPitchBf16 + c * 16);
-        store_once(a.act + ((grow0 + row) * H + h0) * 2 + c * 16, v);
-    }
-    return asked;
 }
 
 __global__ __launch_bounds__(512) void moe_up_kernel_bf16(MoeArgs a) {
     __shared__ __attribute__((aligned(1024))) char lds[tall::kLdsBytes];
     const KernelPlan kp = a.plan->up;
-    const int xcd = (int)(blockIdx.x & 7);
-    const int n_slabs_all = a.K * 2 / tall::kRB;
-    int *counter = &a.plan->counters[xcd];
-    for (int pos = (int)(blockIdx.x >> 3);;) {
-        TallJob j;
-        const int st = resolve_tall_job(8 * pos + xcd, a.n_wtiles, kp, j);
-        if (st < 0) break;
-        if (st == 0) {
-            pos = pass_slot(ask_slot(counter), reinterpret_cast<int *>(lds));
-            continue;
+    int *counter = &a.plan->counters[blockIdx.x & 7];
+    bool pre = false;
+    uint32_t tok_ahead[tall::kMaxFrags / 2] = {};
+    walk_queue(kp, a.tiles, a.n_wtiles, a.K * 2 / tall::kRB, counter, lds, [&](const Work &w, Work &next) {
+        switch (w.fg) {
+            case 1: up_tile_tall<1>(a, kp, w, counter, lds, pre, tok_ahead, next); break;
+            case 2: up_tile_tall<2>(a, kp, w, counter, lds, pre, tok_ahead, next); break;
+            case 3: up_tile_tall<3>(a, kp, w, counter, lds, pre, tok_ahead, next); break;
+            case 4: up_tile_tall<4>(a, kp, w, counter, lds, pre, tok_ahead, next); break;
+            case 5: up_tile_tall<5>(a, kp, w, counter, lds, pre, tok_ahead, next); break;
+            default: up_tile_tall<6>(a, kp, w, counter, lds, pre, tok_ahead, next); break;
         }
-        int asked = 0;
-        const int4 tl = a.tiles[j.tile];
-        int f0 = tl.x, fg = tl.y;
-        const int e = tl.z;
-        int slab0 = 0, n_slabs = n_slabs_all, deep_part = -1;
-        if (kp.deep) {
-            slab0 = j.part * n_slabs_all / j.parts;
-            n_slabs = (j.part + 1) * n_slabs_all / j.parts - slab0;
-            deep_part = j.part;
-        } else if (j.parts > 1) {
-            fg = row_split(f0, fg, j.part, j.parts);
-        }
-        fg = __builtin_amdgcn_readfirstlane(fg);
-        switch (fg) {
-            case 1: asked = up_tile_tall<1>(a, e, f0, j.wt, slab0, n_slabs, deep_part, pos, counter, lds); break;
-            case 2: asked = up_tile_tall<2>(a, e, f0, j.wt, slab0, n_slabs, deep_part, pos, counter, lds); break;
-            case 3: asked = up_tile_tall<3>(a, e, f0, j.wt, slab0, n_slabs, deep_part, pos, counter, lds); break;
-            case 4: asked = up_tile_tall<4>(a, e, f0, j.wt, slab0, n_slabs, deep_part, pos, counter, lds); break;
-            case 5: asked = up_tile_tall<5>(a, e, f0, j.wt, slab0, n_slabs, deep_part, pos, counter, lds); break;
-            case 6: asked = up_tile_tall<6>(a, e, f0, j.wt, slab0, n_slabs, deep_part, pos, counter, lds); break;
-            default: asked = ask_slot(counter); break;
-        }
-        pos = pass_slot(asked, reinterpret_cast<int *>(lds));
-    }
+    });
 }
 
 // Deep mode: adds the partial sums the parts of every up job left in memory and finishes the tiles.  One
@@ -458,107 +549,120 @@ __global__ __launch_bounds__(256) void moe_up_join_kernel(MoeArgs a) {
 // Down kernel tile: y[pairs of the tile's rows, 256 columns of K from 256 wt] = act[rows, :H] . W2[e][cols, :H]^T,
 // the whole reduction over H inside the workgroup; the routing weights are applied later, by finalize_kernel.
 // Weight rows (output columns) sit on the MFMA M side: register i of lane l = output column
-// 64 w4 + 32 f + 8(i/4) + 4(l/32) + i%4 of tile row 32 t + l%32.  A group's 32 FG x 256 tile is rounded to
-// bf16 and transposed through LDS (one group after the other: both do not fit), then all 512 threads store
-// its rows, 512 contiguous bytes each, to y[pair id]; rows without a pair are skipped.
-template <int FG>
-__device__ __forceinline__ int down_tile_tall(const MoeArgs &a, int e, int f0, int wt, int pos, int *counter, char *lds) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = wave >> 2, w4 = wave & 3;
-    const int K = a.K, H = a.H;
-    const int k0 = wt * kWRows;
-    const int64_t row0 = (int64_t)f0 * 32;
-    const uint32_t row_bytes = (uint32_t)H * 2u;
-    const int n_slabs = (int)(row_bytes / tall::kRB);
+// 64 w4 + 32 f + 8(i/4) + 4(l/32) + i%4 of tile row 32 t + l%32.  A wave rounds a fragment of its 64 columns to
+// bf16, transposes it through its LDS scratch and stores whole 128-byte lines to y[pair id]; rows without a pair
+// are skipped.
+struct DownTile {
+    const char *act, *w_lo, *w_hi;
+    uint32_t row_bytes;
+};
+__device__ __forceinline__ DownTile down_operands(const MoeArgs &a, const Work &w) {
+    DownTile d;
+    d.row_bytes = (uint32_t)a.H * 2u;
+    d.act = a.act + (int64_t)w.f0 * 32 * d.row_bytes;
     // weight rows (output columns) k0 .. k0 + 255 of the expert; the last tile of a K that is not a multiple
     // of 256 has 128 of them and reads the first half twice
-    const char *w_lo = a.w2 + ((int64_t)e * K + k0) * H * 2;
-    const char *w_hi = (k0 + 128 < K) ? w_lo + (int64_t)128 * H * 2 : w_lo;
+    const int k0 = w.wt * kWRows;
+    d.w_lo = a.w2 + ((int64_t)w.e * a.K + k0) * d.row_bytes;
+    d.w_hi = (k0 + 128 < a.K) ? d.w_lo + (int64_t)128 * d.row_bytes : d.w_lo;
+    return d;
+}
+template <int FG>
+__device__ __forceinline__ void down_tile_tall(const MoeArgs &a, const KernelPlan &kp, const Work &w, int *counter, char *lds,
+                                               bool &pre, Work &next) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave >> 2, w4 = wave & 3;
+    const int K = a.K;
+    const int k0 = w.wt * kWRows;
+    const DownTile d = down_operands(a, w);
     tall::Loader<FG, false> ld;
-    ld.setup(tid, a.act + row0 * H * 2, w_lo, w_hi, row_bytes, row_bytes, [&](int row) { return (uint32_t)row * row_bytes; });
+    ld.setup(tid, d.act, d.w_lo, d.w_hi, d.row_bytes, d.row_bytes, [&](int row) { return (uint32_t)row * d.row_bytes; });
     const int wrow[2] = {64 * w4, 64 * w4 + 32};
     f32x16 acc[2][FG];
     zero_acc<FG>(acc);
-    const int start = (pos & 7) % n_slabs;  // workgroups that run side by side start their K walks at different slabs
-    tall::main_loop<FG>(acc, ld, lds, n_slabs, wrow, grp * FG, lane, start);
-    const int asked = ask_slot(counter);
+    int asked = 0;
+    // pair ids of the wave's 32 FG rows, one per lane; fetched before the last slab, in the registers its loader no
+    // longer needs
+    constexpr int NP = (FG + 1) / 2;
+    int pairs[NP];
+    tall::main_loop<FG>(acc, ld, lds, w.n_slabs, wrow, grp * FG, lane, k_start(w), pre, [&] { asked = ask_slot(counter); },
+                        [&] {
+#pragma unroll
+                            for (int q = 0; q < NP; ++q) {
+                                const int64_t s = (int64_t)w.f0 * 32 + grp * 32 * FG + 64 * q + lane;
+                                pairs[q] = (64 * q + lane < 32 * FG && s < a.sorted_num) ? a.sorted_ids[s] : -1;
+                            }
+                        });
+    // (they are here before the copies of the next tile queue up behind them)
+#pragma unroll
+    for (int q = 0; q < NP; ++q) asm volatile("" : "+v"(pairs[q]));
 
-    const int r = lane & 31, half = lane >> 5;
-    const int cols = min(kWRows, K - k0);
+    // (the epilogue's addresses are computed from a lane number that the compiler knows nothing about: it would keep
+    // them in registers across the K loop, that is spill them, and a reload here waits for the copies in flight)
+    int lane_e = lane;
+    asm volatile("" : "+v"(lane_e));
+    const int r = lane_e & 31, half = lane_e >> 5;
+    const bool in_cols = k0 + 64 * w4 < K;  // (K is a multiple of 128: a wave's 64 columns are inside or outside)
     const uint32_t n_pairs = (uint32_t)(a.M * a.top_k);
-    const int c = tid & 31;
+    char *scratch = lds + tall::kScratchOff + wave * tall::kScratchBytes;
+    constexpr int kPitch = 144;  // 64 columns + 16 B pad
+    char *dst = a.y + (int64_t)(k0 + 64 * w4) * 2 + (lane_e & 7) * 16;
+    int4 tl = make_int4(0, 0, 0, 0);
+    pre = false;
+    epilogue_with_links<FG, 2>(
+        [&](int t) {
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-        // 32 threads per row (16 bytes each), 16 rows per turn; the pair ids of this thread's rows are fetched
-        // first, so that they are in flight during the LDS round trip
-        int pr[2 * FG];
+            for (int f = 0; f < 2; ++f)
 #pragma unroll
-        for (int i = 0; i < 2 * FG; ++i) {
-            const int64_t s = row0 + g * 32 * FG + (tid >> 5) + 16 * i;
-            pr[i] = s < a.sorted_num ? a.sorted_ids[s] : -1;
-        }
-        if (grp == g) {
+                for (int q = 0; q < 4; ++q) {
+                    uint2 pk;
+                    pk.x = pack2_bf16(acc[f][t][4 * q], acc[f][t][4 * q + 1]);
+                    pk.y = pack2_bf16(acc[f][t][4 * q + 2], acc[f][t][4 * q + 3]);
+                    *reinterpret_cast<uint2 *>(scratch + r * kPitch + 64 * f + 16 * q + 8 * half) = pk;
+                }
+            wave_lds_order();
 #pragma unroll
-            for (int t = 0; t < FG; ++t) {
-                const int row = 32 * t + r;
-#pragma unroll
-                for (int f = 0; f < 2; ++f)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int col = 64 * w4 + 32 * f + 8 * q + 4 * half;
-                        uint2 pk;
-                        pk.x = pack2_bf16(acc[f][t][4 * q], acc[f][t][4 * q + 1]);
-                        pk.y = pack2_bf16(acc[f][t][4 * q + 2], acc[f][t][4 * q + 3]);
-                        *reinterpret_cast<uint2 *>(lds + row * kYPitch + col * 2) = pk;
-                    }
+            for (int i = 0; i < 4; ++i) {
+                const int row = (lane_e >> 3) + 8 * i;
+                const int p = __shfl(pairs[t / 2], 32 * (t & 1) + row, 64);
+                const uint4 v = *reinterpret_cast<const uint4 *>(scratch + row * kPitch + (lane_e & 7) * 16);
+                if (in_cols && (uint32_t)p < n_pairs) store_once(dst + (int64_t)p * K * 2, v);
             }
-        }
-        __syncthreads();
-        if (8 * c < cols) {
-#pragma unroll
-            for (int i = 0; i < 2 * FG; ++i) {
-                const int row = (tid >> 5) + 16 * i;
-                if ((uint32_t)pr[i] < n_pairs) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(lds + row * kYPitch + c * 16);
-                    store_once(a.y + (int64_t)pr[i] * K * 2 + (int64_t)k0 * 2 + c * 16, v);
+            wave_lds_order();
+        },
+        [&](int link) {
+            if (link == 0) {
+                next = slot_work(pass_slot(asked, lds), a.n_wtiles, kp);
+                if (next.state > 0) tl = a.tiles_down[next.tile];
+            } else {
+                if (next.state > 0) tile_work(next, tl, kp, a.H * 2 / tall::kRB);
+                if (next.state > 0) {
+                    const DownTile n = down_operands(a, next);
+                    const int row = 8 * wave + (lane_e >> 3);
+                    const uint32_t off = (uint32_t)row * n.row_bytes + (uint32_t)((lane_e & 7) ^ ((row >> 1) & 7)) * 16u;
+                    tall::pre_issue<false>(next.fg, lds, wave, lane_e, n.act, n.w_lo, n.w_hi, n.row_bytes, n.row_bytes, &off,
+                                           next.n_slabs, k_start(next));
+                    pre = true;
                 }
             }
-        }
-        if (g == 0) __syncthreads();
-    }
-    return asked;
+        });
 }
 
 __global__ __launch_bounds__(512) void moe_down_kernel_bf16(MoeArgs a) {
     __shared__ __attribute__((aligned(1024))) char lds[tall::kLdsBytes];
     const KernelPlan kp = a.plan->down;
-    const int xcd = (int)(blockIdx.x & 7);
-    int *counter = &a.plan->counters[8 + xcd];
-    for (int pos = (int)(blockIdx.x >> 3);;) {
-        TallJob j;
-        const int st = resolve_tall_job(8 * pos + xcd, a.n_wtiles, kp, j);
-        if (st < 0) break;
-        if (st == 0) {
-            pos = pass_slot(ask_slot(counter), reinterpret_cast<int *>(lds));
-            continue;
+    int *counter = &a.plan->counters[8 + (blockIdx.x & 7)];
+    bool pre = false;
+    walk_queue(kp, a.tiles_down, a.n_wtiles, a.H * 2 / tall::kRB, counter, lds, [&](const Work &w, Work &next) {
+        switch (w.fg) {
+            case 1: down_tile_tall<1>(a, kp, w, counter, lds, pre, next); break;
+            case 2: down_tile_tall<2>(a, kp, w, counter, lds, pre, next); break;
+            case 3: down_tile_tall<3>(a, kp, w, counter, lds, pre, next); break;
+            case 4: down_tile_tall<4>(a, kp, w, counter, lds, pre, next); break;
+            case 5: down_tile_tall<5>(a, kp, w, counter, lds, pre, next); break;
+            default: down_tile_tall<6>(a, kp, w, counter, lds, pre, next); break;
         }
-        int asked = 0;
-        const int4 tl = a.tiles_down[j.tile];
-        int f0 = tl.x, fg = tl.y;
-        const int e = tl.z;
-        if (j.parts > 1) fg = row_split(f0, fg, j.part, j.parts);
-        fg = __builtin_amdgcn_readfirstlane(fg);
-        switch (fg) {
-            case 1: asked = down_tile_tall<1>(a, e, f0, j.wt, pos, counter, lds); break;
-            case 2: asked = down_tile_tall<2>(a, e, f0, j.wt, pos, counter, lds); break;
-            case 3: asked = down_tile_tall<3>(a, e, f0, j.wt, pos, counter, lds); break;
-            case 4: asked = down_tile_tall<4>(a, e, f0, j.wt, pos, counter, lds); break;
-            case 5: asked = down_tile_tall<5>(a, e, f0, j.wt, pos, counter, lds); break;
-            case 6: asked = down_tile_tall<6>(a, e, f0, j.wt, pos, counter, lds); break;
-            default: asked = ask_slot(counter); break;
-        }
-        pos = pass_slot(asked, reinterpret_cast<int *>(lds));
-    }
+    });
 }
 
 // Weight-streaming kernels (moe_stream.h).  n_tiles: weight tiles per block (0: the up kernel only inverts).

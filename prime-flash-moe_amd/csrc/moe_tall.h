@@ -34,6 +34,15 @@ constexpr int kWUnitBytes = kWRows * kRB;   // the 256 weight rows of a slab
 constexpr int kLdsBytes = 160 * 1024;
 constexpr int kMaxFrags = 12;
 
+// LDS behind the stages of a tile's first slabs: while the epilogue of one tile runs, the first stages of the next
+// one are already being filled (see pre_issue), so the epilogue stays clear of them.  At most kPreBytes are filled
+// ahead (three stages of the smallest tile; two of 48 KB or one of up to 80 KB otherwise).
+constexpr int kPreBytes = 3 * (2 * kFragBytes + kWUnitBytes);
+constexpr int kWordOff = kPreBytes;                   // a word that hands a number to every wave
+constexpr int kScratchBytes = 32 * 144;               // per wave: 32 rows of 128 B, 16 B pad each
+constexpr int kScratchOff = kLdsBytes - 8 * kScratchBytes;
+static_assert(kWordOff + 16 <= kScratchOff, "the scratch of the epilogues overlaps the stages filled ahead");
+
 template <int FG>
 struct Geo {
     static constexpr int kNTF = 2 * FG;
@@ -60,9 +69,11 @@ struct Loader {
     int lds_piece;         // LDS offset of the wave's first piece inside a 8 KB group of pieces
 
     // row_off(row) = byte offset of tile row `row` (0 .. 64 FG - 1) in `tok` (!GATHER: row * tok_pitch).
+    // Gathered rows: `ahead` holds the offsets (chunk included) of the wave's pieces already (see pre_issue).
     template <typename TokOff>
     __device__ __forceinline__ void setup(int tid, const char *tok, const char *w_half0, const char *w_half1,
-                                          uint32_t w_pitch, uint32_t tok_pitch, TokOff row_off) {
+                                          uint32_t w_pitch, uint32_t tok_pitch, TokOff row_off,
+                                          const uint32_t *ahead = nullptr) {
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
         lds_piece = wave * 1024;
         // piece p (8 rows) of a run of rows: rows 8 p .. 8 p + 7; this wave takes pieces wave + 8 q.  The
@@ -70,7 +81,7 @@ struct Loader {
         const int row = 8 * wave + (lane >> 3);
         const uint32_t chunk = (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
 #pragma unroll
-        for (int q = 0; q < NT; ++q) tok_off[q] = row_off(row + 64 * q) + chunk;
+        for (int q = 0; q < NT; ++q) tok_off[q] = ahead != nullptr ? ahead[q] : row_off(row + 64 * q) + chunk;
         tok_step = 64u * tok_pitch;
         w_off = (uint32_t)row * w_pitch + chunk;
         w_step = 64u * w_pitch;
@@ -95,6 +106,38 @@ struct Loader {
         for (int c = 0; c < Geo<FG>::kCopies; ++c) issue(c, stage, koff);
     }
 };
+
+// The first slabs of a tile of `fg` pairs of fragments, issued ahead of its main_loop (which then starts with
+// PRE): slabs 0 .. min(stages - 1, n_slabs) - 1 into stages 0, 1, ...  `tok_off`: GATHER: the offsets of this
+// wave's pieces (fg of them); otherwise [0] is that of its first piece.  The number of pairs is a run-time value: the
+// code runs once per tile, under the epilogue of a tile of another size.
+template <bool GATHER>
+__device__ __forceinline__ void pre_issue(int fg, char *lds, int wave, int lane, const char *tok, const char *w_half0, const char *w_half1,
+                                          uint32_t w_pitch, uint32_t tok_pitch, const uint32_t *tok_off, int n_slabs,
+                                          int start) {
+    const int row = 8 * wave + (lane >> 3);
+    const uint32_t w_off = (uint32_t)row * w_pitch + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+    tok = ring::uniform_ptr(tok);
+    w_half0 = ring::uniform_ptr(w_half0);
+    w_half1 = ring::uniform_ptr(w_half1);
+    const int tok_bytes = 2 * fg * kFragBytes, stage_bytes = tok_bytes + kWUnitBytes;
+    const int ahead = min(min(4, kLdsBytes / stage_bytes) - 1, n_slabs);
+    for (int s = 0; s < ahead; ++s) {
+        const int slab = s + start >= n_slabs ? s + start - n_slabs : s + start;
+        const uint32_t koff = (uint32_t)slab * kRB;
+        char *stage = lds + s * stage_bytes + wave * 1024;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            ring::copy16((c < 2 ? w_half0 : w_half1) + koff + (c & 1) * (size_t)(64u * w_pitch), w_off,
+                         stage + tok_bytes + c * 8192);
+#pragma unroll
+        for (int q = 0; q < kMaxFrags / 2; ++q)
+            if (q < fg) {
+                if constexpr (GATHER) ring::copy16(tok + koff, tok_off[q], stage + q * 8192);
+                else ring::copy16(tok + koff + q * (size_t)(64u * tok_pitch), tok_off[0], stage + q * 8192);
+            }
+    }
+}
 
 __device__ __forceinline__ bf16x8 lds_frag(const char *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
@@ -159,10 +202,14 @@ __device__ __forceinline__ void slab(f32x16 (&acc)[2][FG], bf16x8 &a0, bf16x8 &a
 
 // K loop of one tile.  acc[f][t]: weight fragment f (rows wrow[f] .. + 31 of the weight tile) against token
 // fragment tok_frag0 + t (weight rows on the MFMA M side).  Slabs are visited in rotated order starting at
-// `start`.  Ends with a barrier: the ring may be reused as scratch afterwards.
-template <int FG, typename LD>
+// `start`.  Ends with a barrier: the ring may be reused as scratch afterwards.  `pre`: the first slabs have been
+// issued (pre_issue).  `near_end()` runs before the last slab but one, `last()` before the last (n_slabs >= 2).
+// What else of this wave is in flight (stores of the previous tile's epilogue, loads of the hooks) only makes the
+// counted waits longer: copies complete in the order of issue.
+template <int FG, typename LD, typename NearEnd, typename Last>
 __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][FG], const LD &ld, char *lds, int n_slabs,
-                                          const int (&wrow)[2], int tok_frag0, int lane, int start) {
+                                          const int (&wrow)[2], int tok_frag0, int lane, int start, bool pre,
+                                          NearEnd near_end, Last last) {
     using G = Geo<FG>;
     constexpr int S = G::kStages, LPS = G::kCopies, SB = G::kStageBytes;
     auto rot = [&](int s) {
@@ -177,7 +224,7 @@ __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][FG], const LD &ld, ch
 
 #pragma unroll
     for (int s = 0; s < S - 1; ++s)
-        if (s < n_slabs) ld.issue_all(lds + s * SB, (uint32_t)rot(s) * kRB);
+        if (!pre && s < n_slabs) ld.issue_all(lds + s * SB, (uint32_t)rot(s) * kRB);
     {
         // slab 0 has landed once at most the copies of the later slabs (up to S - 2) are pending
         const int later = min(S - 2, n_slabs - 1);
@@ -195,6 +242,7 @@ __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][FG], const LD &ld, ch
     for (int kt = 0; kt < n_slabs - 1; ++kt) {
         // the stage slab kt - 1 used is free: everybody is past the barrier that opened slab kt
         const bool fill = kt + S - 1 < n_slabs;
+        if (kt == n_slabs - 2) near_end();
         int fs = cur - 1;
         if (fs < 0) fs += S;
         int nx = cur + 1;
@@ -204,7 +252,14 @@ __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][FG], const LD &ld, ch
                         S == 2 ? 0 : min(S - 2, n_slabs - 2 - kt));
         cur = nx;
     }
+    last();
     slab<FG, true>(acc, a0, a1, b, ld, lds + cur * SB, lds, false, lds, 0u, off0, w_at0, w_at1, t_at, 0);
+    // the sums are complete here: without this the compiler moves matrix instructions of the last slab into the
+    // branches of the epilogue that use their results, and spills the operands it has to keep for them
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int t = 0; t < FG; ++t) asm volatile("" : "+v"(acc[f][t]));
     __syncthreads();  // all reads of the last stage are done: the ring may be reused as scratch
 }
 
