@@ -24,18 +24,6 @@
 
 namespace pmoe {
 
-// Slab width (bytes per row and slab) of the stage-ring tiles.  128: every request is a whole cache line.
-// 64 (twice the stages in the same LDS) stays selectable at build time for measurements: with the
-// non-temporal weight copies it runs the decode shape 32 % and the DeepSeek-like prefill 40 % slower.
-#ifndef PMOE_SKINNY_RB
-#define PMOE_SKINNY_RB 128
-#endif
-#ifndef PMOE_PART_RB
-#define PMOE_PART_RB 128
-#endif
-constexpr int kSkinnyRB = PMOE_SKINNY_RB;  // tiles with one live fragment
-constexpr int kPartRB = PMOE_PART_RB;      // mxfp8 tiles with more
-
 // What one workgroup of an mxfp8 kernel does: `n_sub` consecutive weight tiles from `wt` on for the row tile
 // of `nb` blocks starting at block `first`, expert `e`.
 struct Job {
@@ -324,11 +312,9 @@ __device__ __forceinline__ void setup_ring_loader(ring::Loader<RB> &ld, const ri
 // blockIdx / 8) start 128 bytes apart, 8 distinct phases over a 1 KB period.  The spread keeps the
 // workgroups that share a weight tile off the same HBM channel at the same instant, and stays short
 // enough that they still meet in L2 (a 16-phase, 4 KB spread read 30 % more from HBM for the same time).
-// Even for 64-byte slabs: two of them share a scale dword.
 template <int RB>
 __device__ __forceinline__ int slab_rotation(int n_slabs) {
-    const int phase = (int)((blockIdx.x >> 3) & 7) * (128 / RB);
-    return RB == 64 ? phase % n_slabs & ~1 : phase % n_slabs;
+    return (int)((blockIdx.x >> 3) & 7) % n_slabs;
 }
 
 // Up kernel tile on the stage ring: the live fragments of one or two row blocks x activation
@@ -386,9 +372,9 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, R
         f32x16 acc[2][4];
         zero_acc(acc);
         if (active)
-            ring::main_loop<DT, RB, NTF, true, true>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
+            ring::main_loop<DT, RB, NTF, true>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
         else
-            ring::main_loop<DT, RB, NTF, true, false>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
+            ring::main_loop<DT, RB, NTF, false>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
         const bool more = sub + 1 < n_sub;
         if (more) {
             // same token rows, the next 128 gate and 128 up rows of the expert
@@ -397,7 +383,7 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, R
             if (DT == DT_FP8 && wave >= 4) ld.sc_off += (uint32_t)kt128 * 512u;
             ld.make_uniform();
             stage0 = free0 < NS ? free0 : 0;
-            n_pre = free0 < NS ? min(NS - 1, NS - free0) : 0;
+            n_pre = max(NS - free0, 0);
             ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, stage0, n_pre);
         }
         if (active) swiglu_epilogue<DT, NTF>(acc, tile, sc_tile, w4, lane);
@@ -433,9 +419,9 @@ __global__ __launch_bounds__(512) void moe_up_kernel(MoeArgs a) {
     const int ntf = load_row_info<2>(a, j.first, j.nb, ri);
     if (ntf == 0) return;
     uint32_t *act_sc_lds = reinterpret_cast<uint32_t *>(lds + L::kActScaleOff);
-    if (ntf == 1) up_tile_ring<DT, kSkinnyRB, 1>(a, j, ri, lds, act_sc_lds);
-    else if (ntf == 2) up_tile_ring<DT, kPartRB, 2>(a, j, ri, lds, act_sc_lds);
-    else up_tile_ring<DT, kPartRB, 4>(a, j, ri, lds, act_sc_lds);
+    if (ntf == 1) up_tile_ring<DT, ring::kRB, 1>(a, j, ri, lds, act_sc_lds);
+    else if (ntf == 2) up_tile_ring<DT, ring::kRB, 2>(a, j, ri, lds, act_sc_lds);
+    else up_tile_ring<DT, ring::kRB, 4>(a, j, ri, lds, act_sc_lds);
 }
 
 // Down kernel tile on the stage ring: y[rows, 256 cols of K] = act[rows, :H] . W2[e][cols, :H]^T, the
@@ -493,15 +479,15 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
         f32x16 acc[2][4];
         zero_acc(acc);
         if (active)
-            ring::main_loop<DT, RB, NTF, true, true>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
+            ring::main_loop<DT, RB, NTF, true>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
         else
-            ring::main_loop<DT, RB, NTF, true, false>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
+            ring::main_loop<DT, RB, NTF, false>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
         const bool more = sub + 1 < n_sub;
         if (more) {
             set_weights(k0 + kWRows);
             ld.make_uniform();
             stage0 = free0 < NS ? free0 : 0;
-            n_pre = free0 < NS ? min(NS - 1, NS - free0) : 0;
+            n_pre = max(NS - free0, 0);
             ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, stage0, n_pre);
         }
         const YDst dst = y_destination(a, k0);
@@ -527,9 +513,9 @@ __global__ __launch_bounds__(512) void moe_down_kernel(MoeArgs a) {
     if (!resolve_job(a, j)) return;
     const int ntf = load_row_info<2>(a, j.first, j.nb, ri);
     if (ntf == 0) return;
-    if (ntf == 1) down_tile_ring<DT, kSkinnyRB, 1>(a, j, ri, lds);
-    else if (ntf == 2) down_tile_ring<DT, kPartRB, 2>(a, j, ri, lds);
-    else down_tile_ring<DT, kPartRB, 4>(a, j, ri, lds);
+    if (ntf == 1) down_tile_ring<DT, ring::kRB, 1>(a, j, ri, lds);
+    else if (ntf == 2) down_tile_ring<DT, ring::kRB, 2>(a, j, ri, lds);
+    else down_tile_ring<DT, ring::kRB, 4>(a, j, ri, lds);
 }
 
 // Walk order of the tiles of one mxfp8 kernel: [group of 8 weight tiles][row tile][weight tile in group].

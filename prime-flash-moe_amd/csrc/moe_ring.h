@@ -1,11 +1,12 @@
 // Stage-ring engine of the mxfp8 grouped-GEMM kernels (512 threads), gfx950, and the copy primitives that the
 // bf16 engine (moe_tall.h) shares with it.
 //
-// Tile: token rows x 256 weight rows.  The contraction is consumed in slabs of RB = 64 or 128 bytes
-// per row.  Slabs are copied global -> LDS by the direct-to-LDS path (global_load_lds_*: no staging
-// registers, no ds_write) into a ring of stages; all but one stage are in flight while one is
-// consumed.  One barrier per slab.  RB = 128 asks L2 for whole cache lines (half the requests, half
-// the barriers; a plain stream from HBM runs 8 % faster); RB = 64 has twice the stages in the same LDS.
+// Tile: token rows x 256 weight rows.  The contraction is consumed in slabs of RB = 128 bytes per row: whole cache
+// lines (with 64-byte slabs and twice the stages the decode shape ran 32 %, the DeepSeek-like prefill 40 % slower).
+// Slabs are copied global -> LDS by the direct-to-LDS path (global_load_lds_*: no staging registers, no ds_write)
+// into a ring of stages.  Two barriers per slab: one opens a slab that has landed, one gives its stage back as soon as
+// every wave holds the slab's remaining operands in registers, so that up to all stages are in flight while the last
+// third of the matrix instructions of a slab runs (see main_loop).
 //
 // The ring is sized per tile.  A stage holds only the 32-row token fragments that have live rows
 // (group 0's first, then group 1's), the 256 weight rows and, for mxfp8, the scale dwords of both;
@@ -15,8 +16,7 @@
 //
 // Stage layout: [live token rows][RB] [256 weight rows][RB] [scale dwords: token rows rounded up to a
 // multiple of 64, then weight rows (mxfp8)].
-// A row is RB/16 chunks of 16 B; chunk c of row r sits in slot c ^ swizzle(r) (64 B: (r >> 2) & 3,
-// 128 B: (r >> 1) & 7): the 16-byte MFMA operand reads of 16 consecutive rows then cover all 64 LDS
+// A row is RB/16 chunks of 16 B; chunk c of row r sits in slot c ^ swizzle(r), swizzle(r) = (r >> 1) & 7: the 16-byte MFMA operand reads of 16 consecutive rows then cover all 64 LDS
 // banks exactly once.  The copy engine writes lane l of a wave instruction to bytes [16 l, 16 l + 16)
 // behind a wave-uniform base (one instruction = 1 KB = 1024 / RB rows), so the swizzle is applied on
 // the global side (the lane landing in slot s of row r fetches chunk s ^ swizzle(r)).
@@ -37,9 +37,11 @@ namespace ring {
 
 constexpr int kMaxStages = 8;
 
+constexpr int kRB = 128;  // row bytes of a slab
 template <int RB>
 __device__ __forceinline__ int swz(int row) {
-    return RB == 64 ? (row >> 2) & 3 : (row >> 1) & 7;
+    static_assert(RB == 128, "the swizzle of 128-byte rows");
+    return (row >> 1) & 7;
 }
 
 // Geometry of a tile's ring; every member is wave-uniform.
@@ -107,10 +109,11 @@ template <int N>
 __device__ __forceinline__ void wait_and_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
+// This wave's LDS reads have returned; joins the workgroup barrier.
+__device__ __forceinline__ void all_read() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
 // Waits until at most `n` (wave-uniform, <= 30) of this wave's copies are in flight and its LDS
 // reads have returned, then joins the workgroup barrier.  The wait count is an immediate of the
-// instruction, hence the switch (RB = 64: at most 5 copies per stage x 6 stages behind the current
-// one; RB = 128: 9 x 2).
+// instruction, hence the switch (at most 9 copies per stage x 3 stages behind the current one).
 __device__ __forceinline__ void wait_and_barrier_dyn(int n) {
     switch (n) {
 #define PMOE_WB(k) case k: wait_and_barrier<k>(); break;
@@ -160,71 +163,58 @@ struct Loader {
         w_base[1] = uniform_ptr(w_base[1]);
         sc_base = uniform_ptr(sc_base);
     }
-    __device__ __forceinline__ void issue(char *stage, int slab) const {
+    // Copy c (a constant once the caller's loop is unrolled) of this wave's share of a stage: kWPieces of weight rows,
+    // which every wave issues, then the token rows, then the scales.
+    static constexpr int kWPieces = 2 * N, kPieces = 4 * N + 1;
+    __device__ __forceinline__ void issue_piece(int c, char *stage, int slab) const {
         const uint32_t koff = (uint32_t)slab * RB;
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int q = 0; q < N; ++q)
-                if (tok_dst[b][q] >= 0) {
-                    if (tok_live[b][q]) copy16(tok_base, tok_off[b][q] + koff, stage + tok_dst[b][q]);
-                }
-        if (w_once) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int q = 0; q < N; ++q) copy16_once(w_base[h], w_off[q] + koff, stage + w_dst[h][q]);
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int q = 0; q < N; ++q) copy16(w_base[h], w_off[q] + koff, stage + w_dst[h][q]);
+        const int b = (c / N) & 1, q = c % N;
+        if (c < kWPieces) {
+            if (w_once) copy16_once(w_base[b] + koff, w_off[q], stage + w_dst[b][q]);
+            else copy16(w_base[b] + koff, w_off[q], stage + w_dst[b][q]);
+        } else if (c < 2 * kWPieces) {
+            if (tok_dst[b][q] >= 0) {
+                if (tok_live[b][q]) copy16(tok_base + koff, tok_off[b][q], stage + tok_dst[b][q]);
+            }
+        } else if (sc_dst >= 0) {
+            copy4(sc_base + (uint32_t)slab * sc_step, sc_off, stage + sc_dst);
         }
-        if (sc_dst >= 0) copy4(sc_base, sc_off + (uint32_t)(RB == 64 ? slab >> 1 : slab) * sc_step, stage + sc_dst);
+    }
+    __device__ __forceinline__ void issue(char *stage, int slab) const {
+#pragma unroll
+        for (int c = 0; c < kPieces; ++c) issue_piece(c, stage, slab);
     }
 };
 
-// 64 e4m3 of K = one v_mfma_scale_f32_32x32x64_f8f6f4 per (weight fragment, token fragment); `j` is
-// the 64-byte step inside the slab (0 for RB = 64).  Registers 0-3 of both lane halves form K block 0
-// of the step (lanes < 32 its first 16 bytes, lanes >= 32 the last 16), registers 4-7 form K block 1;
-// the scale of block 0 is taken from lanes < 32 and that of block 1 from lanes >= 32 (measured on
-// gfx950).  `sel` = 8 * (2 * (64-byte step inside its 128-wide K tile) + lane / 32) picks this lane's
-// scale byte out of the row's 4-scale dword.
-template <int RB, int NTF, bool TRANSPOSED>
-__device__ __forceinline__ void mma_fp8_step(f32x16 (&acc)[2][4], const char *tok, const char *wgt,
-                                             const uint32_t *tok_sc, const uint32_t *w_sc,
-                                             const int (&wrow)[2], int lane, int j, int sel) {
-    const int r = lane & 31, half = lane >> 5, sx = swz<RB>(r);
-    const int off = r * RB + (((4 * j + half) ^ sx) << 4);
-    i32x8 a[2];
-    int sa[2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f) {
-        const char *p = wgt + wrow[f] * RB;
-        const i32x4 lo = *reinterpret_cast<const i32x4 *>(p + off);
-        const i32x4 hi = *reinterpret_cast<const i32x4 *>(p + (off ^ 32));
-        a[f] = i32x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        sa[f] = (int)((w_sc[wrow[f] + r] >> sel) & 0xffu);
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-        if (t < NTF) {
-            const char *p = tok + t * 32 * RB;
-            const i32x4 lo = *reinterpret_cast<const i32x4 *>(p + off);
-            const i32x4 hi = *reinterpret_cast<const i32x4 *>(p + (off ^ 32));
-            const i32x8 b = i32x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-            const int sb = (int)((tok_sc[32 * t + r] >> sel) & 0xffu);
-#pragma unroll
-            for (int f = 0; f < 2; ++f) {
-                if constexpr (TRANSPOSED)
-                    acc[f][t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[f], b, acc[f][t], 0, 0, 0, sa[f], 0, sb);
-                else
-                    acc[f][t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(b, a[f], acc[f][t], 0, 0, 0, sb, 0, sa[f]);
-            }
-        }
+// Operands of one 64-wide K step of a wave: weight fragments a[f], token fragments b[t], and for the slab the step
+// belongs to the scale dwords of their rows (4 scales = 128 contraction elements).
+//
+// One v_mfma_scale_f32_32x32x64_f8f6f4 per (weight fragment, token fragment) and step.  Registers 0-3 of both lane
+// halves form K block 0 of the step (lanes < 32 its first 16 bytes, lanes >= 32 the last 16), registers 4-7 K block
+// 1; the scale of block 0 is taken from lanes < 32 and that of block 1 from lanes >= 32 (measured on gfx950).  So a
+// lane's scale byte in step j is byte 2 j + lane / 32 of its dword: shifted right by 8 (lane / 32) once per slab, the
+// instruction picks byte 2 j itself.
+template <int NTF>
+struct Operands {
+    i32x8 a[2], b[NTF];
+    int sa[2], sb[NTF];
+};
+__device__ __forceinline__ i32x8 lds_frag(const char *p, int off) {
+    const i32x4 lo = *reinterpret_cast<const i32x4 *>(p + off);
+    const i32x4 hi = *reinterpret_cast<const i32x4 *>(p + (off ^ 32));
+    return i32x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+}
+// Nothing crosses this point in the instruction schedule: the order written is the order issued.
+#define PMOE_RING_FENCE() __builtin_amdgcn_sched_barrier(0)
+
+// Matrix instructions of weight fragment F with token fragment t in step J.
+template <int NTF, int J, int F>
+__device__ __forceinline__ void mma(f32x16 (&acc)[2][4], const Operands<NTF> &o, int t) {
+    acc[F][t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(o.a[F], o.b[t], acc[F][t], 0, 0, 2 * J, o.sa[F], 2 * J, o.sb[t]);
+    asm volatile("" : "+v"(acc[F][t]));  // stays here: the compiler would sink it past the copies and keep its operands
 }
 
-// Issues slabs 0 .. n - 1 of a tile (at most stages - 1 of them, in rotated order from `start`) into
+// Issues slabs 0 .. n - 1 of a tile (at most as many as there are stages, in rotated order from `start`) into
 // stages stage0, stage0 + 1, ...
 template <int DT, int RB>
 __device__ __forceinline__ void pre_issue(const Loader<RB> &ld, const Layout &lay, char *lds, int n_slabs, int start,
@@ -243,63 +233,189 @@ __device__ __forceinline__ void pre_issue(const Loader<RB> &ld, const Layout &la
 // rows): they only issue their share of the copies and join the barriers.  `tok_region` = byte
 // offset of this wave's group inside a stage's token rows.
 //
-// The slabs are visited in rotated order, starting at slab `start` (even for RB = 64): workgroups
+// The slabs are visited in rotated order, starting at slab `start`: workgroups
 // that run side by side and share rows then ask for different cache lines at any one time instead
 // of queueing on the same ones.  The sum over K does not depend on the order.
 //
-// Geometry and wait counts are wave-uniform run-time values (the wait count goes through a switch).  A
-// variant for tiles of two full blocks with compile-time geometry, 64-byte slabs and 4 stages measured 2 - 3 %
-// slower on large mxfp8 batches than this loop with 128-byte slabs and 2 stages, and is gone.
+// Geometry and wait counts are wave-uniform run-time values (the wait count goes through a switch).
+//
+// A slab's stage is given back (second barrier) before its matrix instructions are done.  NTF <= 2: all operands of a
+// slab are read first.  NTF = 4 has registers for one 64-wide step: the operands of step 1 replace those of step 0 as
+// these are used up, the stage goes back behind step 0, the copies into it are spread over the matrix instructions of
+// step 1 (a wave waits where the CU's copy path does not take its next copy: issued in one run, 9 copies held up the
+// wave's matrix instructions), and the barrier that opens the next slab sits in the middle of step 1, whose second
+// half covers the first reads of that slab.  Before, one barrier per slab opened it and its copies followed in one
+// run: a tile of two full blocks has LDS for two stages, so the copy path went idle once per slab.
+// 24593 tokens on 32 experts (K = N = 2048): 899 -> 855 us for the layer (882 with the copies in one run);
+// 4096 tokens on 256 experts (K 7168, N 4096): 2712 -> 2649 us.  Reading both steps first at NTF = 4 spills registers:
+// 1019 and 2981 us.
 //
 // Slab 0 goes to stage `stage0`, the following ones to the stages behind it (wrapping).  `n_pre`: the
 // caller has already issued slabs 0 .. n_pre - 1 (see pre_issue; a workgroup that runs one tile
 // after another issues them under the previous tile's epilogue).
-template <int DT, int RB, int NTF, bool TRANSPOSED, bool COMPUTE>
+template <int DT, int RB, int NTF, bool COMPUTE>
 __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][4], const Loader<RB> &ld, const Layout &lay, char *lds,
                                           int n_slabs, const int (&wrow)[2], int lane, int tok_region, int start,
                                           int stage0 = 0, int n_pre = 0) {
+    static_assert(DT == DT_FP8 && RB == 128, "two scaled matrix instructions of 64 e4m3 per slab and accumulator");
     const int SB = lay.stage_bytes, NS = lay.stages;
-    const int w_off = lay.w_off, scale_off = lay.scale_off, scale_tok_rows = lay.scale_tok_rows;
     auto rot = [&](int s) {
         s += start;
         return s >= n_slabs ? s - n_slabs : s;
     };
-    for (int s = n_pre; s < NS - 1; ++s) {
+    for (int s = n_pre; s < NS; ++s) {
         int st = stage0 + s;
         if (st >= NS) st -= NS;
         if (s < n_slabs) ld.issue(lds + st * SB, rot(s));
     }
     const int lps = ld.lps;
+    // opens slab k: it has landed once at most the copies of the later slabs (up to NS - 1) are pending
+    // (copies and stores of an epilogue that are in flight too only make the counted waits longer)
+    auto open = [&](int k) { wait_and_barrier_dyn(lps * min(NS - 1, n_slabs - 1 - k)); };
+    // gives the stage of slab k, which every wave has read, to slab k + NS
+    auto refill = [&](int k, int off) {
+        if (k + NS < n_slabs) {
+            all_read();
+            ld.issue(lds + off, rot(k + NS));
+        }
+    };
     int cur_off = stage0 * SB;  // stage of slab kt
-    // stage slab kt + NS - 1 goes to (the one slab kt - 1 used)
-    int fill_off = (stage0 == 0 ? NS - 1 : stage0 - 1) * SB;
-    for (int kt = 0; kt < n_slabs; ++kt) {
-        // slab kt has landed once at most the copies of the later slabs (up to NS - 2) are pending
-        wait_and_barrier_dyn(lps * min(NS - 2, n_slabs - 1 - kt));
-        // the stage consumed in the previous iteration is free: everybody is past the barrier
-        if (kt + NS - 1 < n_slabs) ld.issue(lds + fill_off, rot(kt + NS - 1));
-        if constexpr (COMPUTE) {
-            const char *cur = lds + cur_off;
-            const char *tok = cur + tok_region;
-            const char *wgt = cur + w_off;
-            {
-                const uint32_t *sc = reinterpret_cast<const uint32_t *>(cur + scale_off);
-                const uint32_t *tok_sc = sc + tok_region / RB, *w_sc = sc + scale_tok_rows;
-                if constexpr (RB == 64) {
-                    // start is even: the parity of kt is the parity of the slab inside its 128-wide K tile
-                    mma_fp8_step<RB, NTF, TRANSPOSED>(acc, tok, wgt, tok_sc, w_sc, wrow, lane, 0,
-                                                      8 * (2 * (kt & 1) + (lane >> 5)));
-                } else {
+    auto next = [&](int off) { return off + SB >= NS * SB ? 0 : off + SB; };
+    open(0);
+    if constexpr (COMPUTE) {
+        const int r = lane & 31, half = lane >> 5, sh = 8 * half;
+        const int off0 = r * RB + ((half ^ swz<RB>(r)) << 4);
+        const int w_at[2] = {lay.w_off + wrow[0] * RB, lay.w_off + wrow[1] * RB};
+        const int tok_sc_at = lay.scale_off + (tok_region / RB + r) * 4;
+        const int w_sc_at[2] = {lay.scale_off + (lay.scale_tok_rows + wrow[0] + r) * 4,
+                                lay.scale_off + (lay.scale_tok_rows + wrow[1] + r) * 4};
+        auto read_a = [&](Operands<NTF> &o, int f, const char *st, int j) { o.a[f] = lds_frag(st + w_at[f], off0 ^ (64 * j)); };
+        auto read_b = [&](Operands<NTF> &o, int t, const char *st, int j) { o.b[t] = lds_frag(st + tok_region + t * 32 * RB, off0 ^ (64 * j)); };
+        auto read_sa = [&](Operands<NTF> &o, int f, const char *st) { o.sa[f] = *reinterpret_cast<const int *>(st + w_sc_at[f]); };
+        auto read_sb = [&](Operands<NTF> &o, int t, const char *st) { o.sb[t] = *reinterpret_cast<const int *>(st + tok_sc_at + 128 * t); };
+        if constexpr (NTF <= 2) {
+            for (int kt = 0; kt < n_slabs; ++kt) {
+                const char *st = lds + cur_off;
+                Operands<NTF> o[2];
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        mma_fp8_step<RB, NTF, TRANSPOSED>(acc, tok, wgt, tok_sc, w_sc, wrow, lane, j,
-                                                          8 * (2 * j + (lane >> 5)));
+                for (int f = 0; f < 2; ++f) {
+                    read_sa(o[0], f, st);
+                    read_a(o[0], f, st, 0);
                 }
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) {
+                    read_sb(o[0], t, st);
+                    read_b(o[0], t, st, 0);
+                }
+#pragma unroll
+                for (int f = 0; f < 2; ++f) read_a(o[1], f, st, 1);
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) read_b(o[1], t, st, 1);
+                refill(kt, cur_off);
+#pragma unroll
+                for (int f = 0; f < 2; ++f) o[0].sa[f] = o[1].sa[f] = (int)((uint32_t)o[0].sa[f] >> sh);
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) {
+                    o[0].sb[t] = o[1].sb[t] = (int)((uint32_t)o[0].sb[t] >> sh);
+                    mma<NTF, 0, 0>(acc, o[0], t);
+                    mma<NTF, 0, 1>(acc, o[0], t);
+                }
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) {
+                    mma<NTF, 1, 0>(acc, o[1], t);
+                    mma<NTF, 1, 1>(acc, o[1], t);
+                }
+                cur_off = next(cur_off);
+                if (kt + 1 < n_slabs) open(kt + 1);
+            }
+        } else {
+            Operands<NTF> o;
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                read_a(o, f, lds + cur_off, 0);
+                read_sa(o, f, lds + cur_off);
+            }
+#pragma unroll
+            for (int t = 0; t < NTF; ++t) {
+                read_b(o, t, lds + cur_off, 0);
+                read_sb(o, t, lds + cur_off);
+            }
+            // step 0 of the slab in stage `st`: the operands are replaced as they are used up by those of step 1
+            auto step0 = [&](const char *st) {
+                o.sa[0] = (int)((uint32_t)o.sa[0] >> sh);
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) {
+                    o.sb[t] = (int)((uint32_t)o.sb[t] >> sh);
+                    mma<NTF, 0, 0>(acc, o, t);
+                    PMOE_RING_FENCE();
+                }
+                read_a(o, 0, st, 1);
+                o.sa[1] = (int)((uint32_t)o.sa[1] >> sh);
+                PMOE_RING_FENCE();
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) {
+                    mma<NTF, 0, 1>(acc, o, t);
+                    read_b(o, t, st, 1);
+                    PMOE_RING_FENCE();
+                }
+                read_a(o, 1, st, 1);
+                PMOE_RING_FENCE();
+            };
+            for (int kt = 0; kt < n_slabs - 1; ++kt) {
+                step0(lds + cur_off);
+                const bool fill = kt + NS < n_slabs;
+                char *fill_st = lds + cur_off;
+                const int fslab = rot(fill ? kt + NS : 0);
+                if (fill) all_read();
+                auto copies = [&](int c0, int c1) {
+                    if (fill) {
+#pragma unroll
+                        for (int c = 0; c < Loader<RB>::kPieces; ++c)
+                            if (c >= c0 && c < c1) ld.issue_piece(c, fill_st, fslab);
+                    }
+                    PMOE_RING_FENCE();
+                };
+                constexpr int W = Loader<RB>::kWPieces, P = Loader<RB>::kPieces - W;
+                cur_off = next(cur_off);
+                const char *st = lds + cur_off;
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) {
+                    mma<NTF, 1, 0>(acc, o, t);
+                    copies(t * W / NTF, (t + 1) * W / NTF);
+                }
+                wait_and_barrier_dyn(lps * min(NS - 2, n_slabs - 2 - kt) + (fill ? W : 0));
+                read_a(o, 0, st, 0);
+                read_sa(o, 0, st);
+                PMOE_RING_FENCE();
+#pragma unroll
+                for (int t = 0; t < NTF; ++t) {
+                    mma<NTF, 1, 1>(acc, o, t);
+                    read_b(o, t, st, 0);
+                    read_sb(o, t, st);
+                    copies(W + t * P / NTF, W + (t + 1) * P / NTF);
+                }
+                read_a(o, 1, st, 0);
+                read_sa(o, 1, st);
+                PMOE_RING_FENCE();
+            }
+            step0(lds + cur_off);
+#pragma unroll
+            for (int t = 0; t < NTF; ++t) {
+                mma<NTF, 1, 0>(acc, o, t);
+                mma<NTF, 1, 1>(acc, o, t);
             }
         }
-        fill_off = cur_off;
-        cur_off += SB;
-        if (cur_off >= NS * SB) cur_off = 0;
+        // the sums are complete here: the compiler would move matrix instructions into the branches of the epilogue
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int t = 0; t < NTF; ++t) asm volatile("" : "+v"(acc[f][t]));
+    } else {
+        for (int kt = 0; kt < n_slabs - 1; ++kt) {
+            refill(kt, cur_off);
+            cur_off = next(cur_off);
+            open(kt + 1);
+        }
     }
     __syncthreads();  // all reads of the last stages are done: the ring may be reused as scratch
 }

@@ -261,6 +261,45 @@ def test_validation_errors(device):
         call(xs=shifted)
 
 
+@pytest.mark.parametrize("K,N,per,split", [
+    (256, 256, 0, True),     # two slabs up, one down
+    (512, 512, 0, False),    # as many slabs as the rings of one-fragment tiles have stages; two down
+    (768, 768, 2, True),     # an odd number of slabs; tiles in a row, with all stages of the next one filled ahead
+    (1280, 2048, 3, False),  # more slabs than stages in every ring
+])
+def test_ring_at_fragment_and_slab_edges(K, N, per, split, device):
+    """Row tiles of one and two blocks with 1 to 8 live fragments of 32 rows, each on rings of its own depth."""
+    import prime_moe
+    from prime_moe import _native
+    counts = [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 257, 385]
+    counts[-1] += sum(counts) % 2
+    E = len(counts)
+    ids, wts = _routing_by_counts(counts, 2, device, seed=K)
+    T = ids.shape[0]
+    assert 2 * T > 64 * E  # the rule of the dispatch: with a schedule
+    g, a, deq = _quantised_inputs(T, K, E, N, device, seed=N)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    outs = []
+    try:
+        _native.load().pmoe_set_tiles_per_workgroup(per)
+        for _ in range(2):
+            torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+            out = torch.zeros((T, K), dtype=torch.bfloat16, device=device)
+            prime_moe.fused_moe_mxfp8(a["x"], a["x_scales"], a["w1"], a["w1_scales"], a["w2"], a["w2_scales"], *sched, wts,
+                                      out, 2, 128, 64, 4, 2, 1, split)
+            outs.append(out)
+    finally:
+        _native.load().pmoe_set_tiles_per_workgroup(0)
+    torch.cuda.synchronize()
+    ref, bound = O.fused_moe_dense(deq["x"], deq["w1"], deq["w2"], ids.cpu(), wts.cpu(), act_mx=True,
+                                   flip_delta=MX_FLIP_DELTA)
+    got = outs[0].float().cpu()
+    assert torch.isfinite(got).all()
+    assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
+    mx_elementwise_gates(got, ref, bound)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("per", [2, 3, 16])
 @pytest.mark.parametrize("T,K,E,N,top_k", [
     (300, 1280, 4, 1280, 2),   # wide tiles of every kind; 5 up and 5 down weight tiles (not a multiple of 2 or 3)
