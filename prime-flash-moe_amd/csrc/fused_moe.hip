@@ -844,13 +844,14 @@ static thread_local int g_tiles_per_wg = 0;
 
 // A workgroup of the mxfp8 kernels can keep its token rows and take several weight tiles in a row: it
 // saves the set-up of all but the first and starts each tile's copies under the epilogue of the one
-// before, but the coarser work balances worse over the CUs.  Measured on the DeepSeek-V3-like prefill
-// and decode shapes: two tiles gain 3 % on the down kernel (16 slabs per tile), nothing on the up kernel
-// (56 slabs per tile), more than two lose on both.  So: two for the down kernel when that still leaves
-// 8 rounds of workgroups per CU, one otherwise.
+// before, but the coarser work balances worse over the CUs.  Two tiles when that leaves enough rounds of workgroups
+// per CU: 8 for the down kernel, whose tiles are short, 32 for the up kernel (blocks are paired to row tiles, hence
+// 16 and 64 in terms of blocks).  Two against one tile, K = N = 2048 on 32 experts: down 137 / 145 us at 12000 tokens,
+// 1272 / 1390 at 131072; up 985 / 994 at 65536 tokens (64 per CU), 1893 / 1992 at 131072, but 401 / 394 at 24593 and
+// 234 / 224 at 12000; DeepSeek-V3-like prefill (32 per CU): down 3 % faster, up equal.  Four or eight lose on both.
 static int tiles_per_workgroup(bool down, int n_blocks, int n_wt) {
     if (g_tiles_per_wg > 0) return std::min(g_tiles_per_wg, n_wt);
-    return (down && (int64_t)n_blocks * n_wt >= (int64_t)resident_grid() * 16) ? 2 : 1;
+    return (int64_t)n_blocks * n_wt >= (int64_t)resident_grid() * (down ? 16 : 64) ? std::min(2, n_wt) : 1;
 }
 
 void launch_finalize(const MoeArgs &a, void *out, int split, int n_wt_down, hipStream_t s) {
