@@ -10,6 +10,7 @@
 // accumulated with atomics and every sum has a fixed order: the result is a pure function of the inputs.
 #include <algorithm>
 
+#include "align_sort.h"
 #include "moe_pipeline.h"
 #include "moe_stream.h"
 #include "moe_tall.h"
@@ -82,16 +83,17 @@ __device__ __forceinline__ int choose_tiles(int t_min, int t_cap, int f2, int n_
 //  1. runs of blocks with one expert (a thread per block, block-wide scans per 1024 blocks); the thread of a run's
 //     last block reads that block's 128 ids for the last row that holds a pair: the run has f2 pairs of fragments;
 //  2. per kernel the number of row tiles (see choose_tiles);
-//  3. the runs in the order of falling f2 (a counting sort; runs of one size in the order their threads arrive,
-//     which only moves equal tiles in the schedule): the walk of a kernel then ends with the small tiles, and
-//     what is left over when the CUs run out of jobs is short;
+//  3. the runs in the order of falling f2, runs of one size in their own order (a stable counting sort: a job's place in
+//     the walk sets where its K loop starts, so places given in order of arrival would change the last bits of
+//     the result from call to call): the walk of a kernel then ends with the small tiles, and what is left over
+//     when the CUs run out of jobs is short;
 //  4. the tiles of the two cuts (a run gets the tiles it needs at 6 pairs a tile, and the largest runs one more
 //     each until the chosen number is reached), then the plans with the split of the tails.
 // The list of runs lives in LDS (in the workspace when there are more than kLdsRuns blocks).
 // All workgroups invert the sorted order: inv[pair id] = sorted row.  Entries of pairs that are not in the
 // schedule keep whatever the buffer held; the reader validates an entry against sorted_ids.
 constexpr int kLdsRuns = 2048;
-constexpr int kSizeKeys = 128;  // runs are ordered by min(f2, kSizeKeys - 1)
+constexpr int kSizeKeyBits = 7, kSizeKeys = 1 << kSizeKeyBits;  // runs are ordered by min(f2, kSizeKeys - 1)
 __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel_bf16(MoeArgs a, int n_wt_up, int n_wt_down, int n_cus,
                                                                 int do_invert) {
     const int n_pairs = a.M * a.top_k;
@@ -100,7 +102,7 @@ __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel_bf16(Moe
         __shared__ int s_order[kLdsRuns];
         __shared__ int s_part[kPrologueThreads / 64], s_carry[2], s_want[2], s_tiles[2];
         __shared__ int s_sum[8];            // [0]: tiles of up to 6 pairs the runs need; [4]: pairs of fragments
-        __shared__ int s_hist[kSizeKeys];   // runs per size key, then the first place of each key in the order
+        __shared__ int s_hist[kSizeKeys];   // runs per size key, then the next place of each key in the order
         const int tid = threadIdx.x;
         const int n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
         int4 *runs = n_live <= kLdsRuns ? s_runs : a.runs;
@@ -175,14 +177,16 @@ __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel_bf16(Moe
         }
         const int n_runs = s_carry[1];
         __threadfence_block();
-        // 2. the number of row tiles of each kernel: tid 0 the up kernel's, tid 1 the down kernel's
-        if (tid < 2) {
-            const int n_wt = tid ? n_wt_down : n_wt_up, n_slabs = (tid ? a.H : a.K) * 2 / tall::kRB;
-            s_want[tid] = choose_tiles(s_sum[0], a.n_blocks, s_sum[4], n_wt, n_slabs, n_cus);
+        // 2. the number of row tiles of each kernel: thread 64 the up kernel's, thread 65 the down kernel's (a wave
+        // that has no part in step 3)
+        if ((tid & ~1) == 64) {
+            const int down = tid & 1;
+            const int n_wt = down ? n_wt_down : n_wt_up, n_slabs = (down ? a.H : a.K) * 2 / tall::kRB;
+            s_want[down] = choose_tiles(s_sum[0], a.n_blocks, s_sum[4], n_wt, n_slabs, n_cus);
         }
-        // 3. order of the runs: by falling size key, runs of one key in their own order.  First place of each key ...
+        // 3. order of the runs, by one wave: the first place of each key, then every run takes the next place of its key
         if (tid < 64) {
-            // (one wave: key k's place = runs with a larger key; two keys per lane, largest keys first)
+            // (key k's place = runs with a larger key; two keys per lane, largest keys first)
             const int k_hi = kSizeKeys - 1 - 2 * tid, k_lo = k_hi - 1;
             const int c_hi = s_hist[k_hi], c_lo = s_hist[k_lo];
             int incl = c_hi + c_lo;
@@ -193,10 +197,14 @@ __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel_bf16(Moe
             }
             s_hist[k_hi] = incl - c_hi - c_lo;
             s_hist[k_lo] = incl - c_lo;
+            for (int base = 0; base < n_runs; base += 64) {
+                const int i = base + tid;
+                const int key[1] = {i < n_runs ? min(runs[i].y, kSizeKeys - 1) : -1};
+                int place[1];
+                align::rank_ids<1>(key, place, s_hist, kSizeKeys, kSizeKeyBits, tid);
+                if (i < n_runs) order[place[0]] = i;
+            }
         }
-        __syncthreads();
-        // ... then every run takes the next place of its key
-        for (int i = tid; i < n_runs; i += kPrologueThreads) order[atomicAdd(&s_hist[min(runs[i].y, kSizeKeys - 1)], 1)] = i;
         __syncthreads();
         __threadfence_block();
         // 4. the tiles of the two cuts (one pass when both kernels use the same cut), and the plans

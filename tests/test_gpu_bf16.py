@@ -265,3 +265,65 @@ def test_few_jobs_deep_split_and_join_kernel(T, K, E, N, top_k, exact, device):
         outs.append(out)
     torch.cuda.synchronize()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+def _tall_plan(x, w1, w2, sched, wts, out, top_k):
+    """(number of row tiles, the up kernel's table of row tiles) that the prologue of the tall-tile path builds.
+    The workspace starts with the plan, the run list and the table (bf16_workspace in csrc/fused_moe_bf16.hip)."""
+    from prime_moe import _native
+    lib = _native.load()
+    (M, K), (E, N, _) = x.shape, w1.shape
+    s, e, n = sched
+    nbytes = lib.pmoe_fused_moe_bf16_workspace_bytes(M, K, N, E, s.numel(), top_k, 1)
+    ws = torch.zeros((nbytes,), dtype=torch.uint8, device=x.device)
+    try:
+        lib.pmoe_set_phase_mask(1)  # the prologue alone
+        _native.check(lib.pmoe_fused_moe_bf16(
+            x.data_ptr(), w1.data_ptr(), w2.data_ptr(), out.data_ptr(), s.data_ptr(), e.data_ptr(), n.data_ptr(),
+            wts.data_ptr(), top_k, M, K, N, E, s.numel(), 128, 64, 4, 2, 1, 1, 1, ws.data_ptr(), nbytes,
+            torch.cuda.current_stream().cuda_stream))
+    finally:
+        lib.pmoe_set_phase_mask(15)
+    torch.cuda.synchronize()
+    up = lambda b: (b + 255) // 256 * 256
+    at = 256 + up((s.numel() // 128 + 1) * 20)
+    n_tiles = int(ws[:4].view(torch.int32)[0])
+    return n_tiles, ws[at:at + 16 * n_tiles].view(torch.int32).view(-1, 4)[:, :3].cpu()
+
+
+@pytest.mark.parametrize("E", [130, 1000, 1024])
+def test_row_tiles_of_one_size_keep_their_order(E, device):
+    """The place of a row tile decides where the K loops of its jobs start, that is the order of their sums: tiles of
+    one size come in the order of the schedule, whichever wave of the prologue is first."""
+    from test_gpu_mxfp8 import _routing_by_counts
+    K, N, top_k = 128, 256, 2
+    counts = [36 if e % 3 else 100 for e in range(E)]  # one and two pairs of fragments
+    counts[-1] += sum(counts) % 2
+    ids, wts = _routing_by_counts(counts, top_k, device, seed=E)
+    T = ids.shape[0]
+    assert T * top_k > 32 * E and E >= 128  # the rule of the dispatch: tall tiles
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=E)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    want = [[4 * e, 2 - (c <= 64), e] for e, c in enumerate(counts)]
+    want.sort(key=lambda t: (-t[1], t[0]))
+    for _ in range(4):
+        n_tiles, tiles = _tall_plan(x, w1, w2, sched, wts, out, top_k)
+        assert n_tiles == E
+        assert torch.equal(tiles, torch.tensor(want, dtype=torch.int32))
+
+
+def test_many_tiles_of_one_size_are_bitwise_reproducible(device):
+    import prime_moe
+    T, K, E, N, top_k = 640, 2048, 128, 512, 8
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=4)
+    ids = torch.topk(torch.randn((T, E), device=device, generator=g), top_k).indices.to(torch.int32).contiguous()
+    wts = torch.softmax(torch.randn((T, top_k), device=device, generator=g), -1)
+    assert T * top_k > 32 * E  # tall tiles
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    first = None
+    for _ in range(20):
+        out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, top_k, 128, 64, 4, 2, 1, 1, True)
+        first = out if first is None else first
+        assert torch.equal(first.view(torch.int16), out.view(torch.int16))
