@@ -7,6 +7,8 @@
 //
 // In C++ because the calls a decode step makes are short: checks, allocations and ctypes in Python cost 25 - 30 us a
 // call, which the device spends less than on a single token.
+#include <limits>
+
 #include <torch/csrc/utils/pybind.h>
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -82,12 +84,17 @@ void check_tuning(const char *what, int64_t block_m, int64_t block_n, int64_t wa
 
 // ------------------------------------------------------------------------------- moe_align
 
-// (pad_to, max_padded, max_blocks) as torch_interface.cpp:88-91 computes them.
+// (pad_to, max_padded, max_blocks) as torch_interface.cpp:88-91 computes them.  Ids, positions and sizes are int32 in the
+// kernels and the C ABI: what does not fit is an error here (block_m, bpc > 0, num_experts <= 1024: no step overflows).
 struct AlignSizes {
     int64_t pad_to, max_padded, max_blocks;
     AlignSizes(int64_t n, int64_t num_experts, int64_t block_m, int64_t bpc) {
+        constexpr int64_t kMax = std::numeric_limits<int32_t>::max();
+        REQUIRE(n <= kMax, "moe_align: ", n, " ids do not fit 32 bits");
+        REQUIRE(block_m <= kMax && bpc <= kMax / block_m, "moe_align: block_m * bpc does not fit 32 bits (", block_m, " * ", bpc, ")");
         pad_to = block_m * bpc;
         max_padded = (n + num_experts * (pad_to - 1) + pad_to - 1) / pad_to * pad_to;
+        REQUIRE(max_padded <= kMax, "moe_align: a schedule of ", max_padded, " rows does not fit 32 bits");
         max_blocks = max_padded / block_m;
     }
 };
@@ -99,6 +106,7 @@ void validate_align(const Tensor &topk_ids, int64_t num_experts, int64_t block_m
     REQUIRE(topk_ids.scalar_type() == at::kInt, "moe_align: topk_ids must be int32");
     REQUIRE(block_m > 0 && bpc > 0 && num_experts > 0, "moe_align: block_m, bpc and num_experts must be positive");
     REQUIRE(num_experts <= 1024, "moe_align supports at most 1024 experts, got ", num_experts);
+    AlignSizes(topk_ids.numel(), num_experts, block_m, bpc);
 }
 
 struct Schedule {

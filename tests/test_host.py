@@ -214,6 +214,19 @@ def test_align_validation_and_sizes():
             prime_moe._validate_align(*a, placement=False)
 
 
+@pytest.mark.parametrize("block_m,bpc", [
+    (1 << 32, 1 << 32),        # the product wraps to 0 in 64 bits
+    (1 << 62, 4), (1 << 33, 1 << 30), ((1 << 32) + 128, 1), (1 << 16, 1 << 15),
+    (1 << 30, 1),              # the product fits, 4 experts' padding does not
+])
+def test_align_sizes_beyond_32_bits_are_an_error(block_m, bpc):
+    import prime_moe
+    ok = torch.zeros((8,), dtype=torch.int32)
+    with pytest.raises(RuntimeError, match="32 bits"):
+        prime_moe._validate_align(ok, 4, block_m, bpc, placement=False)
+    prime_moe._validate_align(ok, 4, 1 << 20, 1 << 8, placement=False)
+
+
 def test_ops_refuse_cpu_tensors():
     import prime_moe
     with pytest.raises((NotImplementedError, RuntimeError)):
