@@ -15,8 +15,6 @@ three ops trace), :func:`quantize_mx`, the OCP-MX quantiser in front of the mxfp
 """
 from __future__ import annotations
 
-import os
-
 import torch
 
 BLOCK = 32  # MX scale block size
@@ -40,15 +38,22 @@ try:
     # host side of the ops (csrc/torch_ops.cpp): registers their CUDA-key implementations, does the argument checks
     from . import _torch_ops
 except ImportError as _err:
-    if os.path.exists(os.path.join(os.path.dirname(os.path.abspath(__file__)), "_torch_ops.so")):
-        raise
+    # Not built, or built against another torch or library: the package still imports (its build module has to), and
+    # everything that needs the native code raises.
+    class _Unavailable:
+        def __init__(self, reason):
+            self._reason = reason
 
-    class _NotBuilt:
+        def _raise(self, *args, **kwargs):
+            raise RuntimeError(f"prime_moe: _torch_ops.so cannot be loaded ({self._reason}). Build the native code "
+                               "first: python prime-flash-moe_amd/prime_moe/build.py (there is no fallback path).")
+
         def __getattr__(self, name):
-            raise RuntimeError("prime_moe: _torch_ops.so is missing. Build the native code first: "
-                               "python prime-flash-moe_amd/prime_moe/build.py (there is no fallback path).")
+            return self._raise
 
-    _torch_ops = _NotBuilt()
+    _torch_ops = _Unavailable(str(_err))
+    for _op in ("moe_align", "fused_moe_bf16", "fused_moe_mxfp8"):
+        _LIB.impl(_op, _torch_ops._raise, "CUDA")
 
 
 # ------------------------------------------------------------------------------- moe_align

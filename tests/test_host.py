@@ -79,6 +79,44 @@ def test_missing_library_fails_loudly(monkeypatch):
         _native.load()
 
 
+@pytest.mark.parametrize("state", ["not built", "library missing", "not a library"])
+def test_package_without_native_code_imports_and_every_call_raises(state, tmp_path):
+    """`python -m prime_moe.build` imports the package first: it has to work in every state that a build repairs."""
+    import shutil
+    import subprocess
+    import sys
+    src = os.path.join(ROOT, "prime-flash-moe_amd", "prime_moe")
+    pkg = tmp_path / "prime_moe"
+    pkg.mkdir()
+    for f in os.listdir(src):
+        if f.endswith(".py"):
+            shutil.copy(os.path.join(src, f), pkg / f)
+    if state == "library missing":  # _torch_ops.so finds libprime_moe_hip.so next to itself only
+        shutil.copy(os.path.join(src, "_torch_ops.so"), pkg / "_torch_ops.so")
+    elif state == "not a library":
+        (pkg / "_torch_ops.so").write_bytes(b"not an ELF file")
+    code = """
+import torch, prime_moe, prime_moe.build
+ids = torch.zeros((8,), dtype=torch.int32)
+calls = [lambda: prime_moe.route(torch.zeros((2, 4)), 2), lambda: prime_moe.quantize_mx(torch.zeros((2, 32))),
+         lambda: prime_moe._validate_align(ids, 4, 128, 1, False)]
+for op in ("moe_align", "fused_moe_bf16", "fused_moe_mxfp8"):
+    assert torch._C._dispatch_has_kernel_for_dispatch_key("prime_moe::" + op, "CUDA")
+    calls.append(lambda: prime_moe._torch_ops._raise())
+for call in calls:
+    try:
+        call()
+    except RuntimeError as err:
+        assert "build.py" in str(err) and "no fallback" in str(err), err
+    else:
+        raise AssertionError("no error")
+print("fine")
+"""
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=tmp_path,
+                         env={**os.environ, "PYTHONPATH": str(tmp_path)})
+    assert res.returncode == 0 and "fine" in res.stdout, res.stderr[-2000:]
+
+
 def test_schemas_match_reference_surface():
     import prime_moe  # noqa: F401
     s = str(torch.ops.prime_moe.fused_moe_bf16.default._schema)
