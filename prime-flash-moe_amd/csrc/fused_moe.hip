@@ -683,7 +683,8 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
 template <bool UP>
 __global__ __launch_bounds__(512, 4) void moe_stream_kernel_mx(MoeArgs a, int n_tiles) {
     __shared__ __attribute__((aligned(1024))) stream::Shared sh;
-    stream::for_each_job<UP>(a, n_tiles, [&](int blk, int e, int tile, int id) { stream::mx_run_job<UP>(a, sh, blk, e, tile, id); });
+    stream::for_each_job<UP>(a, n_tiles, [](int) { return false; },
+                             [&](int blk, int e, int tile, int id) { stream::mx_run_job<UP>(a, sh, blk, e, tile, id); });
 }
 
 // Down GEMM for H = RB without a prologue (see stream::for_each_turn).

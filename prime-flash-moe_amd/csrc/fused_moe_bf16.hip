@@ -17,6 +17,43 @@
 
 namespace pmoe {
 
+// Crowded schedules.  Whether the streaming kernels (moe_stream.h) are the faster ones is a matter of the rows per
+// block, and the host, which enqueues them when there are few rows per expert on average, does not know how the
+// tokens are spread: with all of them on a few experts a block is full, its weights are read once per 64 rows, and the
+// short down kernel reads the activation once per 32 columns.  The length of the schedule tells: `pairs` rows on
+// n_live blocks.  So where crowding can matter (crowding_possible), both kinds of kernels are enqueued and decide by
+// this function, the same in all of them, which of them works: bit 0 the up kernel, bit 1 the down kernel is a tall one.
+//  * up, and down with H > 256: more than 64 rows per live block, that is, more than one pass over most weights, and enough
+//    bytes in a pass that the prologue (8 us) is small against it;
+//  * down with H <= 256: the fragments of 32 rows beyond the first of a block cost a pass over its rows of W2 each.
+// Streaming / tall / as decided here, us, whole op.  K 2048, N 1536, 512 tokens x top 8 on 85 of 128 experts (48 rows per
+// block): 188 / 199 / 194, on 64: 168 / 163 / 175, on 51: 188 / 152 / 155, on 21: 138 / 85 / 91; K 4096, N 28672, 128 x 2 on
+// 4 of 8 (64 rows): 400 / 419 / 406, on 3: 423 / 342 / 348; K 7168, N 512, 900 x 9 on all 257 (31 rows): 662 / 659 / 630,
+// on 63: 532 / 246 / 233, 256 x 9 on 57 (40 rows): 169 / 199 / 162.
+// The kernels that are enqueued and find nothing to do cost 2 us each, so they are enqueued where crowding would cost more:
+// an expert has at most M rows (more only if a token names it twice, which is not looked for), M <= 64 is one pass.
+constexpr float kCrowdedUpBytes = 64e6f, kCrowdedDownBytes = 96e6f;
+__device__ __forceinline__ int crowding(const MoeArgs &a, int ntpp) {
+    if (!a.crowd) return 0;
+    const float n_live = (float)min((ntpp + kBlockRows - 1) / kBlockRows, a.n_blocks);
+    if (n_live < 1.f) return 0;
+    const float rows = (float)(a.M * a.top_k) / n_live, w2_bytes = 2.f * (float)a.K * (float)a.H;
+    int tall = rows > 64.f && n_live * 2.f * w2_bytes >= kCrowdedUpBytes ? 3 : 0;
+    if (a.H <= 256) {
+        // rows of a block spread round the mean: the second fragment appears from 24 rows on
+        const float extra = fminf((rows - 24.f) * (1.f / 16.f), rows * (1.f / 32.f) - 0.5f);
+        if (n_live * extra * w2_bytes >= kCrowdedDownBytes) tall |= 2;
+    }
+    return tall & a.crowd;
+}
+// The tall kernels to enqueue (bits as in crowding()).
+static int crowding_possible(const MoeArgs &a) {
+    const double pairs = (double)a.M * a.top_k, w2_bytes = 2.0 * a.K * a.H;
+    int tall = a.M > 64 && pairs / 64 * 2 * w2_bytes >= 2 * kCrowdedUpBytes ? 3 : 0;
+    if (a.H <= 256 && a.M > 24 && 0.75 * pairs / 32 * w2_bytes >= kCrowdedDownBytes) tall |= 2;
+    return tall;
+}
+
 constexpr int kPrologueThreads = 1024;
 // Inclusive scan of one int per thread over the workgroup of the prologue; `s_part` holds an int per wave.
 __device__ __forceinline__ int block_scan(int v, int *s_part) {
@@ -96,6 +133,7 @@ constexpr int kLdsRuns = 2048;
 constexpr int kSizeKeyBits = 7, kSizeKeys = 1 << kSizeKeyBits;  // runs are ordered by min(f2, kSizeKeys - 1)
 __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel_bf16(MoeArgs a, int n_wt_up, int n_wt_down, int n_cus,
                                                                 int do_invert) {
+    if (a.crowd && crowding(a, a.ntpp[0]) == 0) return;
     const int n_pairs = a.M * a.top_k;
     if (blockIdx.x == 0) {
         __shared__ int4 s_runs[kLdsRuns];  // {first block, f2, expert, 0}
@@ -497,6 +535,7 @@ __device__ __forceinline__ void walk_queue(const KernelPlan &kp, const int4 *til
 
 __global__ __launch_bounds__(512) void moe_up_kernel_bf16(MoeArgs a) {
     __shared__ __attribute__((aligned(1024))) char lds[tall::kLdsBytes];
+    if (a.crowd && !(crowding(a, a.ntpp[0]) & 1)) return;
     const KernelPlan kp = a.plan->up;
     int *counter = &a.plan->counters[blockIdx.x & 7];
     bool pre = false;
@@ -658,6 +697,7 @@ __device__ __forceinline__ void down_tile_tall(const MoeArgs &a, const KernelPla
 
 __global__ __launch_bounds__(512) void moe_down_kernel_bf16(MoeArgs a) {
     __shared__ __attribute__((aligned(1024))) char lds[tall::kLdsBytes];
+    if (a.crowd && !(crowding(a, a.ntpp[0]) & 2)) return;
     const KernelPlan kp = a.plan->down;
     int *counter = &a.plan->counters[8 + (blockIdx.x & 7)];
     bool pre = false;
@@ -677,13 +717,15 @@ __global__ __launch_bounds__(512) void moe_down_kernel_bf16(MoeArgs a) {
 template <bool UP, int U>
 __global__ __launch_bounds__(512, 4) void moe_stream_kernel(MoeArgs a, int n_tiles) {
     __shared__ __attribute__((aligned(1024))) stream::Shared sh;
-    stream::for_each_job<UP>(a, n_tiles, [&](int blk, int e, int tile, int id) { stream::run_job<UP, U>(a, sh, blk, e, tile, id); });
+    stream::for_each_job<UP>(a, n_tiles, [&](int ntpp) { return (crowding(a, ntpp) & (UP ? 1 : 2)) != 0; },
+                             [&](int blk, int e, int tile, int id) { stream::run_job<UP, U>(a, sh, blk, e, tile, id); });
 }
 
 // Down GEMM of the streaming path for H = RB / 2 (see stream::for_each_turn).
 template <int RB>
 __global__ __launch_bounds__(256, RB == 256 ? 4 : 2) void moe_stream_down_short_kernel(MoeArgs a) {
     __shared__ __attribute__((aligned(1024))) char bufs[4][stream::ShortDown<RB>::kBytes];
+    if (a.crowd && (crowding(a, a.ntpp[0]) & 2)) return;
     stream::ShortDown<RB> eng(a, bufs[__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)]);
     stream::for_each_turn(a, a.K / 32, eng);
 }
@@ -703,8 +745,11 @@ static bool use_stream(const MoeArgs &a) {
 }
 
 static int launch_stream_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
-    const int mask = phase_mask();
-    const int n_wgs = 2 * resident_grid();
+    const int mask = phase_mask(), n_cus = resident_grid();
+    const int n_wgs = 2 * n_cus;
+    const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
+    const int tall = a.n_blocks > 0 ? crowding_possible(a) : 0;
+    a.crowd = tall;
     // units of 32 weight rows a job takes: two when that still leaves a job for every workgroup
     const int64_t blocks = std::min<int64_t>(a.n_blocks, std::min<int64_t>(a.E, (int64_t)a.M * a.top_k));
     auto launch = [&](auto one, auto two, int units) {
@@ -715,14 +760,23 @@ static int launch_stream_pipeline(MoeArgs a, void *out, int split, hipStream_t s
     };
     if (mask & PMOE_PHASE_UP) launch(moe_stream_kernel<true, 1>, moe_stream_kernel<true, 2>, a.H / 16);
     else if (mask & PMOE_PHASE_PROLOGUE) launch(moe_stream_kernel<true, 1>, moe_stream_kernel<true, 2>, 0);
+    if (tall) {
+        MoeArgs t = a;
+        t.deep_ok = 0;
+        hipLaunchKernelGGL(moe_prologue_kernel_bf16, dim3(1), dim3(kPrologueThreads), 0, s, t, n_wt_up, n_wt_down, n_cus, 0);
+        t.n_wtiles = n_wt_up;
+        if ((tall & 1) && (mask & PMOE_PHASE_UP)) hipLaunchKernelGGL(moe_up_kernel_bf16, dim3(n_cus), dim3(512), 0, s, t);
+        t.n_wtiles = n_wt_down;
+        if (mask & PMOE_PHASE_DOWN) hipLaunchKernelGGL(moe_down_kernel_bf16, dim3(n_cus), dim3(512), 0, s, t);
+    }
     if ((mask & PMOE_PHASE_DOWN) && a.H <= 256 && a.n_blocks > 0) {
-        const int grid = (int)std::min<int64_t>((int64_t)a.n_blocks * (a.K / 128), (a.H == 128 ? 4 : 2) * resident_grid());
+        const int grid = (int)std::min<int64_t>((int64_t)a.n_blocks * (a.K / 128), (a.H == 128 ? 4 : 2) * n_cus);
         if (a.H == 128) hipLaunchKernelGGL(moe_stream_down_short_kernel<256>, dim3(grid), dim3(256), 0, s, a);
         else hipLaunchKernelGGL(moe_stream_down_short_kernel<512>, dim3(grid), dim3(256), 0, s, a);
     } else if (mask & PMOE_PHASE_DOWN) {
         launch(moe_stream_kernel<false, 1>, moe_stream_kernel<false, 2>, a.K / 32);
     }
-    if (mask & PMOE_PHASE_FINALIZE) launch_finalize(a, out, split, (a.K + kWRows - 1) / kWRows, s);
+    if (mask & PMOE_PHASE_FINALIZE) launch_finalize(a, out, split, n_wt_down, s);
     return check_launch("fused_moe_bf16 launch");
 }
 

@@ -237,10 +237,10 @@ __device__ __forceinline__ void invert(const MoeArgs &a, int threads) {
     }
 }
 
-// The jobs of this workgroup: job(block, expert, weight tile, sorted id of this thread's row).  The up kernel also
-// inverts the sorted order.
-template <bool UP, typename Job>
-__device__ __forceinline__ void for_each_job(const MoeArgs &a, int n_tiles, Job job) {
+// The jobs of this workgroup: job(block, expert, weight tile, sorted id of this thread's row), none if skip(length of
+// the schedule).  The up kernel also inverts the sorted order.
+template <bool UP, typename Skip, typename Job>
+__device__ __forceinline__ void for_each_job(const MoeArgs &a, int n_tiles, Skip skip, Job job) {
     const int tid = threadIdx.x, grid = (int)gridDim.x;
     // sorted id (threads 0 .. 127) and expert of a job's block, fetched under the job before; for the first job
     // without waiting for the length of the schedule
@@ -258,6 +258,7 @@ __device__ __forceinline__ void for_each_job(const MoeArgs &a, int n_tiles, Job 
     const int ntpp = a.ntpp[0];
     const int n_jobs = min((ntpp + kBlockRows - 1) / kBlockRows, a.n_blocks) * n_tiles;
     if (UP) invert(a, 512);
+    if (skip(ntpp)) return;
     for (int j = (int)blockIdx.x; j < n_jobs; j += grid) {
         const int blk = j / n_tiles;
         int next_id, next_e;

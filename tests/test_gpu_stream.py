@@ -68,6 +68,43 @@ def test_stream_kernels_with_dropped_rows_and_blocks(device):
         assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
 
 
+@pytest.mark.parametrize("K,N,E,T,top_k,hot,want", [
+    (1024, 768, 168, 1340, 4, 50, 3),    # general down kernel: all pairs on 50 experts, 107 rows each
+    (1024, 768, 168, 1340, 4, 168, 0),   # the same call with its pairs spread out
+    (2048, 512, 150, 1200, 4, 80, 2),    # short down kernel (H = 256): 60 rows per block crowd it, not the up kernel
+    (4096, 256, 150, 1200, 4, 30, 3),    # H = 128, blocks of one expert
+    (7168, 512, 60, 60, 32, 1, 2),       # one expert named 32 times by each token: only the tall down kernel is enqueued
+])
+def test_crowded_schedules_take_the_tall_kernels(K, N, E, T, top_k, hot, want, device):
+    """Few rows per expert on average, all of them on few experts: the kernels decide on the device which of them work
+    (1: the tall up kernel, 2: the tall down kernel), and whichever did, every pair is computed once."""
+    from prime_moe import _native
+    lib = _native.load()
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=K)
+    perm = torch.randperm(E, device=device, generator=g)[:hot].to(torch.int32)
+    pick = torch.randn((T, max(hot, top_k)), device=device, generator=g).topk(top_k).indices % hot
+    ids = perm[pick].contiguous()
+    wts = torch.softmax(torch.randn((T, top_k), device=device, generator=g), -1)
+    assert T * top_k <= 32 * E  # the rule of the dispatch: streaming kernels are enqueued
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    nbytes = lib.pmoe_fused_moe_bf16_workspace_bytes(T, K, N, E, s.numel(), top_k, 1)
+    ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device=device)
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    _native.check(lib.pmoe_fused_moe_bf16(
+        x.data_ptr(), w1.data_ptr(), w2.data_ptr(), out.data_ptr(), s.data_ptr(), e.data_ptr(), n.data_ptr(),
+        wts.data_ptr(), top_k, T, K, N, E, s.numel(), 128, 64, 4, 2, 1, 1, 1, ws.data_ptr(), nbytes,
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    # the plan of the tall kernels: two descriptions of 16 bytes, then the next slot of every queue (8 up, 8 down)
+    up, down = ws[32:96].view(torch.int32).view(2, 8).cpu()
+    first = torch.cuda.get_device_properties(device).multi_processor_count // 8
+    took = (1 if bool((up > first).any()) else 0) | (2 if bool((down > first).any()) else 0)
+    assert took == want
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    got = out.float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
 SPARSE = [129, 65, 64, 33, 32, 5] + [1] * 60
 
 
