@@ -59,6 +59,8 @@ int pmoe_moe_align(const int32_t *topk_ids, int32_t *sorted_token_ids, int32_t *
  * does so (0 for n <= 16384), the second what spreads it as far as it pays (0 for
  * n <= 8192); where a query returns 0 `workspace` may be null, and with a null or too small
  * workspace the call falls back to a single workgroup.  Same output, bit for bit.
+ * A workspace that is not 4-byte aligned is an error where the first query asks for one and
+ * gets it, and not used otherwise.
  */
 size_t pmoe_moe_align_workspace_bytes(int n, int num_experts);
 size_t pmoe_moe_align_workspace_bytes_fast(int n, int num_experts);

@@ -313,12 +313,15 @@ extern "C" int pmoe_moe_align_ws(const int32_t *topk_ids, int32_t *sorted_token_
     hipStream_t s = static_cast<hipStream_t>(stream);
     const Outputs o{sorted_token_ids, expert_ids, num_tokens_post_padded, block_m, pad_to, max_padded, max_blocks};
     if (n > kFewIds && workspace != nullptr) {
+        // A misaligned pointer is an error only where the call cannot do without the scratch it was given for; where the
+        // first query asks for none, or for more than this, it is not looked at.
+        const bool aligned = (reinterpret_cast<uintptr_t>(workspace) & 3) == 0;
+        PMOE_REQUIRE(aligned || n <= kSingleMaxIds || workspace_bytes < pmoe_moe_align_workspace_bytes(n, num_experts),
+                     "moe_align: workspace must be 4-byte aligned");
         // the finest slices whose counts fit the scratch
-        for (int slice = slice_ids(n); slice <= kMaxSliceIds; slice *= 2)
-            if (sizeof(int32_t) * (size_t)n_slices(n, slice) * num_experts <= workspace_bytes) {
-                PMOE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3) == 0, "moe_align: workspace must be 4-byte aligned");
+        for (int slice = slice_ids(n); aligned && slice <= kMaxSliceIds; slice *= 2)
+            if (sizeof(int32_t) * (size_t)n_slices(n, slice) * num_experts <= workspace_bytes)
                 return launch_multi(topk_ids, o, n, num_experts, slice, static_cast<int32_t *>(workspace), s);
-            }
     }
     return launch_single(topk_ids, o, n, num_experts, s);
 }

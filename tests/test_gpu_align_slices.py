@@ -40,6 +40,30 @@ def test_align_at_slice_edges_with_every_scratch(n, E, device):
             np.testing.assert_array_equal(got.cpu().numpy(), want, err_msg=f"{nbytes} bytes of scratch")
 
 
+@pytest.mark.parametrize("n,E,short,refused", [(8193, 37, 0, False), (16384, 8, 0, False), (16385, 8, 4, False), (16385, 8, 0, True)])
+def test_a_misaligned_workspace_is_an_error_only_where_scratch_is_needed(n, E, short, refused, device):
+    """The first query asks for no scratch up to 16384 ids, and a smaller one than it asks for is as good as none: such a
+    pointer may be anything."""
+    import prime_moe
+    from prime_moe import _native
+    lib = _native.load()
+    ids = np.random.default_rng(n).integers(0, E, size=n).astype(np.int32)
+    pad_to, max_padded, max_blocks = prime_moe.align_sizes(n, E, 128, 1)
+    need = lib.pmoe_moe_align_workspace_bytes(n, E)
+    assert (need == 0) == (n <= 16384)
+    nbytes = (need or 1 << 20) - short
+    ws = torch.full((nbytes + 8,), 0x5a, dtype=torch.uint8, device=device)
+    dev_ids = torch.from_numpy(ids).to(device)
+    s, e, t = (torch.empty((c,), dtype=torch.int32, device=device) for c in (max_padded, max_blocks, 1))
+    rc = lib.pmoe_moe_align_ws(dev_ids.data_ptr(), s.data_ptr(), e.data_ptr(), t.data_ptr(), n, E, 128, pad_to, max_padded,
+                               max_blocks, ws.data_ptr() + 1, nbytes, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert (rc != 0) == refused
+    if not refused:
+        for got, want in zip((s, e, t), O.moe_align_fast(ids, E, 128, 1)):
+            np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("T,E,k", [(16, 512, 32), (17, 512, 8), (8, 513, 32), (9, 1024, 4), (16, 64, 32), (2, 33, 32)])
 def test_route_around_the_one_kernel_form(T, E, k, device):
     g = torch.Generator(device=device).manual_seed(T + E + k)
