@@ -46,7 +46,7 @@ __global__ __launch_bounds__(NW * 64) void moe_align_kernel(const int32_t *__res
     sort_in_workgroup<NW, PER>(id, o, E, id_bits, smem);
 }
 
-// ---- many ids: the same sort spread over workgroups, two launches.
+// ---- many ids: the same sort spread over workgroups, two launches (three for very many).
 //   count:   workgroup g counts ids [g S, (g + 1) S) per expert -> counts[g][e]
 //   scatter: every workgroup sums counts[.][e] itself (all slices: totals and the padded prefix; the slices before
 //            its own: its bases), ranks its slice as above and writes pair id i to offs[e] + base + rank; it also
@@ -54,6 +54,8 @@ __global__ __launch_bounds__(NW * 64) void moe_align_kernel(const int32_t *__res
 //            expert_ids.  No slot is written twice and no order between workgroups is needed.
 // Slices are contiguous and ascending in g, waves inside a slice likewise: the order inside an expert is
 // ascending pair id, bit for bit what the single workgroup produces.
+// That reading of all counts by every workgroup grows with the square of the number of slices: above kSelfScanWords
+// a kernel between the two turns counts[.][e] into bases and totals (align_bases_kernel).
 // Ranking is what a slice costs (ballots, a few hundred instructions per 64 ids of a wave), so slices are as small as
 // the scratch allows, from 1024 ids on, up to 64 of them: 65536 ids of 128 experts take 20 us in 8 slices.
 constexpr int kMinSliceIds = 1024, kMaxSliceIds = 8192;
@@ -87,9 +89,44 @@ __global__ __launch_bounds__(NW * 64) void align_count_kernel(const int32_t *__r
     }
 }
 
+// counts[g][e] -> ids of e in the slices before g, for 1 << bits experts per workgroup; their totals -> totals[e].  A
+// thread sums a run of slices, the runs before it come from LDS, and a second pass over its run writes the bases.
+__global__ __launch_bounds__(1024) void align_bases_kernel(int32_t *counts, int32_t *totals, int G, int E, int bits) {
+    __shared__ int32_t sums[1024];
+    constexpr int kBatch = 16;  // loads in flight
+    const int tid = threadIdx.x, cols = 1 << bits, parts = 1024 >> bits, col = tid & (cols - 1), part = tid >> bits;
+    const int e = blockIdx.x * cols + col, per = (G + parts - 1) / parts, end = min((part + 1) * per, G);
+    int sum = 0;
+    if (e < E) {
+#pragma unroll 16
+        for (int s = part * per; s < end; ++s) sum += counts[(size_t)s * E + e];
+    }
+    sums[tid] = sum;
+    __syncthreads();
+    int run = 0, all = 0;
+    for (int p = 0; p < parts; ++p) {
+        const int v = sums[p * cols + col];
+        run += p < part ? v : 0;
+        all += v;
+    }
+    if (e >= E) return;
+    if (part == 0) totals[e] = all;
+    for (int s = part * per; s < end; s += kBatch) {
+        int c[kBatch];
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) c[i] = s + i < end ? counts[(size_t)(s + i) * E + e] : 0;
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            if (s + i < end) counts[(size_t)(s + i) * E + e] = run;
+            run += c[i];
+        }
+    }
+}
+
+// `totals`: counts holds the bases already (align_bases_kernel); null: it holds the counts.
 template <int NW, int PER>
 __global__ __launch_bounds__(NW * 64) void align_scatter_kernel(const int32_t *__restrict__ topk_ids, const int32_t *__restrict__ counts,
-                                                                Outputs o, int n, int E, int id_bits) {
+                                                                const int32_t *__restrict__ totals, Outputs o, int n, int E, int id_bits) {
     extern __shared__ int32_t smem[];
     constexpr int NT = NW * 64;
     int32_t *offs = smem, *padc = smem + E + 1, *table = smem + 2 * E + 1;  // table: [NW][E]
@@ -99,7 +136,12 @@ __global__ __launch_bounds__(NW * 64) void align_scatter_kernel(const int32_t *_
     load_ids<NW, PER>(id, topk_ids, (int64_t)g * NT * PER, n);
     for (int i = tid; i < (NW + 2) * E; i += NT) table[i] = 0;
     __syncthreads();
-    {
+    if (totals != nullptr) {
+        for (int e = tid; e < E; e += NT) {
+            tot[e] = totals[e];
+            before[e] = counts[(size_t)g * E + e];
+        }
+    } else {
         // thread (part, e) sums every parts-th slice
         const int bits = 32 - __builtin_clz(max(E - 1, 1)), pitch = 1 << bits, parts = max(1, NT >> bits);
         for (int i = tid; i < pitch * parts; i += NT) {
@@ -199,10 +241,10 @@ __global__ __launch_bounds__(NW * 64) void align_runs_kernel(const int32_t *__re
     }
 }
 
-// Scratch of the entry point that allocates nothing (pmoe_moe_align_static): counts[G][E] (and 2 E + 1 words more)
-// of the multi-workgroup sort for up to kStaticMaxIds ids and kMaxExperts experts, 520 KB held by
-// every device the library runs on until the process ends.  In host code this name is only a handle for
-// hipGetSymbolAddress; kernels get the address that call returns.
+// Scratch of the entry point that allocates nothing (pmoe_moe_align_static): what the first query asks for, that is
+// 2 E + 1 words more than the counts[G][E] in use, for the multi-workgroup sort of up to kStaticMaxIds ids and kMaxExperts
+// experts: 520 KB held by every device the library runs on until the process ends.  In host code this name is only a
+// handle for hipGetSymbolAddress; kernels get the address that call returns.
 constexpr int kStaticMaxIds = PMOE_ALIGN_STATIC_MAX_IDS;
 constexpr size_t kStaticWords = (size_t)(kStaticMaxIds / kMaxSliceIds) * kMaxExperts + 2 * kMaxExperts + 1;
 static __device__ __align__(256) int32_t scratch[kStaticWords];
@@ -227,17 +269,25 @@ int launch_single(const int32_t *topk_ids, const Outputs &o, int n, int E, hipSt
     return pmoe::check_launch("moe_align launch");
 }
 
-// The two launches of the multi-workgroup sort in slices of `slice` ids; `words` holds n_slices * E int32 of device
-// scratch, every one of which is written before it is read.
-int launch_multi(const int32_t *topk_ids, const Outputs &o, int n, int E, int slice, int32_t *words, hipStream_t s) {
+// The launches of the multi-workgroup sort in slices of `slice` ids; `words` holds n_slices * E int32 of device
+// scratch, or E more (n_words), every one of which is written before it is read.
+// What the scatter kernel reads if it adds up the counts itself, in words of all its workgroups, against one launch more:
+// equal at 1 << 20 ids of 1024 experts (48 us, 16.8 M words) and 1 << 21 of 128 (27 / 29 us, 8.4 M); 21 / 28 us at 1 << 22 of 8
+// (2.1 M), 140 / 72 at 1 << 22 of 1024 (268 M), 247 / 139 at 1 << 24 of 128, 1144 / 219 at 1 << 24 of 1024, 15097 / 731 at 1 << 26.
+constexpr int64_t kSelfScanWords = 1 << 24;
+int launch_multi(const int32_t *topk_ids, const Outputs &o, int n, int E, int slice, int32_t *words, size_t n_words, hipStream_t s) {
     const int id_bits = id_bits_for(E);
     const int G = n_slices(n, slice);
+    int32_t *totals = (int64_t)G * G * E > kSelfScanWords && n_words >= (size_t)(G + 1) * E ? words + (size_t)G * E : nullptr;
     auto launch = [&](auto nw, auto p) {
         constexpr int NW = decltype(nw)::value, PER = decltype(p)::value;
         hipLaunchKernelGGL((align_count_kernel<NW, PER>), dim3(G), dim3(NW * 64), sizeof(int32_t) * (size_t)NW * E, s, topk_ids, n, E,
                            id_bits, words);
+        const int bits = std::min(id_bits, 6);
+        if (totals != nullptr)
+            hipLaunchKernelGGL(align_bases_kernel, dim3((E + (1 << bits) - 1) >> bits), dim3(1024), 0, s, words, totals, G, E, bits);
         hipLaunchKernelGGL((align_scatter_kernel<NW, PER>), dim3(G), dim3(NW * 64), sizeof(int32_t) * (size_t)(sort_words(NW, E) + 2 * E), s,
-                           topk_ids, words, o, n, E, id_bits);
+                           topk_ids, words, totals, o, n, E, id_bits);
     };
     auto with_per = [&](auto nw) {
         constexpr int NW = decltype(nw)::value;
@@ -285,7 +335,7 @@ int static_scratch(const void *data, int32_t **out) {
 
 extern "C" size_t pmoe_moe_align_workspace_bytes(int n, int num_experts) {
     if (n <= kSingleMaxIds || num_experts <= 0 || num_experts > kMaxExperts) return 0;
-    const size_t G = (size_t)n_slices(n, kMaxSliceIds);
+    const size_t G = (size_t)n_slices(n, kMaxSliceIds);  // counts, totals; E + 1 words more than are used, as callers know it
     return sizeof(int32_t) * (G * (size_t)num_experts + 2 * (size_t)num_experts + 1);
 }
 
@@ -321,7 +371,7 @@ extern "C" int pmoe_moe_align_ws(const int32_t *topk_ids, int32_t *sorted_token_
         // the finest slices whose counts fit the scratch
         for (int slice = slice_ids(n); aligned && slice <= kMaxSliceIds; slice *= 2)
             if (sizeof(int32_t) * (size_t)n_slices(n, slice) * num_experts <= workspace_bytes)
-                return launch_multi(topk_ids, o, n, num_experts, slice, static_cast<int32_t *>(workspace), s);
+                return launch_multi(topk_ids, o, n, num_experts, slice, static_cast<int32_t *>(workspace), workspace_bytes / sizeof(int32_t), s);
     }
     return launch_single(topk_ids, o, n, num_experts, s);
 }
@@ -342,5 +392,5 @@ extern "C" int pmoe_moe_align_static(const int32_t *topk_ids, int32_t *sorted_to
     // the finest slices whose counts fit the array
     int slice = slice_ids(n);
     while (slice < kMaxSliceIds && (size_t)n_slices(n, slice) * num_experts > kStaticWords) slice *= 2;
-    return launch_multi(topk_ids, o, n, num_experts, slice, words, s);
+    return launch_multi(topk_ids, o, n, num_experts, slice, words, kStaticWords, s);
 }

@@ -64,6 +64,32 @@ def test_a_misaligned_workspace_is_an_error_only_where_scratch_is_needed(n, E, s
             np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("n,E,words", [
+    ((1 << 21) + 1, 1024, "all"),  # the kernel that turns counts into bases: 257 slices, 16 workgroups of experts
+    ((1 << 22) - 77, 100, "all"),  # its last workgroup has experts to spare
+    ((1 << 23) + 5, 17, "all"),    # one workgroup, 32 columns
+    ((1 << 22) - 77, 100, "counts"),  # scratch for the counts alone: the scatter kernel adds them up
+])
+def test_align_of_very_many_ids(n, E, words, device):
+    import prime_moe
+    from prime_moe import _native
+    lib = _native.load()
+    slices = -(-n // 8192)
+    assert slices * slices * E > 1 << 24  # the rule of the dispatch
+    ids = np.random.default_rng(n).integers(0, E, size=n).astype(np.int32)
+    ids[n // 2: n // 2 + n // 8] = E // 2
+    pad_to, max_padded, max_blocks = prime_moe.align_sizes(n, E, 128, 1)
+    nbytes = lib.pmoe_moe_align_workspace_bytes(n, E) if words == "all" else 4 * slices * E
+    ws = torch.full((nbytes,), 0x5a, dtype=torch.uint8, device=device)
+    dev_ids = torch.from_numpy(ids).to(device)
+    s, e, t = (torch.full((c,), 0x5a5a5a5a, dtype=torch.int32, device=device) for c in (max_padded, max_blocks, 1))
+    _native.check(lib.pmoe_moe_align_ws(dev_ids.data_ptr(), s.data_ptr(), e.data_ptr(), t.data_ptr(), n, E, 128, pad_to,
+                                        max_padded, max_blocks, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    for got, want in zip((s, e, t), O.moe_align_fast(ids, E, 128, 1)):
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("T,E,k", [(16, 512, 32), (17, 512, 8), (8, 513, 32), (9, 1024, 4), (16, 64, 32), (2, 33, 32)])
 def test_route_around_the_one_kernel_form(T, E, k, device):
     g = torch.Generator(device=device).manual_seed(T + E + k)
