@@ -93,10 +93,14 @@ __device__ __forceinline__ void fill_minus_one(const Outputs &o, int n_threads) 
     if ((reinterpret_cast<uintptr_t>(o.sorted_token_ids) & 15) == 0) {
         int4 *dst = reinterpret_cast<int4 *>(o.sorted_token_ids);
         for (int i = tid; i < o.max_padded / 4; i += n_threads) dst[i] = make_int4(-1, -1, -1, -1);
-        for (int i = (o.max_padded & ~3) + tid; i < o.max_padded; i += n_threads) o.sorted_token_ids[i] = -1;
+        for (int64_t i = (o.max_padded & ~3) + (int64_t)tid; i < o.max_padded; i += n_threads) o.sorted_token_ids[i] = -1;
     } else {
-        for (int i = tid; i < o.max_padded; i += n_threads) o.sorted_token_ids[i] = -1;
+        for (int64_t i = tid; i < o.max_padded; i += n_threads) o.sorted_token_ids[i] = -1;
     }
+}
+
+__device__ __forceinline__ void write_expert_ids(const Outputs &o, const int32_t *offs, int E, int n_threads) {
+    for (int64_t j = threadIdx.x; j < o.max_blocks; j += n_threads) o.expert_ids[j] = owner_of(offs, E, (int)j * o.block_m);
 }
 
 // LDS words of sort_in_workgroup.
@@ -128,7 +132,7 @@ __device__ __forceinline__ void sort_in_workgroup(const int (&id)[PER], const Ou
     scan_experts(padc, offs, E);
     __syncthreads();
     if (tid == 0) o.num_tokens_post_padded[0] = offs[E];
-    for (int j = tid; j < o.max_blocks; j += NT) o.expert_ids[j] = owner_of(offs, E, j * o.block_m);
+    write_expert_ids(o, offs, E, NT);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int e = id[i];

@@ -4,7 +4,7 @@
 // except that the within-expert order is made unique (ascending pair id) instead of being
 // left to an atomic race.  Up to kSingleMaxIds ids one workgroup does it (align_sort.h): ranks inside the waves,
 // per-expert counts of the waves -> bases, padded totals -> prefix, scatter.  More ids spread over workgroups.
-// All arithmetic is int32 and the output is a pure function of the input.
+// Ids, positions and sizes are int32 (loops that step past a size near 2^31 count in int64), and the output is a pure function of the input.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(NW * 64) void align_scatter_kernel(const int32_t *_
     __syncthreads();
     const int total = offs[E];
     if (g == 0 && tid == 0) o.num_tokens_post_padded[0] = total;
-    for (int j = g * NT + tid; j < o.max_blocks; j += G * NT) o.expert_ids[j] = owner_of(offs, E, j * o.block_m);
+    for (int64_t j = g * NT + tid; j < o.max_blocks; j += G * NT) o.expert_ids[j] = owner_of(offs, E, (int)j * o.block_m);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int e = id[i];
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(NW * 64) void align_scatter_kernel(const int32_t *_
     }
     // padding: an expert's by one wave, the slots past the total by everybody
     for (int e = g * NW + wave; e < E; e += G * NW)
-        for (int pos = offs[e] + tot[e] + lane; pos < offs[e + 1]; pos += 64) o.sorted_token_ids[pos] = -1;
+        for (int64_t pos = (int64_t)offs[e] + tot[e] + lane; pos < offs[e + 1]; pos += 64) o.sorted_token_ids[pos] = -1;
     for (int64_t pos = (int64_t)total + g * NT + tid; pos < o.max_padded; pos += (int64_t)G * NT) o.sorted_token_ids[pos] = -1;
 }
 
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(NW * 64) void align_runs_kernel(const int32_t *__re
     scan_experts(padc, offs, E);
     __syncthreads();
     if (tid == 0) o.num_tokens_post_padded[0] = offs[E];
-    for (int j = tid; j < o.max_blocks; j += NT) o.expert_ids[j] = owner_of(offs, E, j * o.block_m);
+    write_expert_ids(o, offs, E, NT);
     for (int64_t r = 0; r < n; r += RUN) {
         load_ids<NW, PER>(id, topk_ids, r, n);
         for (int i = tid; i < NW * E; i += NT) table[i] = 0;

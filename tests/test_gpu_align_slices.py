@@ -90,6 +90,36 @@ def test_align_of_very_many_ids(n, E, words, device):
         np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
+def test_align_next_to_2_31_blocks_by_one_workgroup(device):
+    """Blocks of one row and padding to 2^30 - 1: two of them make 2^31 - 2 blocks, and every loop over rows or blocks steps
+    past 2^31 before it ends."""
+    import prime_moe  # noqa: F401
+    bpc = (1 << 30) - 1
+    s, e, t = torch.ops.prime_moe.moe_align(torch.zeros((8,), dtype=torch.int32, device=device), 1, 1, bpc)
+    assert s.numel() == e.numel() == 2 * bpc and int(t) == bpc
+    assert torch.equal(s[:8], torch.arange(8, dtype=torch.int32, device=device))
+    for at in range(0, 2 * bpc, 1 << 29):
+        assert int(s[max(at, 8):at + (1 << 29)].max()) == -1 == int(s[max(at, 8):at + (1 << 29)].min())
+        assert int(e[at:at + (1 << 29)].max()) == 0 == int(e[at:at + (1 << 29)].min())
+
+
+def test_align_next_to_2_31_ids_by_many_workgroups(device):
+    import prime_moe  # noqa: F401
+    n, step = (1 << 31) - 1, 1 << 29
+    ids = torch.empty((n,), dtype=torch.int32, device=device)
+    for at in range(0, n, step):
+        ids[at:at + step] = torch.arange(at, min(at + step, n), dtype=torch.int32, device=device).bitwise_and_(1)
+    s, e, t = torch.ops.prime_moe.moe_align(ids, 2, 1, 1)
+    half = (n + 1) // 2  # the even ids, then the odd ones
+    assert s.numel() == e.numel() == int(t) == n
+    for at in range(0, n, step):
+        end = min(at + step, n)
+        want = torch.arange(at, end, dtype=torch.int64, device=device)
+        owner = (want >= half).to(torch.int32)
+        want = torch.where(want < half, 2 * want, 2 * (want - half) + 1).to(torch.int32)
+        assert torch.equal(s[at:end], want) and torch.equal(e[at:end], owner)
+
+
 @pytest.mark.parametrize("T,E,k", [(16, 512, 32), (17, 512, 8), (8, 513, 32), (9, 1024, 4), (16, 64, 32), (2, 33, 32)])
 def test_route_around_the_one_kernel_form(T, E, k, device):
     g = torch.Generator(device=device).manual_seed(T + E + k)
