@@ -313,9 +313,15 @@ __device__ __forceinline__ void setup_ring_loader(ring::Loader<RB> &ld, const ri
 // blockIdx / 8) start 128 bytes apart, 8 distinct phases over a 1 KB period.  The spread keeps the
 // workgroups that share a weight tile off the same HBM channel at the same instant, and stays short
 // enough that they still meet in L2 (a 16-phase, 4 KB spread read 30 % more from HBM for the same time).
+// Without a work list and with rows of whole 4 KB there are 32 phases.  Neighbouring weight tiles then run side by side all
+// over the chip and the same bytes of all their rows lie on few channels: with 8 phases the up kernel took 194 us at 24
+// tokens x top 2 on 8 experts of K 4096 x N 28672 (168 with 32 phases; 171 in the order of the work lists), the down kernel 101
+// at 16384 x 7168 (80; 106), both kernels 301 at 64 tokens on 32 experts of K 4096 x N 8192 (273; 307).  Rows of other
+// lengths start on different channels by themselves (K 7168: 155 and 155).
 template <int RB>
-__device__ __forceinline__ int slab_rotation(int n_slabs) {
-    return (int)((blockIdx.x >> 3) & 7) % n_slabs;
+__device__ __forceinline__ int slab_rotation(const MoeArgs &a, int n_slabs) {
+    const int phases = a.work == nullptr && (n_slabs * RB) % 4096 == 0 ? 4096 / RB : 8;
+    return (int)((blockIdx.x >> 3) & (phases - 1)) % n_slabs;
 }
 
 // Up kernel tile on the stage ring: the live fragments of one or two row blocks x activation
@@ -357,7 +363,7 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, R
         [&](int row) { return (uint32_t)blocked_scale_off((row < 128 ? h0 : H + h0 - 128) + row, 0, K >> 7); });
 
     const int wrow[2] = {32 * w4, 128 + 32 * w4};
-    const int start = slab_rotation<RB>(n_slabs);
+    const int start = slab_rotation<RB>(a, n_slabs);
     const int tok_region = grp ? lay.group1_off : 0;
     // the ring is free after main_loop (it ends with a barrier): its head holds the activation tiles
     constexpr int kPitch = kActPitchFp8;
@@ -467,7 +473,7 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
         [&](int row) { return (uint32_t)blocked_scale_off(min(k0 + row, K - 1), 0, ht128); });
 
     const int wrow[2] = {64 * w4, 64 * w4 + 32};
-    const int start = slab_rotation<RB>(n_slabs);
+    const int start = slab_rotation<RB>(a, n_slabs);
     const int tok_region = grp ? lay.group1_off : 0;
     const int SB = lay.stage_bytes, NS = lay.stages;
     // the ring is free after main_loop (it ends with a barrier): its head holds the 128 x 256 output

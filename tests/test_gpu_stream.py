@@ -115,6 +115,7 @@ SPARSE = [129, 65, 64, 33, 32, 5] + [1] * 60
     (256, 2048, 40, EDGES, False),     # ring kernels without a work list
     (256, 768, 256, SPARSE, True),     # general streaming down kernel, H = 384: the last slab has one half
     (1024, 512 + 256, 256, SPARSE, False),
+    (2048, 8192, 11, [129, 33, 31, 20, 15, 10, 8, 6, 5, 4, 3], True),  # ring kernels, activation rows of 4 KB: 32 phases of the K walk
 ])
 def test_mx_kernels_without_a_schedule_at_row_edges(K, N, E, counts, split, device):
     import prime_moe
