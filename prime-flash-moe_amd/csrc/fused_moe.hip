@@ -31,6 +31,26 @@ struct Job {
     bool w_once;  // no other row tile of this expert: nobody else reads the weight rows of this job
 };
 
+// Crowded schedules.  Without work lists (few rows per expert on average, see use_direct) neighbouring workgroups work on
+// neighbouring weight tiles of one block.  With the tokens crowded on a few experts these have several full blocks: paired
+// to row tiles, and 8 weight tiles by 4 row tiles to an XCD, their token rows are read from its L2.  How the tokens are
+// spread is known on the device only, so where it may matter (crowding_possible_mx) the prologue is enqueued too, and
+// it and the two kernels decide by this function whether they use its lists: more than 64 rows per live block, and more
+// jobs than one round of the CUs, which pairing would leave idle.  Us without lists / as decided here, K 7168, N 4096,
+// tokens x top 8 on some of 256 experts: 256 on 8 (no lists) 154 / 159, on 16 250 / 188, on 64 (no lists) 491 / 495; 300 on 8
+// 231 / 182, on 16 260 / 210; 512 on 8 267 / 212, on 32 411 / 354; 768 on 32 500 / 406, on 64 582 / 570, Zipf 1938 / 1938.
+// The prologue that finds nothing to do costs 2 to 4 us.
+__host__ __device__ __forceinline__ bool crowded_mx(int64_t pairs, int64_t n_live, int n_wt_up, int n_cus) {
+    return pairs > 64 * n_live && n_live * n_wt_up > n_cus;
+}
+__device__ __forceinline__ bool crowded_mx(const int32_t *ntpp, int n_blocks, int64_t pairs, int n_wt_up, int n_cus) {
+    return crowded_mx(pairs, min((ntpp[0] + kBlockRows - 1) / kBlockRows, n_blocks), n_wt_up, n_cus);
+}
+// The arguments as the kernels use them: without the work list if nobody filled it.
+__device__ __forceinline__ void settle_lists(MoeArgs &a) {
+    if (a.crowd && !crowded_mx(a.ntpp, a.n_blocks, (int64_t)a.M * a.top_k, a.H / 128, a.crowd)) a.work = nullptr;
+}
+
 // Workgroup id -> job.  With a work list: one load from it, which the prologue lays out by workgroup id (see
 // emit_work); entries of workgroups without work are -1.  Without one (few rows per expert, see use_direct): every
 // live block is a row tile of its own, its jobs are consecutive workgroups.
@@ -420,6 +440,7 @@ __global__ __launch_bounds__(512) void moe_up_kernel(MoeArgs a) {
     using L = SplitLds<DT>;
     __shared__ __attribute__((aligned(1024))) char lds[L::kTotal];
     RowInfo<2> &ri = *reinterpret_cast<RowInfo<2> *>(lds + L::kRowInfoOff);
+    settle_lists(a);
     if (a.work == nullptr) stream::invert(a, 512);  // (no prologue did)
     Job j;
     if (!resolve_job(a, j)) return;
@@ -516,6 +537,7 @@ __global__ __launch_bounds__(512) void moe_down_kernel(MoeArgs a) {
     using L = SplitLds<DT>;
     __shared__ __attribute__((aligned(1024))) char lds[L::kTotal];
     RowInfo<2> &ri = *reinterpret_cast<RowInfo<2> *>(lds + L::kRowInfoOff);
+    settle_lists(a);
     Job j;
     if (!resolve_job(a, j)) return;
     const int ntf = load_row_info<2>(a, j.first, j.nb, ri);
@@ -563,7 +585,8 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
                                                            int grid_down, int num_experts,
                                                            const int32_t *sorted_ids, int sorted_num, int32_t *inv,
                                                            int n_pairs, int do_invert, const uint8_t *x_scales,
-                                                           uint32_t *xs_tiled, int nkt, int top_k, int M) {
+                                                           uint32_t *xs_tiled, int nkt, int top_k, int M, int crowd) {
+    if (crowd && !crowded_mx(ntpp, n_blocks, n_pairs, n_wt_up, crowd)) return;
     if (blockIdx.x == 0 && tiles != nullptr) {
         __shared__ int s_max[4], s_sum[4], s_carry[2];
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -908,27 +931,56 @@ static bool use_direct(const MoeArgs &a) {
     return (int64_t)a.M * a.top_k <= rows * a.E;
 }
 
-static int launch_direct_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
+// The prologue, with work lists for grids of grid_up and grid_down workgroups that take per_up and per_down weight tiles.
+static void launch_prologue(const MoeArgs &a, const SchedBuffers &sb, int per_up, int grid_up, int per_down, int grid_down,
+                            hipStream_t s) {
+    // the work lists are needed by the two kernels even when the rest of the prologue is masked off
+    const int do_invert = (g_phase_mask & PMOE_PHASE_PROLOGUE) ? 1 : 0;
+    const int blocks = do_invert ? std::max(1, std::min((a.sorted_num + 255) / 256, a.crowd ? 48 : 1024)) : 1;
+    hipLaunchKernelGGL(moe_prologue_kernel, dim3(blocks), dim3(256), 0, s, a.expert_ids, a.ntpp, a.n_blocks, sb.tiles, sb.n_tiles,
+                       sb.work_up, a.H / 128, per_up, grid_up, sb.work_down, (a.K + kWRows - 1) / kWRows, per_down, grid_down, a.E,
+                       a.sorted_ids, a.sorted_num, a.inv, a.M * a.top_k, do_invert, a.x_scales, a.xs_tiled, a.K >> 7, a.top_k, a.M,
+                       a.crowd);
+}
+
+// An expert has at most M rows (more only if a token names it twice, which is not looked for): up to 128 it has one block.
+// Crowded blocks hold 96 rows or more on average.
+static bool crowding_possible_mx(const MoeArgs &a, int n_cus) {
+    const int64_t pairs = (int64_t)a.M * a.top_k;
+    return a.M > kBlockRows && crowded_mx(pairs, pairs / 96, a.H / 128, n_cus);
+}
+
+static int launch_direct_pipeline(MoeArgs a, const SchedBuffers &sb, void *out, int split, hipStream_t s) {
     const int mask = g_phase_mask, n_cus = resident_grid();
     const int64_t blocks = expected_blocks(a);
+    const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
+    // narrow jobs while wide tiles do not give every CU one (us at 128 / 256 / 640 / 1024 wide jobs, stream against
+    // ring, whole op: 75.5 / 81.7, 130 / 129, 291 / 290, 419 / 406)
+    const bool stream_up = blocks * n_wt_up < n_cus;
+    // (256 experts, K 7168, H 2048, stream against ring, whole op: 71.6 / 75.5 us at 1 token, 126 / 130 at 2,
+    // 288 / 291 at 5, 408 / 406 at 8; 32 experts with 8 rows each, K 2048, H 1024: 45.0 / 44.6)
+    const bool stream_down = a.H <= 256 || (blocks * n_wt_down < 5 * n_cus && (int64_t)a.M * a.top_k <= 4 * blocks);
     auto launch_stream = [&](auto kernel, int n_tiles) {
         const int grid = (int)std::min<int64_t>((int64_t)a.n_blocks * std::max(n_tiles, 1), 2 * n_cus);
         if (grid > 0) hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, s, a, n_tiles);
     };
-    auto launch_ring = [&](auto kernel, bool down, int n_wt) {
+    const int per_up = tiles_per_workgroup(false, (int)blocks, n_wt_up), per_down = tiles_per_workgroup(true, (int)blocks, n_wt_down);
+    const int grid_up = grid_for(a.n_blocks * ((n_wt_up + per_up - 1) / per_up));
+    const int grid_down = grid_for(a.n_blocks * ((n_wt_down + per_down - 1) / per_down));
+    auto launch_ring = [&](auto kernel, const int4 *list, int n_wt, int per_job, int grid) {
         MoeArgs d = a;
-        d.work = nullptr;
+        d.work = a.crowd ? list : nullptr;
         d.n_wtiles = n_wt;
-        d.per_job = tiles_per_workgroup(down, (int)blocks, n_wt);
-        const int grid = a.n_blocks * ((n_wt + d.per_job - 1) / d.per_job);
+        d.per_job = per_job;
         if (grid > 0) hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, s, d);
     };
-    const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
+    if (!stream_up && !stream_down && crowding_possible_mx(a, n_cus)) {
+        a.crowd = n_cus;
+        launch_prologue(a, sb, per_up, grid_up, per_down, grid_down, s);
+    }
     if (mask & PMOE_PHASE_UP) {
-        // narrow jobs while wide tiles do not give every CU one (us at 128 / 256 / 640 / 1024 wide jobs, stream against
-        // ring, whole op: 75.5 / 81.7, 130 / 129, 291 / 290, 419 / 406)
-        if (blocks * n_wt_up < n_cus) launch_stream(moe_stream_kernel_mx<true>, a.H / 32);
-        else launch_ring(moe_up_kernel<DT_FP8>, false, n_wt_up);
+        if (stream_up) launch_stream(moe_stream_kernel_mx<true>, a.H / 32);
+        else launch_ring(moe_up_kernel<DT_FP8>, sb.work_up, n_wt_up, per_up, grid_up);
     } else if (mask & PMOE_PHASE_PROLOGUE) {
         launch_stream(moe_stream_kernel_mx<true>, 0);
     }
@@ -940,12 +992,10 @@ static int launch_direct_pipeline(MoeArgs a, void *out, int split, hipStream_t s
                 if (a.H == 128) hipLaunchKernelGGL(moe_stream_down_short_kernel_mx<128>, dim3(grid), dim3(256), 0, s, a);
                 else hipLaunchKernelGGL(moe_stream_down_short_kernel_mx<256>, dim3(grid), dim3(256), 0, s, a);
             }
-        } else if (blocks * n_wt_down < 5 * n_cus && (int64_t)a.M * a.top_k <= 4 * blocks) {
-            // (256 experts, K 7168, H 2048, stream against ring, whole op: 71.6 / 75.5 us at 1 token, 126 / 130 at 2,
-            // 288 / 291 at 5, 408 / 406 at 8; 32 experts with 8 rows each, K 2048, H 1024: 45.0 / 44.6)
+        } else if (stream_down) {
             launch_stream(moe_stream_kernel_mx<false>, a.K / 64);
         } else {
-            launch_ring(moe_down_kernel<DT_FP8>, true, n_wt_down);
+            launch_ring(moe_down_kernel<DT_FP8>, sb.work_down, n_wt_down, per_down, grid_down);
         }
     }
     if (mask & PMOE_PHASE_FINALIZE) launch_finalize(a, out, split, n_wt_down, s);
@@ -956,23 +1006,14 @@ static int launch_mxfp8_pipeline(MoeArgs a, const SchedBuffers &sb, void *out, i
     constexpr int DT = DT_FP8;
     const int mask = g_phase_mask;
     a.n_blocks = (a.sorted_num + kBlockRows - 1) / kBlockRows;
-    if (use_direct(a)) return launch_direct_pipeline(a, out, split, s);
+    if (use_direct(a)) return launch_direct_pipeline(a, sb, out, split, s);
     a.n_wtiles = a.H / 128;
     const int n_wt_down = (a.K + kWRows - 1) / kWRows;
     const int per_up = tiles_per_workgroup(false, a.n_blocks, a.n_wtiles);
     const int per_down = tiles_per_workgroup(true, a.n_blocks, n_wt_down);
     const int grid_up = grid_for(a.n_blocks * ((a.n_wtiles + per_up - 1) / per_up));
     const int grid_down = grid_for(a.n_blocks * ((n_wt_down + per_down - 1) / per_down));
-    {
-        // the work lists are needed by the two kernels even when the rest of the prologue is masked off
-        const int do_invert = (mask & PMOE_PHASE_PROLOGUE) ? 1 : 0;
-        const int blocks = do_invert ? std::max(1, std::min((a.sorted_num + 255) / 256, 1024)) : 1;
-        hipLaunchKernelGGL(moe_prologue_kernel, dim3(blocks), dim3(256), 0, s, a.expert_ids, a.ntpp, a.n_blocks,
-                           sb.tiles, sb.n_tiles, sb.work_up, a.n_wtiles, per_up, grid_up,
-                           sb.work_down, n_wt_down, per_down, grid_down, a.E,
-                           a.sorted_ids, a.sorted_num, a.inv, a.M * a.top_k, do_invert, a.x_scales, a.xs_tiled,
-                           a.K >> 7, a.top_k, a.M);
-    }
+    launch_prologue(a, sb, per_up, grid_up, per_down, grid_down, s);
     if (a.n_blocks > 0) {
         a.work = sb.work_up;
         if (mask & PMOE_PHASE_UP) hipLaunchKernelGGL((moe_up_kernel<DT>), dim3(grid_up), dim3(512), 0, s, a);

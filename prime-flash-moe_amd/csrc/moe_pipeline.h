@@ -125,7 +125,8 @@ struct MoeArgs {
     int4 *runs;           // prologue scratch: the runs of blocks with one expert
     float *up_partials;   // deep mode: fp32 partial sums, [part][fragment][weight tile][32 KB]
     int deep_ok;          // deep mode may be planned (the workspace holds up_partials)
-    int crowd;            // bf16: tall kernels enqueued beside the streaming ones (bits: 1 up, 2 down), see crowding()
+    int crowd;            // bf16: tall kernels enqueued beside the streaming ones (bits: 1 up, 2 down), see crowding();
+                          // mxfp8: the work list is one for crowded schedules only (the number of CUs), see crowded_mx()
     int top_k, M, K, N, H, E, sorted_num;
     int n_blocks;  // sorted_num / 128 (rounded up)
     int n_wtiles;  // weight tiles along the free dimension: H/128 (up) or ceil(K/256) (down)

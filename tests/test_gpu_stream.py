@@ -140,3 +140,42 @@ def test_mx_kernels_without_a_schedule_at_row_edges(K, N, E, counts, split, devi
     assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
     mx_elementwise_gates(got, ref, bound)
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("counts,lists", [
+    ([180, 180, 130, 128, 75, 75, 75, 21], True),  # 79 rows per block: the lists of the prologue, paired blocks
+    ([24] * 36, False),                            # the same call spread out: jobs by arithmetic
+    ([216] * 4, False),                            # crowded, but on fewer jobs than CUs
+])
+def test_mx_crowded_schedules_use_work_lists(counts, lists, device):
+    """Few rows per expert on average, all of them on few experts: the prologue and the two kernels decide on the device
+    whether there are work lists."""
+    import prime_moe
+    from prime_moe import _native
+    lib = _native.load()
+    K, E, N, top_k = 256, 36, 8192, 4
+    counts = counts + [0] * (E - len(counts))
+    ids, wts = _routing_by_counts(counts, top_k, device, seed=sum(counts[:3]))
+    T = ids.shape[0]
+    cus, n_wt = torch.cuda.get_device_properties(device).multi_processor_count, N // 256
+    assert T > 128 and T * top_k <= 24 * E and T * top_k // 96 * n_wt > cus  # the rules of the dispatch
+    n_live = sum(-(-c // 128) for c in counts)
+    assert lists == (T * top_k > 64 * n_live and n_live * n_wt > cus)
+    g, a, deq = _quantised_inputs(T, K, E, N, device, seed=N)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    nbytes = lib.pmoe_fused_moe_mxfp8_workspace_bytes(T, K, N, E, s.numel(), top_k, 1)
+    ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device=device)
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    _native.check(lib.pmoe_fused_moe_mxfp8(
+        *(a[k].data_ptr() for k in ("x", "x_scales", "w1", "w1_scales", "w2", "w2_scales")), out.data_ptr(), s.data_ptr(),
+        e.data_ptr(), n.data_ptr(), wts.data_ptr(), top_k, T, K, N, E, s.numel(), 128, 64, 4, 2, 1, 1, ws.data_ptr(), nbytes,
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    n_tiles = int(ws[:4].view(torch.int32)[0])  # the workspace starts with the number of row tiles of the lists
+    assert n_tiles == (sum(-(-c // 256) for c in counts) if lists else -1)
+    ref, bound = O.fused_moe_dense(deq["x"], deq["w1"], deq["w2"], ids.cpu(), wts.cpu(), act_mx=True,
+                                   flip_delta=MX_FLIP_DELTA)
+    got = out.float().cpu()
+    assert torch.isfinite(got).all()
+    assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
+    mx_elementwise_gates(got, ref, bound)
