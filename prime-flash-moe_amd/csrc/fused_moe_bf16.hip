@@ -31,7 +31,11 @@ namespace pmoe {
 // 4 of 8 (64 rows): 400 / 419 / 406, on 3: 423 / 342 / 348; K 7168, N 512, 900 x 9 on all 257 (31 rows): 662 / 659 / 630,
 // on 63: 532 / 246 / 233, 256 x 9 on 57 (40 rows): 169 / 199 / 162.
 // The kernels that are enqueued and find nothing to do cost 2 us each, so they are enqueued where crowding would cost more:
-// an expert has at most M rows (more only if a token names it twice, which is not looked for), M <= 64 is one pass.
+// an expert has at most M rows (more only if a token names it twice, which is not looked for), M <= 64 is one pass.  The
+// tall up kernel comes with the prologue and the tall down kernel, unless these are there already.  Crowded, without / with it,
+// and spread out, without / with it, us: K 2048, N 1536 top 8: 200 tokens on 16 experts 70 / 66, on all 128 216 / 222 (157 MB:
+// not enqueued), 256 on 16 103 / 74, on 128 220 / 227; K = N = 2048, 256 x 4 on 6 of 32 experts 71 / 63, on 4 54 / 63, on 32 91 / 96
+// (134 MB: not enqueued); K 7168, N 512, 160 x 9 on 9 of 257 130 / 101, on all 481 / 485.
 constexpr float kCrowdedUpBytes = 64e6f, kCrowdedDownBytes = 96e6f;
 __device__ __forceinline__ int crowding(const MoeArgs &a, int ntpp) {
     if (!a.crowd) return 0;
@@ -49,8 +53,8 @@ __device__ __forceinline__ int crowding(const MoeArgs &a, int ntpp) {
 // The tall kernels to enqueue (bits as in crowding()).
 static int crowding_possible(const MoeArgs &a) {
     const double pairs = (double)a.M * a.top_k, w2_bytes = 2.0 * a.K * a.H;
-    int tall = a.M > 64 && pairs / 64 * 2 * w2_bytes >= 2 * kCrowdedUpBytes ? 3 : 0;
-    if (a.H <= 256 && a.M > 24 && 0.75 * pairs / 32 * w2_bytes >= kCrowdedDownBytes) tall |= 2;
+    int tall = a.H <= 256 && a.M > 24 && 0.75 * pairs / 32 * w2_bytes >= kCrowdedDownBytes ? 2 : 0;
+    if (a.M > 64 && pairs / 64 * 2 * w2_bytes >= (tall ? 2 : 3) * kCrowdedUpBytes) tall = 3;
     return tall;
 }
 

@@ -69,8 +69,9 @@ def test_stream_kernels_with_dropped_rows_and_blocks(device):
 
 
 @pytest.mark.parametrize("K,N,E,T,top_k,hot,want", [
-    (1024, 768, 168, 1340, 4, 50, 3),    # general down kernel: all pairs on 50 experts, 107 rows each
-    (1024, 768, 168, 1340, 4, 168, 0),   # the same call with its pairs spread out
+    (1024, 768, 246, 1960, 4, 73, 3),    # general down kernel: all pairs on 73 experts, 107 rows each
+    (1024, 768, 246, 1960, 4, 246, 0),   # the same call with its pairs spread out
+    (1024, 768, 168, 1340, 4, 50, 0),    # crowded, but too small to enqueue the tall kernels
     (2048, 512, 150, 1200, 4, 80, 2),    # short down kernel (H = 256): 60 rows per block crowd it, not the up kernel
     (4096, 256, 150, 1200, 4, 30, 3),    # H = 128, blocks of one expert
     (7168, 512, 60, 60, 32, 1, 2),       # one expert named 32 times by each token: only the tall down kernel is enqueued
