@@ -58,15 +58,14 @@ __device__ __forceinline__ bool resolve_job(const MoeArgs &a, Job &j) {
     if (a.work == nullptr) {
         const int n_jobs = (a.n_wtiles + a.per_job - 1) / a.per_job;
         j.first = (int)blockIdx.x / n_jobs;
-        const int n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
-        if (j.first >= n_live) return false;
+        if (j.first >= min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks)) return false;
         j.e = a.expert_ids[j.first];
         if (j.e < 0 || j.e >= a.E) return false;
         j.nb = 1;
         j.wt = ((int)blockIdx.x - j.first * n_jobs) * a.per_job;
         j.n_sub = min(a.per_job, a.n_wtiles - j.wt);
         j.w_once = (j.first == 0 || a.expert_ids[j.first - 1] != j.e) &&
-                   (j.first + 1 >= n_live || a.expert_ids[j.first + 1] != j.e);
+                   (j.first + 1 >= a.n_blocks || a.expert_ids[j.first + 1] != j.e);
         return true;
     }
     const int4 w = a.work[blockIdx.x];
