@@ -103,6 +103,41 @@ def test_tokens_beyond_m_are_dropped(device):
     assert rel_clamp(out.float().cpu(), ref, 1.0) <= BF16_GATE
 
 
+def shuffle_runs(s, counts, gen):
+    """The rows of every expert's run in another order: what is dropped then leaves holes between live rows."""
+    s, at = s.clone(), 0
+    for c in counts:
+        s[at:at + c] = s[at:at + c][torch.randperm(c, device=s.device, generator=gen)]
+        at += (c + 127) // 128 * 128
+    return s
+
+
+@pytest.mark.parametrize("T,K,E,N", [
+    (1625, 256, 5, 8192),  # up kernel: 10 row tiles x 32 weight tiles, workgroups go from tile to tile
+    (1625, 8192, 5, 256),  # down kernel: likewise; up kernel: deep split
+])
+def test_tokens_beyond_m_are_dropped_on_tall_tiles(T, K, E, N, device):
+    import prime_moe
+    top_k, keep = 2, 1000
+    assert T * top_k > 32 * E  # the rule of the dispatch: tall tiles
+    g, x, w1, w2 = _inputs(T, K, E, N, device, 5)
+    ids, wts = reference_routing(T, E, top_k, device, g, hot_last=False)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    s = shuffle_runs(s, torch.bincount(ids.flatten(), minlength=E).tolist(), g)
+    n_tiles, _ = _tall_plan(x, w1, w2, (s, e, n), wts, torch.empty_like(x), top_k)
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    assert n_tiles * (N // 256 if N > K else K // 256) > cus
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())[:keep]
+    # the whole schedule, and the rows that its length names and no more (no padding behind them)
+    for length in (s.numel(), int(n[0])):
+        torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+        out = torch.empty((keep, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_bf16(x[:keep].contiguous(), w1, w2, s[:length].contiguous(), e[:length // 128].contiguous(), n, wts,
+                                 out, top_k, 128, 32, 8, 1, 1, 1, True)
+        torch.cuda.synchronize()
+        assert rel_clamp(out.float().cpu(), ref, 1.0) <= BF16_GATE
+
+
 def test_validation_errors(device):
     import prime_moe
     T, K, E, N, top_k = 16, 256, 2, 256, 2
@@ -240,23 +275,30 @@ def test_block_without_expert_and_duplicate_pair(device):
         assert rel_clamp(got[keep], ref[keep], 1.0) <= BF16_GATE
 
 
-@pytest.mark.parametrize("T,K,E,N,top_k,exact", [
-    (256, 4096, 8, 512, 4, False),   # the README shape: 8 - 16 row tiles x 2 weight tiles, every tile split 8 ways
-    (40, 2048, 4, 256, 2, False),    # one weight tile, tiles of one or two fragments
-    (130, 6144, 3, 512, 3, True),    # exact-size schedule, a second block with two live rows
-    (1, 2048, 1, 256, 1, False),     # one row
-    (300, 2176, 2, 1024, 2, False),  # 17 slabs: parts of unequal length
+@pytest.mark.parametrize("T,K,E,N,top_k,exact,deep", [
+    (256, 4096, 8, 512, 4, False, True),    # the README shape: 8 - 16 row tiles x 2 weight tiles, every tile split 8 ways
+    (100, 2048, 4, 256, 2, False, True),    # one weight tile, tiles of two to four fragments
+    (130, 6144, 3, 512, 3, True, True),     # exact-size schedule, a second block with two live rows
+    (33, 2048, 1, 256, 1, False, True),     # one weight tile, a second fragment with one live row
+    (300, 2176, 2, 1024, 2, False, True),   # 17 slabs: parts of unequal length
+    (40, 2048, 4, 256, 2, False, False),    # up to 32 rows per expert: the streaming kernels, no deep split
+    (1, 2048, 1, 256, 1, False, False),     # one row, likewise
 ])
-def test_few_jobs_deep_split_and_join_kernel(T, K, E, N, top_k, exact, device):
+def test_few_jobs_deep_split_and_join_kernel(T, K, E, N, top_k, exact, deep, device):
     """Few up jobs for the chip and a long contraction: every up tile is split over up to 8 workgroups that
     only store their partial sums, and a kernel of its own joins them and applies SwiGLU.  Against the
     oracle, and bit for bit the same on a second call (the join adds the parts in part order)."""
     import prime_moe
+    n_blocks = (T * top_k + E * 127 + 127) // 128
+    assert deep == (T * top_k > 32 * E) and n_blocks * (N // 256) <= 32 and K >= 2048  # the rules of the dispatch
     for split in (True, False):
         _run_case(T, K, E, N, top_k, split, device, seed=T + K, use_op_align=not exact, exact=exact, hot_last=False)
     g, x, w1, w2 = _inputs(T, K, E, N, device, T + K)
     ids, wts = reference_routing(T, E, top_k, device, g, hot_last=False)
     sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    if deep:
+        plan = _prologue_workspace(x, w1, w2, sched, wts, torch.empty_like(x), top_k)[:16].view(torch.int32).tolist()
+        assert plan[1] >= 2 and plan[3] == 1  # (row tiles, parts, split jobs, deep) of the up kernel
     outs = []
     for _ in range(2):
         torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
@@ -267,9 +309,9 @@ def test_few_jobs_deep_split_and_join_kernel(T, K, E, N, top_k, exact, device):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
-def _tall_plan(x, w1, w2, sched, wts, out, top_k):
-    """(number of row tiles, the up kernel's table of row tiles) that the prologue of the tall-tile path builds.
-    The workspace starts with the plan, the run list and the table (bf16_workspace in csrc/fused_moe_bf16.hip)."""
+def _prologue_workspace(x, w1, w2, sched, wts, out, top_k):
+    """The workspace after the prologue of the tall-tile path: it starts with the plan, the run list and the table of row
+    tiles (bf16_workspace in csrc/fused_moe_bf16.hip)."""
     from prime_moe import _native
     lib = _native.load()
     (M, K), (E, N, _) = x.shape, w1.shape
@@ -285,8 +327,14 @@ def _tall_plan(x, w1, w2, sched, wts, out, top_k):
     finally:
         lib.pmoe_set_phase_mask(15)
     torch.cuda.synchronize()
+    return ws
+
+
+def _tall_plan(x, w1, w2, sched, wts, out, top_k):
+    """(number of row tiles, the up kernel's table of row tiles) that the prologue of the tall-tile path builds."""
+    ws = _prologue_workspace(x, w1, w2, sched, wts, out, top_k)
     up = lambda b: (b + 255) // 256 * 256
-    at = 256 + up((s.numel() // 128 + 1) * 20)
+    at = 256 + up((sched[0].numel() // 128 + 1) * 20)
     n_tiles = int(ws[:4].view(torch.int32)[0])
     return n_tiles, ws[at:at + 16 * n_tiles].view(torch.int32).view(-1, 4)[:, :3].cpu()
 
