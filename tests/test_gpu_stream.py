@@ -8,7 +8,7 @@ import torch
 from helpers import (BF16_GATE, MX_COS_GATE, MX_FLIP_DELTA, MX_RELL2_GATE, cosine, mx_elementwise_gates, rel_clamp,
                      rel_l2)
 from oracle import moe_oracle as O
-from test_gpu_bf16 import _inputs
+from test_gpu_bf16 import _inputs, shuffle_runs
 from test_gpu_mxfp8 import _quantised_inputs, _routing_by_counts
 
 pytestmark = pytest.mark.gpu
@@ -180,3 +180,57 @@ def test_mx_crowded_schedules_use_work_lists(counts, lists, device):
     assert torch.isfinite(got).all()
     assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
     mx_elementwise_gates(got, ref, bound)
+
+
+@pytest.mark.parametrize("K,N,E,counts,rows", [
+    (256, 256, 40, EDGES, "stream"),    # streaming up kernel, H = 128 down
+    (512, 512, 40, EDGES, "stream"),    # H = 256 down
+    (256, 768, 256, SPARSE, "mixed"),    # ring up kernel, general streaming down kernel with half a slab (H = 384)
+    (512, 768, 64, [33, 16, 12] + [1] * 9, "stream"),  # general streaming kernels in both directions
+    (256, 2048, 40, EDGES, "ring"),     # ring kernels without a work list
+    (256, 512, 4, [400, 300, 257, 129], "list"),  # ring kernels with one
+])
+def test_mx_kernels_with_dropped_rows_and_blocks(K, N, E, counts, rows, device):
+    """x with fewer rows than the schedule names (single holes and whole groups of four rows inside live fragments: a copy
+    instruction of the loaders each), a block of an expert that does not exist, a schedule cut behind its last pair."""
+    import prime_moe
+    counts = counts + [0] * (E - len(counts))
+    counts[-1] += sum(counts) % 2
+    ids, wts = _routing_by_counts(counts, 2, device, seed=K + N)
+    T = ids.shape[0]
+    keep = (3 * T) // 5
+    jobs, cus = min(E, 2 * keep) * (N // 256), torch.cuda.get_device_properties(device).multi_processor_count
+    assert (rows == "list") == (2 * keep > (64 if jobs < cus // 2 else 24) * E)  # the rules of the dispatch
+    assert rows != "ring" or (jobs >= cus and N > 512 and 2 * keep > 4 * E)
+    g, a, deq = _quantised_inputs(T, K, E, N, device, seed=N)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    s = shuffle_runs(s, counts, g)
+    at = groups = 0
+    for c in counts:  # rows 4 .. 7 of a run: a group without a token where the run has four dropped rows
+        gone = (s[at:at + c] >= 2 * keep).nonzero().flatten()[:4]
+        if c >= 12 and gone.numel() == 4:
+            run = s[at:at + c].clone()
+            rest = torch.ones(c, dtype=torch.bool, device=device)
+            rest[gone] = False
+            s[at:at + c] = torch.cat([run[rest][:4], run[gone], run[rest][4:]])
+            groups += 1
+        at += (c + 127) // 128 * 128
+    assert groups >= 2
+    e_bad = e.clone()
+    e_bad[1] = E + 3
+    w_ref = wts.clone()
+    lost = s[128:256]
+    w_ref.view(-1)[lost[lost >= 0].long()] = 0.0
+    ref, bound = O.fused_moe_dense(deq["x"], deq["w1"], deq["w2"], ids.cpu(), w_ref.cpu(), act_mx=True, flip_delta=MX_FLIP_DELTA)
+    ref, bound = ref[:keep], bound[:keep]
+    last = int((s >= 0).nonzero().max()) + 1
+    for length in (s.numel(), last):
+        torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+        out = torch.empty((keep, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_mxfp8(a["x"][:keep].contiguous(), a["x_scales"][:keep].contiguous(), a["w1"], a["w1_scales"], a["w2"],
+                                  a["w2_scales"], s[:length].contiguous(), e_bad, n, wts, out, 2, 128, 64, 4, 2, 1, True)
+        torch.cuda.synchronize()
+        got = out.float().cpu()
+        assert torch.isfinite(got).all()
+        assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
+        mx_elementwise_gates(got, ref, bound)
