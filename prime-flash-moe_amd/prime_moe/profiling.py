@@ -17,6 +17,11 @@ figures, the derived table) and replaces the config's lines in ``<out>/kernel_fi
 table ``bench.py`` reads its ``roofline.traffic`` from:
 
     <config> <kernel> avg_us <float> fetch_bytes <int> write_bytes <int> mfma_busy <float> lds_conflict <float>
+
+    python prime-flash-moe_amd/prime_moe/profiling.py --layers bf16_decode_1,bf16_decode_29 [--out profiles]
+
+traces whole layers instead (router or moe_align, quantiser, fused op; the cases of ``perf/cases.py``), which reach the kernels
+that the benchmark workloads do not take, and writes the duration of every kernel to ``<out>/layers.md``.
 """
 from __future__ import annotations
 
@@ -30,8 +35,13 @@ import subprocess
 import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
-KERNELS = ("moe_up_kernel", "moe_up_join_kernel", "moe_down_kernel", "finalize_kernel", "moe_prologue_kernel",
-           "copy_calibration_kernel")
+# key -> what a kernel's demangled name holds
+KERNELS = {k: k for k in ("moe_up_kernel", "moe_up_join_kernel", "moe_down_kernel", "finalize_kernel", "moe_prologue_kernel")}
+KERNELS.update({"moe_stream_up_kernel": "moe_stream_kernel<true", "moe_stream_down_kernel": "moe_stream_kernel<false",
+                "moe_stream_up_kernel_mx": "moe_stream_kernel_mx<true", "moe_stream_down_kernel_mx": "moe_stream_kernel_mx<false"})
+KERNELS.update({k: k for k in ("moe_stream_down_short_kernel", "route_topk_kernel", "route_small_kernel", "moe_align_kernel",
+                               "align_runs_kernel", "align_count_kernel", "align_bases_kernel", "align_scatter_kernel",
+                               "quantize_mx_kernel", "copy_calibration_kernel")})
 SQ_COUNTERS = ["SQ_BUSY_CYCLES", "SQ_VALU_MFMA_BUSY_CYCLES", "SQ_INSTS_VALU_MFMA_MOPS_{DT}", "SQ_LDS_BANK_CONFLICT",
                "SQ_ACTIVE_INST_LDS", "SQ_WAIT_INST_LDS", "SQ_WAVE_CYCLES", "SQ_WAIT_ANY"]
 EA_COUNTERS = ["TCC_EA0_RDREQ_sum", "TCC_EA0_RDREQ_LEVEL_sum", "TCC_EA0_RDREQ_DRAM_CREDIT_STALL_sum", "TCC_BUSY_sum"]
@@ -39,8 +49,8 @@ GIB_KIB = 1048576.0
 
 
 def short(name: str) -> str:
-    for k in KERNELS:
-        if k in name:
+    for k, part in KERNELS.items():
+        if part in name:
             return k
     return ""
 
@@ -99,13 +109,64 @@ def simds_per_shader_engine(out_dir) -> float:
     return 32.0
 
 
+def run_layer(name, passes):
+    """Passes of one case of perf/cases.py: what --layers traces."""
+    sys.path.insert(0, ROOT)
+    os.chdir(ROOT)
+    import torch
+    from perf import cases
+    state = cases.prepare(next(c for c in cases.listed() if c["name"] == name), 0)
+    torch.cuda.synchronize()
+    for _ in range(passes):
+        cases.run(state)
+    torch.cuda.synchronize()
+
+
+def profile_layers(names, out, workdir):
+    lines = ["# rocprofv3 summary: whole layers", "",
+             "Cases of `perf/cases.py` (router or `moe_align`, quantiser, fused op), one MI355X.  Written by",
+             f"`python prime-flash-moe_amd/prime_moe/profiling.py --layers {','.join(names)}`, which runs for each case",
+             "`rocprofv3 --kernel-trace --stats -- python3 prime-flash-moe_amd/prime_moe/profiling.py --run-layer <case>`.",
+             "Launches of the 20 passes and of the preparation of the inputs (mxfp8 weights are quantised there); a kernel's median",
+             "is that of a pass.", "", "| case | kernel | launches | median us | shortest us |", "|---|---|---|---|---|"]
+    for name in names:
+        d = os.path.join(workdir, "layer_" + name)
+        shutil.rmtree(d, ignore_errors=True)
+        cmd = ["timeout", "-s", "KILL", "120", "rocprofv3", "--kernel-trace", "--stats", "-d", d, "-o", "out", "--output-format", "csv",
+               "--", "python3", os.path.abspath(__file__), "--run-layer", name]
+        res = subprocess.run(cmd, cwd="/tmp", env=dict(os.environ, TMPDIR="/tmp"), capture_output=True, text=True)
+        if res.returncode != 0:
+            sys.exit(f"profiler run of {name} failed (rc {res.returncode}):\n{res.stdout[-2000:]}\n{res.stderr[-2000:]}")
+        times = collections.defaultdict(list)
+        for f in glob.glob(os.path.join(d, "**", "*kernel_trace.csv"), recursive=True):
+            for r in csv.DictReader(open(f)):
+                k = short(r["Kernel_Name"])
+                if k:
+                    times[k].append((int(r["Start_Timestamp"]), int(r["End_Timestamp"]) - int(r["Start_Timestamp"])))
+        for k, v in sorted(times.items(), key=lambda kv: min(kv[1])[0]):
+            ns = sorted(t for _, t in v)
+            lines.append(f"| {name} | {k} | {len(ns)} | {ns[len(ns) // 2] / 1e3:.1f} | {ns[0] / 1e3:.1f} |")
+        print(f"traced {name}", flush=True)
+    os.makedirs(out, exist_ok=True)
+    with open(os.path.join(out, "layers.md"), "w") as f:
+        f.write("\n".join(lines) + "\n")
+    print("\n".join(lines))
+
+
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--config", required=True)
+    what = ap.add_mutually_exclusive_group(required=True)
+    what.add_argument("--config")
+    what.add_argument("--layers", help="cases of perf/cases.py, comma separated")
+    what.add_argument("--run-layer", help=argparse.SUPPRESS)
     ap.add_argument("--split", type=int, default=1)
     ap.add_argument("--out", default=os.path.join(ROOT, "profiles"))
     ap.add_argument("--workdir", default=os.path.join(ROOT, "gpurun_out", "prof"))
     a = ap.parse_args()
+    if a.run_layer:
+        return run_layer(a.run_layer, 20)
+    if a.layers:
+        return profile_layers(a.layers.split(","), a.out, a.workdir)
     sys.path.insert(0, os.path.join(ROOT, "prime-flash-moe_amd"))
     dt = "bf16" if "bf16" in a.config else "mxfp8"
     sq = [c.replace("{DT}", "BF16" if dt == "bf16" else "F8") for c in SQ_COUNTERS]
@@ -138,8 +199,8 @@ def main():
               "| kernel | avg duration | fetched past L2 | written past L2 | sum | algorithmic bytes | rate | MFMA busy | LDS conflict cycles / LDS active | waiting on LDS | read latency past L2 | DRAM credit stalls |",
               "|---|---|---|---|---|---|---|---|---|---|---|---|"]
     figs = []
-    for k in KERNELS[:5]:
-        if k not in stats:
+    for k in KERNELS:
+        if k not in stats or k == "copy_calibration_kernel":
             continue
         us = stats[k]["avg_ns"] / 1e3
         fb = fetch.get(k, {}).get("FETCH_SIZE", (0.0, 0))[0] * 1024 * f_scale
