@@ -55,9 +55,9 @@ int pmoe_moe_align(const int32_t *topk_ids, int32_t *sorted_token_ids, int32_t *
 /*
  * The same sort with scratch memory from the caller, which lets it spread over many
  * workgroups (two launches) when n is large; no counterpart in the reference, whose
- * kernel is one thread block for any n.  The first query returns the least scratch that
- * does so (0 for n <= 16384), the second what spreads it as far as it pays (0 for
- * n <= 8192); where a query returns 0 `workspace` may be null, and with a null or too small
+ * kernel is one thread block for any n.  The first query returns scratch that does so for
+ * any n (0 for n <= 16384; a few words more than the sort uses), the second what spreads it
+ * as far as it pays (0 for n <= 8192); where a query returns 0 `workspace` may be null, and with a null or too small
  * workspace the call falls back to a single workgroup.  Same output, bit for bit.
  * A workspace that is not 4-byte aligned is an error where the first query asks for one and
  * gets it, and not used otherwise.

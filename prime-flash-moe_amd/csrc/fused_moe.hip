@@ -64,6 +64,9 @@ __device__ __forceinline__ bool resolve_job(const MoeArgs &a, Job &j) {
         j.nb = 1;
         j.wt = ((int)blockIdx.x - j.first * n_jobs) * a.per_job;
         j.n_sub = min(a.per_job, a.n_wtiles - j.wt);
+        // (Ids past the total name the last expert, so that one's last block counts as shared.  Compared with live blocks only
+        // its weights would be read with the hint too: 100 tokens that all name the last of 257 experts, K 7168, N 512, took
+        // 260 us instead of 245, the tail of the up kernel being that expert's two tiles.)
         j.w_once = (j.first == 0 || a.expert_ids[j.first - 1] != j.e) &&
                    (j.first + 1 >= a.n_blocks || a.expert_ids[j.first + 1] != j.e);
         return true;
@@ -333,10 +336,10 @@ __device__ __forceinline__ void setup_ring_loader(ring::Loader<RB> &ld, const ri
 // workgroups that share a weight tile off the same HBM channel at the same instant, and stays short
 // enough that they still meet in L2 (a 16-phase, 4 KB spread read 30 % more from HBM for the same time).
 // Without a work list and with rows of whole 4 KB there are 32 phases.  Neighbouring weight tiles then run side by side all
-// over the chip and the same bytes of all their rows lie on few channels: with 8 phases the up kernel took 194 us at 24
-// tokens x top 2 on 8 experts of K 4096 x N 28672 (168 with 32 phases; 171 in the order of the work lists), the down kernel 101
-// at 16384 x 7168 (80; 106), both kernels 301 at 64 tokens on 32 experts of K 4096 x N 8192 (273; 307).  Rows of other
-// lengths start on different channels by themselves (K 7168: 155 and 155).
+// over the chip and the same bytes of all their rows lie on few channels.  Us with 8 phases / with 32 / in the order of
+// the work lists: up kernel at 24 tokens x top 2 on 8 experts of K 4096 x N 28672 192 / 160 / 177, down kernel of K 7168 x N
+// 16384 at 64 tokens 94 / 81 / 106, the whole op at 64 tokens on 32 experts of K 4096 x N 8192 298 / 272 / 305.  Rows of other
+// lengths start on different channels by themselves (K 7168: 152 and 152).
 template <int RB>
 __device__ __forceinline__ int slab_rotation(const MoeArgs &a, int n_slabs) {
     const int phases = a.work == nullptr && (n_slabs * RB) % 4096 == 0 ? 4096 / RB : 8;
@@ -497,8 +500,9 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
     const int tok_region = grp ? lay.group1_off : 0;
     const int SB = lay.stage_bytes, NS = lay.stages;
     // the ring is free after main_loop (it ends with a barrier): its head holds the 128 x 256 output
-    // tiles of the live groups (none for tiles of one fragment, which store from registers); the
-    // next weight tile's copies start in the first stage clear of them, under this tile's epilogue
+    // tiles of the live groups (none for tiles of one fragment, which store from registers); the next weight
+    // tile's copies start in the first stage clear of them, under this tile's epilogue (if there is one: the tiles of two full
+    // blocks take both stages)
     const int epi_bytes = NTF == 1 ? 0 : (ntf1 > 0 ? 2 : 1) * kBlockRows * kYPitch;
     const int free0 = (epi_bytes + SB - 1) / SB;
     int stage0 = 0, n_pre = 0;
@@ -873,8 +877,10 @@ int phase_mask() { return g_phase_mask; }
 static thread_local int g_tiles_per_wg = 0;
 
 // A workgroup of the mxfp8 kernels can keep its token rows and take several weight tiles in a row: it
-// saves the set-up of all but the first and starts each tile's copies under the epilogue of the one
-// before, but the coarser work balances worse over the CUs.  Two tiles when that leaves enough rounds of workgroups
+// saves the set-up of all but the first and starts each tile's copies under the epilogue of the one before, as far as
+// the ring has stages behind the epilogue's tiles (up kernel: one of two on tiles of two full blocks; down kernel: one of
+// three on a full block, none on two, whose y tiles take the whole ring), but the coarser work balances worse over the
+// CUs.  Two tiles when that leaves enough rounds of workgroups
 // per CU: 8 for the down kernel, whose tiles are short, 32 for the up kernel (blocks are paired to row tiles, hence
 // 16 and 64 in terms of blocks).  Two against one tile, K = N = 2048 on 32 experts: down 137 / 145 us at 12000 tokens,
 // 1272 / 1390 at 131072; up 985 / 994 at 65536 tokens (64 per CU), 1893 / 1992 at 131072, but 401 / 394 at 24593 and

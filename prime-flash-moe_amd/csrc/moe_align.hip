@@ -2,8 +2,9 @@
 //
 // Semantics follow the reference kernel (prime_moe/csrc/kernels/fused_moe_bf16_kernel.cu:853-907)
 // except that the within-expert order is made unique (ascending pair id) instead of being
-// left to an atomic race.  Up to kSingleMaxIds ids one workgroup does it (align_sort.h): ranks inside the waves,
-// per-expert counts of the waves -> bases, padded totals -> prefix, scatter.  More ids spread over workgroups.
+// left to an atomic race.  Up to kFewIds ids, or any number without scratch memory, one workgroup does it (align_sort.h):
+// ranks inside the waves, per-expert counts of the waves -> bases, padded totals -> prefix, scatter.  More ids spread over
+// workgroups if the caller gives scratch (pmoe_moe_align_static, which has its own, does so above kSingleMaxIds).
 // Ids, positions and sizes are int32 (loops that step past a size near 2^31 count in int64), and the output is a pure function of the input.
 #include <algorithm>
 #include <mutex>

@@ -143,9 +143,9 @@ __device__ __forceinline__ void store_once(void *p, uint4 q) {
     v[0] = (int)q.x; v[1] = (int)q.y; v[2] = (int)q.z; v[3] = (int)q.w;
     __builtin_nontemporal_store(v, reinterpret_cast<i32x4 *>(p));
 }
-constexpr int kActPitchBf16 = 272;  // 128 bf16 + 16 B pad: 16-byte aligned rows, 2-way conflicts at most
-constexpr int kActPitchFp8 = 144;   // 128 e4m3 + 16 B pad
-constexpr int kYPitch = 528;        // 256 bf16 + 16 B pad
+// Epilogue tiles of the mxfp8 kernels in LDS: 16-byte aligned rows.
+constexpr int kActPitchFp8 = 144;  // 128 e4m3 + 16 B pad
+constexpr int kYPitch = 528;       // 256 bf16 + 16 B pad
 
 // CU count of the current device, rounded down to a multiple of the 8 XCDs.
 int resident_grid();

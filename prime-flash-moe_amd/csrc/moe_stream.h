@@ -53,7 +53,8 @@ struct Loader {
     bool tok_live[2];       // this lane's token row holds a token
     bool tok_any[2];        // wave-uniform: some lane's does
     int lps;                // instructions per stage
-    bool w_once;            // wave-uniform: the weights are read by this pass only
+    bool w_once;            // wave-uniform: the block reads the weights in one pass (other blocks of the expert, rare where
+                            // these kernels run, are not looked for)
 
     __device__ __forceinline__ void issue(char *stage, int tok_bytes, int wave, uint32_t koff) const {
 #pragma unroll
