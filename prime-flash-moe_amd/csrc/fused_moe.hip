@@ -962,9 +962,12 @@ static int launch_direct_pipeline(MoeArgs a, const SchedBuffers &sb, void *out, 
     // narrow jobs while wide tiles do not give every CU one (us at 128 / 256 / 640 / 1024 wide jobs, stream against
     // ring, whole op: 75.5 / 81.7, 130 / 129, 291 / 290, 419 / 406)
     const bool stream_up = blocks * n_wt_up < n_cus;
-    // (256 experts, K 7168, H 2048, stream against ring, whole op: 71.6 / 75.5 us at 1 token, 126 / 130 at 2,
-    // 288 / 291 at 5, 408 / 406 at 8; 32 experts with 8 rows each, K 2048, H 1024: 45.0 / 44.6)
-    const bool stream_down = a.H <= 256 || (blocks * n_wt_down < 5 * n_cus && (int64_t)a.M * a.top_k <= 4 * blocks);
+    // Narrow jobs while the wide tiles are few and hold a row each, or do not give every CU one and hold a few (stream
+    // against ring, whole op, us; 256 experts, K 7168, H 2048: 71.6 / 75.5 at 1 token, 126 / 130 at 2, 288 / 291 at 5, 408 / 406
+    // at 8; 8 experts, K 4096, H 14336: 206 / 232 at 4 tokens x top 2, 266 / 295 at 16; 64 experts, K 2048, tokens x top 4: H 384
+    // 33.8 / 34.1 at 12, 47.8 / 41.9 at 32, H 1536 75.1 / 82.2, 105 / 105; 128 experts, K 2048, H 768, top 8: 125.9 / 120.1 at 64)
+    const int64_t down_jobs = blocks * n_wt_down;
+    const bool stream_down = a.H <= 256 || (down_jobs < 5 * n_cus && (int64_t)a.M * a.top_k <= (down_jobs <= n_cus ? 4 : 1) * blocks);
     auto launch_stream = [&](auto kernel, int n_tiles) {
         const int grid = (int)std::min<int64_t>((int64_t)a.n_blocks * std::max(n_tiles, 1), 2 * n_cus);
         if (grid > 0) hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, s, a, n_tiles);

@@ -115,7 +115,9 @@ SPARSE = [129, 65, 64, 33, 32, 5] + [1] * 60
     (2304, 512, 40, EDGES, True),      # more slabs than stages, a last group of turns that is not full
     (256, 2048, 40, EDGES, False),     # ring kernels without a work list
     (256, 768, 256, SPARSE, True),     # general streaming down kernel, H = 384: the last slab has one half
-    (1024, 512 + 256, 256, SPARSE, False),
+    (1024, 512 + 256, 256, SPARSE, False),  # ring down kernel: two rows a tile, four tiles per CU
+    (1024, 512 + 256, 60, [33, 16, 5] + [2] * 40, True),  # general streaming down kernel, up to four rows a tile
+    (1024, 512 + 256, 300, [1] * 200, False),             # likewise, a row each and more tiles than CUs
     (2048, 8192, 11, [129, 33, 31, 20, 15, 10, 8, 6, 5, 4, 3], True),  # ring kernels, activation rows of 4 KB: 32 phases of the K walk
 ])
 def test_mx_kernels_without_a_schedule_at_row_edges(K, N, E, counts, split, device):
