@@ -581,6 +581,8 @@ __device__ __forceinline__ void emit_work(int4 *work, int n_wt, int per_job, int
 // block-wide scans per 256 blocks, then one pass over the tiles that writes the two walk orders).
 // All workgroups invert the sorted order: inv[pair id] = sorted row.  Entries of pairs that are not
 // in the schedule keep whatever the buffer held; the reader validates an entry against sorted_ids.
+// CROWD: only for crowded schedules (`n_cus`: see crowded_mx).
+template <bool CROWD>
 __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert_ids, const int32_t *ntpp,
                                                            int n_blocks, int2 *tiles, int *n_tiles,
                                                            int4 *work_up, int n_wt_up, int per_job_up, int grid_up,
@@ -588,8 +590,8 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
                                                            int grid_down, int num_experts,
                                                            const int32_t *sorted_ids, int sorted_num, int32_t *inv,
                                                            int n_pairs, int do_invert, const uint8_t *x_scales,
-                                                           uint32_t *xs_tiled, int nkt, int top_k, int M, int crowd) {
-    if (crowd && !crowded_mx(ntpp, n_blocks, n_pairs, n_wt_up, crowd)) return;
+                                                           uint32_t *xs_tiled, int nkt, int top_k, int M, int n_cus) {
+    if (CROWD && !crowded_mx(ntpp, n_blocks, n_pairs, n_wt_up, n_cus)) return;
     if (blockIdx.x == 0 && tiles != nullptr) {
         __shared__ int s_max[4], s_sum[4], s_carry[2];
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -942,7 +944,7 @@ static void launch_prologue(const MoeArgs &a, const SchedBuffers &sb, int per_up
     // the work lists are needed by the two kernels even when the rest of the prologue is masked off
     const int do_invert = (g_phase_mask & PMOE_PHASE_PROLOGUE) ? 1 : 0;
     const int blocks = do_invert ? std::max(1, std::min((a.sorted_num + 255) / 256, a.crowd ? 48 : 1024)) : 1;
-    hipLaunchKernelGGL(moe_prologue_kernel, dim3(blocks), dim3(256), 0, s, a.expert_ids, a.ntpp, a.n_blocks, sb.tiles, sb.n_tiles,
+    hipLaunchKernelGGL(a.crowd ? moe_prologue_kernel<true> : moe_prologue_kernel<false>, dim3(blocks), dim3(256), 0, s, a.expert_ids, a.ntpp, a.n_blocks, sb.tiles, sb.n_tiles,
                        sb.work_up, a.H / 128, per_up, grid_up, sb.work_down, (a.K + kWRows - 1) / kWRows, per_down, grid_down, a.E,
                        a.sorted_ids, a.sorted_num, a.inv, a.M * a.top_k, do_invert, a.x_scales, a.xs_tiled, a.K >> 7, a.top_k, a.M,
                        a.crowd);
