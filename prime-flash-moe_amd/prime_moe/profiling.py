@@ -33,6 +33,7 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 # key -> what a kernel's demangled name holds
@@ -60,7 +61,7 @@ def run_pass(tag, prof_args, bench_args, workdir, log):
     shutil.rmtree(out_dir, ignore_errors=True)
     cmd = ["rocprofv3", *prof_args, "-d", out_dir, "-o", "out", "--output-format", "csv", "--",
            "python3", os.path.join(ROOT, "bench.py"), *bench_args]
-    log.append(" ".join(cmd).replace(ROOT, "$R").replace(workdir.replace(ROOT, "$R"), "$R/gpurun_out/prof"))
+    log.append(" ".join(cmd).replace(workdir, "$OUT").replace(ROOT, "$R"))
     env = dict(os.environ, TMPDIR="/tmp")
     res = subprocess.run(["timeout", "-s", "KILL", "240", *cmd], cwd="/tmp", env=env, capture_output=True, text=True)
     if res.returncode != 0:
@@ -161,7 +162,7 @@ def main():
     what.add_argument("--run-layer", help=argparse.SUPPRESS)
     ap.add_argument("--split", type=int, default=1)
     ap.add_argument("--out", default=os.path.join(ROOT, "profiles"))
-    ap.add_argument("--workdir", default=os.path.join(ROOT, "gpurun_out", "prof"))
+    ap.add_argument("--workdir", default=os.path.join(tempfile.gettempdir(), "prime_moe_profile"))
     a = ap.parse_args()
     if a.run_layer:
         return run_layer(a.run_layer, 20)
@@ -190,7 +191,7 @@ def main():
     lines = [f"# rocprofv3 summary: fused-MoE pipeline, {a.config}", "",
              f"Workload `{a.config}` of `prime_moe/workloads.py`, `split={bool(a.split)}`, one MI355X.  Written by",
              f"`python prime-flash-moe_amd/prime_moe/profiling.py --config {a.config} --split {a.split}`, which runs (from `/tmp`,",
-             "`TMPDIR=/tmp`, `$R` = repository root):", ""]
+             "`TMPDIR=/tmp`, `$R` = repository root, `$OUT` = the working directory of the profiler):", ""]
     lines += ["    " + c for c in cmds]
     lines += ["", "`--calibrate-copy` adds launches of `copy_calibration_kernel`, a plain copy that reads 1 GiB and writes 1 GiB:",
               f"FETCH_SIZE reads {cal_f:,.0f} KiB for it (scale factor {f_scale:.2f}), WRITE_SIZE {cal_w:,.0f} KiB (scale factor {w_scale:.2f}).",
