@@ -82,49 +82,29 @@ __device__ __forceinline__ bool resolve_job(const MoeArgs &a, Job &j) {
     return true;
 }
 
-template <int NG>
+// The sorted rows of a row tile: two blocks, one per group of four waves.
 struct RowInfo {
-    int tok[kBlockRows * NG];   // token index of each sorted row, -1 for padding / dropped rows
-    int pair[kBlockRows * NG];  // its pair id (the row of y it writes), -1 likewise
-    int nvalid[NG];             // per group: 1 + index of the last live row
+    int id[2 * kBlockRows];  // up kernel: token, down kernel: pair id (the row of y it writes); -1 for padding / dropped rows
+    int nvalid[2];           // per group: 1 + index of the last live row
 };
 
 // Fills RowInfo for the `nb` blocks starting at `first`; returns the largest number of 32-row
-// fragments holding live rows in any group.
-template <int NG>
-__device__ __forceinline__ int load_row_info(const MoeArgs &a, int first, int nb, RowInfo<NG> &ri) {
+// fragments up to the last live row in any group.
+template <bool TOKENS>
+__device__ __forceinline__ int load_row_info(const MoeArgs &a, int first, int nb, RowInfo &ri) {
     const int tid = threadIdx.x;
-    if (tid < NG) ri.nvalid[tid] = 0;
+    if (tid < 2) ri.nvalid[tid] = 0;
     __syncthreads();
-    if (tid < kBlockRows * NG) {
-        const int g = tid >> 7;
-        int tok = -1, pair = -1;
-        if (g < nb) {
-            const int s = first * kBlockRows + tid;
-            const int p = (s < a.sorted_num) ? a.sorted_ids[s] : -1;
-            if (p >= 0 && p / a.top_k < a.M) {
-                tok = p / a.top_k;
-                pair = p;
-            }
-        }
-        ri.tok[tid] = tok;
-        ri.pair[tid] = pair;
-        if (tok >= 0) atomicMax(&ri.nvalid[g], (tid & 127) + 1);
+    if (tid < 2 * kBlockRows) {
+        const int g = tid >> 7, s = first * kBlockRows + tid;
+        const int p = g < nb && s < a.sorted_num ? a.sorted_ids[s] : -1;
+        const int tok = p / a.top_k;
+        const bool ok = p >= 0 && tok < a.M;
+        ri.id[tid] = ok ? (TOKENS ? tok : p) : -1;
+        if (ok) atomicMax(&ri.nvalid[g], (tid & 127) + 1);
     }
     __syncthreads();
-    int m = 0;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) m = max(m, (ri.nvalid[g] + 31) >> 5);
-    return m;
-}
-
-__device__ __forceinline__ void zero_acc(f32x16 (&acc)[2][4]) {
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[f][t][i] = 0.f;
+    return (max(ri.nvalid[0], ri.nvalid[1]) + 31) >> 5;
 }
 
 // Epilogue of the down GEMM.  Weight rows (output columns) sit on the MFMA M side: register i of lane
@@ -269,12 +249,11 @@ __device__ __forceinline__ void store_act_tile(const MoeArgs &a, const char *til
 // halves start at w_base[0/1] with `w_pitch` bytes per row.  Scales (mxfp8): `tok_sc_off(row)` /
 // `w_sc_off(row)` are the byte offsets of the row's first 4-scale dword; the dword of the next 128-wide
 // K tile lies 512 bytes on in the blocked weight scales, tok_sc_step in the token side's (512 if they are tiled,
-// 4 in a row-major matrix).  Only the live 32-row
-// fragments of the two blocks (ntf0, ntf1 of them) are copied; they are packed one after the other in
-// the stage (see ring::Layout).
+// 4 in a row-major matrix).  Only rows up to the last live one of each block are copied; those of the two blocks are
+// packed one after the other in the stage (see ring::Layout).
 template <int DT, int RB, typename TokOff, typename TokScOff, typename WScOff>
 __device__ __forceinline__ void setup_ring_loader(ring::Loader<RB> &ld, const ring::Layout &lay, int tid,
-                                                  uint32_t w_pitch, int ntf0, int ntf1, const RowInfo<2> &ri,
+                                                  uint32_t w_pitch, const RowInfo &ri,
                                                   bool w_once, TokOff tok_row_off,
                                                   const uint8_t *tok_sc_base, uint32_t tok_sc_step, TokScOff tok_sc_off,
                                                   const uint8_t *w_sc_base, WScOff w_sc_off) {
@@ -288,35 +267,35 @@ __device__ __forceinline__ void setup_ring_loader(ring::Loader<RB> &ld, const ri
         ld.w_off[q] = (uint32_t)row * w_pitch + gchunk;
         ld.w_dst[0][q] = lay.w_off + row0 * RB;
         ld.w_dst[1][q] = ld.w_dst[0][q] + 128 * RB;
-        const int frag = row0 >> 5;  // the instruction's rows lie in this 32-row fragment
-        ld.tok_dst[0][q] = ld.tok_dst[1][q] = -1;
-        ld.tok_off[0][q] = ld.tok_off[1][q] = 0;
-        ld.tok_live[0][q] = frag < ntf0 && ri.tok[row] >= 0;
-        ld.tok_live[1][q] = frag < ntf1 && ri.tok[kBlockRows + row] >= 0;
-        if (__ballot(ld.tok_live[0][q]) != 0) {
-            ld.tok_dst[0][q] = row0 * RB;
-            ld.tok_off[0][q] = tok_row_off(row) + gchunk;
-        }
-        if (__ballot(ld.tok_live[1][q]) != 0) {
-            ld.tok_dst[1][q] = lay.group1_off + row0 * RB;
-            ld.tok_off[1][q] = tok_row_off(kBlockRows + row) + gchunk;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            ld.tok_dst[g][q] = -1;
+            ld.tok_off[g][q] = 0;
+            ld.tok_live[g][q] = ri.id[g * kBlockRows + row] >= 0;
+            if (__ballot(ld.tok_live[g][q]) != 0) {
+                ld.tok_dst[g][q] = g * lay.group1_off + row0 * RB;
+                ld.tok_off[g][q] = tok_row_off(g * kBlockRows + row) + gchunk;
+            }
         }
     }
     ld.sc_base = nullptr;
     ld.sc_off = 0;
     ld.sc_step = 0;
     ld.sc_dst = -1;
+    ld.sc_live = true;
     if constexpr (DT == DT_FP8) {
         if (wave >= 4) {  // weight rows 64 (wave - 4) + lane
             const int row = 64 * (wave - 4) + lane;
             ld.sc_base = reinterpret_cast<const char *>(w_sc_base);
             ld.sc_off = w_sc_off(row);
             ld.sc_step = 512u;
-            ld.sc_dst = lay.scale_off + (lay.scale_tok_rows + 64 * (wave - 4)) * 4;
+            ld.sc_dst = lay.scale_off + (lay.tok_rows + 64 * (wave - 4)) * 4;
         } else if (64 * wave < lay.tok_rows) {
-            // packed token rows 64 wave + lane (the lanes past the last live row repeat it)
-            const int c = min(64 * wave + lane, lay.tok_rows - 1);
-            const int row = c < 32 * ntf0 ? c : kBlockRows + c - 32 * ntf0;
+            // packed token rows 64 wave + lane
+            const int c = 64 * wave + lane;
+            ld.sc_live = c < lay.tok_rows;
+            const int cc = min(c, lay.tok_rows - 1);
+            const int row = cc < lay.rows0 ? cc : kBlockRows + cc - lay.rows0;
             ld.sc_base = reinterpret_cast<const char *>(tok_sc_base);
             ld.sc_off = tok_sc_off(row);
             ld.sc_step = tok_sc_step;
@@ -346,23 +325,43 @@ __device__ __forceinline__ int slab_rotation(const MoeArgs &a, int n_slabs) {
     return (int)((blockIdx.x >> 3) & (phases - 1)) % n_slabs;
 }
 
-// Up kernel tile on the stage ring: the live fragments of one or two row blocks x activation
+template <int NTF>
+__device__ __forceinline__ void zero_acc(f32x16 (&acc)[2][4]) {
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int t = 0; t < NTF; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[f][t][i] = 0.f;
+}
+// Runs the tile code of a group with `ntf` live fragments.  The two groups of a workgroup may take different cases: the
+// barriers of all of them are the same.
+template <typename Run>
+__device__ __forceinline__ void by_fragments(int ntf, Run run) {
+    switch (ntf) {
+        case 0: run(std::integral_constant<int, 0>{}); break;
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        default: run(std::integral_constant<int, 4>{}); break;
+    }
+}
+
+// Bytes of a group's activation tile and its scales, one behind the other at the head of the ring.
+constexpr int kActTileBytes = kBlockRows * kActPitchFp8 + kBlockRows * 4;
+
+// Up kernel tile on the stage ring: the live rows of one or two row blocks x activation
 // columns [128 ht, 128 ht + 128).  LDS weight rows 0..127 are gate rows, 128..255 the matching up rows;
 // wave v of a group owns gate/up rows 32v..32v+31 so gate and up of one activation element sit in the
 // same lane and register.
 template <int DT, int RB, int NTF>
-__device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, RowInfo<2> &ri, char *lds,
-                                             uint32_t *act_sc_lds) {
+__device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, int rows0, int rows1, const RowInfo &ri, char *lds) {
     constexpr int ES = 1;  // bytes per element
     const int first = job.first, ht = job.wt, n_sub = job.n_sub, e = job.e;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, w4 = wave & 3, gt = tid & 255;
     const int K = a.K, H = a.H, N = a.N;
-    const int ntf0 = __builtin_amdgcn_readfirstlane((ri.nvalid[0] + 31) >> 5);
-    const int ntf1 = __builtin_amdgcn_readfirstlane((ri.nvalid[1] + 31) >> 5);
-    const int my_ntf = grp ? ntf1 : ntf0;
-    const bool active = my_ntf > 0;
-    const ring::Layout lay = ring::make_layout<DT, RB>(ntf0, ntf1, ring::ring_bytes<DT>());
+    const ring::Layout lay = ring::make_layout<DT, RB>(rows0, rows1, ring::ring_bytes<DT>());
 
     int h0 = ht * 128;
     const int n_slabs = (K * ES) / RB;
@@ -372,14 +371,14 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, R
     ld.w_base[1] = ld.w_base[0] + (int64_t)H * K * ES;
     const uint32_t row_bytes = (uint32_t)(K * ES);
     const int kb = K >> 5, kt128 = K >> 7;
+    auto token = [&](int row) { return (uint32_t)max(ri.id[row], 0); };
     setup_ring_loader<DT, RB>(
-        ld, lay, tid, row_bytes, ntf0, ntf1, ri, job.w_once,
-        [&](int row) { return (uint32_t)max(ri.tok[row], 0) * row_bytes; },
+        ld, lay, tid, row_bytes, ri, job.w_once, [&](int row) { return token(row) * row_bytes; },
         a.work != nullptr ? reinterpret_cast<const uint8_t *>(a.xs_tiled + (int64_t)first * kt128 * kBlockRows) : a.x_scales,
         a.work != nullptr ? 512u : 4u,
         [&](int row) {
             return a.work != nullptr ? (uint32_t)(((row >> 7) * kt128 * kBlockRows + (row & 127)) * 4)
-                                     : (uint32_t)(max(ri.tok[row], 0) * kb);
+                                     : (uint32_t)(token(row) * kb);
         },
         a.w1_scales + (int64_t)e * N * kb,
         [&](int row) { return (uint32_t)blocked_scale_off((row < 128 ? h0 : H + h0 - 128) + row, 0, K >> 7); });
@@ -388,22 +387,17 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, R
     const int start = slab_rotation<RB>(a, n_slabs);
     const int tok_region = grp ? lay.group1_off : 0;
     // the ring is free after main_loop (it ends with a barrier): its head holds the activation tiles
-    constexpr int kPitch = kActPitchFp8;
-    char *tile = lds + grp * (kBlockRows * kPitch);
-    uint32_t *sc_tile = act_sc_lds + grp * kBlockRows;
+    char *tile = lds + grp * kActTileBytes;
+    uint32_t *sc_tile = reinterpret_cast<uint32_t *>(tile + kBlockRows * kActPitchFp8);
     const int SB = lay.stage_bytes, NS = lay.stages;
     // first stage clear of the activation tiles: the next weight tile's copies start there, under
     // the epilogue of this one
-    const int epi_bytes = (ntf1 > 0 ? 2 : 1) * kBlockRows * kPitch;
-    const int free0 = (epi_bytes + SB - 1) / SB;
+    const int free0 = ((rows1 > 0 ? 2 : 1) * kActTileBytes + SB - 1) / SB;
     int stage0 = 0, n_pre = 0;
     for (int sub = 0; sub < n_sub; ++sub) {
         f32x16 acc[2][4];
-        zero_acc(acc);
-        if (active)
-            ring::main_loop<DT, RB, NTF, true>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
-        else
-            ring::main_loop<DT, RB, NTF, false>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
+        zero_acc<NTF>(acc);
+        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
         const bool more = sub + 1 < n_sub;
         if (more) {
             // same token rows, the next 128 gate and 128 up rows of the expert
@@ -415,63 +409,56 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, R
             n_pre = max(NS - free0, 0);
             ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, stage0, n_pre);
         }
-        if (active) swiglu_epilogue<DT, NTF>(acc, tile, sc_tile, w4, lane);
+        swiglu_epilogue<DT, NTF>(acc, tile, sc_tile, w4, lane);
         __syncthreads();
-        if (active) store_act_tile<DT>(a, tile, sc_tile, (int64_t)(first + grp) * kBlockRows, h0, my_ntf, gt);
+        if (NTF > 0) store_act_tile<DT>(a, tile, sc_tile, (int64_t)(first + grp) * kBlockRows, h0, NTF, gt);
         if (more) __syncthreads();  // the tiles have been read: the head of the ring may be filled again
         h0 += 128;
     }
 }
 
-// LDS plan of the mxfp8 kernels: ring, row table, activation scales side by side.
+// LDS plan of the mxfp8 kernels: ring and row table.
 template <int DT>
 struct SplitLds {
-    static constexpr int kRowInfoBytes = 2304;  // >= sizeof(RowInfo<2>)
     static constexpr int kRing = ring::ring_bytes<DT>();
     static constexpr int kRowInfoOff = kRing;
-    static constexpr int kActScaleOff = kRowInfoOff + kRowInfoBytes;
-    static constexpr int kTotal = kActScaleOff + kBlockRows * 2 * 4;
-    static_assert(sizeof(RowInfo<2>) <= kRowInfoBytes, "row table does not fit its slot");
+    static constexpr int kTotal = 160 * 1024;
+    static_assert(kRowInfoOff + sizeof(RowInfo) <= kTotal, "row table does not fit its slot");
     // the epilogues reuse the head of the ring: two y tiles (down kernel) or two activation tiles (up kernel)
     static_assert(2 * kBlockRows * kYPitch <= kRing, "y tiles of the epilogue overrun their LDS");
-    static_assert(2 * kBlockRows * kActPitchFp8 <= kRing, "activation tiles of the epilogue overrun the ring");
+    static_assert(2 * kActTileBytes <= kRing, "activation tiles of the epilogue overrun the ring");
 };
 
 template <int DT>
 __global__ __launch_bounds__(512) void moe_up_kernel(MoeArgs a) {
     using L = SplitLds<DT>;
     __shared__ __attribute__((aligned(1024))) char lds[L::kTotal];
-    RowInfo<2> &ri = *reinterpret_cast<RowInfo<2> *>(lds + L::kRowInfoOff);
+    RowInfo &ri = *reinterpret_cast<RowInfo *>(lds + L::kRowInfoOff);
     settle_lists(a);
     if (a.work == nullptr) stream::invert(a, 512);  // (no prologue did)
     Job j;
     if (!resolve_job(a, j)) return;
-    const int ntf = load_row_info<2>(a, j.first, j.nb, ri);
-    if (ntf == 0) return;
-    uint32_t *act_sc_lds = reinterpret_cast<uint32_t *>(lds + L::kActScaleOff);
-    if (ntf == 1) up_tile_ring<DT, ring::kRB, 1>(a, j, ri, lds, act_sc_lds);
-    else if (ntf == 2) up_tile_ring<DT, ring::kRB, 2>(a, j, ri, lds, act_sc_lds);
-    else up_tile_ring<DT, ring::kRB, 4>(a, j, ri, lds, act_sc_lds);
+    if (load_row_info<true>(a, j.first, j.nb, ri) == 0) return;
+    const int rows0 = __builtin_amdgcn_readfirstlane(ri.nvalid[0]), rows1 = __builtin_amdgcn_readfirstlane(ri.nvalid[1]);
+    const int my_rows = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) ? rows1 : rows0;
+    by_fragments((my_rows + 31) >> 5, [&](auto n) { up_tile_ring<DT, ring::kRB, decltype(n)::value>(a, j, rows0, rows1, ri, lds); });
 }
 
 // Down kernel tile on the stage ring: y[rows, 256 cols of K] = act[rows, :H] . W2[e][cols, :H]^T, the
 // whole reduction over H inside the workgroup; the
-// routing weights are applied later, by finalize_kernel.
+// routing weights are applied later, by finalize_kernel.  `ntf`: fragments of the larger group.
 template <int DT, int RB, int NTF>
-__device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job, RowInfo<2> &ri, char *lds) {
+__device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job, int ntf, int rows0, int rows1, const RowInfo &ri,
+                                               char *lds) {
     constexpr int ES = 1;  // bytes per element
     const int first = job.first, kt = job.wt, n_sub = job.n_sub, e = job.e;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, w4 = wave & 3, gt = tid & 255;
     const int K = a.K, H = a.H;
     const int64_t row0 = (int64_t)first * kBlockRows;
-    const int ntf0 = __builtin_amdgcn_readfirstlane((ri.nvalid[0] + 31) >> 5);
-    const int ntf1 = __builtin_amdgcn_readfirstlane((ri.nvalid[1] + 31) >> 5);
-    const int my_ntf = grp ? ntf1 : ntf0;
-    const int my_rows = ri.nvalid[grp];  // rows past the last live one are never read back
-    const int my_pair = ri.pair[grp * kBlockRows + (lane & 31)];  // (tiles of one fragment store from registers)
-    const bool active = my_ntf > 0;
-    const ring::Layout lay = ring::make_layout<DT, RB>(ntf0, ntf1, ring::ring_bytes<DT>());
+    const int my_rows = grp ? rows1 : rows0;  // rows past the last live one are never read back
+    const int my_pair = ri.id[grp * kBlockRows + (lane & 31)];  // (tiles of one fragment store from registers)
+    const ring::Layout lay = ring::make_layout<DT, RB>(rows0, rows1, ring::ring_bytes<DT>());
 
     int k0 = kt * kWRows;
     const uint32_t row_bytes = (uint32_t)(H * ES);
@@ -489,7 +476,7 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
     };
     set_weights(k0);
     setup_ring_loader<DT, RB>(
-        ld, lay, tid, row_bytes, ntf0, ntf1, ri, job.w_once, [&](int row) { return (uint32_t)row * row_bytes; },
+        ld, lay, tid, row_bytes, ri, job.w_once, [&](int row) { return (uint32_t)row * row_bytes; },
         reinterpret_cast<const uint8_t *>(a.act_scales + (int64_t)first * ht128 * kBlockRows), 512u,
         [&](int row) { return (uint32_t)(((row >> 7) * ht128 * kBlockRows + (row & 127)) * 4); },
         a.w2_scales + (int64_t)e * K * hb,
@@ -503,16 +490,13 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
     // tiles of the live groups (none for tiles of one fragment, which store from registers); the next weight
     // tile's copies start in the first stage clear of them, under this tile's epilogue (if there is one: the tiles of two full
     // blocks take both stages)
-    const int epi_bytes = NTF == 1 ? 0 : (ntf1 > 0 ? 2 : 1) * kBlockRows * kYPitch;
+    const int epi_bytes = ntf == 1 ? 0 : (rows1 > 0 ? 2 : 1) * kBlockRows * kYPitch;
     const int free0 = (epi_bytes + SB - 1) / SB;
     int stage0 = 0, n_pre = 0;
     for (int sub = 0; sub < n_sub; ++sub) {
         f32x16 acc[2][4];
-        zero_acc(acc);
-        if (active)
-            ring::main_loop<DT, RB, NTF, true>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
-        else
-            ring::main_loop<DT, RB, NTF, false>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
+        zero_acc<NTF>(acc);
+        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
         const bool more = sub + 1 < n_sub;
         if (more) {
             set_weights(k0 + kWRows);
@@ -522,13 +506,13 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
             ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, stage0, n_pre);
         }
         const YDst dst = y_destination(a, k0);
-        if constexpr (NTF == 1) {
-            if (active) store_y_direct(dst, acc, my_rows, w4, lane, my_pair);
+        if (ntf == 1) {
+            if (NTF > 0) store_y_direct(dst, acc, my_rows, w4, lane, my_pair);
         } else {
             char *tile = lds + grp * (kBlockRows * kYPitch);
-            if (active) y_epilogue<NTF>(acc, tile, w4, lane);
+            y_epilogue<NTF>(acc, tile, w4, lane);
             __syncthreads();
-            if (active) store_y_tile(dst, tile, my_rows, gt, ri.pair + grp * kBlockRows);
+            if (NTF > 0) store_y_tile(dst, tile, my_rows, gt, ri.id + grp * kBlockRows);
             if (more) __syncthreads();  // the tiles have been read: the head of the ring may be filled again
         }
         k0 += kWRows;
@@ -539,15 +523,15 @@ template <int DT>
 __global__ __launch_bounds__(512) void moe_down_kernel(MoeArgs a) {
     using L = SplitLds<DT>;
     __shared__ __attribute__((aligned(1024))) char lds[L::kTotal];
-    RowInfo<2> &ri = *reinterpret_cast<RowInfo<2> *>(lds + L::kRowInfoOff);
+    RowInfo &ri = *reinterpret_cast<RowInfo *>(lds + L::kRowInfoOff);
     settle_lists(a);
     Job j;
     if (!resolve_job(a, j)) return;
-    const int ntf = load_row_info<2>(a, j.first, j.nb, ri);
+    const int ntf = load_row_info<false>(a, j.first, j.nb, ri);
     if (ntf == 0) return;
-    if (ntf == 1) down_tile_ring<DT, ring::kRB, 1>(a, j, ri, lds);
-    else if (ntf == 2) down_tile_ring<DT, ring::kRB, 2>(a, j, ri, lds);
-    else down_tile_ring<DT, ring::kRB, 4>(a, j, ri, lds);
+    const int rows0 = __builtin_amdgcn_readfirstlane(ri.nvalid[0]), rows1 = __builtin_amdgcn_readfirstlane(ri.nvalid[1]);
+    const int my_rows = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) ? rows1 : rows0;
+    by_fragments((my_rows + 31) >> 5, [&](auto n) { down_tile_ring<DT, ring::kRB, decltype(n)::value>(a, j, ntf, rows0, rows1, ri, lds); });
 }
 
 // Walk order of the tiles of one mxfp8 kernel: [group of 8 weight tiles][row tile][weight tile in group].

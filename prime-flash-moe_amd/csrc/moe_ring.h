@@ -8,14 +8,15 @@
 // every wave holds the slab's remaining operands in registers, so that up to all stages are in flight while the last
 // third of the matrix instructions of a slab runs (see main_loop).
 //
-// The ring is sized per tile.  A stage holds only the 32-row token fragments that have live rows
-// (group 0's first, then group 1's), the 256 weight rows and, for mxfp8, the scale dwords of both;
-// as many stages as fit the LDS budget are used, at most 8.  The fewer token rows a tile has, the
+// The ring is sized per tile.  A stage holds only the token rows up to a group's last live one (group 0's first,
+// then group 1's, each rounded up to the 8 rows of a copy instruction), the 256 weight rows and the scale dwords of
+// both; as many stages as fit the LDS budget are used, at most 8.  The fewer token rows a tile has, the
 // closer it is to a pure stream of weights from HBM, and what keeps HBM busy then is weight bytes in
-// flight per CU.
+// flight per CU.  (Rounded up to whole 32-row fragments, tiles of 129 to 160 rows had two stages instead of three: with
+// 128 rows per expert on average that is every second expert.)
 //
-// Stage layout: [live token rows][RB] [256 weight rows][RB] [scale dwords: token rows rounded up to a
-// multiple of 64, then weight rows (mxfp8)].
+// Stage layout: [token rows][RB] [256 weight rows][RB] [scale dwords: token rows, weight rows].  Operand reads of a group's
+// last fragment run past its rows into what lies behind them, which only reaches output rows nobody reads.
 // A row is RB/16 chunks of 16 B; chunk c of row r sits in slot c ^ swizzle(r), swizzle(r) = (r >> 1) & 7: the 16-byte MFMA operand reads of 16 consecutive rows then cover all 64 LDS
 // banks exactly once.  The copy engine writes lane l of a wave instruction to bytes [16 l, 16 l + 16)
 // behind a wave-uniform base (one instruction = 1 KB = 1024 / RB rows), so the swizzle is applied on
@@ -46,32 +47,34 @@ __device__ __forceinline__ int swz(int row) {
 
 // Geometry of a tile's ring; every member is wave-uniform.
 struct Layout {
-    int tok_rows;        // live token rows of both groups: 32 (ntf0 + ntf1)
-    int group1_off;      // byte offset of group 1's token rows inside a stage
-    int w_off;           // byte offset of the weight rows
-    int scale_off;       // byte offset of the scale dwords (mxfp8)
-    int scale_tok_rows;  // token scale dwords reserved: tok_rows rounded up to 64
+    int rows0;        // token rows of group 0 in a stage, a multiple of 8
+    int tok_rows;     // of both groups
+    int group1_off;   // byte offset of group 1's token rows inside a stage
+    int w_off;        // byte offset of the weight rows
+    int scale_off;    // byte offset of the scale dwords (mxfp8)
     int stage_bytes;
     int stages;
 };
+// rows0, rows1: 1 + index of each group's last live row.
 template <int DT, int RB>
-__device__ __forceinline__ Layout make_layout(int ntf0, int ntf1, int budget) {
+__device__ __forceinline__ Layout make_layout(int rows0, int rows1, int budget) {
     Layout l;
-    l.tok_rows = 32 * (ntf0 + ntf1);
-    l.group1_off = 32 * ntf0 * RB;
+    l.rows0 = (rows0 + 7) & ~7;
+    l.tok_rows = l.rows0 + ((rows1 + 7) & ~7);
+    l.group1_off = l.rows0 * RB;
     l.w_off = l.tok_rows * RB;
     l.scale_off = l.w_off + kWRows * RB;
-    l.scale_tok_rows = (l.tok_rows + 63) & ~63;
-    const int bytes = l.scale_off + (DT == DT_FP8 ? (l.scale_tok_rows + kWRows) * 4 : 0);
+    const int bytes = l.scale_off + (DT == DT_FP8 ? (l.tok_rows + kWRows) * 4 : 0);
     l.stage_bytes = (bytes + 255) & ~255;
     l.stages = min(kMaxStages, budget / l.stage_bytes);
     return l;
 }
-// LDS the ring may use, a multiple of 1 KB (the split kernels put their row table behind it).
+// LDS the ring may use, a multiple of 256 bytes (the kernels put their row table behind it).  Three stages hold up to 152
+// token rows.
 template <int DT>
 constexpr int ring_bytes() {
     static_assert(DT == DT_FP8, "the stage ring serves the mxfp8 kernels");
-    return 156 * 1024;
+    return 160 * 1024 - 1280;
 }
 
 __device__ __forceinline__ uint32_t lds_addr(const char *p) {
@@ -128,8 +131,8 @@ __device__ __forceinline__ void wait_and_barrier_dyn(int n) {
 
 // Per-thread description of the copies of one stage.  A 128-row block of token rows or half of the
 // weight tile takes N = RB / 64 instructions of every wave: instruction q of wave w moves rows
-// q * 8 * rpc + rpc * w .. + rpc - 1 of it (rpc = 1024 / RB rows per instruction).  Token rows of
-// fragments without live rows are not copied, nor are the rows without a token inside a live fragment
+// q * 8 * rpc + rpc * w .. + rpc - 1 of it (rpc = 1024 / RB rows per instruction).  Token rows behind the last
+// live one are not copied, nor are rows without a token in front of it
 // (an instruction whose rows all lack one is dropped: the wait counts rely on every issued
 // instruction having an active lane).  Scales: at most one 4-byte-per-lane instruction per
 // wave.
@@ -144,6 +147,7 @@ struct Loader {
     const char *sc_base;  // wave-uniform: activation scales or weight scales
     uint32_t sc_off;      // this lane's row in them
     uint32_t sc_step;     // bytes between consecutive 128-wide K tiles: 4 (row major) or 512 (blocked)
+    bool sc_live;         // this lane has a row
     int tok_dst[2][N];    // LDS offset inside a stage of this wave's token rows; -1: nothing to copy
     bool tok_live[2][N];  // this lane's row holds a token (rows without one are not fetched: what the
                           // stage holds for them only reaches their own, unused, output rows)
@@ -177,7 +181,7 @@ struct Loader {
                 if (tok_live[b][q]) copy16(tok_base + koff, tok_off[b][q], stage + tok_dst[b][q]);
             }
         } else if (sc_dst >= 0) {
-            copy4(sc_base + (uint32_t)slab * sc_step, sc_off, stage + sc_dst);
+            if (sc_live) copy4(sc_base + (uint32_t)slab * sc_step, sc_off, stage + sc_dst);
         }
     }
     __device__ __forceinline__ void issue(char *stage, int slab) const {
@@ -229,8 +233,9 @@ __device__ __forceinline__ void pre_issue(const Loader<RB> &ld, const Layout &la
         ld.issue(lds + st * SB, slab);
     }
 }
-// K loop.  COMPUTE = false is the loop of the waves without matrix work (a group without live
-// rows): they only issue their share of the copies and join the barriers.  `tok_region` = byte
+// K loop of a group with NTF live fragments.  NTF = 0 is the loop of the waves without matrix work (a group without live
+// rows): they only issue their share of the copies and join the barriers, which are the same ones for every
+// NTF: the two groups of a tile need not have the same number.  `tok_region` = byte
 // offset of this wave's group inside a stage's token rows.
 //
 // The slabs are visited in rotated order, starting at slab `start`: workgroups
@@ -240,7 +245,7 @@ __device__ __forceinline__ void pre_issue(const Loader<RB> &ld, const Layout &la
 // Geometry and wait counts are wave-uniform run-time values (the wait count goes through a switch).
 //
 // A slab's stage is given back (second barrier) before its matrix instructions are done.  NTF <= 2: all operands of a
-// slab are read first.  NTF = 4 has registers for one 64-wide step: the operands of step 1 replace those of step 0 as
+// slab are read first.  NTF = 3 and 4 have registers for one 64-wide step: the operands of step 1 replace those of step 0 as
 // these are used up, the stage goes back behind step 0, the copies into it are spread over the matrix instructions of
 // step 1 (a wave waits where the CU's copy path does not take its next copy: issued in one run, 9 copies held up the
 // wave's matrix instructions), and the barrier that opens the next slab sits in the middle of step 1, whose second
@@ -253,7 +258,7 @@ __device__ __forceinline__ void pre_issue(const Loader<RB> &ld, const Layout &la
 // Slab 0 goes to stage `stage0`, the following ones to the stages behind it (wrapping).  `n_pre`: the
 // caller has already issued slabs 0 .. n_pre - 1 (see pre_issue; a workgroup that runs one tile
 // after another issues them under the previous tile's epilogue).
-template <int DT, int RB, int NTF, bool COMPUTE>
+template <int DT, int RB, int NTF>
 __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][4], const Loader<RB> &ld, const Layout &lay, char *lds,
                                           int n_slabs, const int (&wrow)[2], int lane, int tok_region, int start,
                                           int stage0 = 0, int n_pre = 0) {
@@ -282,13 +287,13 @@ __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][4], const Loader<RB> 
     int cur_off = stage0 * SB;  // stage of slab kt
     auto next = [&](int off) { return off + SB >= NS * SB ? 0 : off + SB; };
     open(0);
-    if constexpr (COMPUTE) {
+    if constexpr (NTF > 0) {
         const int r = lane & 31, half = lane >> 5, sh = 8 * half;
         const int off0 = r * RB + ((half ^ swz<RB>(r)) << 4);
         const int w_at[2] = {lay.w_off + wrow[0] * RB, lay.w_off + wrow[1] * RB};
         const int tok_sc_at = lay.scale_off + (tok_region / RB + r) * 4;
-        const int w_sc_at[2] = {lay.scale_off + (lay.scale_tok_rows + wrow[0] + r) * 4,
-                                lay.scale_off + (lay.scale_tok_rows + wrow[1] + r) * 4};
+        const int w_sc_at[2] = {lay.scale_off + (lay.tok_rows + wrow[0] + r) * 4,
+                                lay.scale_off + (lay.tok_rows + wrow[1] + r) * 4};
         auto read_a = [&](Operands<NTF> &o, int f, const char *st, int j) { o.a[f] = lds_frag(st + w_at[f], off0 ^ (64 * j)); };
         auto read_b = [&](Operands<NTF> &o, int t, const char *st, int j) { o.b[t] = lds_frag(st + tok_region + t * 32 * RB, off0 ^ (64 * j)); };
         auto read_sa = [&](Operands<NTF> &o, int f, const char *st) { o.sa[f] = *reinterpret_cast<const int *>(st + w_sc_at[f]); };

@@ -87,6 +87,30 @@ def _routing_by_counts(counts, top_k, device, seed):
     return ids.to(device), wts.to(device)
 
 
+@pytest.mark.parametrize("K,N,split", [(1024, 768, True), (2048, 512, False)])
+def test_row_counts_round_the_edges_of_fragments_and_copies(K, N, split, device):
+    # a tile's token rows are copied in runs of 8 and multiplied in fragments of 32, the two halves of a tile may have
+    # different numbers of fragments, and the number of LDS stages changes with the rows (152 / 153)
+    import prime_moe
+    counts = [1, 7, 8, 9, 24, 25, 32, 33, 63, 64, 65, 95, 96, 97, 103, 127, 128, 129, 136, 137, 144, 145, 152, 153, 160, 161,
+              192, 193, 224, 225, 255, 256, 257, 384, 385]
+    counts.append(sum(counts) % 2)
+    E, top_k = len(counts), 2
+    ids, wts = _routing_by_counts(counts, top_k, device, seed=7)
+    T = ids.shape[0]
+    g, a, deq = _quantised_inputs(T, K, E, N, device, seed=23)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    out = torch.zeros((T, K), dtype=torch.bfloat16, device=device)
+    prime_moe.fused_moe_mxfp8(a["x"], a["x_scales"], a["w1"], a["w1_scales"], a["w2"], a["w2_scales"],
+                              *sched, wts, out, top_k, 128, 64, 4, 2, 1, split)
+    torch.cuda.synchronize()
+    ref, bound = O.fused_moe_dense(deq["x"], deq["w1"], deq["w2"], ids.cpu(), wts.cpu(), act_mx=True,
+                                   flip_delta=MX_FLIP_DELTA)
+    got = out.float().cpu()
+    assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
+    mx_elementwise_gates(got, ref, bound)
+
+
 @pytest.mark.parametrize("split", [True, False])
 def test_experts_with_one_and_with_several_row_tiles(split, device):
     # expert 0: 700 rows = three row tiles that share its weight rows; experts 1 - 3: one row tile of two
