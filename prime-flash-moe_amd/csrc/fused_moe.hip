@@ -108,32 +108,11 @@ __device__ __forceinline__ int load_row_info(const MoeArgs &a, int first, int nb
 }
 
 // Epilogue of the down GEMM.  Weight rows (output columns) sit on the MFMA M side: register i of lane
-// l = output column 64 w4 + 32 f + 8(i/4) + 4(l/32) + i%4 of sorted row 32 t + l%32.  The group's
-// 128 x 256 tile is rounded to bf16 into `tile` (row pitch kYPitch) ...
-template <int NTF>
-__device__ __forceinline__ void y_epilogue(const f32x16 (&acc)[2][4], char *tile, int w4, int lane) {
-    const int r = lane & 31, half = lane >> 5;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        if (t < NTF) {
-            const int row = 32 * t + r;
-#pragma unroll
-            for (int f = 0; f < 2; ++f)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int col = 64 * w4 + 32 * f + 8 * g + 4 * half;
-                    uint2 pk;
-                    pk.x = pack2_bf16(acc[f][t][4 * g], acc[f][t][4 * g + 1]);
-                    pk.y = pack2_bf16(acc[f][t][4 * g + 2], acc[f][t][4 * g + 3]);
-                    *reinterpret_cast<uint2 *>(tile + row * kYPitch + col * 2) = pk;
-                }
-        }
-    }
-}
-// Where a group's 128 x 256 output tile goes: the y rows of its pairs (y is indexed by pair id, row pitch
+// l = output column 64 w4 + 32 f + 8(i/4) + 4(l/32) + i%4 of sorted row 32 t + l%32.  Where the outputs of a tile of 256
+// columns go: the y rows of its pairs (y is indexed by pair id, row pitch
 // K; the last tile of a K that is not a multiple of 256 has 128 columns).
 struct YDst {
-    char *base;     // first column of the group's tile in row 0 of y
+    char *base;     // first column of the tile in row 0 of y
     int64_t pitch;  // bytes per row
     int cols;       // columns to write
 };
@@ -165,79 +144,78 @@ __device__ __forceinline__ void store_y_direct(const YDst &d, const f32x16 (&acc
             }
         }
 }
-// ... and its first n_rows rows are copied to the destination; gt = thread index inside the group,
-// `pair` = the pair ids of the group's 128 rows (rows without one are skipped).
-__device__ __forceinline__ void store_y_tile(const YDst &d, const char *tile, int n_rows, int gt, const int *pair) {
-    const int c = gt & 31;
-    if (8 * c >= d.cols) return;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int row = (gt >> 5) + 8 * i;
-        if (row < n_rows) {
-            const int dst_row = pair[row];
-            if (dst_row >= 0) {
-                const uint4 v = *reinterpret_cast<const uint4 *>(tile + row * kYPitch + c * 16);
-                store_once(d.base + dst_row * d.pitch + c * 16, v);
-            }
-        }
-    }
+// LDS written by some lanes of a wave is read by others of the same wave: LDS operations of a wave are executed in
+// order, only the compiler has to keep them so.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-// SwiGLU epilogue of the up GEMM, in registers: the 2H-wide gate/up tensor never leaves the chip.
-// acc[0] holds gate rows, acc[1] the matching up rows (weight rows on the MFMA M side: register i
-// of lane l = activation column 32 w4 + 8(i/4) + 4(l/32) + i%4 of token row 32 t + l%32).  The
-// 128 x 128 activation tile of the group is written to `tile` with row pitch kActPitch*, for the
-// coalesced copy to the workspace.
-// mxfp8: per token row and 32 columns, amax -> e8m0 scale + e4m3 values; a lane holds 16 of the 32
-// columns of one MX block, the partner lane (l ^ 32) the others.
-template <int DT, int NTF>
-__device__ __forceinline__ void swiglu_epilogue(const f32x16 (&acc)[2][4], char *tile, uint32_t *sc_tile,
-                                                int w4, int lane) {
+// Larger tiles: a wave rounds a fragment (token rows 32 t .. of its group) of its 64 columns to bf16, transposes it through a
+// scratch of its own, 16 rows at a time, and stores whole 128-byte lines.  `pair` = the pair ids of the fragment's rows (rows
+// without one are skipped).  Before, the groups' 128 x 256 tiles went through 132 KB of LDS: on two full blocks the first slabs of
+// the next weight tile could not be requested meanwhile, now they can (down kernel, 131072
+// tokens on 32 experts of K = N = 2048: 1331 -> 1298 us; 24593 tokens, K 2048 x N 8192: 812 -> 800).
+constexpr int kScratchRows = 16, kScratchPitch = 144;  // 128 B, 16 B pad
+constexpr int kScratchBytes = kScratchRows * kScratchPitch;
+__device__ __forceinline__ void store_y_fragment(const YDst &d, const f32x16 &lo, const f32x16 &hi, char *scratch, int w4, int lane,
+                                                 const int *pair) {
     const int r = lane & 31, half = lane >> 5;
+    const bool in_cols = 64 * w4 < d.cols;  // (a multiple of 128: a wave's 64 columns are inside or outside)
+    char *dst = d.base + 128 * w4 + (lane & 7) * 16;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        if (t < NTF) {
-            float v[16];
+    for (int h = 0; h < 2; ++h) {
+        if ((r >> 4) == h) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = swiglu(acc[0][t][i], acc[1][t][i]);
-            const int row = 32 * t + r;
-            static_assert(DT == DT_FP8, "the bf16 epilogue lives in fused_moe_bf16.hip");
-            float amax = 0.f;
+            for (int f = 0; f < 2; ++f)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
-            amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-            uint32_t e8;
-            float inv;
-            mx_block_scale(amax, e8, inv);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int hl = 32 * w4 + 8 * g + 4 * half;
-                const uint32_t q = pack4_e4m3(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3], inv);
-                *reinterpret_cast<uint32_t *>(tile + row * kActPitchFp8 + hl) = q;
-            }
-            if (half == 0) reinterpret_cast<uint8_t *>(sc_tile)[row * 4 + w4] = (uint8_t)e8;
+                for (int g = 0; g < 4; ++g) {
+                    const f32x16 &v = f ? hi : lo;
+                    uint2 pk;
+                    pk.x = pack2_bf16(v[4 * g], v[4 * g + 1]);
+                    pk.y = pack2_bf16(v[4 * g + 2], v[4 * g + 3]);
+                    *reinterpret_cast<uint2 *>(scratch + (r & 15) * kScratchPitch + 64 * f + 16 * g + 8 * half) = pk;
+                }
         }
+        wave_lds_order();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int row = (lane >> 3) + 8 * i, p = pair[16 * h + row];
+            const uint4 v = *reinterpret_cast<const uint4 *>(scratch + row * kScratchPitch + (lane & 7) * 16);
+            if (in_cols && p >= 0) store_once(dst + (int64_t)p * d.pitch, v);
+        }
+        wave_lds_order();
     }
 }
 
-// Coalesced copy of the first 32*ntf rows of a group's activation tile (pitch kActPitch*) to the
-// workspace rows row0.., columns [h0, h0+128); gt = thread index inside the group (0..255).
-template <int DT>
-__device__ __forceinline__ void store_act_tile(const MoeArgs &a, const char *tile, const uint32_t *sc_tile,
-                                               int64_t row0, int h0, int ntf, int gt) {
-    const int H = a.H;
-    static_assert(DT == DT_FP8, "the bf16 epilogue lives in fused_moe_bf16.hip");
-    const int c = gt & 7;
+// SwiGLU of the up GEMM, in registers: the 2H-wide gate/up tensor never leaves the chip.  `gate` and `up` hold gate rows and
+// the matching up rows of one token fragment (weight rows on the MFMA M side: register i of lane l = activation column
+// 8(i/4) + 4(l/32) + i%4 of the wave's 32 and of token row l%32).  Per token row amax -> e8m0 scale + e4m3 values: the wave's 32
+// columns are one MX block, of which a lane holds 16 and the lane 32 on the others.  The two swap what makes their 16 bytes
+// contiguous, and a row is stored in 32 bytes without a detour through LDS (`act`: the first of the wave's columns in the lane's
+// row, `scale`: the row's scale byte; `live`: the row is wanted).  Before, the group's 128 x 128 tile was collected in LDS and
+// stored in whole lines: two barriers, and the next weight tile's first slabs had to
+// stay clear of the 38 KB (with the down kernel's change below, both kernels at 131072 tokens on 32 experts of K = N = 2048:
+// 3455 -> 3400 us).
+__device__ __forceinline__ void swiglu_store(const f32x16 &gate, const f32x16 &up, char *act, uint8_t *scale, bool live, int half) {
+    float v[16], amax = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = (gt >> 3) + 32 * i;
-        if (i < ntf) {
-            uint4 v = *reinterpret_cast<const uint4 *>(tile + row * kActPitchFp8 + c * 16);
-            store_once(a.act + (row0 + row) * H + h0 + c * 16, v);
-        }
+    for (int i = 0; i < 16; ++i) v[i] = swiglu(gate[i], up[i]);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
+    amax = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+    uint32_t e8, q[4];
+    float inv;
+    mx_block_scale(amax, e8, inv);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) q[g] = pack4_e4m3(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3], inv);
+    // lanes < 32: both halves of q[0], q[1] (columns 0 .. 15), lanes >= 32: those of q[2], q[3]
+    const auto a = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false), b = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
+    if (live) {
+        store_once(act + 16 * half, make_uint4(a[0], a[1], b[0], b[1]));
+        if (half == 0) *scale = (uint8_t)e8;
     }
-    if (gt < 32 * ntf)
-        a.act_scales[((row0 >> 7) * (H >> 7) + (h0 >> 7)) * kBlockRows + gt] = sc_tile[gt];
 }
 
 // ==========================================================================================
@@ -347,9 +325,6 @@ __device__ __forceinline__ void by_fragments(int ntf, Run run) {
     }
 }
 
-// Bytes of a group's activation tile and its scales, one behind the other at the head of the ring.
-constexpr int kActTileBytes = kBlockRows * kActPitchFp8 + kBlockRows * 4;
-
 // Up kernel tile on the stage ring: the live rows of one or two row blocks x activation
 // columns [128 ht, 128 ht + 128).  LDS weight rows 0..127 are gate rows, 128..255 the matching up rows;
 // wave v of a group owns gate/up rows 32v..32v+31 so gate and up of one activation element sit in the
@@ -359,7 +334,8 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, i
     constexpr int ES = 1;  // bytes per element
     const int first = job.first, ht = job.wt, n_sub = job.n_sub, e = job.e;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = wave >> 2, w4 = wave & 3, gt = tid & 255;
+    const int grp = wave >> 2, w4 = wave & 3;
+    const int my_rows = grp ? rows1 : rows0;
     const int K = a.K, H = a.H, N = a.N;
     const ring::Layout lay = ring::make_layout<DT, RB>(rows0, rows1, ring::ring_bytes<DT>());
 
@@ -386,33 +362,27 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, i
     const int wrow[2] = {32 * w4, 128 + 32 * w4};
     const int start = slab_rotation<RB>(a, n_slabs);
     const int tok_region = grp ? lay.group1_off : 0;
-    // the ring is free after main_loop (it ends with a barrier): its head holds the activation tiles
-    char *tile = lds + grp * kActTileBytes;
-    uint32_t *sc_tile = reinterpret_cast<uint32_t *>(tile + kBlockRows * kActPitchFp8);
-    const int SB = lay.stage_bytes, NS = lay.stages;
-    // first stage clear of the activation tiles: the next weight tile's copies start there, under
-    // the epilogue of this one
-    const int free0 = ((rows1 > 0 ? 2 : 1) * kActTileBytes + SB - 1) / SB;
-    int stage0 = 0, n_pre = 0;
+    const int64_t row0 = (int64_t)(first + grp) * kBlockRows;
+    int n_pre = 0;
     for (int sub = 0; sub < n_sub; ++sub) {
         f32x16 acc[2][4];
         zero_acc<NTF>(acc);
-        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
-        const bool more = sub + 1 < n_sub;
-        if (more) {
-            // same token rows, the next 128 gate and 128 up rows of the expert
+        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, 0, n_pre);
+        if (sub + 1 < n_sub) {
+            // same token rows, the next 128 gate and 128 up rows of the expert; their first slabs under this tile's epilogue
             ld.w_base[0] += (int64_t)128 * K * ES;
             ld.w_base[1] += (int64_t)128 * K * ES;
             if (DT == DT_FP8 && wave >= 4) ld.sc_off += (uint32_t)kt128 * 512u;
             ld.make_uniform();
-            stage0 = free0 < NS ? free0 : 0;
-            n_pre = max(NS - free0, 0);
-            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, stage0, n_pre);
+            n_pre = lay.stages;
+            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, 0, n_pre);
         }
-        swiglu_epilogue<DT, NTF>(acc, tile, sc_tile, w4, lane);
-        __syncthreads();
-        if (NTF > 0) store_act_tile<DT>(a, tile, sc_tile, (int64_t)(first + grp) * kBlockRows, h0, NTF, gt);
-        if (more) __syncthreads();  // the tiles have been read: the head of the ring may be filled again
+#pragma unroll
+        for (int t = 0; t < NTF; ++t) {
+            const int row = 32 * t + (lane & 31);
+            uint8_t *scale = reinterpret_cast<uint8_t *>(a.act_scales + ((row0 >> 7) * (H >> 7) + (h0 >> 7)) * kBlockRows + row) + w4;
+            swiglu_store(acc[0][t], acc[1][t], a.act + (row0 + row) * H + h0 + 32 * w4, scale, row < my_rows, lane >> 5);
+        }
         h0 += 128;
     }
 }
@@ -424,9 +394,6 @@ struct SplitLds {
     static constexpr int kRowInfoOff = kRing;
     static constexpr int kTotal = 160 * 1024;
     static_assert(kRowInfoOff + sizeof(RowInfo) <= kTotal, "row table does not fit its slot");
-    // the epilogues reuse the head of the ring: two y tiles (down kernel) or two activation tiles (up kernel)
-    static_assert(2 * kBlockRows * kYPitch <= kRing, "y tiles of the epilogue overrun their LDS");
-    static_assert(2 * kActTileBytes <= kRing, "activation tiles of the epilogue overrun the ring");
 };
 
 template <int DT>
@@ -453,7 +420,7 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
     constexpr int ES = 1;  // bytes per element
     const int first = job.first, kt = job.wt, n_sub = job.n_sub, e = job.e;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = wave >> 2, w4 = wave & 3, gt = tid & 255;
+    const int grp = wave >> 2, w4 = wave & 3;
     const int K = a.K, H = a.H;
     const int64_t row0 = (int64_t)first * kBlockRows;
     const int my_rows = grp ? rows1 : rows0;  // rows past the last live one are never read back
@@ -486,34 +453,31 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
     const int start = slab_rotation<RB>(a, n_slabs);
     const int tok_region = grp ? lay.group1_off : 0;
     const int SB = lay.stage_bytes, NS = lay.stages;
-    // the ring is free after main_loop (it ends with a barrier): its head holds the 128 x 256 output
-    // tiles of the live groups (none for tiles of one fragment, which store from registers); the next weight
-    // tile's copies start in the first stage clear of them, under this tile's epilogue (if there is one: the tiles of two full
-    // blocks take both stages)
-    const int epi_bytes = ntf == 1 ? 0 : (rows1 > 0 ? 2 : 1) * kBlockRows * kYPitch;
-    const int free0 = (epi_bytes + SB - 1) / SB;
-    int stage0 = 0, n_pre = 0;
+    // the ring is free after main_loop (it ends with a barrier): its end holds the scratch of the waves (tiles of one fragment
+    // store from registers); the next weight tile's copies start in the stages in front of it, under this tile's epilogue
+    constexpr int kScratchOff = ring::ring_bytes<DT>() - 8 * kScratchBytes;
+    const int ahead = __builtin_amdgcn_readfirstlane(ntf == 1 ? NS : min(NS, kScratchOff / SB));
+    char *scratch = lds + kScratchOff + wave * kScratchBytes;
+    int n_pre = 0;
     for (int sub = 0; sub < n_sub; ++sub) {
         f32x16 acc[2][4];
         zero_acc<NTF>(acc);
-        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, stage0, n_pre);
+        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, 0, n_pre);
         const bool more = sub + 1 < n_sub;
         if (more) {
             set_weights(k0 + kWRows);
             ld.make_uniform();
-            stage0 = free0 < NS ? free0 : 0;
-            n_pre = max(NS - free0, 0);
-            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, stage0, n_pre);
+            n_pre = ahead;
+            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, 0, n_pre);
         }
         const YDst dst = y_destination(a, k0);
         if (ntf == 1) {
             if (NTF > 0) store_y_direct(dst, acc, my_rows, w4, lane, my_pair);
         } else {
-            char *tile = lds + grp * (kBlockRows * kYPitch);
-            y_epilogue<NTF>(acc, tile, w4, lane);
-            __syncthreads();
-            if (NTF > 0) store_y_tile(dst, tile, my_rows, gt, ri.id + grp * kBlockRows);
-            if (more) __syncthreads();  // the tiles have been read: the head of the ring may be filled again
+#pragma unroll
+            for (int t = 0; t < NTF; ++t)
+                store_y_fragment(dst, acc[0][t], acc[1][t], scratch, w4, lane, ri.id + grp * kBlockRows + 32 * t);
+            if (more && ahead < NS) __syncthreads();  // the scratch has been read: the ring may be filled there
         }
         k0 += kWRows;
     }
@@ -864,16 +828,15 @@ static thread_local int g_tiles_per_wg = 0;
 
 // A workgroup of the mxfp8 kernels can keep its token rows and take several weight tiles in a row: it
 // saves the set-up of all but the first and starts each tile's copies under the epilogue of the one before, as far as
-// the ring has stages behind the epilogue's tiles (up kernel: one of two on tiles of two full blocks; down kernel: one of
-// three on a full block, none on two, whose y tiles take the whole ring), but the coarser work balances worse over the
+// the ring has stages in front of the epilogue's scratch, but the coarser work balances worse over the
 // CUs.  Two tiles when that leaves enough rounds of workgroups
-// per CU: 8 for the down kernel, whose tiles are short, 32 for the up kernel (blocks are paired to row tiles, hence
-// 16 and 64 in terms of blocks).  Two against one tile, K = N = 2048 on 32 experts: down 137 / 145 us at 12000 tokens,
-// 1272 / 1390 at 131072; up 985 / 994 at 65536 tokens (64 per CU), 1893 / 1992 at 131072, but 401 / 394 at 24593 and
-// 234 / 224 at 12000; DeepSeek-V3-like prefill (32 per CU): down 3 % faster, up equal.  Four or eight lose on both.
+// per CU: 8 for the down kernel, whose tiles are short, 20 for the up kernel (blocks are paired to row tiles, hence
+// 16 and 40 in terms of blocks).  Two against one tile, K = N = 2048 on 32 experts: down 137 / 145 us at 12000 tokens,
+// 1272 / 1390 at 131072; up 974 / 1012 at 60000 tokens (59 blocks x weight tiles per CU), 1893 / 1992 at 131072, but 450 / 442 at
+// 24593 and 240 / 231 at 12000; DeepSeek-V3-like prefill (32 per CU): down 3 % faster, up equal.  Four or eight lose on both.
 static int tiles_per_workgroup(bool down, int n_blocks, int n_wt) {
     if (g_tiles_per_wg > 0) return std::min(g_tiles_per_wg, n_wt);
-    return (int64_t)n_blocks * n_wt >= (int64_t)resident_grid() * (down ? 16 : 64) ? std::min(2, n_wt) : 1;
+    return (int64_t)n_blocks * n_wt >= (int64_t)resident_grid() * (down ? 16 : 40) ? std::min(2, n_wt) : 1;
 }
 
 void launch_finalize(const MoeArgs &a, void *out, int split, int n_wt_down, hipStream_t s) {

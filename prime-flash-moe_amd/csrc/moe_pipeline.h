@@ -143,10 +143,6 @@ __device__ __forceinline__ void store_once(void *p, uint4 q) {
     v[0] = (int)q.x; v[1] = (int)q.y; v[2] = (int)q.z; v[3] = (int)q.w;
     __builtin_nontemporal_store(v, reinterpret_cast<i32x4 *>(p));
 }
-// Epilogue tiles of the mxfp8 kernels in LDS: 16-byte aligned rows.
-constexpr int kActPitchFp8 = 144;  // 128 e4m3 + 16 B pad
-constexpr int kYPitch = 528;       // 256 bf16 + 16 B pad
-
 // CU count of the current device, rounded down to a multiple of the 8 XCDs.
 int resident_grid();
 // Which phases of the pipeline the fused entry points enqueue (see pmoe_set_phase_mask).
