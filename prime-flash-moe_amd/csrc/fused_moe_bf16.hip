@@ -286,19 +286,8 @@ __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel_bf16(Moe
             KernelPlan kp{};
             kp.n_tiles = s_tiles[tid];
             estimate_kernel(kp.n_tiles, s_sum[4], n_wt, n_slabs, n_cus, kp.parts, kp.tail);
-            if (tid == 0) {
-                const int jobs_up = kp.n_tiles * n_wt_up;
-                int deep_parts = 1;
-                if (a.deep_ok && jobs_up > 0) deep_parts = min(min(kDeepParts, n_slabs / 4), n_cus / jobs_up);
-                if (deep_parts >= 2) {
-                    kp.deep = 1;
-                    kp.parts = deep_parts;
-                    kp.tail = 0;
-                }
-                a.plan->up = kp;
-            } else {
-                a.plan->down = kp;
-            }
+            if (tid == 0) a.plan->up = kp;
+            else a.plan->down = kp;
         }
     }
     if (do_invert) {
@@ -330,11 +319,10 @@ __device__ __forceinline__ int row_split(int &f0, int fg, int part, int parts) {
     return hi - lo;
 }
 
-// Where deep-mode partial sums of (part, fragment, weight tile) live: 2048 float4 = the two accumulators
-// (gate, up) of the four waves that own the fragment, [f][q][wave % 4][lane].
-__device__ __forceinline__ float4 *partial_block(const MoeArgs &a, int part, int frag, int wt) {
-    return reinterpret_cast<float4 *>(a.up_partials) +
-           (((int64_t)part * (4 * a.n_blocks) + frag) * a.n_wtiles + wt) * 2048;
+// Where the partial sums of (part of `parts`, fragment, weight tile) live: 2048 float4 = the two accumulators
+// (gate, up) of the four waves that own the fragment, [f][q][wave % 4][lane].  Fragments are numbered through the tiles.
+__device__ __forceinline__ float4 *partial_block(const MoeArgs &a, int part, int parts, int frag, int wt) {
+    return reinterpret_cast<float4 *>(a.up_partials) + (((int64_t)frag * a.n_wtiles + wt) * parts + part) * 2048;
 }
 
 // The queue of an XCD: its workgroups (workgroup w is number w / 8 of XCD w mod 8) start with the slot of their own
@@ -418,7 +406,8 @@ __device__ __forceinline__ void wave_lds_order() {
 // contraction slabs [slab0, slab0 + n_slabs).  LDS weight rows 0..127 are gate rows, 128..255 the matching up
 // rows; wave v of a group owns gate/up rows 32v..32v+31, so gate and up of one activation element sit in the
 // same lane and register: SwiGLU in registers, the 2H-wide tensor never leaves the chip.
-// deep_part >= 0: the contraction is shared (deep mode); the fp32 sums go to up_partials instead.
+// QUEUE = false (deep mode): the workgroup has this one job, whose contraction is shared; the fp32 sums go to up_partials
+// instead, from fragment number `deep_frag` on.
 // `pre`: the first slabs are on their way (tok_ahead: the offsets of their token rows); `next` returns the
 // job after this one, with `pre` and tok_ahead for it.
 struct UpTile {
@@ -438,9 +427,10 @@ __device__ __forceinline__ uint32_t gather_off(const MoeArgs &a, int64_t s, uint
     const int p = s < a.sorted_num ? a.sorted_ids[s] : -1;
     return ((uint32_t)p < (uint32_t)(a.M * a.top_k) ? (uint32_t)p / (uint32_t)a.top_k : 0u) * row_bytes;
 }
-template <int FG>
+template <int FG, bool QUEUE = true>
 __device__ __forceinline__ void up_tile_tall(const MoeArgs &a, const KernelPlan &kp, const Work &w, int *counter, char *lds,
-                                             bool &pre, uint32_t (&tok_ahead)[tall::kMaxFrags / 2], Work &next) {
+                                             bool &pre, uint32_t (&tok_ahead)[tall::kMaxFrags / 2], Work &next,
+                                             int deep_frag = 0) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, w4 = wave & 3;
     const int H = a.H;
@@ -454,28 +444,34 @@ __device__ __forceinline__ void up_tile_tall(const MoeArgs &a, const KernelPlan 
     f32x16 acc[2][FG];
     zero_acc<FG>(acc);
     int asked = 0;
-    tall::main_loop<FG>(acc, ld, lds, w.n_slabs, wrow, grp * FG, lane, k_start(w), pre, [&] { asked = ask_slot(counter); },
+    tall::main_loop<FG>(acc, ld, lds, w.n_slabs, wrow, grp * FG, lane, k_start(w), pre,
+                        [&] {
+                            if constexpr (QUEUE) asked = ask_slot(counter);
+                        },
                         [] {});
 
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
     const int r = lane_e & 31, half = lane_e >> 5;
+    if constexpr (!QUEUE) {
+#pragma unroll
+        for (int t = 0; t < FG; ++t) {
+            float4 *dst = partial_block(a, w.deep_part, w.parts, deep_frag + grp * FG + t, w.wt);
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    dst[((f * 4 + q) * 4 + w4) * 64 + lane_e] =
+                        make_float4(acc[f][t][4 * q], acc[f][t][4 * q + 1], acc[f][t][4 * q + 2], acc[f][t][4 * q + 3]);
+        }
+        return;
+    }
     char *scratch = lds + tall::kScratchOff + wave * tall::kScratchBytes;
     constexpr int kPitch = 80;  // 32 activation columns + 16 B pad
     int4 tl = make_int4(0, 0, 0, 0);
     pre = false;
     epilogue_with_links<FG, 3>(
         [&](int t) {
-            if (w.deep_part >= 0) {
-                float4 *dst = partial_block(a, w.deep_part, w.f0 + grp * FG + t, w.wt);
-#pragma unroll
-                for (int f = 0; f < 2; ++f)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        dst[((f * 4 + q) * 4 + w4) * 64 + lane_e] =
-                            make_float4(acc[f][t][4 * q], acc[f][t][4 * q + 1], acc[f][t][4 * q + 2], acc[f][t][4 * q + 3]);
-                return;
-            }
             // register i of lane_e l = activation column 32 w4 + 8(i/4) + 4(l/32) + i%4 of token row 32 t + l%32
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -556,32 +552,137 @@ __global__ __launch_bounds__(512) void moe_up_kernel_bf16(MoeArgs a) {
     });
 }
 
-// Deep mode: adds the partial sums the parts of every up job left in memory and finishes the tiles.  One
-// workgroup of 4 waves per (row tile, fragment of it, weight tile, quarter of the accumulator registers):
+// Few up jobs (at most kDeepJobs (block, weight tile) pairs, K >= 2048).  All of them together leave most CUs idle, so every
+// job's contraction is shared among up to kDeepParts workgroups, which store fp32 partial sums; moe_up_join_kernel adds them in
+// part order and applies SwiGLU.  There are at most 32 blocks: a wave of every workgroup works out the row tiles (a lane per
+// block) while the last workgroup writes what the kernels behind need, and no prologue runs in front.  Prologue, up kernel and join
+// before / up kernel and join, 8 experts of K 4096, N 512, top 4, us: 256 tokens 8.9 + 17.1 + 6.0 / 18.0 + 5.6, 100 tokens 8.4 + 12.1 +
+// 4.4 / 12.0 + 4.3.  With 12 and 16 parts the K loop is shorter by what the sums are longer: 25.1 and 25.2 us instead of 23.6 at 256.
+struct DeepTiles {
+    int4 tile[kDeepJobs];  // {first fragment, pairs of fragments, expert, first fragment's number}
+    int rows[kDeepJobs];   // of every block: 1 + its last live row
+    KernelPlan plan;
+};
+__global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_down, int n_cus, int plan_only) {
+    __shared__ __attribute__((aligned(1024))) char lds[tall::kLdsBytes];
+    DeepTiles &s = *reinterpret_cast<DeepTiles *>(lds);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned n_pairs = (unsigned)(a.M * a.top_k);
+    const int n_slabs = a.K * 2 / tall::kRB;
+    const int ntpp = a.ntpp[0], e_all = lane < a.n_blocks ? a.expert_ids[lane] : -1;
+    // the last live row of every block, a block per wave and turn
+    for (int blk = wave; blk < a.n_blocks; blk += 8) {
+        const int64_t at = (int64_t)blk * kBlockRows + lane;
+        const int id0 = at < a.sorted_num ? a.sorted_ids[at] : -1, id1 = at + 64 < a.sorted_num ? a.sorted_ids[at + 64] : -1;
+        const uint64_t m0 = __ballot((unsigned)id0 < n_pairs), m1 = __ballot((unsigned)id1 < n_pairs);
+        if (lane == 0) s.rows[blk] = m1 ? 128 - __builtin_clzll(m1) : m0 ? 64 - __builtin_clzll(m0) : 0;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int n_live = min((ntpp + kBlockRows - 1) / kBlockRows, a.n_blocks);
+        const bool live = lane < n_live;
+        const int e = live ? e_all : -1;
+        const uint64_t starts = __ballot(live && (lane == 0 || __shfl_up(e, 1, 64) != e));
+        const bool last = live && (lane + 1 == n_live || ((starts >> (lane + 1)) & 1));
+        const int run = 63 - __builtin_clzll((starts & ((2ull << lane) - 1)) | 1);  // first block of the lane's run
+        const int f2 = last && e >= 0 && e < a.E ? ((lane - run) * kBlockRows + s.rows[lane] + 63) >> 6 : 0;
+        const int n = (f2 + 5) / 6;
+        // tiles, runs and pairs of fragments (at most 32, 32 and 64) up to and including this lane, added up together
+        auto up_to = [&](int v) {
+#pragma unroll
+            for (int d = 1; d < kDeepJobs; d <<= 1) {
+                const int t = __shfl_up(v, d, 64);
+                if (lane >= d) v += t;
+            }
+            return v;
+        };
+        const int sums = up_to(n | (f2 > 0 ? 1 << 8 : 0) | f2 << 16), all = __shfl(sums, kDeepJobs - 1, 64);
+        const int tiles = sums & 0xff, runs = (sums >> 8) & 0xff, pairs = sums >> 16;
+        const int n_tiles = all & 0xff, n_runs = (all >> 8) & 0xff, n_f2 = all >> 16;
+        auto cut = [&](int4 *dst, int at, int count) {  // this lane's run in `count` tiles
+            int frag = 4 * run, number = 2 * (pairs - f2);
+            for (int q = 0; q < count; ++q) {
+                const int fg = f2 / count + (q < f2 % count ? 1 : 0);
+                dst[at + q] = make_int4(frag, fg, e, number);
+                frag += 2 * fg;
+                number += 2 * fg;
+            }
+        };
+        cut(s.tile, tiles - n, n);
+        KernelPlan kp{};
+        kp.n_tiles = n_tiles;
+        kp.deep = 1;
+        kp.parts = max(1, min(min(kDeepParts, n_slabs / 4), (int)gridDim.x / max(n_tiles * a.n_wtiles, 1)));
+        if (lane == 0) s.plan = kp;
+        if (blockIdx.x == gridDim.x - 1) {
+            // for the kernels behind: the tiles and plans, the sorted numbers of the fragments
+            const int want = choose_tiles(n_tiles, a.n_blocks, n_f2, n_wt_down, a.H * 2 / tall::kRB, n_cus), extra = max(want - n_tiles, 0);
+            const int mine = f2 > 0 ? min(f2, n + extra / n_runs + (runs <= extra % n_runs ? 1 : 0)) : 0;
+            const int at = up_to(mine), n_down = __shfl(at, kDeepJobs - 1, 64);
+            cut(a.tiles, tiles - n, n);
+            cut(a.tiles_down, at - mine, mine);
+            int *numbers = reinterpret_cast<int *>(a.runs);
+            for (int q = 0; q < 2 * f2; ++q) numbers[2 * (pairs - f2) + q] = 4 * run + q;
+            if (lane < 16) a.plan->counters[lane] = n_cus / 8;
+            if (lane == 0) {
+                KernelPlan down{};
+                down.n_tiles = n_down;
+                estimate_kernel(n_down, n_f2, n_wt_down, a.H * 2 / tall::kRB, n_cus, down.parts, down.tail);
+                a.plan->up = kp;
+                a.plan->down = down;
+                a.plan->deep_frags = 2 * n_f2;
+            }
+        }
+    }
+    __syncthreads();
+    KernelPlan kp{};
+    kp.n_tiles = __builtin_amdgcn_readfirstlane(s.plan.n_tiles);
+    kp.parts = __builtin_amdgcn_readfirstlane(s.plan.parts);
+    kp.deep = 1;
+    Work w = slot_work((int)(blockIdx.x >> 3), a.n_wtiles, kp);
+    // The sorted order is inverted by the workgroups without a job, or by all of them at the end.
+    const int busy = kp.n_tiles * a.n_wtiles * kp.parts, first = !plan_only && (int)gridDim.x - busy >= 16 ? busy : 0;
+    if (plan_only || w.state <= 0) {
+        if ((int)blockIdx.x >= first) stream::invert(a, 512, first);
+        return;
+    }
+    const int4 tl = s.tile[w.tile];
+    const int deep_frag = __builtin_amdgcn_readfirstlane(tl.w);
+    tile_work(w, tl, kp, n_slabs);
+    __syncthreads();  // the tiles have been read: the ring may be filled
+    bool pre = false;
+    uint32_t tok_ahead[tall::kMaxFrags / 2] = {};
+    Work next;
+    switch (w.fg) {
+        case 1: up_tile_tall<1, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
+        case 2: up_tile_tall<2, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
+        case 3: up_tile_tall<3, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
+        case 4: up_tile_tall<4, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
+        case 5: up_tile_tall<5, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
+        default: up_tile_tall<6, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
+    }
+    if (first == 0) stream::invert(a, 512);
+}
+
+// Adds the partial sums the parts of every up job left in memory and finishes the tiles.  One
+// workgroup of 4 waves per (fragment, weight tile, quarter of the accumulator registers):
 // thread (v, lane) takes over registers 4q .. 4q + 3 of what thread (v, lane) of the fragment's group held, gate
 // and up sums, adds the parts in part order, applies SwiGLU and writes its 4 activation values.  All loads of
 // a thread are in flight together: the kernel is one memory latency long.
 __global__ __launch_bounds__(256) void moe_up_join_kernel(MoeArgs a) {
-    const KernelPlan kp = a.plan->up;
-    if (!kp.deep) return;
-    int b = blockIdx.x;
-    const int q = b & 3;
-    b >>= 2;
-    const int wt = b % a.n_wtiles;
-    b /= a.n_wtiles;
-    const int t = b % tall::kMaxFrags, tile = b / tall::kMaxFrags;
-    if (tile >= kp.n_tiles) return;
-    const int4 tl = a.tiles[tile];
-    if (t >= 2 * tl.y) return;
-    const int frag = tl.x + t, parts = kp.parts;
+    const int q = blockIdx.x & 3, b = (int)blockIdx.x >> 2;
+    const int number = b / a.n_wtiles, wt = b - number * a.n_wtiles;
+    const int parts = a.plan->up.parts;
+    const int frag = reinterpret_cast<const int *>(a.runs)[number];
+    if (number >= a.plan->deep_frags) return;
     const int tid = threadIdx.x, lane = tid & 63, v = tid >> 6;
     float4 vg[kDeepParts], vu[kDeepParts];
+    const float4 *src = partial_block(a, 0, parts, number, wt) + (q * 4 + v) * 64 + lane;
 #pragma unroll
     for (int p = 0; p < kDeepParts; ++p)
         if (p < parts) {
-            const float4 *src = partial_block(a, p, frag, wt);
-            vg[p] = src[((0 * 4 + q) * 4 + v) * 64 + lane];
-            vu[p] = src[((1 * 4 + q) * 4 + v) * 64 + lane];
+            vg[p] = src[p * 2048];
+            vu[p] = src[p * 2048 + 1024];
         }
     float g[4] = {0.f, 0.f, 0.f, 0.f}, u[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -771,7 +872,6 @@ static int launch_stream_pipeline(MoeArgs a, void *out, int split, hipStream_t s
     }
     if (tall) {
         MoeArgs t = a;
-        t.deep_ok = 0;
         hipLaunchKernelGGL(moe_prologue_kernel_bf16, dim3(1), dim3(kPrologueThreads), 0, s, t, n_wt_up, n_wt_down, n_cus, 0);
         t.n_wtiles = n_wt_up;
         if ((tall & 1) && (mask & PMOE_PHASE_UP)) hipLaunchKernelGGL(moe_up_kernel_bf16, dim3(n_cus), dim3(512), 0, s, t);
@@ -807,7 +907,7 @@ size_t bf16_workspace(MoeArgs &a, char *ws) {
     // (a cut has at most one tile per block: choose_tiles)
     a.tiles = reinterpret_cast<int4 *>(take((blocks + 1) * sizeof(int4)));
     a.tiles_down = reinterpret_cast<int4 *>(take((blocks + 1) * sizeof(int4)));
-    // few up jobs for the chip and a contraction long enough to share: deep mode may be planned
+    // few up jobs for the chip and a contraction long enough to share
     a.deep_ok = (blocks * n_wt_up <= (size_t)kDeepJobs && a.K >= 2048) ? 1 : 0;
     a.up_partials = reinterpret_cast<float *>(
         take(a.deep_ok ? (size_t)kDeepParts * 4 * blocks * n_wt_up * 2048 * sizeof(float4) : 0));
@@ -824,21 +924,22 @@ int launch_bf16_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
     if (use_stream(a)) return launch_stream_pipeline(a, out, split, s);
     const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
     const int n_cus = resident_grid();
-    {
+    a.n_wtiles = n_wt_up;
+    if (a.deep_ok && a.n_blocks > 0) {
+        // (the plan is part of the up kernel)
+        hipLaunchKernelGGL(moe_deep_up_kernel, dim3(n_cus), dim3(512), 0, s, a, n_wt_down, n_cus,
+                               (mask & PMOE_PHASE_UP) ? 0 : 1);
+        if (mask & PMOE_PHASE_UP) hipLaunchKernelGGL(moe_up_join_kernel, dim3(a.n_blocks * 4 * n_wt_up * 4), dim3(256), 0, s, a);
+    } else {
         // the plan is needed by the two kernels even when the rest of the prologue is masked off
         const int do_invert = (mask & PMOE_PHASE_PROLOGUE) ? 1 : 0;
         const int blocks = do_invert ? std::max(1, std::min((a.sorted_num + kPrologueThreads - 1) / kPrologueThreads, 512)) : 1;
         hipLaunchKernelGGL(moe_prologue_kernel_bf16, dim3(blocks), dim3(kPrologueThreads), 0, s, a, n_wt_up, n_wt_down, n_cus,
                            do_invert);
+        // resident kernels: a workgroup per CU (their 160 KB of LDS leave room for one)
+        if (a.n_blocks > 0 && (mask & PMOE_PHASE_UP)) hipLaunchKernelGGL(moe_up_kernel_bf16, dim3(n_cus), dim3(512), 0, s, a);
     }
     if (a.n_blocks > 0) {
-        // resident kernels: a workgroup per CU (their 160 KB of LDS leave room for one)
-        a.n_wtiles = n_wt_up;
-        if (mask & PMOE_PHASE_UP) {
-            hipLaunchKernelGGL(moe_up_kernel_bf16, dim3(n_cus), dim3(512), 0, s, a);
-            if (a.deep_ok)
-                hipLaunchKernelGGL(moe_up_join_kernel, dim3(a.n_blocks * tall::kMaxFrags * n_wt_up * 4), dim3(256), 0, s, a);
-        }
         MoeArgs d = a;
         d.n_wtiles = n_wt_down;
         if (mask & PMOE_PHASE_DOWN) hipLaunchKernelGGL(moe_down_kernel_bf16, dim3(n_cus), dim3(512), 0, s, d);

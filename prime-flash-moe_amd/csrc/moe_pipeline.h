@@ -33,10 +33,10 @@ namespace pmoe {
 //    each (no sums to join: a part is a smaller tile).  The parts > 0 follow the main list on the XCD of their
 //    part 0 (they read the same weight rows): b = main_end + 8 m + xcd is the m-th (job, part) pair of that XCD.
 //
-// Deep mode (up kernel only, up.deep != 0): so few jobs that even all of them together leave most CUs
-// idle (the README shape: 16 jobs).  Then every job's contraction is shared among up.parts workgroups,
-// b = job * parts + part; each stores its fp32 partial sums and moe_up_join_kernel adds them in part order and
-// finishes the tiles.
+// Deep mode (up.deep != 0): so few up jobs that even all of them together leave most CUs
+// idle (the README shape: 16 jobs).  Then every job's contraction is shared among up.parts workgroups of
+// moe_deep_up_kernel, b = job * parts + part, which also plans; each stores its fp32 partial sums and moe_up_join_kernel adds
+// them in part order and finishes the tiles.
 struct KernelPlan {
     int n_tiles;
     int parts;  // 1: no split
@@ -45,6 +45,7 @@ struct KernelPlan {
 };
 struct TallPlan {
     KernelPlan up, down;
+    int deep_frags;  // deep mode: fragments of all tiles
     int counters[16];  // next slot of every XCD's queue: up kernel [0, 8), down kernel [8, 16)
 };
 struct TallJob {
@@ -52,7 +53,7 @@ struct TallJob {
     int part, parts;
 };
 constexpr int kDeepParts = 8;    // most parts of an up job in deep mode
-constexpr int kDeepJobs = 32;    // deep mode is considered up to this many (row block, weight tile) pairs
+constexpr int kDeepJobs = 32;    // deep mode is taken up to this many (row block, weight tile) pairs
 
 // Position l of a kernel's walk -> job.
 __device__ __forceinline__ void walk_to_job(int l, int nt, int n_wt, int &tile, int &wt) {
@@ -122,9 +123,9 @@ struct MoeArgs {
     TallPlan *plan;
     int4 *tiles;          // row tiles of this kernel (the up kernel's or the down kernel's cut)
     int4 *tiles_down;     // the down kernel's cut
-    int4 *runs;           // prologue scratch: the runs of blocks with one expert
-    float *up_partials;   // deep mode: fp32 partial sums, [part][fragment][weight tile][32 KB]
-    int deep_ok;          // deep mode may be planned (the workspace holds up_partials)
+    int4 *runs;           // prologue scratch: the runs of blocks with one expert; deep mode: sorted number of each fragment
+    float *up_partials;   // deep mode: fp32 partial sums, [fragment][weight tile][part][32 KB]
+    int deep_ok;          // deep mode (the workspace holds up_partials)
     int crowd;            // bf16: tall kernels enqueued beside the streaming ones (bits: 1 up, 2 down), see crowding();
                           // mxfp8: the work list is one for crowded schedules only (the number of CUs), see crowded_mx()
     int top_k, M, K, N, H, E, sorted_num;

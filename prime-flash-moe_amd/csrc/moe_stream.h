@@ -229,10 +229,10 @@ __device__ __forceinline__ void run_job(const MoeArgs &a, Shared &sh, int blk, i
 }
 
 // Inverts the sorted order for finalize: inv[pair id] = sorted row (entries of pairs that are not in the schedule keep
-// what the buffer held; the reader validates them).  All workgroups of the grid, `threads` threads each.
-__device__ __forceinline__ void invert(const MoeArgs &a, int threads) {
+// what the buffer held; the reader validates them).  The workgroups of the grid from `first` on, `threads` threads each.
+__device__ __forceinline__ void invert(const MoeArgs &a, int threads, int first = 0) {
     const int n_rows = min(a.ntpp[0], a.sorted_num), n_pairs = a.M * a.top_k;
-    for (int s = (int)blockIdx.x * threads + (int)threadIdx.x; s < n_rows; s += (int)gridDim.x * threads) {
+    for (int s = ((int)blockIdx.x - first) * threads + (int)threadIdx.x; s < n_rows; s += ((int)gridDim.x - first) * threads) {
         const int p = a.sorted_ids[s], es = a.expert_ids[s >> 7];
         if (p >= 0 && p < n_pairs && es >= 0 && es < a.E) a.inv[p] = s;
     }

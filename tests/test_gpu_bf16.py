@@ -309,6 +309,40 @@ def test_few_jobs_deep_split_and_join_kernel(T, K, E, N, top_k, exact, deep, dev
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("K,N,counts", [
+    (2048, 256, [40] * 9 + [1, 0, 63, 64, 65, 127, 128, 129, 0, 33]),  # 28 blocks: most runs a block long, some experts without rows
+    (2304, 768, [385, 3]),                                            # a run of four blocks with one row in the last, two tiles
+    (4096, 512, [0, 700, 0]),                                         # two runs of six blocks
+])
+def test_deep_up_kernel_cuts_and_plans(K, N, counts, device):
+    """The tiles that every workgroup of the deep up kernel works out for itself: also with tokens beyond M (holes in a block),
+    a block of an expert that does not exist and a schedule cut behind its last pair."""
+    from test_gpu_mxfp8 import _routing_by_counts
+    import prime_moe
+    E, top_k = len(counts) + 1, 2
+    counts = counts + [max(counts) + sum(counts + [max(counts)]) % 2]  # (no expert has more rows than there are tokens)
+    ids, wts = _routing_by_counts(counts, top_k, device, seed=K)
+    T = ids.shape[0]
+    keep = T - T // 8
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    assert keep * top_k > 32 * E and s.numel() // 128 * (N // 256) <= 32 and K >= 2048  # the rules of the dispatch
+    e_bad = e.clone()
+    e_bad[1] = E + 3
+    w_ref = wts.clone()
+    lost = s[128:256]
+    w_ref.view(-1)[lost[lost >= 0].long()] = 0.0
+    last = int((s >= 0).nonzero().max()) + 1
+    for e_, w_, m, length in ((e, wts, T, s.numel()), (e_bad, w_ref, keep, last)):
+        ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), w_.cpu())[:m]
+        torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+        out = torch.empty((m, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_bf16(x[:m].contiguous(), w1, w2, s[:length].contiguous(), e_, n, wts, out, top_k, 128, 64, 4, 2, 1, 1, True)
+        torch.cuda.synchronize()
+        got = out.float().cpu()
+        assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
 def _prologue_workspace(x, w1, w2, sched, wts, out, top_k):
     """The workspace after the prologue of the tall-tile path: it starts with the plan, the run list and the table of row
     tiles (bf16_workspace in csrc/fused_moe_bf16.hip)."""
