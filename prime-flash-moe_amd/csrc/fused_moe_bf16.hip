@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "align_sort.h"
+#include "moe_few.h"
 #include "moe_pipeline.h"
 #include "moe_stream.h"
 #include "moe_tall.h"
@@ -837,7 +838,40 @@ __global__ __launch_bounds__(256, RB == 256 ? 4 : 2) void moe_stream_down_short_
     stream::for_each_turn(a, a.K / 32, eng);
 }
 
+// A handful of pairs (moe_few.h).  The down kernel ends the pipeline, nothing is left for finalize.
+__global__ __launch_bounds__(64) void moe_few_up_kernel(MoeArgs a) {
+    const int n_tiles = a.H / 4, n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
+    for (int j = (int)blockIdx.x; j < n_live * n_tiles; j += (int)gridDim.x) {
+        const int blk = j / n_tiles;
+        few::up_job(a, blk, j - blk * n_tiles, n_live);
+    }
+}
+__global__ __launch_bounds__(512) void moe_few_down_kernel(MoeArgs a, char *out, int accumulate) {
+    __shared__ few::DownShared sh;
+    const int n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
+    for (int j = (int)blockIdx.x; j < a.K / 8; j += (int)gridDim.x) few::down_job(a, sh, j, n_live, out, accumulate != 0);
+}
+
 // ------------------------------------------------------------------------------------------ host
+
+// One token or two: weights straight into registers.  Whole layer, streaming kernels / these, us: K 2048, N 1536, 8 of 128
+// experts 29.7 / 23.7 at 1 token, 39.2 / 36.0 at 2; K 4096, N 512, 4 of 8 24.3 / 16.6, 25.4 / 21.0; K 4096, N 28672, 2 of 8 121.8 /
+// 115.9, 193.7 / 171.9.  The op alone: K 4096, N 4096, 2 of 64 at 2 tokens 41.5 / 38.3, both on the same two experts 26.3 / 27.5.
+// From three tokens on blocks have more rows than are multiplied at a time, and the weights are read again: 53.4 / 47.6 at
+// 3 tokens on 128 experts, but all on the same 8 21.8 / 30.0.  With K beyond 4096 a CU has more than two workgroups' worth of
+// output columns, whose latencies add up: K 7168, N 4096, 1 token 116 / 124 (down kernel 41 / 50), N 512, 2 tokens 38 / 44.
+static bool use_few(const MoeArgs &a) {
+    return a.M <= 2 && a.M * a.top_k <= few::kMaxPairs && a.K <= 4096 && a.n_blocks > 0;
+}
+static int launch_few_pipeline(const MoeArgs &a, void *out, int split, hipStream_t s) {
+    const int mask = phase_mask();
+    const int64_t blocks = std::min<int64_t>(a.n_blocks, std::min<int64_t>(a.E, (int64_t)a.M * a.top_k));
+    if (mask & PMOE_PHASE_UP)
+        hipLaunchKernelGGL(moe_few_up_kernel, dim3((unsigned)std::min<int64_t>(blocks * (a.H / 4), 1 << 16)), dim3(64), 0, s, a);
+    if (mask & PMOE_PHASE_DOWN)
+        hipLaunchKernelGGL(moe_few_down_kernel, dim3(a.K / 8), dim3(512), 0, s, a, static_cast<char *>(out), split ? 0 : 1);
+    return check_launch("fused_moe_bf16 launch");
+}
 
 // Few rows per expert on average: what the problem costs is the stream of the weights (moe_stream.h).  Whole op,
 // stream against tall tiles, us (graph replays): 8 large experts (K 4096, N 28672, top 2) 117 / 300 at 1 token, 424 /
@@ -921,6 +955,7 @@ size_t bf16_workspace(MoeArgs &a, char *ws) {
 int launch_bf16_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
     const int mask = phase_mask();
     a.n_blocks = (a.sorted_num + kBlockRows - 1) / kBlockRows;
+    if (use_few(a)) return launch_few_pipeline(a, out, split, s);
     if (use_stream(a)) return launch_stream_pipeline(a, out, split, s);
     const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
     const int n_cus = resident_grid();

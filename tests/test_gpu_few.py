@@ -1,0 +1,68 @@
+"""One token or two through the bf16 layer (csrc/moe_few.h): one step of the contraction, whole batches of steps and a remainder,
+one to sixteen blocks (of four or fewer, several waves share a contraction), experts named by both tokens, a token that names
+an expert more than twice, tokens beyond M, blocks of experts that do not exist, pairs listed twice."""
+import pytest
+import torch
+
+from helpers import BF16_GATE, rel_clamp
+from oracle import moe_oracle as O
+from test_gpu_bf16 import _inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(x, w1, w2, sched, wts, top_k, split, device):
+    import prime_moe
+    M, K = x.shape
+    torch.empty((8 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+    out = torch.full((M, K), float("nan") if split else 0.25, dtype=torch.bfloat16, device=device)
+    prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, top_k, 128, 64, 4, 2, 1, 1, split)
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("K,N,E,ids", [
+    (128, 256, 4, [[2]]),                                   # one step, one block: eight parts of one step
+    (1024, 2048, 6, [[5, 0]]),                              # whole batches of 8 steps, two blocks
+    (1152, 2304, 8, [[0, 1, 2], [2, 1, 0]]),                # a remainder of one step, three blocks of two rows
+    (4096, 512, 8, [[7, 6, 5, 4], [3, 2, 1, 0]]),           # eight blocks
+    (256, 768, 40, [list(range(0, 9)), list(range(5, 14))]),  # fourteen blocks, four of them with two rows
+    (384, 256, 3, [[1, 1, 1], [1, 0, 1]]),                  # an expert with five rows
+    (640, 512, 40, [list(range(32)), list(range(8, 40))]),  # 64 pairs
+])
+def test_one_and_two_tokens(K, N, E, ids, split, device):
+    import prime_moe  # noqa: F401 (registers the ops)
+    ids = torch.tensor(ids, dtype=torch.int32, device=device)
+    T, top_k = ids.shape
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=K + N)
+    wts = torch.softmax(torch.randn((T, top_k), device=device, generator=g), -1)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu()) + (0.0 if split else 0.25)
+    outs = [_run(x, w1, w2, sched, wts, top_k, split, device) for _ in range(2)]
+    got = outs[0].float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+def test_odd_schedules(device):
+    import prime_moe  # noqa: F401 (registers the ops)
+    K, N, E, top_k = 512, 512, 6, 3
+    ids = torch.tensor([[0, 3, 5], [3, 1, 0], [3, 5, 2]], dtype=torch.int32, device=device)  # the third token is beyond M
+    g, x, w1, w2 = _inputs(3, K, E, N, device, seed=1)
+    wts = torch.softmax(torch.randn((3, top_k), device=device, generator=g), -1)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    ref = lambda w: O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), w.cpu())[:2]
+    check = lambda sched, w, want: rel_clamp(_run(x[:2].contiguous(), w1, w2, sched, w, top_k, True, device).float().cpu(), want, 1.0) <= BF16_GATE
+    assert check((s, e, n), wts, ref(wts))
+    last = int((s >= 0).nonzero().max()) + 1
+    assert check((s[:last].contiguous(), e, n), wts, ref(wts))  # cut behind the last pair
+    e_bad = e.clone()
+    e_bad[0] = E + 1  # expert 0's block
+    w_ref = wts.clone()
+    w_ref[ids == 0] = 0.0
+    assert check((s, e_bad, n), wts, ref(w_ref))
+    s_dup = s.clone()
+    s_dup[1 if int(s[1]) < 0 else int((s[:128] >= 0).sum())] = s[0]  # a pair id twice in its block contributes once
+    assert check((s_dup, e, n), wts, ref(wts))
+    assert check((s, e, torch.zeros_like(n)), wts, torch.zeros_like(ref(wts)))  # nothing scheduled
