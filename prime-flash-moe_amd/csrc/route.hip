@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const T *__restrict__ l
     }
 }
 
-// Top-k of all tokens (a wave each) and the sort of their ids: n_tokens <= NW, n_tokens * top_k <= NW * 64.
+// Top-k of all tokens (wave w: tokens w, w + NW, ...) and the sort of their ids: n_tokens * top_k <= NW * 64.
 template <int NW, int EPL, typename T>
 __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restrict__ logits, const float *__restrict__ bias,
                                                               int32_t *__restrict__ topk_ids, float *__restrict__ topk_weights,
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restric
     extern __shared__ int32_t smem[];
     __shared__ int32_t ids[NW * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (const int t = wave; t < n_tokens) {
+    for (int t = wave; t < n_tokens; t += NW) {
         int id;
         float w;
         topk_of_token<EPL, T>(logits, bias, t, E, top_k, lane, id, w);
@@ -143,11 +143,12 @@ __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restric
     pmoe::align::sort_in_workgroup<NW, 1>(id, o, E, id_bits, smem);
 }
 
-// Tokens that one workgroup routes and sorts faster than two launches do: one per wave (1 token of 128 experts: 5.9 us
-// against 9.8; four per wave: 16.8 against 10.3).
+// Tokens that one workgroup routes and sorts faster than two launches do: a token per wave, or as many as take a wave four rounds
+// of the top-k (one launch / two, us: 1 token, top 8 of 128 5.9 / 9.8, four per wave 16.8 / 10.3; top 2 of 8, two per wave 4.6 /
+// 6.2, four 6.9 / 6.3; top 4 of 64, two per wave 6.6 / 6.9).
 bool fits_small(int n_tokens, int E, int top_k) {
     const int nw = E <= 512 ? 16 : 8;
-    return n_tokens <= nw && n_tokens * top_k <= nw * 64;
+    return (n_tokens <= nw || (n_tokens + nw - 1) / nw * top_k <= 4) && n_tokens * top_k <= nw * 64;
 }
 
 template <typename T>

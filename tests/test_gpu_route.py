@@ -62,6 +62,14 @@ def test_route_shapes(T, E, k, device):
     _check(torch.randn((T, E), generator=g, device=device), k)
 
 
+@pytest.mark.parametrize("T,E,k", [(16, 8, 2), (17, 8, 2), (32, 8, 2), (33, 8, 2), (64, 8, 1), (65, 8, 1), (49, 70, 1), (17, 300, 2),
+                                   (9, 600, 2), (16, 600, 2), (17, 600, 2)])
+def test_several_tokens_per_wave_of_one_workgroup(T, E, k, device):
+    # at and beyond the most tokens that are routed and sorted by one workgroup
+    g = torch.Generator(device=device).manual_seed(T + E + k)
+    _check(torch.randn((T, E), generator=g, device=device), k)
+
+
 def test_route_ties_go_to_the_lower_index(device):
     # few distinct values: almost every selection is decided by the tie rule
     g = torch.Generator(device=device).manual_seed(3)
