@@ -684,22 +684,29 @@ __global__ __launch_bounds__(256, 2) void moe_stream_down_short_kernel_mx(MoeArg
 // that the schedule lists more than once contributes once (if its rows lie in blocks of different experts,
 // which of them is unspecified).
 //
-// One wave per (token, run of `chunks` pieces of 512 columns): lanes 0 .. top_k - 1 resolve the token's pairs
-// once (inv, sorted_ids, expert_ids, routing weight), the result is broadcast, and then every lane streams its
-// 8 columns of the top_k rows of y (contiguous: y is indexed by pair id), G loads in flight at a time.
+// One wave per (token, piece of 512 columns): lanes 0 .. top_k - 1 resolve the token's pairs (inv, sorted_ids,
+// expert_ids, routing weight), the result is broadcast, and then every lane reads its 8 columns of the top_k rows of y
+// (contiguous: y is indexed by pair id), G loads in flight at a time.
+//
+// Bound by the read of y and by the chain of loads that resolves the pairs in front of it, so waves must be many, each
+// with little to do: a wave per piece resolves the pairs again for every piece (from L2) and is faster all the same than
+// one that keeps them for a run of pieces, and a launch as large as the work than 16384 workgroups that each come back for
+// more.  Before / after, K 2048 unless said: 58.6 / 50.9 us at 8192 tokens x top 8 (5.9 TB/s), 117.5 / 98 at 16000 x 8,
+// 345 / 316 at 100000 x 4, 100 / 88 at 4096 x 8 with K 7168; 15.4 / 14.7 at 2000 x 8, the same at 200 x 9.  Eight loads
+// in flight instead of four cost registers: 15.6 us at 2000 x 8, 7.4 / 7.0 at 200 x 9, nothing gained above.
 template <bool ACCUMULATE, int G>
 __global__ __launch_bounds__(256) void finalize_kernel(const char *y, const int32_t *inv, const int32_t *sorted_ids,
                                                        const int32_t *ntpp, int sorted_num, const float *topk_w,
                                                        int top_k, int M, int K, char *out,
-                                                       const int32_t *expert_ids, int num_experts, int chunks,
-                                                       int groups_per_token) {
+                                                       const int32_t *expert_ids, int num_experts, int pieces) {
     const int lane = threadIdx.x & 63;
     const int n_rows = min(ntpp[0], sorted_num);
-    const int64_t n_items = (int64_t)M * groups_per_token;
+    const int64_t n_items = (int64_t)M * pieces;
     const int64_t wave_stride = (int64_t)gridDim.x * (blockDim.x >> 6);
     for (int64_t item = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); item < n_items; item += wave_stride) {
-        const int t = (int)(item / groups_per_token), grp = (int)(item - (int64_t)t * groups_per_token);
-        const int col_lo = grp * chunks * 512;
+        const int t = (int)(item / pieces);
+        const int col = (int)(item - (int64_t)t * pieces) * 512 + lane * 8;
+        const bool in_range = col < K;
         for (int r0 = 0; r0 < top_k; r0 += 64) {
             // lane r resolves pair r0 + r: its weight, or 0 with `ok` unset
             float w_mine = 0.f;
@@ -717,50 +724,45 @@ __global__ __launch_bounds__(256) void finalize_kernel(const char *y, const int3
             }
             const uint64_t ok_mask = __ballot(ok);
             const int n_here = min(64, top_k - r0);
-            for (int ch = 0; ch < chunks; ++ch) {
-                const int col = col_lo + ch * 512 + lane * 8;
-                if (col_lo + ch * 512 >= K) break;
-                const bool in_range = col < K;
-                float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                if (r0 > 0 || ACCUMULATE) {
-                    if (in_range) {
-                        const uint4 prev = *reinterpret_cast<const uint4 *>(out + ((int64_t)t * K + col) * 2);
-                        const uint32_t u[4] = {prev.x, prev.y, prev.z, prev.w};
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            v[2 * j] = bf16_bits_to_f32(u[j] & 0xffffu);
-                            v[2 * j + 1] = bf16_bits_to_f32(u[j] >> 16);
-                        }
-                    }
-                }
-                for (int g0 = 0; g0 < n_here; g0 += G) {
-                    uint4 q[G];
-                    float w[G];
-#pragma unroll
-                    for (int g = 0; g < G; ++g) {
-                        const int r = g0 + g;  // wave-uniform
-                        const bool live = r < n_here && ((ok_mask >> r) & 1);
-                        w[g] = __shfl(w_mine, r < 64 ? r : 0, 64);
-                        q[g] = make_uint4(0, 0, 0, 0);
-                        if (live && in_range) q[g] = load_once(y + ((int64_t)(t * top_k + r0 + r) * K + col) * 2);
-                        if (!live) w[g] = 0.f;
-                    }
-#pragma unroll
-                    for (int g = 0; g < G; ++g) {
-                        const uint32_t u[4] = {q[g].x, q[g].y, q[g].z, q[g].w};
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            v[2 * j] += w[g] * bf16_bits_to_f32(u[j] & 0xffffu);
-                            v[2 * j + 1] += w[g] * bf16_bits_to_f32(u[j] >> 16);
-                        }
-                    }
-                }
+            float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (r0 > 0 || ACCUMULATE) {
                 if (in_range) {
-                    uint32_t o[4];
+                    const uint4 prev = *reinterpret_cast<const uint4 *>(out + ((int64_t)t * K + col) * 2);
+                    const uint32_t u[4] = {prev.x, prev.y, prev.z, prev.w};
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) o[j] = pack2_bf16(v[2 * j], v[2 * j + 1]);
-                    store_once(out + ((int64_t)t * K + col) * 2, make_uint4(o[0], o[1], o[2], o[3]));
+                    for (int j = 0; j < 4; ++j) {
+                        v[2 * j] = bf16_bits_to_f32(u[j] & 0xffffu);
+                        v[2 * j + 1] = bf16_bits_to_f32(u[j] >> 16);
+                    }
                 }
+            }
+            for (int g0 = 0; g0 < n_here; g0 += G) {
+                uint4 q[G];
+                float w[G];
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const int r = g0 + g;  // wave-uniform
+                    const bool live = r < n_here && ((ok_mask >> r) & 1);
+                    w[g] = __shfl(w_mine, r < 64 ? r : 0, 64);
+                    q[g] = make_uint4(0, 0, 0, 0);
+                    if (live && in_range) q[g] = load_once(y + ((int64_t)(t * top_k + r0 + r) * K + col) * 2);
+                    if (!live) w[g] = 0.f;
+                }
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const uint32_t u[4] = {q[g].x, q[g].y, q[g].z, q[g].w};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        v[2 * j] += w[g] * bf16_bits_to_f32(u[j] & 0xffffu);
+                        v[2 * j + 1] += w[g] * bf16_bits_to_f32(u[j] >> 16);
+                    }
+                }
+            }
+            if (in_range) {
+                uint32_t o[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = pack2_bf16(v[2 * j], v[2 * j + 1]);
+                store_once(out + ((int64_t)t * K + col) * 2, make_uint4(o[0], o[1], o[2], o[3]));
             }
         }
     }
@@ -841,25 +843,19 @@ static int tiles_per_workgroup(bool down, int n_blocks, int n_wt) {
 
 void launch_finalize(const MoeArgs &a, void *out, int split, int n_wt_down, hipStream_t s) {
     (void)n_wt_down;
-    // a wave per (token, group of 512-column pieces); enough waves to fill the chip even for a few tokens
     const int pieces = (a.K + 511) / 512;
-    int groups = std::min<int64_t>(pieces, std::max<int64_t>(1, 8192 / std::max(a.M, 1)));
-    const int chunks = (pieces + groups - 1) / groups;
-    groups = (pieces + chunks - 1) / chunks;
-    const int64_t waves = (int64_t)a.M * groups;
-    const int blocks = (int)std::min<int64_t>((waves + 3) / 4, 16384);
+    const int64_t waves = (int64_t)a.M * pieces;
+    const int blocks = (int)std::min<int64_t>((waves + 3) / 4, 1 << 20);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, a.y, a.inv, a.sorted_ids, a.ntpp, a.sorted_num,
-                           a.topk_w, a.top_k, a.M, a.K, static_cast<char *>(out), a.expert_ids, a.E, chunks, groups);
+                           a.topk_w, a.top_k, a.M, a.K, static_cast<char *>(out), a.expert_ids, a.E, pieces);
     };
     if (split) {
         if (a.top_k <= 2) launch(finalize_kernel<false, 2>);
-        else if (a.top_k <= 4) launch(finalize_kernel<false, 4>);
-        else launch(finalize_kernel<false, 8>);
+        else launch(finalize_kernel<false, 4>);
     } else {
         if (a.top_k <= 2) launch(finalize_kernel<true, 2>);
-        else if (a.top_k <= 4) launch(finalize_kernel<true, 4>);
-        else launch(finalize_kernel<true, 8>);
+        else launch(finalize_kernel<true, 4>);
     }
 }
 
