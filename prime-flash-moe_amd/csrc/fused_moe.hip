@@ -10,6 +10,8 @@
 //             row; mxfp8: re-tiles the scales of the gathered x rows)
 //   -> up kernel (gate/up GEMM + SwiGLU, activation tile -> workspace)
 //   -> down kernel (y[pair id, :K] = act . W2[e]^T, bf16, -> workspace)
+//      (bf16, few up jobs: the up kernel plans for itself and its join follows, no prologue; one token or two:
+//      moe_few.h, where the down kernel writes `out` itself)
 //   -> finalize: out[t] = bf16(sum over the token's pairs p of w[p] * y[p]), fp32 sum in pair order;
 //      split == 0: added to `out` (the reference's accumulate-into-out contract of its single-kernel
 //      path), split != 0: `out` overwritten.

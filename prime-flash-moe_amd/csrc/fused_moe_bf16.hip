@@ -5,8 +5,9 @@
 // prime_moe/csrc/kernels/fused_moe_bf16_kernel.cu:21-733 (gather :21-47, gate/up GEMM + SwiGLU :196-229,
 // down GEMM :496-542).
 //
-// No work list: a workgroup derives its job from its id and a 48-byte plan that workgroup 0 of the
-// prologue writes (see TallPlan), so the prologue only builds the table of row tiles.  No value is
+// No work list: a workgroup derives its job from its id and a plan that workgroup 0 of the prologue writes
+// (see TallPlan), so the prologue only builds the table of row tiles.  Problems of few up jobs have no prologue: the
+// workgroups of moe_deep_up_kernel plan for themselves.  One token or two: the kernels of moe_few.h.  No value is
 // accumulated with atomics and every sum has a fixed order: the result is a pure function of the inputs.
 #include <algorithm>
 

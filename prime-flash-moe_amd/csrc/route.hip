@@ -13,7 +13,7 @@
 // register, where shuffles through LDS cost ten times the latency), finds the lowest expert that holds it with a ballot
 // per key register, and retires it.  The softmax of the top_k winners is computed by the lanes that keep them.
 //
-// Few tokens (one workgroup's work): top-k and sort in one kernel, the ids handed over in LDS (align_sort.h).
+// Few tokens (one workgroup's work, up to four rounds of top-k per wave): top-k and sort in one kernel, the ids handed over in LDS (align_sort.h).
 #include <type_traits>
 
 #include "align_sort.h"
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restric
 // 6.2, four 6.9 / 6.3; top 4 of 64, two per wave 6.6 / 6.9).
 bool fits_small(int n_tokens, int E, int top_k) {
     const int nw = E <= 512 ? 16 : 8;
-    return (n_tokens <= nw || (n_tokens + nw - 1) / nw * top_k <= 4) && n_tokens * top_k <= nw * 64;
+    return n_tokens * top_k <= nw * 64 && (n_tokens <= nw || (n_tokens + nw - 1) / nw * top_k <= 4);
 }
 
 template <typename T>

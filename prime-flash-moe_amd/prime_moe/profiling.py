@@ -40,7 +40,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)
 KERNELS = {k: k for k in ("moe_up_kernel", "moe_up_join_kernel", "moe_down_kernel", "finalize_kernel", "moe_prologue_kernel")}
 KERNELS.update({"moe_stream_up_kernel": "moe_stream_kernel<true", "moe_stream_down_kernel": "moe_stream_kernel<false",
                 "moe_stream_up_kernel_mx": "moe_stream_kernel_mx<true", "moe_stream_down_kernel_mx": "moe_stream_kernel_mx<false"})
-KERNELS.update({k: k for k in ("moe_stream_down_short_kernel", "route_topk_kernel", "route_small_kernel", "moe_align_kernel",
+KERNELS.update({k: k for k in ("moe_deep_up_kernel", "moe_few_up_kernel", "moe_few_down_kernel", "moe_stream_down_short_kernel", "route_topk_kernel", "route_small_kernel", "moe_align_kernel",
                                "align_runs_kernel", "align_count_kernel", "align_bases_kernel", "align_scatter_kernel",
                                "quantize_mx_kernel", "copy_calibration_kernel")})
 SQ_COUNTERS = ["SQ_BUSY_CYCLES", "SQ_VALU_MFMA_BUSY_CYCLES", "SQ_INSTS_VALU_MFMA_MOPS_{DT}", "SQ_LDS_BANK_CONFLICT",
