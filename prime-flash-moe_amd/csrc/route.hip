@@ -13,7 +13,8 @@
 // register, where shuffles through LDS cost ten times the latency), finds the lowest expert that holds it with a ballot
 // per key register, and retires it.  The softmax of the top_k winners is computed by the lanes that keep them.
 //
-// Few tokens (one workgroup's work, up to four rounds of top-k per wave): top-k and sort in one kernel, the ids handed over in LDS (align_sort.h).
+// Few tokens (one workgroup's work, see fits_small): top-k and sort in one kernel, the ids handed over in LDS
+// (align_sort.h).
 #include <type_traits>
 
 #include "align_sort.h"
