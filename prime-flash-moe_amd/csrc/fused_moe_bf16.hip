@@ -584,7 +584,8 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
         const int n_live = min((ntpp + kBlockRows - 1) / kBlockRows, a.n_blocks);
         const bool live = lane < n_live;
         const int e = live ? e_all : -1;
-        const uint64_t starts = __ballot(live && (lane == 0 || __shfl_up(e, 1, 64) != e));
+        const int before = __shfl_up(e, 1, 64);  // (with all lanes active: a lane that is switched off hands out 0)
+        const uint64_t starts = __ballot(live && (lane == 0 || before != e));
         const bool last = live && (lane + 1 == n_live || ((starts >> (lane + 1)) & 1));
         const int run = 63 - __builtin_clzll((starts & ((2ull << lane) - 1)) | 1);  // first block of the lane's run
         const int f2 = last && e >= 0 && e < a.E ? ((lane - run) * kBlockRows + s.rows[lane] + 63) >> 6 : 0;

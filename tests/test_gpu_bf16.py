@@ -343,6 +343,47 @@ def test_deep_up_kernel_cuts_and_plans(K, N, counts, device):
         assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
 
 
+@pytest.mark.parametrize("counts,order", [
+    ([0, 700, 0, 700], None),                            # ascending, expert 0 without rows: two runs of six blocks
+    ([130, 60, 40, 230], [4, 0, 1, 2, 3, 5]),            # experts 3 0 0 1 2 3: another expert in front of expert 0
+    ([130, 60, 40, 230], [2, 0, 4, 1, 5, 3]),            # experts 1 0 3 0 3 2: no expert's blocks side by side
+    ([40, 230, 60, 130], [1, 2, 0, 4, 5, 3]),            # experts 1 1 0 3 3 2
+])
+def test_deep_up_kernel_takes_blocks_in_any_order(counts, order, device):
+    """expert_ids says which expert a block belongs to, in whatever order the blocks come; neighbours of one expert are one run."""
+    from test_gpu_mxfp8 import _routing_by_counts
+    import prime_moe
+    K, N, E, top_k = 2048, 256, len(counts), 2
+    ids, wts = _routing_by_counts(counts, top_k, device, seed=sum(counts))
+    T = ids.shape[0]
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    assert T * top_k > 32 * E and s.numel() // 128 * (N // 256) <= 32  # the rules of the dispatch
+    n_live = int(n[0]) // 128
+    if order is not None:
+        assert len(order) == n_live
+        s, e = s.clone(), e.clone()
+        s.view(-1, 128)[:n_live] = s.view(-1, 128)[order]
+        e[:n_live] = e[order]
+    # pairs of fragments of every run: whole blocks and the rows of the last one
+    f2, exp, rows = [], e[:n_live].tolist(), (s.view(-1, 128)[:n_live] >= 0).sum(1).tolist()
+    for b in range(n_live):
+        if b == 0 or exp[b] != exp[b - 1]:
+            start = b
+        if b + 1 == n_live or exp[b + 1] != exp[b]:
+            f2.append((128 * (b - start) + rows[b] + 63) // 64)
+    ws = _prologue_workspace(x, w1, w2, (s, e, n), wts, torch.empty_like(x), top_k)
+    plan = ws[:36].view(torch.int32).tolist()
+    assert plan[0] == sum((f + 5) // 6 for f in f2) and plan[3] == 1  # the up kernel's tiles, deep
+    assert plan[8] == 2 * sum(f2)                                     # fragments
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    prime_moe.fused_moe_bf16(x, w1, w2, s, e, n, wts, out, top_k, 128, 64, 4, 2, 1, 1, True)
+    torch.cuda.synchronize()
+    got = out.float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
 def _prologue_workspace(x, w1, w2, sched, wts, out, top_k):
     """The workspace after the prologue of the tall-tile path: it starts with the plan, the run list and the table of row
     tiles (bf16_workspace in csrc/fused_moe_bf16.hip)."""
