@@ -105,12 +105,19 @@ __device__ __forceinline__ void by_rows(int n_rows, Group group) {
         for (int r = 0; r < n_rows; r += 2) group(std::integral_constant<int, 2>{}, r);
 }
 
-// act[rows, 4 columns from 4 tile] = swiglu(x W1^T)
+// act[rows, 4 columns from 4 tile] = swiglu(x W1^T).  The wave of a block's first columns also writes the sorted row of each of
+// its pairs to `inv`: of a pair that blocks of two experts list one row stays there, and the down kernel, where several waves
+// may share a contraction, takes that row alone.
 __device__ __forceinline__ void up_job(const MoeArgs &a, int blk, int tile, int n_live) {
     const int lane = threadIdx.x & 63, sub = lane >> 4, chunk = (lane & 15) * 16;
     const int K = a.K, H = a.H, col = 4 * tile + sub;
     const Block b = load_block(a, blk, n_live);
     if (b.e < 0) return;
+    if (tile == 0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if ((unsigned)b.id[i] < (unsigned)(a.M * a.top_k)) a.inv[b.id[i]] = blk * kBlockRows + lane + 64 * i;
+    }
     const char *const gate = a.w1 + ((int64_t)b.e * a.N + col) * K * 2 + chunk;
     const char *const w[2] = {gate, gate + (int64_t)H * K * 2};
     by_rows(b.n_rows, [&](auto n, int row0) {
@@ -156,18 +163,19 @@ __device__ __forceinline__ void down_job(const MoeArgs &a, DownShared &sh, int t
         by_rows(b.n_rows, [&](auto n, int row0) {
             constexpr int NR = decltype(n)::value;
             const char *x[NR];
-            int p[NR];
+            int p[NR], stands[NR];  // the pair, the row that stands for it
             float acc[2][NR] = {};
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 p[r] = pair_of(a, b, row0 + r);
+                stands[r] = a.inv[max(p[r], 0)];
                 x[r] = a.act + ((int64_t)blk * kBlockRows + (p[r] >= 0 ? row0 + r : 0)) * H * 2 + chunk + s0 * 256;
             }
             dots<NR>(acc, w, x, s1 - s0);
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 const float lo = row_sum(acc[0][r]), hi = row_sum(acc[1][r]);
-                if (p[r] >= 0 && (lane & 15) == 0) {
+                if (p[r] >= 0 && stands[r] == blk * kBlockRows + row0 + r && (lane & 15) == 0) {
                     sh.y[part][p[r]][sub] = lo;
                     sh.y[part][p[r]][4 + sub] = hi;
                     sh.ok[p[r]] = 1;

@@ -66,3 +66,28 @@ def test_odd_schedules(device):
     s_dup[1 if int(s[1]) < 0 else int((s[:128] >= 0).sum())] = s[0]  # a pair id twice in its block contributes once
     assert check((s_dup, e, n), wts, ref(wts))
     assert check((s, e, torch.zeros_like(n)), wts, torch.zeros_like(ref(wts)))  # nothing scheduled
+
+
+@pytest.mark.parametrize("ids,place", [
+    ([[0, 1]], 1),                       # two blocks: four waves per contraction
+    ([[1, 0, 3], [3, 0, 2]], 2),         # four blocks: two
+    ([list(range(9))], 5),               # nine: one, and two blocks of one wave
+])
+def test_pair_under_two_experts(ids, place, device):
+    """One of the two rows stands for the pair, for every column of its token."""
+    import prime_moe  # noqa: F401 (registers the ops)
+    K, N, E = 2048, 2048, 9
+    ids = torch.tensor(ids, dtype=torch.int32, device=device)
+    T, top_k = ids.shape
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=place)
+    wts = torch.softmax(torch.randn((T, top_k), device=device, generator=g), -1)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    n_live = int(n[0]) // 128
+    for src, dst in ((0, n_live - 1), (n_live - 1, 0), (place - 1, place)):
+        pair, s_far, ids_far = int(s[128 * src]), s.clone(), ids.clone()
+        s_far[128 * dst + int((s[128 * dst:128 * dst + 128] >= 0).sum())] = pair
+        ids_far.view(-1)[pair] = int(e[dst])
+        refs = [O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), i.cpu(), wts.cpu()) for i in (ids, ids_far)]
+        for _ in range(4):
+            got = _run(x, w1, w2, (s_far, e, n), wts, top_k, True, device).float().cpu()
+            assert min(rel_clamp(got, r, 1.0) for r in refs) <= BF16_GATE
