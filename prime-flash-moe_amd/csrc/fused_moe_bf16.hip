@@ -842,16 +842,16 @@ __global__ __launch_bounds__(256, RB == 256 ? 4 : 2) void moe_stream_down_short_
 
 // A handful of pairs (moe_few.h).  The down kernel ends the pipeline, nothing is left for finalize.
 __global__ __launch_bounds__(64) void moe_few_up_kernel(MoeArgs a) {
-    const int n_tiles = a.H / 4, n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
+    const int n_rows = few::schedule_rows(a), n_live = (n_rows + kBlockRows - 1) / kBlockRows, n_tiles = a.H / 4;
     for (int j = (int)blockIdx.x; j < n_live * n_tiles; j += (int)gridDim.x) {
         const int blk = j / n_tiles;
-        few::up_job(a, blk, j - blk * n_tiles, n_live);
+        few::up_job(a, blk, j - blk * n_tiles, n_rows);
     }
 }
 __global__ __launch_bounds__(512) void moe_few_down_kernel(MoeArgs a, char *out, int accumulate) {
     __shared__ few::DownShared sh;
-    const int n_live = min((a.ntpp[0] + kBlockRows - 1) / kBlockRows, a.n_blocks);
-    for (int j = (int)blockIdx.x; j < a.K / 8; j += (int)gridDim.x) few::down_job(a, sh, j, n_live, out, accumulate != 0);
+    const int n_rows = few::schedule_rows(a);
+    for (int j = (int)blockIdx.x; j < a.K / 8; j += (int)gridDim.x) few::down_job(a, sh, j, n_rows, out, accumulate != 0);
 }
 
 // ------------------------------------------------------------------------------------------ host

@@ -78,15 +78,17 @@ __device__ __forceinline__ float row_sum(float v) {
 struct Block {
     int e, id[2], n_rows;
 };
-__device__ __forceinline__ Block load_block(const MoeArgs &a, int blk, int n_live) {
+// Rows of the schedule.
+__device__ __forceinline__ int schedule_rows(const MoeArgs &a) { return min(a.ntpp[0], a.sorted_num); }
+__device__ __forceinline__ Block load_block(const MoeArgs &a, int blk, int n_rows) {
     const int lane = threadIdx.x & 63;
     const unsigned n_pairs = (unsigned)(a.M * a.top_k);
     Block b;
     const int64_t at = (int64_t)blk * kBlockRows + lane;
-    b.id[0] = at < a.sorted_num ? a.sorted_ids[at] : -1;
-    b.id[1] = at + 64 < a.sorted_num ? a.sorted_ids[at + 64] : -1;
+    b.id[0] = at < n_rows ? a.sorted_ids[at] : -1;
+    b.id[1] = at + 64 < n_rows ? a.sorted_ids[at + 64] : -1;
     b.e = __builtin_amdgcn_readfirstlane(a.expert_ids[blk]);
-    if (b.e < 0 || b.e >= a.E || blk >= n_live) b.e = -1;
+    if (b.e < 0 || b.e >= a.E) b.e = -1;
     const uint64_t m0 = __ballot((unsigned)b.id[0] < n_pairs), m1 = __ballot((unsigned)b.id[1] < n_pairs);
     b.n_rows = m1 ? 128 - __builtin_clzll(m1) : m0 ? 64 - __builtin_clzll(m0) : 0;
     return b;
@@ -108,10 +110,10 @@ __device__ __forceinline__ void by_rows(int n_rows, Group group) {
 // act[rows, 4 columns from 4 tile] = swiglu(x W1^T).  The wave of a block's first columns also writes the sorted row of each of
 // its pairs to `inv`: of a pair that blocks of two experts list one row stays there, and the down kernel, where several waves
 // may share a contraction, takes that row alone.
-__device__ __forceinline__ void up_job(const MoeArgs &a, int blk, int tile, int n_live) {
+__device__ __forceinline__ void up_job(const MoeArgs &a, int blk, int tile, int n_rows) {
     const int lane = threadIdx.x & 63, sub = lane >> 4, chunk = (lane & 15) * 16;
     const int K = a.K, H = a.H, col = 4 * tile + sub;
-    const Block b = load_block(a, blk, n_live);
+    const Block b = load_block(a, blk, n_rows);
     if (b.e < 0) return;
     if (tile == 0) {
 #pragma unroll
@@ -147,16 +149,17 @@ struct DownShared {
     int ok[kMaxPairs];
 };
 // out[:, 8 columns from 8 tile] (+)= sum over the pairs, in their order, of weight x (act W2^T)
-__device__ __forceinline__ void down_job(const MoeArgs &a, DownShared &sh, int tile, int n_live, char *out, bool accumulate) {
+__device__ __forceinline__ void down_job(const MoeArgs &a, DownShared &sh, int tile, int n_rows, char *out, bool accumulate) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = lane >> 4, chunk = (lane & 15) * 16;
     const int K = a.K, H = a.H, n_pairs = a.M * a.top_k, n_steps = H >> 7;
+    const int n_live = (n_rows + kBlockRows - 1) / kBlockRows;
     const int parts = n_live > 4 ? 1 : n_live > 2 ? 2 : n_live == 2 ? 4 : 8;
     const int part = wave & (parts - 1), s0 = part * n_steps / parts, s1 = (part + 1) * n_steps / parts;
     if (tid < n_pairs) sh.ok[tid] = 0;
     __syncthreads();
     for (int blk = wave / parts; blk < n_live; blk += 8 / parts) {
-        const Block b = load_block(a, blk, n_live);
+        const Block b = load_block(a, blk, n_rows);
         if (b.e < 0) continue;
         const char *const first = a.w2 + ((int64_t)b.e * K + 8 * tile + sub) * H * 2 + chunk + s0 * 256;
         const char *const w[2] = {first, first + (int64_t)4 * H * 2};

@@ -91,3 +91,20 @@ def test_pair_under_two_experts(ids, place, device):
         for _ in range(4):
             got = _run(x, w1, w2, (s_far, e, n), wts, top_k, True, device).float().cpu()
             assert min(rel_clamp(got, r, 1.0) for r in refs) <= BF16_GATE
+
+
+def test_rows_behind_the_end_of_the_schedule_are_no_pairs(device):
+    """num_tokens_post_padded may end inside a block: what lies behind it is not part of the schedule."""
+    import prime_moe  # noqa: F401 (registers the ops)
+    K, N, E, top_k = 512, 512, 6, 3
+    ids = torch.tensor([[0, 3, 5], [3, 1, 5]], dtype=torch.int32, device=device)
+    g, x, w1, w2 = _inputs(2, K, E, N, device, seed=2)
+    wts = torch.softmax(torch.randn((2, top_k), device=device, generator=g), -1)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)  # blocks of experts 0, 1, 3 (two rows), 5 (two rows)
+    for end in (1, 129, 257, 258, 385, 386):
+        w_ref = wts.clone()
+        lost = s[end:]
+        w_ref.view(-1)[lost[lost >= 0].long()] = 0.0
+        ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), w_ref.cpu())
+        got = _run(x, w1, w2, (s, e, torch.full_like(n, end)), wts, top_k, True, device).float().cpu()
+        assert rel_clamp(got, ref, 1.0) <= BF16_GATE, end
