@@ -862,8 +862,29 @@ __global__ __launch_bounds__(512) void moe_few_down_kernel(MoeArgs a, char *out,
 // From three tokens on blocks have more rows than are multiplied at a time, and the weights are read again: 53.4 / 47.6 at
 // 3 tokens on 128 experts, but all on the same 8 21.8 / 30.0.  With K beyond 4096 a CU has more than two workgroups' worth of
 // output columns, whose latencies add up: K 7168, N 4096, 1 token 116 / 124 (down kernel 41 / 50), N 512, 2 tokens 38 / 44.
+// What a call gains is a fixed 5 to 7 us of latency; what it loses grows with the pairs.  The op on weights that are not in the
+// caches, streaming / these, us:
+//  * up to four pairs these are faster nearly everywhere: K 2048, N 1536 17.1 / 13.9 at 4, K 512, N 512 11.3 / 7.6; at worst
+//    K 2048, N 8192 41.8 / 43.0 at 4;
+//  * a workgroup of the down kernel has 8 output columns, and with fewer workgroups than CUs the others idle while it reads
+//    pairs x N x 8 bytes: kFewIdle is what that may cost.  K 512, N 1536 18.6 / 17.9 at 16 pairs, 26.9 / 31.1 at 32; K 512, N 4096
+//    20.6 / 20.1 at 8, 29.1 / 34.2 at 16; K 1024, N 2048 27.7 / 27.1 at 16, 43.5 / 45.9 at 32; K 1024, N 4096 26.6 / 27.0 at 8,
+//    42.6 / 45.4 at 16;
+//  * with more workgroups than CUs every step of a workgroup is paid twice: K 4096, N 512 22.5 / 21.2 at 8 pairs, 29.1 / 31.4 at 16,
+//    N 1536 38.0 / 34.3 at 8, 59.2 / 59.9 at 16; N 2048 43.0 / 42.8 at 8, and 26.3 / 27.9 where two tokens share their four experts;
+//  * of more than eight blocks a wave takes several, one behind the other, and each has to be long: K 2048, N 512 20.1 / 19.7 at 16
+//    pairs, 30.1 / 30.9 at 32, N 1024 28.6 / 26.9 and 45.6 / 43.6; K 512, N 512 14.3 / 13.0 and 17.5 / 19.7; K 1024, N 1024
+//    20.6 / 18.6 and 29.3 / 30.8 (with less room for idle CUs, too);
+//  * large experts stream at the rate of memory either way: K 2048, N 4096 42.8 / 40.9 at 8 pairs, N 8192 73.8 / 74.0 (40.4 / 44.1
+//    where two tokens share their four experts), 140 / 135 at 16.
+constexpr int64_t kFewIdle = 50 << 20;
 static bool use_few(const MoeArgs &a) {
-    return a.M <= 2 && a.M * a.top_k <= few::kMaxPairs && a.K <= 4096 && a.n_blocks > 0;
+    if (a.M > 2 || a.K > 4096 || a.n_blocks == 0) return false;
+    const int64_t pairs = (int64_t)a.M * a.top_k, idle = 8 * resident_grid() - a.K;  // output columns the CUs have room for beside K
+    if (pairs <= 4) return true;
+    if (idle < 0) return pairs <= 8 && a.N <= 1536;
+    if (pairs <= 16) return pairs * a.N * idle <= kFewIdle;
+    return pairs <= few::kMaxPairs && a.N >= 1024 && pairs * a.N * idle <= kFewIdle / 4;
 }
 static int launch_few_pipeline(const MoeArgs &a, void *out, int split, hipStream_t s) {
     const int mask = phase_mask();

@@ -108,3 +108,44 @@ def test_rows_behind_the_end_of_the_schedule_are_no_pairs(device):
         ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), w_ref.cpu())
         got = _run(x, w1, w2, (s, e, torch.full_like(n, end)), wts, top_k, True, device).float().cpu()
         assert rel_clamp(got, ref, 1.0) <= BF16_GATE, end
+
+
+def _few_runs(T, K, N, top_k, device):
+    """Whether a call takes the kernels of moe_few.h: with finalize masked off they alone write `out`."""
+    from prime_moe import _native
+    import prime_moe
+    E = max(2, T * top_k)
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
+    ids = torch.randperm(E, generator=g, device=device)[:T * top_k].view(T, top_k).to(torch.int32)
+    wts = torch.softmax(torch.randn((T, top_k), device=device, generator=g), -1)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    out = torch.full((T, K), float("nan"), dtype=torch.bfloat16, device=device)
+    lib = _native.load()
+    try:
+        lib.pmoe_set_phase_mask(6)  # the up and the down kernel
+        prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, top_k, 128, 64, 4, 2, 1, 1, True)
+    finally:
+        lib.pmoe_set_phase_mask(15)
+    torch.cuda.synchronize()
+    written = torch.isfinite(out.float()).all().item()
+    assert written or torch.isnan(out.float()).all().item()
+    got = _run(x, w1, w2, sched, wts, top_k, True, device).float().cpu()
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+    return written
+
+
+@pytest.mark.parametrize("T,K,N,top_k,few", [
+    (2, 256, 8192, 2, True), (1, 256, 8192, 5, False),      # four pairs of any size; more, and most CUs idle
+    (1, 512, 2048, 16, True), (1, 512, 2304, 16, False),    # the idle CUs' share
+    (2, 640, 512, 8, True), (1, 640, 512, 17, False), (2, 640, 512, 32, False),  # short rows of W2: 16 pairs, 17, 64
+    (1, 2048, 8192, 5, True), (2, 2048, 1024, 32, True), (1, 2048, 1024, 65, False), (2, 2048, 768, 9, False),  # no idle CU
+    (2, 1792, 1024, 24, True), (2, 1664, 1024, 24, False),  # few idle CUs, more than 16 pairs
+    (2, 2176, 1536, 4, True), (1, 2176, 1536, 9, False), (1, 2176, 1792, 5, False), (2, 4096, 2048, 2, True),  # K beyond the CUs
+    (1, 4224, 256, 1, False), (3, 256, 256, 1, False),      # K beyond 4096, three tokens
+])
+def test_which_calls_take_these_kernels(T, K, N, top_k, few, device):
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    if cus != 256:
+        pytest.skip("the lines are drawn for 256 CUs")
+    assert _few_runs(T, K, N, top_k, device) == few
