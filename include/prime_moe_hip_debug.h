@@ -36,6 +36,13 @@ void pmoe_set_phase_mask(int mask);
 void pmoe_set_tiles_per_workgroup(int n);
 
 /*
+ * Test aid with no counterpart in the reference: the launches of the calling thread are sized as on a device of `n` CUs (from 8
+ * on, rounded down to a multiple of 8); 0 (the default): what the device has.  The result depends on it only in
+ * the order of its sums.
+ */
+void pmoe_set_compute_units(int n);
+
+/*
  * Second profiling aid without a counterpart in the reference: a plain device copy of `bytes`
  * bytes (multiple of 16) done by a kernel named copy_calibration_kernel.  Its known traffic
  * (bytes read, bytes written) scales the FETCH_SIZE / WRITE_SIZE hardware counters of a

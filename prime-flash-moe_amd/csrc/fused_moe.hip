@@ -809,8 +809,11 @@ static WorkspaceLayout workspace_layout(int M, int K, int N, int sorted_num, int
 
 static int grid_for(int n_tiles) { return (n_tiles + 7) / 8 * 8; }
 
+// CUs that launches are sized for (0: those of the device); see pmoe_set_compute_units in the header.
+static thread_local int g_compute_units = 0;
 int resident_grid() {
     static thread_local int cached_dev = -1, cached = 0;
+    if (g_compute_units > 0) return g_compute_units;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 256;
     if (dev != cached_dev) {
@@ -986,6 +989,7 @@ static int launch_mxfp8_pipeline(MoeArgs a, const SchedBuffers &sb, void *out, i
 using namespace pmoe;
 
 extern "C" void pmoe_set_phase_mask(int mask) { g_phase_mask = mask; }
+extern "C" void pmoe_set_compute_units(int n) { g_compute_units = n <= 0 ? 0 : std::max(n / 8 * 8, 8); }
 extern "C" void pmoe_set_tiles_per_workgroup(int n) { g_tiles_per_wg = n < 0 ? 0 : (n > 16 ? 16 : n); }
 
 extern "C" size_t pmoe_fused_moe_bf16_workspace_bytes(int M, int K, int N, int num_experts,

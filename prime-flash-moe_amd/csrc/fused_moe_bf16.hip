@@ -964,7 +964,8 @@ size_t bf16_workspace(MoeArgs &a, char *ws) {
     // (a cut has at most one tile per block: choose_tiles)
     a.tiles = reinterpret_cast<int4 *>(take((blocks + 1) * sizeof(int4)));
     a.tiles_down = reinterpret_cast<int4 *>(take((blocks + 1) * sizeof(int4)));
-    // few up jobs for the chip and a contraction long enough to share
+    // few up jobs for the chip and a contraction long enough to share (whether the chip has room is seen at the launch: the
+    // size does not depend on the device)
     a.deep_ok = (blocks * n_wt_up <= (size_t)kDeepJobs && a.K >= 2048) ? 1 : 0;
     a.up_partials = reinterpret_cast<float *>(
         take(a.deep_ok ? (size_t)kDeepParts * 4 * blocks * n_wt_up * 2048 * sizeof(float4) : 0));
@@ -983,7 +984,9 @@ int launch_bf16_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
     const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
     const int n_cus = resident_grid();
     a.n_wtiles = n_wt_up;
-    if (a.deep_ok && a.n_blocks > 0) {
+    // A workgroup of moe_deep_up_kernel has one job and comes back for no other: the grid holds every job, however the blocks
+    // fall into tiles, and shares it between two workgroups at least.
+    if (a.deep_ok && a.n_blocks > 0 && 2 * a.n_blocks * n_wt_up <= n_cus) {
         // (the plan is part of the up kernel)
         hipLaunchKernelGGL(moe_deep_up_kernel, dim3(n_cus), dim3(512), 0, s, a, n_wt_down, n_cus,
                                (mask & PMOE_PHASE_UP) ? 0 : 1);

@@ -32,6 +32,7 @@ SIGNATURES = {
     "pmoe_route": (_c_int, [_c_void_p, _c_int] + [_c_void_p] * 6 + [_c_int] * 7 + [_c_void_p, _c_size_t, _c_void_p]),
     "pmoe_set_phase_mask": (None, [_c_int]),
     "pmoe_set_tiles_per_workgroup": (None, [_c_int]),
+    "pmoe_set_compute_units": (None, [_c_int]),
     "pmoe_copy_calibration": (_c_int, [_c_void_p, _c_void_p, ctypes.c_int64, _c_void_p]),
     "pmoe_poison_lds": (_c_int, [_c_void_p, _c_void_p]),
 }

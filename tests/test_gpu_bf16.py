@@ -384,6 +384,32 @@ def test_deep_up_kernel_takes_blocks_in_any_order(counts, order, device):
     assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
 
 
+@pytest.mark.parametrize("cus", [8, 16, 24, 40, 64, 256])
+def test_few_up_jobs_on_fewer_cus(cus, device):
+    """Every job runs, also where there are more of them than workgroups: 16 here (8 experts of one block, 2 weight tiles)."""
+    from test_gpu_mxfp8 import _routing_by_counts
+    import prime_moe
+    from prime_moe import _native
+    counts, K, N, top_k = [90, 100, 70, 128, 1, 90, 111, 66], 2048, 512, 2
+    E = len(counts)
+    ids, wts = _routing_by_counts(counts, top_k, device, seed=cus)
+    T = ids.shape[0]
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=cus)
+    s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    assert T * top_k > 32 * E and s.numel() // 128 * (N // 256) <= 32 and int(n[0]) == 8 * 128  # the rules of the dispatch
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    try:
+        _native.load().pmoe_set_compute_units(cus)
+        prime_moe.fused_moe_bf16(x, w1, w2, s, e, n, wts, out, top_k, 128, 64, 4, 2, 1, 1, True)
+    finally:
+        _native.load().pmoe_set_compute_units(0)
+    torch.cuda.synchronize()
+    got = out.float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
 def _prologue_workspace(x, w1, w2, sched, wts, out, top_k):
     """The workspace after the prologue of the tall-tile path: it starts with the plan, the run list and the table of row
     tiles (bf16_workspace in csrc/fused_moe_bf16.hip)."""
