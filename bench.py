@@ -104,9 +104,15 @@ def phase_time(step, mask, steps, inner=1):
     the host's launch path, which at a few tens of microseconds per call would drown the small shapes."""
     from prime_moe import _native
     lib = _native.load()
+    mark = torch.zeros((1,), device="cuda")
+
+    def marked():
+        mark.zero_()  # a mask may leave nothing to capture; the fill is part of every phase's time and cancels in differences
+        step()
+
     lib.pmoe_set_phase_mask(mask)
     try:
-        return graph_time(step, steps, inner)
+        return graph_time(marked, steps, inner)
     finally:
         lib.pmoe_set_phase_mask(PHASE_ALL)
 
@@ -232,12 +238,15 @@ def run_config(cfg, split, steps, warmup, device, with_cpu, log):
     step = make_step(cfg, inp, sched, out, split)
     sec = time_steps(step, steps, warmup)
     ev_mean, ev_med = time_events(step, steps)
-    # the part of the prologue that builds the schedule runs whatever the mask: it is timed alone and taken off
-    # the two kernels' times, so that they are the kernels' own
+    # the pipeline cut short behind the prologue, the up kernel and the down kernel: a kernel's time is what its launch adds.
+    # (What builds the schedule runs under every mask and cancels; where the up kernel plans for itself, nothing runs in front.)
     inner = 8 if sec < 200e-6 else 1
-    t_plan = phase_time(step, 0, steps, inner)
-    t_up = max(phase_time(step, PHASE_UP, steps, inner) - t_plan, 1e-9)
-    t_down = max(phase_time(step, PHASE_DOWN, steps, inner) - t_plan, 1e-9)
+    # (Several calls per graph: with one, the replays of the first phase time the host's launches, those of the others 25 to 45 us
+    # of gap at the graph's ends.)
+    t_plan, t_plan_up, t_plan_up_down = (phase_time(step, mask, steps, 16 if sec < 200e-6 else 4)
+                                         for mask in (0, PHASE_UP, PHASE_UP | PHASE_DOWN))
+    t_up = max(t_plan_up - t_plan, 1e-9)
+    t_down = max(t_plan_up_down - t_plan_up, 1e-9)
     t_graph = graph_time(step, steps, inner)
     step()
     torch.cuda.synchronize()

@@ -21,7 +21,8 @@ extern "C" {
  * kernels the two fused entry points enqueue, so a harness can time one kernel of the pipeline
  * with events around the call.  Results are only meaningful with PMOE_PHASE_ALL (the default).
  */
-#define PMOE_PHASE_PROLOGUE 1 /* inversion of the sorted order (work lists and plans are always built) */
+#define PMOE_PHASE_PROLOGUE 1 /* inversion of the sorted order (work lists and plans are built under every mask; few up jobs in
+                               * bf16: the up kernel plans, a launch does with DOWN or PROLOGUE but without UP, none otherwise) */
 #define PMOE_PHASE_UP 2       /* gate/up GEMM + SwiGLU */
 #define PMOE_PHASE_DOWN 4     /* down GEMM; with one token or two in bf16 also the routing-weight reduction */
 #define PMOE_PHASE_FINALIZE 8 /* routing-weight reduction into bf16 `out` */

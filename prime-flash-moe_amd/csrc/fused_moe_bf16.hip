@@ -987,8 +987,9 @@ int launch_bf16_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
     // A workgroup of moe_deep_up_kernel has one job and comes back for no other: the grid holds every job, however the blocks
     // fall into tiles, and shares it between two workgroups at least.
     if (a.deep_ok && a.n_blocks > 0 && 2 * a.n_blocks * n_wt_up <= n_cus) {
-        // (the plan is part of the up kernel)
-        hipLaunchKernelGGL(moe_deep_up_kernel, dim3(n_cus), dim3(512), 0, s, a, n_wt_down, n_cus,
+        // (the plan is part of the up kernel, and a launch of its own only where the down kernel runs without it)
+        if (mask & (PMOE_PHASE_UP | PMOE_PHASE_DOWN | PMOE_PHASE_PROLOGUE))
+            hipLaunchKernelGGL(moe_deep_up_kernel, dim3(n_cus), dim3(512), 0, s, a, n_wt_down, n_cus,
                                (mask & PMOE_PHASE_UP) ? 0 : 1);
         if (mask & PMOE_PHASE_UP) hipLaunchKernelGGL(moe_up_join_kernel, dim3(a.n_blocks * 4 * n_wt_up * 4), dim3(256), 0, s, a);
     } else {
