@@ -369,7 +369,7 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, i
     for (int sub = 0; sub < n_sub; ++sub) {
         f32x16 acc[2][4];
         zero_acc<NTF>(acc);
-        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, 0, n_pre);
+        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, n_pre);
         if (sub + 1 < n_sub) {
             // same token rows, the next 128 gate and 128 up rows of the expert; their first slabs under this tile's epilogue
             ld.w_base[0] += (int64_t)128 * K * ES;
@@ -377,7 +377,7 @@ __device__ __forceinline__ void up_tile_ring(const MoeArgs &a, const Job &job, i
             if (DT == DT_FP8 && wave >= 4) ld.sc_off += (uint32_t)kt128 * 512u;
             ld.make_uniform();
             n_pre = lay.stages;
-            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, 0, n_pre);
+            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, n_pre);
         }
 #pragma unroll
         for (int t = 0; t < NTF; ++t) {
@@ -464,13 +464,13 @@ __device__ __forceinline__ void down_tile_ring(const MoeArgs &a, const Job &job,
     for (int sub = 0; sub < n_sub; ++sub) {
         f32x16 acc[2][4];
         zero_acc<NTF>(acc);
-        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, 0, n_pre);
+        ring::main_loop<DT, RB, NTF>(acc, ld, lay, lds, n_slabs, wrow, lane, tok_region, start, n_pre);
         const bool more = sub + 1 < n_sub;
         if (more) {
             set_weights(k0 + kWRows);
             ld.make_uniform();
             n_pre = ahead;
-            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, 0, n_pre);
+            ring::pre_issue<DT, RB>(ld, lay, lds, n_slabs, start, n_pre);
         }
         const YDst dst = y_destination(a, k0);
         if (ntf == 1) {

@@ -618,15 +618,14 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
         kp.parts = max(1, min(min(kDeepParts, n_slabs / 4), (int)gridDim.x / max(n_tiles * a.n_wtiles, 1)));
         if (lane == 0) s.plan = kp;
         if (blockIdx.x == gridDim.x - 1) {
-            // for the kernels behind: the tiles and plans, the sorted numbers of the fragments
+            // for the kernels behind: the down kernel's tiles and queues, the plans, the sorted numbers of the fragments
             const int want = choose_tiles(n_tiles, a.n_blocks, n_f2, n_wt_down, a.H * 2 / tall::kRB, n_cus), extra = max(want - n_tiles, 0);
             const int mine = f2 > 0 ? min(f2, n + extra / n_runs + (runs <= extra % n_runs ? 1 : 0)) : 0;
             const int at = up_to(mine), n_down = __shfl(at, kDeepJobs - 1, 64);
-            cut(a.tiles, tiles - n, n);
             cut(a.tiles_down, at - mine, mine);
             int *numbers = reinterpret_cast<int *>(a.runs);
             for (int q = 0; q < 2 * f2; ++q) numbers[2 * (pairs - f2) + q] = 4 * run + q;
-            if (lane < 16) a.plan->counters[lane] = n_cus / 8;
+            if (lane < 8) a.plan->counters[8 + lane] = n_cus / 8;
             if (lane == 0) {
                 KernelPlan down{};
                 down.n_tiles = n_down;

@@ -219,18 +219,16 @@ __device__ __forceinline__ void mma(f32x16 (&acc)[2][4], const Operands<NTF> &o,
 }
 
 // Issues slabs 0 .. n - 1 of a tile (at most as many as there are stages, in rotated order from `start`) into
-// stages stage0, stage0 + 1, ...
+// stages 0, 1, ...
 template <int DT, int RB>
 __device__ __forceinline__ void pre_issue(const Loader<RB> &ld, const Layout &lay, char *lds, int n_slabs, int start,
-                                          int stage0, int n) {
-    const int SB = lay.stage_bytes, NS = lay.stages;
+                                          int n) {
+    const int SB = lay.stage_bytes;
     for (int s = 0; s < n; ++s) {
         if (s >= n_slabs) break;
         int slab = s + start;
         if (slab >= n_slabs) slab -= n_slabs;
-        int st = stage0 + s;
-        if (st >= NS) st -= NS;
-        ld.issue(lds + st * SB, slab);
+        ld.issue(lds + s * SB, slab);
     }
 }
 // K loop of a group with NTF live fragments.  NTF = 0 is the loop of the waves without matrix work (a group without live
@@ -255,24 +253,21 @@ __device__ __forceinline__ void pre_issue(const Loader<RB> &ld, const Layout &la
 // 4096 tokens on 256 experts (K 7168, N 4096): 2712 -> 2649 us.  Reading both steps first at NTF = 4 spills registers:
 // 1019 and 2981 us.
 //
-// Slab 0 goes to stage `stage0`, the following ones to the stages behind it (wrapping).  `n_pre`: the
+// Slab 0 goes to stage 0, the following ones to the stages behind it (wrapping).  `n_pre`: the
 // caller has already issued slabs 0 .. n_pre - 1 (see pre_issue; a workgroup that runs one tile
 // after another issues them under the previous tile's epilogue).
 template <int DT, int RB, int NTF>
 __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][4], const Loader<RB> &ld, const Layout &lay, char *lds,
                                           int n_slabs, const int (&wrow)[2], int lane, int tok_region, int start,
-                                          int stage0 = 0, int n_pre = 0) {
+                                          int n_pre) {
     static_assert(DT == DT_FP8 && RB == 128, "two scaled matrix instructions of 64 e4m3 per slab and accumulator");
     const int SB = lay.stage_bytes, NS = lay.stages;
     auto rot = [&](int s) {
         s += start;
         return s >= n_slabs ? s - n_slabs : s;
     };
-    for (int s = n_pre; s < NS; ++s) {
-        int st = stage0 + s;
-        if (st >= NS) st -= NS;
-        if (s < n_slabs) ld.issue(lds + st * SB, rot(s));
-    }
+    for (int s = n_pre; s < NS; ++s)
+        if (s < n_slabs) ld.issue(lds + s * SB, rot(s));
     const int lps = ld.lps;
     // opens slab k: it has landed once at most the copies of the later slabs (up to NS - 1) are pending
     // (copies and stores of an epilogue that are in flight too only make the counted waits longer)
@@ -284,7 +279,7 @@ __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][4], const Loader<RB> 
             ld.issue(lds + off, rot(k + NS));
         }
     };
-    int cur_off = stage0 * SB;  // stage of slab kt
+    int cur_off = 0;  // stage of slab kt
     auto next = [&](int off) { return off + SB >= NS * SB ? 0 : off + SB; };
     open(0);
     if constexpr (NTF > 0) {
