@@ -115,7 +115,7 @@ size_t pmoe_fused_moe_mxfp8_workspace_bytes(int M, int K, int N, int num_experts
  * The workspace is scratch of this one call: calls that may run at the same time need
  * their own.
  * A schedule that lists a pair id twice: inside one block the pair contributes once; in blocks
- * of different experts one of the two rows stands for the pair, which one is unspecified
+ * of different experts one of the two rows stands for the pair in every column, which one is unspecified
  * (nothing faults, the rest of the output is unaffected).
  */
 int pmoe_fused_moe_bf16(const void *x, const void *w, const void *w2, void *out,

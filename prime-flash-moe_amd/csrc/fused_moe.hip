@@ -838,9 +838,11 @@ static thread_local int g_tiles_per_wg = 0;
 // the ring has stages in front of the epilogue's scratch, but the coarser work balances worse over the
 // CUs.  Two tiles when that leaves enough rounds of workgroups
 // per CU: 8 for the down kernel, whose tiles are short, 20 for the up kernel (blocks are paired to row tiles, hence
-// 16 and 40 in terms of blocks).  Two against one tile, K = N = 2048 on 32 experts: down 137 / 145 us at 12000 tokens,
-// 1272 / 1390 at 131072; up 974 / 1012 at 60000 tokens (59 blocks x weight tiles per CU), 1893 / 1992 at 131072, but 450 / 442 at
-// 24593 and 240 / 231 at 12000; DeepSeek-V3-like prefill (32 per CU): down 3 % faster, up equal.  Four or eight lose on both.
+// 16 and 40 in terms of blocks).  Two against one tile, K = N = 2048 on 32 experts, each kernel behind the one in
+// front of it: down 123 / 125 us at 12000 tokens (14 blocks x weight tiles per CU), 461 / 518 at 60000, 1027 / 1190 at 131072; up
+// 959 / 973 at 60000 tokens (59), 2090 / 2108 at 131072, but 207 / 199 at 12000; DeepSeek-V3-like prefill (down 30, up 17 per CU):
+// down 725 / 756, up 1550 / 1533.  Three and four tiles (which need not divide the weight tiles): down 130 and 136 at 12000,
+// 464 and 474 at 60000, 1157 and 1112 at 131072, up 995 and 966 at 60000.
 static int tiles_per_workgroup(bool down, int n_blocks, int n_wt) {
     if (g_tiles_per_wg > 0) return std::min(g_tiles_per_wg, n_wt);
     return (int64_t)n_blocks * n_wt >= (int64_t)resident_grid() * (down ? 16 : 40) ? std::min(2, n_wt) : 1;

@@ -357,7 +357,11 @@ __device__ __forceinline__ Work slot_work(int pos, int n_wt, const KernelPlan &k
     w.wt = j.wt;
     return w;
 }
-// Completes a job with its row tile's entry `tl`.
+// Completes a job with its row tile's entry `tl`.  Only moe_deep_up_kernel takes the branches on kp.deep, here and in
+// resolve_tall_job.  In the resident kernels they stand for the sake of the register allocation: with the deep kernel's jobs set
+// up by code of its own, and no such branch, the compiler spills 33 registers of the resident up kernel and 3 of the down
+// kernel instead of none, and the layers take longer: 4096 tokens on 8 experts of K 4096 x N 28672 2424 -> 2977 us, 8192 on 128 of
+// K 2048 x N 1536 729 -> 772, 131072 on 32 of K = N = 2048 5832 -> 7782 (the README layer at 400 to 3000 tokens: the same).
 __device__ __forceinline__ void tile_work(Work &w, const int4 &tl, const KernelPlan &kp, int n_slabs) {
     w.f0 = __builtin_amdgcn_readfirstlane(tl.x);
     w.fg = __builtin_amdgcn_readfirstlane(tl.y);
@@ -557,7 +561,9 @@ __global__ __launch_bounds__(512) void moe_up_kernel_bf16(MoeArgs a) {
 // Few up jobs (at most kDeepJobs (block, weight tile) pairs, K >= 2048).  All of them together leave most CUs idle, so every
 // job's contraction is shared among up to kDeepParts workgroups, which store fp32 partial sums; moe_up_join_kernel adds them in
 // part order and applies SwiGLU.  There are at most 32 blocks: a wave of every workgroup works out the row tiles (a lane per
-// block) while the last workgroup writes what the kernels behind need, and no prologue runs in front.  Prologue, up kernel and join
+// block) while the last workgroup writes what the kernels behind need, and no prologue runs in front.  (The instance of six
+// pairs of fragments spills 7 registers, which its K loop reloads: 370 rows of one expert, K 4096, N 512, take 39.6 us a call, 310
+// rows 35.1; prologue and resident kernel took 46.3 and 42.7.)  Prologue, up kernel and join
 // before / up kernel and join, 8 experts of K 4096, N 512, top 4, us: 256 tokens 8.9 + 17.1 + 6.0 / 18.0 + 5.6, 100 tokens 8.4 + 12.1 +
 // 4.4 / 12.0 + 4.3.  With 12 and 16 parts the K loop is shorter by what the sums are longer: 25.1 and 25.2 us instead of 23.6 at 256.
 struct DeepTiles {

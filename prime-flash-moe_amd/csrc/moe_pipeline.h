@@ -63,7 +63,7 @@ __device__ __forceinline__ void walk_to_job(int l, int nt, int n_wt, int &tile, 
     wt = wg * 8 + rem - tile * gw;
 }
 // Slot number b -> job.  Returns 1 with the job, 0 if the slot is empty, -1 if the queue of this slot's XCD has
-// ended (every later slot is empty).
+// ended (every later slot is empty).  (The branch on kp.deep: see tile_work in fused_moe_bf16.hip.)
 __device__ __forceinline__ int resolve_tall_job(int b, int n_wt, const KernelPlan &kp, TallJob &j) {
     const int nt = kp.n_tiles, n_jobs = nt * n_wt;
     j.part = 0;

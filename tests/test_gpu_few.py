@@ -1,6 +1,7 @@
 """One token or two through the bf16 layer (csrc/moe_few.h): one step of the contraction, whole batches of steps and a remainder,
-one to sixteen blocks (of four or fewer, several waves share a contraction), experts named by both tokens, a token that names
-an expert more than twice, tokens beyond M, blocks of experts that do not exist, pairs listed twice."""
+one to forty blocks (of four or fewer, several waves share a contraction, of more than eight a wave takes several), experts named
+by both tokens, a token that names an expert more than twice, tokens beyond M, blocks of experts that do not exist, pairs listed
+twice; calls on both sides of the lines behind which other kernels run."""
 import pytest
 import torch
 
@@ -29,7 +30,9 @@ def _run(x, w1, w2, sched, wts, top_k, split, device):
     (4096, 512, 8, [[7, 6, 5, 4], [3, 2, 1, 0]]),           # eight blocks
     (256, 768, 40, [list(range(0, 9)), list(range(5, 14))]),  # fourteen blocks, four of them with two rows
     (384, 256, 3, [[1, 1, 1], [1, 0, 1]]),                  # an expert with five rows
-    (640, 512, 40, [list(range(32)), list(range(8, 40))]),  # 64 pairs
+    (640, 512, 40, [list(range(32)), list(range(8, 40))]),  # 64 pairs (streaming kernels, as the fourteen blocks above)
+    (512, 768, 12, [list(range(8)), list(range(4, 12))]),   # sixteen pairs on twelve blocks, four of them with two rows
+    (2048, 1024, 40, [list(range(32)), list(range(8, 40))]),  # 64 pairs on forty blocks
 ])
 def test_one_and_two_tokens(K, N, E, ids, split, device):
     import prime_moe  # noqa: F401 (registers the ops)
