@@ -428,10 +428,12 @@ __device__ __forceinline__ UpTile up_operands(const MoeArgs &a, const Work &w) {
     u.w_up = u.w_gate + (int64_t)a.H * a.K * 2;
     return u;
 }
-// Byte offset in x of the token of sorted row `s`; dead rows read token 0.
-__device__ __forceinline__ uint32_t gather_off(const MoeArgs &a, int64_t s, uint32_t row_bytes) {
-    const int p = s < a.sorted_num ? a.sorted_ids[s] : -1;
+// Byte offset in x of the token of pair id `p`, and of that of sorted row `s`; dead rows read token 0.
+__device__ __forceinline__ uint32_t token_off(const MoeArgs &a, int p, uint32_t row_bytes) {
     return ((uint32_t)p < (uint32_t)(a.M * a.top_k) ? (uint32_t)p / (uint32_t)a.top_k : 0u) * row_bytes;
+}
+__device__ __forceinline__ uint32_t gather_off(const MoeArgs &a, int64_t s, uint32_t row_bytes) {
+    return token_off(a, s < a.sorted_num ? a.sorted_ids[s] : -1, row_bytes);
 }
 template <int FG, bool QUEUE = true>
 __device__ __forceinline__ void up_tile_tall(const MoeArgs &a, const KernelPlan &kp, const Work &w, int *counter, char *lds,
@@ -445,7 +447,7 @@ __device__ __forceinline__ void up_tile_tall(const MoeArgs &a, const KernelPlan 
     const UpTile u = up_operands(a, w);
     tall::Loader<FG, true> ld;
     ld.setup(tid, u.x, u.w_gate, u.w_up, u.row_bytes, u.row_bytes,
-             [&](int row) { return gather_off(a, row0 + row, u.row_bytes); }, pre ? tok_ahead : nullptr);
+             [&](int row) { return gather_off(a, row0 + row, u.row_bytes); }, pre || !QUEUE ? tok_ahead : nullptr);
     const int wrow[2] = {32 * w4, 128 + 32 * w4};
     f32x16 acc[2][FG];
     zero_acc<FG>(acc);
@@ -561,14 +563,19 @@ __global__ __launch_bounds__(512) void moe_up_kernel_bf16(MoeArgs a) {
 // Few up jobs (at most kDeepJobs (block, weight tile) pairs, K >= 2048).  All of them together leave most CUs idle, so every
 // job's contraction is shared among up to kDeepParts workgroups, which store fp32 partial sums; moe_up_join_kernel adds them in
 // part order and applies SwiGLU.  There are at most 32 blocks: a wave of every workgroup works out the row tiles (a lane per
-// block) while the last workgroup writes what the kernels behind need, and no prologue runs in front.  (The instance of six
-// pairs of fragments spills 7 registers, which its K loop reloads: 370 rows of one expert, K 4096, N 512, take 39.6 us a call, 310
-// rows 35.1; prologue and resident kernel took 46.3 and 42.7.)  Prologue, up kernel and join
-// before / up kernel and join, 8 experts of K 4096, N 512, top 4, us: 256 tokens 8.9 + 17.1 + 6.0 / 18.0 + 5.6, 100 tokens 8.4 + 12.1 +
-// 4.4 / 12.0 + 4.3.  With 12 and 16 parts the K loop is shorter by what the sums are longer: 25.1 and 25.2 us instead of 23.6 at 256.
+// block) while the last workgroup writes what the kernels behind need, and no prologue runs in front.
+// What bounds a workgroup is a chain: 1.4 us until it has the last rows of the blocks, 0.9 to cut them, 1.3 to its first
+// copies, 2 - 3 until these land, 0.7 - 1 per slab of its share (an eighth of K), 1 for the sums.  So the tiles are small, one
+// pair of fragments or two: there are twice as many busy CUs as with tiles of up to six pairs, a slab takes 0.72 instead of 1.0
+// us, and half as many sums leave through each CU (a run of blocks has at most twice as many pairs as blocks, so tiles of two
+// leave every job its eight parts on 256 CUs).  The weight rows that two tiles of a run share come from one L2: part p of every
+// job runs on XCD p.  The token rows are gathered by the ids read for the plan.  8 experts of K 4096, N 512, top 4, the layer at
+// 256 tokens 41.7 -> 39.8 us (this kernel 18.6 -> 17.4), with up to six / up to two pairs a tile.  With 12 and 16 parts the K
+// loop is shorter by what the sums are longer: 25.1 and 25.2 us with the join instead of 23.6 (six pairs a tile).
 struct DeepTiles {
     int4 tile[kDeepJobs];  // {first fragment, pairs of fragments, expert, first fragment's number}
     int rows[kDeepJobs];   // of every block: 1 + its last live row
+    int ids[kDeepJobs * kBlockRows];  // sorted ids: the rows of a tile are gathered by them
     KernelPlan plan;
 };
 __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_down, int n_cus, int plan_only) {
@@ -583,6 +590,8 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
         const int64_t at = (int64_t)blk * kBlockRows + lane;
         const int id0 = at < a.sorted_num ? a.sorted_ids[at] : -1, id1 = at + 64 < a.sorted_num ? a.sorted_ids[at + 64] : -1;
         const uint64_t m0 = __ballot((unsigned)id0 < n_pairs), m1 = __ballot((unsigned)id1 < n_pairs);
+        s.ids[blk * kBlockRows + lane] = id0;
+        s.ids[blk * kBlockRows + 64 + lane] = id1;
         if (lane == 0) s.rows[blk] = m1 ? 128 - __builtin_clzll(m1) : m0 ? 64 - __builtin_clzll(m0) : 0;
     }
     __syncthreads();
@@ -596,7 +605,9 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
         const int run = 63 - __builtin_clzll((starts & ((2ull << lane) - 1)) | 1);  // first block of the lane's run
         const int f2 = last && e >= 0 && e < a.E ? ((lane - run) * kBlockRows + s.rows[lane] + 63) >> 6 : 0;
         const int n = (f2 + 5) / 6;
-        // tiles, runs and pairs of fragments (at most 32, 32 and 64) up to and including this lane, added up together
+        const int halves = (f2 + 1) / 2;  // tiles of two pairs
+        // tiles, runs, pairs of fragments and tiles of two pairs (at most 32, 32, 64 and 32) up to and including this lane,
+        // added up together
         auto up_to = [&](int v) {
 #pragma unroll
             for (int d = 1; d < kDeepJobs; d <<= 1) {
@@ -605,9 +616,9 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
             }
             return v;
         };
-        const int sums = up_to(n | (f2 > 0 ? 1 << 8 : 0) | f2 << 16), all = __shfl(sums, kDeepJobs - 1, 64);
-        const int tiles = sums & 0xff, runs = (sums >> 8) & 0xff, pairs = sums >> 16;
-        const int n_tiles = all & 0xff, n_runs = (all >> 8) & 0xff, n_f2 = all >> 16;
+        const int sums = up_to(n | (f2 > 0 ? 1 << 8 : 0) | f2 << 16 | halves << 24), all = __shfl(sums, kDeepJobs - 1, 64);
+        const int tiles = sums & 0xff, runs = (sums >> 8) & 0xff, pairs = (sums >> 16) & 0xff;
+        const int n_tiles = all & 0xff, n_runs = (all >> 8) & 0xff, n_f2 = (all >> 16) & 0xff;
         auto cut = [&](int4 *dst, int at, int count) {  // this lane's run in `count` tiles
             int frag = 4 * run, number = 2 * (pairs - f2);
             for (int q = 0; q < count; ++q) {
@@ -617,11 +628,14 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
                 number += 2 * fg;
             }
         };
-        cut(s.tile, tiles - n, n);
+        // The up kernel's tiles: one pair of fragments where that leaves a workgroup for every part of every job, or two.
+        const bool single = n_f2 * a.n_wtiles * kDeepParts <= (int)gridDim.x;
+        const int n_up = single ? f2 : halves, n_up_tiles = single ? n_f2 : all >> 24;
+        cut(s.tile, (single ? pairs : sums >> 24) - n_up, n_up);
         KernelPlan kp{};
-        kp.n_tiles = n_tiles;
+        kp.n_tiles = n_up_tiles;
         kp.deep = 1;
-        kp.parts = max(1, min(min(kDeepParts, n_slabs / 4), (int)gridDim.x / max(n_tiles * a.n_wtiles, 1)));
+        kp.parts = max(1, min(min(kDeepParts, n_slabs / 4), (int)gridDim.x / max(n_up_tiles * a.n_wtiles, 1)));
         if (lane == 0) s.plan = kp;
         if (blockIdx.x == gridDim.x - 1) {
             // for the kernels behind: the down kernel's tiles and queues, the plans, the sorted numbers of the fragments
@@ -637,6 +651,7 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
                 down.n_tiles = n_down;
                 estimate_kernel(n_down, n_f2, n_wt_down, a.H * 2 / tall::kRB, n_cus, down.parts, down.tail);
                 a.plan->up = kp;
+                a.plan->up.n_tiles = n_tiles;  // (as the down kernel's choice counts them: tiles of up to six pairs)
                 a.plan->down = down;
                 a.plan->deep_frags = 2 * n_f2;
             }
@@ -657,18 +672,19 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
     const int4 tl = s.tile[w.tile];
     const int deep_frag = __builtin_amdgcn_readfirstlane(tl.w);
     tile_work(w, tl, kp, n_slabs);
-    __syncthreads();  // the tiles have been read: the ring may be filled
     bool pre = false;
     uint32_t tok_ahead[tall::kMaxFrags / 2] = {};
-    Work next;
-    switch (w.fg) {
-        case 1: up_tile_tall<1, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
-        case 2: up_tile_tall<2, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
-        case 3: up_tile_tall<3, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
-        case 4: up_tile_tall<4, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
-        case 5: up_tile_tall<5, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
-        default: up_tile_tall<6, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag); break;
+    {
+        const int row = 8 * wave + (lane >> 3);
+        const uint32_t chunk = (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (q < w.fg) tok_ahead[q] = token_off(a, s.ids[w.f0 * 32 + row + 64 * q], (uint32_t)a.K * 2u) + chunk;
     }
+    __syncthreads();  // the tiles and ids have been read: the ring may be filled
+    Work next;
+    if (w.fg == 1) up_tile_tall<1, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag);
+    else up_tile_tall<2, false>(a, kp, w, nullptr, lds, pre, tok_ahead, next, deep_frag);
     if (first == 0) stream::invert(a, 512);
 }
 

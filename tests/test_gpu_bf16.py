@@ -343,6 +343,33 @@ def test_deep_up_kernel_cuts_and_plans(K, N, counts, device):
         assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
 
 
+@pytest.mark.parametrize("K,N,counts", [
+    (2048, 512, [193, 512, 130, 126]),         # 4 + 8 + 3 + 2 = 17 pairs of fragments x 2 weight tiles: one more than tiles of one pair
+    (2048, 512, [192, 512, 130, 126]),         # 16: the most that tiles of one pair take
+    (2048, 256, [64] * 10 + [700, 640, 65]),   # 33 pairs x 1
+    (4096, 256, [64] * 10 + [700, 640]),       # 31 pairs x 1
+    (2304, 1024, [300, 129]),                  # 8 pairs x 4: as many as there is room for; a share of 4 or 5 slabs
+    (2048, 1280, [321, 63]),                   # 7 pairs x 5: one tile of two pairs and a single one
+])
+def test_deep_up_kernel_tiles_of_one_pair_and_two(K, N, counts, device):
+    """The edge between tiles of one pair of fragments and of two (256 CUs: pairs x weight tiles x 8 parts), against the oracle."""
+    import prime_moe
+    E = len(counts)
+    ids = torch.repeat_interleave(torch.arange(E, dtype=torch.int32, device=device), torch.tensor(counts, device=device))
+    ids = ids[torch.randperm(ids.numel(), generator=torch.Generator().manual_seed(K)).to(device)].view(-1, 1).contiguous()
+    T = ids.shape[0]
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
+    wts = torch.rand((T, 1), generator=g, device=device)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    assert T > 32 * E and sched[0].numel() // 128 * (N // 256) <= 32 and K >= 2048  # the rules of the dispatch
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, 1, 128, 64, 4, 2, 1, 1, True)
+    torch.cuda.synchronize()
+    got = out.float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
 @pytest.mark.parametrize("counts,order", [
     ([0, 700, 0, 700], None),                            # ascending, expert 0 without rows: two runs of six blocks
     ([130, 60, 40, 230], [4, 0, 1, 2, 3, 5]),            # experts 3 0 0 1 2 3: another expert in front of expert 0
