@@ -863,16 +863,20 @@ __global__ __launch_bounds__(256, RB == 256 ? 4 : 2) void moe_stream_down_short_
 
 // A handful of pairs (moe_few.h).  The down kernel ends the pipeline, nothing is left for finalize.
 __global__ __launch_bounds__(64) void moe_few_up_kernel(MoeArgs a) {
-    const int n_rows = few::schedule_rows(a), n_live = (n_rows + kBlockRows - 1) / kBlockRows, n_tiles = a.H / 4;
-    for (int j = (int)blockIdx.x; j < n_live * n_tiles; j += (int)gridDim.x) {
-        const int blk = j / n_tiles;
-        few::up_job(a, blk, j - blk * n_tiles, n_rows);
+    const int n_tiles = a.H / 4;
+    int j = (int)blockIdx.x, blk = j / n_tiles;
+    few::Block b = few::request_block(a, blk);
+    const int n_rows = few::schedule_rows(a), n_live = (n_rows + kBlockRows - 1) / kBlockRows;
+    while (j < n_live * n_tiles) {
+        few::up_job(a, b, blk, j - blk * n_tiles, n_rows);
+        j += (int)gridDim.x;
+        blk = j / n_tiles;
+        b = few::request_block(a, blk);
     }
 }
-__global__ __launch_bounds__(512) void moe_few_down_kernel(MoeArgs a, char *out, int accumulate) {
+__global__ __launch_bounds__(512) void moe_few_down_kernel(MoeArgs a, char *out, int blocks, int accumulate) {
     __shared__ few::DownShared sh;
-    const int n_rows = few::schedule_rows(a);
-    for (int j = (int)blockIdx.x; j < a.K / 8; j += (int)gridDim.x) few::down_job(a, sh, j, n_rows, out, accumulate != 0);
+    for (int j = (int)blockIdx.x; j < a.K / 8; j += (int)gridDim.x) few::down_job(a, sh, j, blocks, out, accumulate != 0);
 }
 
 // ------------------------------------------------------------------------------------------ host
@@ -913,7 +917,7 @@ static int launch_few_pipeline(const MoeArgs &a, void *out, int split, hipStream
     if (mask & PMOE_PHASE_UP)
         hipLaunchKernelGGL(moe_few_up_kernel, dim3((unsigned)std::min<int64_t>(blocks * (a.H / 4), 1 << 16)), dim3(64), 0, s, a);
     if (mask & PMOE_PHASE_DOWN)
-        hipLaunchKernelGGL(moe_few_down_kernel, dim3(a.K / 8), dim3(512), 0, s, a, static_cast<char *>(out), split ? 0 : 1);
+        hipLaunchKernelGGL(moe_few_down_kernel, dim3(a.K / 8), dim3(512), 0, s, a, static_cast<char *>(out), (int)blocks, split ? 0 : 1);
     return check_launch("fused_moe_bf16 launch");
 }
 
