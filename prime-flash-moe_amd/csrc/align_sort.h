@@ -88,14 +88,14 @@ struct Outputs {
     int block_m, pad_to, max_padded, max_blocks;
 };
 
-__device__ __forceinline__ void fill_minus_one(const Outputs &o, int n_threads) {
-    const int tid = threadIdx.x;
-    if ((reinterpret_cast<uintptr_t>(o.sorted_token_ids) & 15) == 0) {
-        int4 *dst = reinterpret_cast<int4 *>(o.sorted_token_ids);
-        for (int i = tid; i < o.max_padded / 4; i += n_threads) dst[i] = make_int4(-1, -1, -1, -1);
-        for (int64_t i = (o.max_padded & ~3) + (int64_t)tid; i < o.max_padded; i += n_threads) o.sorted_token_ids[i] = -1;
+// Thread `me` of `n_threads` that fill `count` words.
+__device__ __forceinline__ void fill_minus_one(int32_t *out, int count, int me, int n_threads) {
+    if ((reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+        int4 *dst = reinterpret_cast<int4 *>(out);
+        for (int i = me; i < count / 4; i += n_threads) dst[i] = make_int4(-1, -1, -1, -1);
+        for (int64_t i = (count & ~3) + (int64_t)me; i < count; i += n_threads) out[i] = -1;
     } else {
-        for (int64_t i = tid; i < o.max_padded; i += n_threads) o.sorted_token_ids[i] = -1;
+        for (int64_t i = me; i < count; i += n_threads) out[i] = -1;
     }
 }
 
@@ -106,15 +106,18 @@ __device__ __forceinline__ void write_expert_ids(const Outputs &o, const int32_t
 // LDS words of sort_in_workgroup.
 __host__ __device__ constexpr int sort_words(int n_waves, int E) { return 2 * E + 1 + n_waves * E; }
 
-// The whole sort by one workgroup of NW waves whose ids are in registers (load_ids from 0; n <= NW * 64 * PER).
+// The whole sort by one workgroup of NW waves whose ids are in registers (load_ids from 0; n <= NW * 64 * PER), in two steps
+// with a barrier between them.  What does not need the ids:
+template <int NW>
+__device__ __forceinline__ void begin_sort(const Outputs &o, int E, int32_t *smem) {
+    fill_minus_one(o.sorted_token_ids, o.max_padded, threadIdx.x, NW * 64);  // complete before any pair id lands on top of it: barriers follow
+    for (int i = threadIdx.x; i < NW * E; i += NW * 64) smem[2 * E + 1 + i] = 0;
+}
 template <int NW, int PER>
-__device__ __forceinline__ void sort_in_workgroup(const int (&id)[PER], const Outputs &o, int E, int id_bits, int32_t *smem) {
+__device__ __forceinline__ void finish_sort(const int (&id)[PER], const Outputs &o, int E, int id_bits, int32_t *smem) {
     constexpr int NT = NW * 64;
     int32_t *offs = smem, *padc = smem + E + 1, *table = smem + 2 * E + 1;  // table: [NW][E] counts, then bases
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    fill_minus_one(o, NT);  // complete before any pair id lands on top of it: barriers follow
-    for (int i = tid; i < NW * E; i += NT) table[i] = 0;
-    __syncthreads();
     int ord[PER];
     rank_ids<PER>(id, ord, table + wave * E, E, id_bits, lane);
     __syncthreads();
@@ -139,6 +142,12 @@ __device__ __forceinline__ void sort_in_workgroup(const int (&id)[PER], const Ou
         if ((unsigned)e < (unsigned)E)
             o.sorted_token_ids[offs[e] + table[wave * E + e] + ord[i]] = (wave * PER + i) * 64 + lane;
     }
+}
+template <int NW, int PER>
+__device__ __forceinline__ void sort_in_workgroup(const int (&id)[PER], const Outputs &o, int E, int id_bits, int32_t *smem) {
+    begin_sort<NW>(o, E, smem);
+    __syncthreads();
+    finish_sort<NW, PER>(id, o, E, id_bits, smem);
 }
 
 inline int id_bits_for(int num_experts) {

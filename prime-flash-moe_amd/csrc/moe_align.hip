@@ -197,7 +197,7 @@ __global__ __launch_bounds__(NW * 64) void align_runs_kernel(const int32_t *__re
     constexpr int NT = NW * 64, PER = 16, RUN = NT * PER;
     int32_t *offs = smem, *padc = smem + E + 1, *table = smem + 2 * E + 1, *base = table + NW * E;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    fill_minus_one(o, NT);
+    fill_minus_one(o.sorted_token_ids, o.max_padded, tid, NT);
     for (int i = tid; i < (NW + 1) * E; i += NT) table[i] = 0;
     __syncthreads();
     int id[PER], ord[PER];

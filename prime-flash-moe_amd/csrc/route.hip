@@ -15,6 +15,7 @@
 //
 // Few tokens (one workgroup's work, see fits_small): top-k and sort in one kernel, the ids handed over in LDS
 // (align_sort.h).
+#include <algorithm>
 #include <type_traits>
 
 #include "align_sort.h"
@@ -121,14 +122,28 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const T *__restrict__ l
     }
 }
 
-// Top-k of all tokens (wave w: tokens w, w + NW, ...) and the sort of their ids: n_tokens * top_k <= NW * 64.
+// Top-k of all tokens (wave w: tokens w, w + NW, ...) and the sort of their ids: n_tokens * top_k <= NW * 64.  Workgroup 0 does
+// that for the rows that the pairs can reach (`reach`, a multiple of block_m or max_padded: every pair in an expert of its own);
+// the others write what is known of the rest, -1 and the last expert.  (A token of 128 experts has room for 16264 rows and
+// reaches 1024, five of 256 experts 32552 and 5120; one CU takes 0.5 and 1 us to fill them.  One token of 128 experts, the whole
+// layer, all rows behind the top-k / in front of it / with other workgroups 24.75 / 24.55 / 24.35 us.)
 template <int NW, int EPL, typename T>
 __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restrict__ logits, const float *__restrict__ bias,
                                                               int32_t *__restrict__ topk_ids, float *__restrict__ topk_weights,
-                                                              pmoe::align::Outputs o, int n_tokens, int E, int top_k, int id_bits) {
+                                                              pmoe::align::Outputs o, int reach, int n_tokens, int E, int top_k, int id_bits) {
     extern __shared__ int32_t smem[];
     __shared__ int32_t ids[NW * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int reach_blocks = min((reach + o.block_m - 1) / o.block_m, o.max_blocks);
+    if (blockIdx.x > 0) {
+        const int n = (int)(gridDim.x - 1) * NW * 64, me = (int)(blockIdx.x - 1) * NW * 64 + tid;
+        pmoe::align::fill_minus_one(o.sorted_token_ids + reach, o.max_padded - reach, me, n);
+        for (int64_t j = reach_blocks + (int64_t)me; j < o.max_blocks; j += n) o.expert_ids[j] = E - 1;
+        return;
+    }
+    o.max_padded = reach;
+    o.max_blocks = reach_blocks;
+    pmoe::align::begin_sort<NW>(o, E, smem);  // (its stores are on their way while the logits are)
     for (int t = wave; t < n_tokens; t += NW) {
         int id;
         float w;
@@ -141,7 +156,7 @@ __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restric
     }
     __syncthreads();
     const int id[1] = {tid < n_tokens * top_k ? ids[tid] : -1};
-    pmoe::align::sort_in_workgroup<NW, 1>(id, o, E, id_bits, smem);
+    pmoe::align::finish_sort<NW, 1>(id, o, E, id_bits, smem);
 }
 
 // Tokens that one workgroup routes and sorts faster than two launches do: a token per wave, or as many as take a wave four rounds
@@ -166,8 +181,13 @@ int launch_topk(const T *logits, const float *bias, int32_t *topk_ids, float *to
     if (o != nullptr) {
         with_epl([&](auto e) {
             constexpr int EPL = decltype(e)::value, NW = EPL <= 8 ? 16 : 8;
-            hipLaunchKernelGGL((route_small_kernel<NW, EPL, T>), dim3(1), dim3(NW * 64), sizeof(int32_t) * (size_t)pmoe::align::sort_words(NW, E),
-                               s, logits, bias, topk_ids, topk_weights, *o, n_tokens, E, top_k, pmoe::align::id_bits_for(E));
+            const int n = n_tokens * top_k;
+            const int64_t rows = n + (int64_t)std::min(n, E) * (o->pad_to - 1);
+            const int reach = (int)std::min<int64_t>(o->max_padded, (rows + o->block_m - 1) / o->block_m * o->block_m);
+            const int rest = std::max(o->max_padded - reach, 4 * (o->max_blocks - reach / o->block_m));
+            const int fillers = std::min((rest + NW * 256 - 1) / (NW * 256), 15);  // 16 bytes a thread and turn
+            hipLaunchKernelGGL((route_small_kernel<NW, EPL, T>), dim3(1 + fillers), dim3(NW * 64), sizeof(int32_t) * (size_t)pmoe::align::sort_words(NW, E),
+                               s, logits, bias, topk_ids, topk_weights, *o, reach, n_tokens, E, top_k, pmoe::align::id_bits_for(E));
         });
         return pmoe::check_launch("route launch");
     }

@@ -70,6 +70,20 @@ def test_several_tokens_per_wave_of_one_workgroup(T, E, k, device):
     _check(torch.randn((T, E), generator=g, device=device), k)
 
 
+@pytest.mark.parametrize("block_m,bpc", [(128, 1), (128, 2), (20, 1), (7, 3)])
+@pytest.mark.parametrize("T,E,k,spread", [(1, 128, 8, True), (2, 16, 8, True), (5, 256, 8, False), (3, 1024, 32, True), (16, 3, 3, False),
+                                          (1, 1, 1, True)])
+def test_rows_that_no_pair_can_reach(T, E, k, spread, block_m, bpc, device):
+    """The workgroup that sorts fills the rows that the pairs can reach, others the rest: every expert another pair (the schedule
+    ends where the reach does) or all tokens on the same experts, in memory that held something else."""
+    logits = torch.zeros((T, E), device=device)
+    for t in range(T):
+        first = t * k if spread else 0
+        logits[t, [(first + i) % E for i in range(k)]] = torch.arange(k, 0, -1, device=device, dtype=torch.float32)
+    torch.empty((1 << 22,), dtype=torch.int32, device=device).fill_(12345)  # dirty the allocator's blocks
+    _check(logits, k, block_m=block_m, bpc=bpc)
+
+
 def test_route_ties_go_to_the_lower_index(device):
     # few distinct values: almost every selection is decided by the tie rule
     g = torch.Generator(device=device).manual_seed(3)
