@@ -510,28 +510,45 @@ __global__ __launch_bounds__(512) void moe_down_kernel(MoeArgs a) {
 // y = first weight tile | expert << 16 | (weight tiles - 1) << 26 (experts < 1024, up to 16 weight
 // tiles), w = 1 if the row tile is the only one of its expert.
 //
-// Writes the work list entry of job `j` (of the (n_wt + per_job - 1) / per_job of the row tile; a workgroup
-// takes `per_job` consecutive weight tiles).
-__device__ __forceinline__ void emit_work(int4 *work, int n_wt, int per_job, int tile, int n_tiles, int first, int nb,
-                                          int e, int j, int flags) {
+// The work list of a kernel with n_wt weight tiles, of which a workgroup takes `per_job` consecutive ones, over `n_tiles` row
+// tiles {first block | blocks << 28, expert}: thread `me` of `threads` writes entries me, me + threads, ... of the `grid` there are,
+// -1 where the walk has ended or a block names no expert.  By position, so that neighbouring threads write neighbouring entries
+// and nobody has to clear the list before.
+__device__ __forceinline__ void emit_work(int4 *work, int grid, int n_wt, int per_job, const int2 *tiles, int n_tiles, int num_experts,
+                                          int me, int threads) {
     constexpr int GW = 8;
-    const int n_jobs = (n_wt + per_job - 1) / per_job;
-    const int per_xcd = (n_tiles * n_jobs + 7) >> 3;
-    const int wg = j / GW;
-    const int gw = min(GW, n_jobs - wg * GW);
-    const int l = wg * GW * n_tiles + tile * gw + (j - wg * GW);
-    const int wt = j * per_job, cnt = min(per_job, n_wt - wt);
-    const int x = first | (nb << 28), y = wt | (e << 16) | ((cnt - 1) << 26);
-    const int pos = l % per_xcd, xcd = l / per_xcd;
-    work[8 * pos + xcd] = make_int4(x, y, 0, flags);
+    const int n_jobs = (n_wt + per_job - 1) / per_job, total = n_tiles * n_jobs;
+    const int per_xcd = (total + 7) >> 3;
+    for (int w = me; w < grid; w += threads) {
+        const int pos = w >> 3, l = (w & 7) * per_xcd + pos;
+        int4 entry = make_int4(-1, -1, 0, 0);
+        if (pos < per_xcd && l < total) {
+            const int wg = l / (GW * n_tiles), rem = l - wg * GW * n_tiles;
+            const int gw = min(GW, n_jobs - wg * GW), t = rem / gw, j = wg * GW + rem - t * gw;
+            const int2 tl = tiles[t];
+            if (tl.y >= 0 && tl.y < num_experts) {
+                // (the only row tile of its expert: then nobody else reads that expert's weight rows)
+                const bool shared = (t > 0 && tiles[t - 1].y == tl.y) || (t + 1 < n_tiles && tiles[t + 1].y == tl.y);
+                const int wt = j * per_job, cnt = min(per_job, n_wt - wt);
+                entry = make_int4(tl.x, wt | (tl.y << 16) | ((cnt - 1) << 26), 0, shared ? 0 : 1);
+            }
+        }
+        work[w] = entry;
+    }
 }
 
-// Prologue of an mxfp8 call.  Workgroup 0 builds the row tiles and work lists of the two-group kernels:
+// Prologue of an mxfp8 call.  The first workgroups build the row tiles and work lists of the two-group kernels:
 // consecutive blocks of one expert are paired, an expert's odd last block stays single (one pass of
-// block-wide scans per 256 blocks, then one pass over the tiles that writes the two walk orders).
+// block-wide scans per 256 blocks, then the two walk orders).  Each of them works out all tiles, in LDS, and writes its
+// share of the lists; only of more than kLdsTiles blocks workgroup 0 writes them alone, from tiles in the workspace.  What bounds it is
+// the chain of scans; the lists of 4096 tokens on 256 experts have 22440 entries, 11264 of them jobs.
+// The re-tiling of the x scales took 28 us there for want of loads in flight (a row and its token at a time): eight rows of
+// every lane, a block per workgroup and no division in the loop.  Prologue, before / now, us: 4096 tokens on 256 experts (K 7168,
+// N 4096) 28.7 / 10.9, 24593 on 32 (K = N = 2048) 17.7 / 10.8; the layers 2474 / 2462 and 818 / 814.
 // All workgroups invert the sorted order: inv[pair id] = sorted row.  Entries of pairs that are not
 // in the schedule keep whatever the buffer held; the reader validates an entry against sorted_ids.
 // CROWD: only for crowded schedules (`n_cus`: see crowded_mx).
+constexpr int kLdsTiles = kBlockRows * 65 / 2;
 template <bool CROWD>
 __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert_ids, const int32_t *ntpp,
                                                            int n_blocks, int2 *tiles, int *n_tiles,
@@ -542,12 +559,13 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
                                                            int n_pairs, int do_invert, const uint8_t *x_scales,
                                                            uint32_t *xs_tiled, int nkt, int top_k, int M, int n_cus) {
     if (CROWD && !crowded_mx(ntpp, n_blocks, n_pairs, n_wt_up, n_cus)) return;
-    if (blockIdx.x == 0 && tiles != nullptr) {
+    const int n_live = min((ntpp[0] + kBlockRows - 1) / kBlockRows, n_blocks);
+    const int builders = min(max((int)gridDim.x / 4, 1), 32);
+    __shared__ uint32_t s_sc[kBlockRows][65];  // row tiles first
+    if ((int)blockIdx.x < (n_live <= kLdsTiles ? builders : 1)) {
         __shared__ int s_max[4], s_sum[4], s_carry[2];
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-        for (int i = tid; i < grid_up; i += 256) work_up[i] = make_int4(-1, -1, 0, 0);
-        for (int i = tid; i < grid_down; i += 256) work_down[i] = make_int4(-1, -1, 0, 0);
-        const int n_live = min((ntpp[0] + kBlockRows - 1) / kBlockRows, n_blocks);
+        int2 *table = n_live <= kLdsTiles ? reinterpret_cast<int2 *>(&s_sc[0][0]) : tiles;
         if (tid == 0) { s_carry[0] = 0; s_carry[1] = 0; }
         __syncthreads();
         for (int base = 0; base < n_live; base += 256) {
@@ -578,43 +596,19 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
             __syncthreads();
             int off = s_carry[1];
             for (int w = 0; w < wave; ++w) off += s_sum[w];
-            if (leader) tiles[off + incl - 1] = make_int2(b, paired ? 2 : 1);
+            if (leader) table[off + incl - 1] = make_int2(b | (paired ? 2 : 1) << 28, e);
             __syncthreads();
             if (tid == 255) { s_carry[0] = run_start; s_carry[1] = off + incl; }
             __syncthreads();
         }
         const int nt = s_carry[1];
-        if (tid == 0) n_tiles[0] = nt;
+        if (blockIdx.x == 0 && tid == 0) n_tiles[0] = nt;
         __threadfence_block();
         __syncthreads();  // tiles written above are read below by other threads
-        const int jobs_up = (n_wt_up + per_job_up - 1) / per_job_up, jobs_down = (n_wt_down + per_job_down - 1) / per_job_down;
-        const int per_tile = jobs_up + jobs_down;
-        // 1 if row tile t is the only one of its expert e (then nobody else reads that expert's weight rows)
-        auto only_tile = [&](int t, int e) {
-            const bool before = t > 0 && expert_ids[tiles[t - 1].x] == e;
-            const bool after = t + 1 < nt && expert_ids[tiles[t + 1].x] == e;
-            return (before || after) ? 0 : 1;
-        };
-        if (nt >= 64) {  // a row tile per thread and turn, its jobs one after the other
-            for (int t = tid; t < nt; t += 256) {
-                const int2 tl = tiles[t];
-                const int e = expert_ids[tl.x];
-                if (e < 0 || e >= num_experts) continue;  // nothing to compute for a block without an expert
-                const int fl = only_tile(t, e);
-                for (int j = 0; j < jobs_up; ++j) emit_work(work_up, n_wt_up, per_job_up, t, nt, tl.x, tl.y, e, j, fl);
-                for (int j = 0; j < jobs_down; ++j) emit_work(work_down, n_wt_down, per_job_down, t, nt, tl.x, tl.y, e, j, fl);
-            }
-        } else {  // few row tiles for 256 threads: an entry per thread and turn
-            for (int i = tid; i < nt * per_tile; i += 256) {
-                const int t = i / per_tile, j = i - t * per_tile;
-                const int2 tl = tiles[t];
-                const int e = expert_ids[tl.x];
-                if (e < 0 || e >= num_experts) continue;
-                const int fl = only_tile(t, e);
-                if (j < jobs_up) emit_work(work_up, n_wt_up, per_job_up, t, nt, tl.x, tl.y, e, j, fl);
-                else emit_work(work_down, n_wt_down, per_job_down, t, nt, tl.x, tl.y, e, j - jobs_up, fl);
-            }
-        }
+        const int me = (int)blockIdx.x * 256 + tid, threads = (n_live <= kLdsTiles ? builders : 1) * 256;
+        emit_work(work_up, grid_up, n_wt_up, per_job_up, table, nt, num_experts, me, threads);
+        emit_work(work_down, grid_down, n_wt_down, per_job_down, table, nt, num_experts, me, threads);
+        __syncthreads();  // (a workgroup that re-tiles, too, uses the LDS again)
     }
     if (do_invert) {
         const int n_rows = min(ntpp[0], sorted_num);
@@ -629,13 +623,11 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
         // the e8m0 scales of the gathered x rows, re-tiled for the up kernel's loader (see
         // MoeArgs::xs_tiled); rows without a token get 2^0.  One sorted block per turn, through LDS so
         // that both the reads (a row's scales) and the writes (128 rows of one K tile) are contiguous.
-        // Workgroup 0 builds the tiles above and takes no share unless it is alone.
+        // The workgroups that build the lists take no share unless there is only one.
         __shared__ int s_tok[kBlockRows];
-        __shared__ uint32_t s_sc[kBlockRows][65];
         const int tid = threadIdx.x;
-        const int n_live = min((ntpp[0] + kBlockRows - 1) / kBlockRows, n_blocks);
-        const int workers = gridDim.x > 1 ? (int)gridDim.x - 1 : 1;
-        const int me = gridDim.x > 1 ? (int)blockIdx.x - 1 : 0;
+        const int workers = gridDim.x > 1 ? (int)gridDim.x - builders : 1;
+        const int me = gridDim.x > 1 ? (int)blockIdx.x - builders : 0;
         const uint32_t *xs = reinterpret_cast<const uint32_t *>(x_scales);  // nkt dwords per token
         for (int b = me; b >= 0 && b < n_live; b += workers) {
             if (tid < kBlockRows) {
@@ -648,12 +640,21 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
             __syncthreads();
             for (int c0 = 0; c0 < nkt; c0 += 64) {
                 const int cw = min(64, nkt - c0);
-                for (int i = tid; i < kBlockRows * cw; i += 256) {
-                    const int r = i / cw, c = i - r * cw;
-                    const int tok = s_tok[r];
-                    s_sc[r][c] = tok >= 0 ? xs[(int64_t)tok * nkt + c0 + c] : 0x7f7f7f7fu;
+                // a row's dwords by 2^sh lanes, eight rows of every lane in flight
+                const int sh = cw > 1 ? 32 - __builtin_clz(cw - 1) : 0, c = tid & ((1 << sh) - 1), rows = 256 >> sh;
+                for (int r0 = tid >> sh; r0 < kBlockRows; r0 += 8 * rows) {
+                    uint32_t v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const int r = r0 + u * rows, tok = r < kBlockRows && c < cw ? s_tok[r] : -1;
+                        v[u] = tok >= 0 ? xs[(int64_t)tok * nkt + c0 + c] : 0x7f7f7f7fu;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (r0 + u * rows < kBlockRows && c < cw) s_sc[r0 + u * rows][c] = v[u];
                 }
                 __syncthreads();
+#pragma unroll 4
                 for (int i = tid; i < kBlockRows * cw; i += 256) {
                     const int c = i >> 7, r = i & 127;
                     xs_tiled[((int64_t)b * nkt + c0 + c) * kBlockRows + r] = s_sc[r][c];
@@ -893,7 +894,7 @@ static void launch_prologue(const MoeArgs &a, const SchedBuffers &sb, int per_up
                             hipStream_t s) {
     // the work lists are needed by the two kernels even when the rest of the prologue is masked off
     const int do_invert = (g_phase_mask & PMOE_PHASE_PROLOGUE) ? 1 : 0;
-    const int blocks = do_invert ? std::max(1, std::min((a.sorted_num + 255) / 256, a.crowd ? 48 : 1024)) : 1;
+    const int blocks = do_invert ? std::max(1, std::min((a.sorted_num + kBlockRows - 1) / kBlockRows, a.crowd ? 48 : 1024)) : 1;
     hipLaunchKernelGGL(a.crowd ? moe_prologue_kernel<true> : moe_prologue_kernel<false>, dim3(blocks), dim3(256), 0, s, a.expert_ids, a.ntpp, a.n_blocks, sb.tiles, sb.n_tiles,
                        sb.work_up, a.H / 128, per_up, grid_up, sb.work_down, (a.K + kWRows - 1) / kWRows, per_down, grid_down, a.E,
                        a.sorted_ids, a.sorted_num, a.inv, a.M * a.top_k, do_invert, a.x_scales, a.xs_tiled, a.K >> 7, a.top_k, a.M,

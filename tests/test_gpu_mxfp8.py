@@ -353,3 +353,31 @@ def test_several_weight_tiles_per_workgroup(T, K, E, N, top_k, per, device):
     ref = O.fused_moe_dense(deq["x"], deq["w1"], deq["w2"], ids.cpu(), wts.cpu(), act_mx=True)
     got = outs[1].float().cpu()
     assert cosine(got, ref) >= MX_COS_GATE and rel_l2(got, ref) <= MX_RELL2_GATE
+
+
+@pytest.mark.parametrize("blocks", [4157, 4160])  # live blocks: at most 4159, and 4161 or more; the row tiles of 4160 fit the prologue's LDS
+def test_prologue_tables_in_lds_and_in_the_workspace(blocks, device):
+    """Tokens are independent and both contractions are too short for the order of their sums to show: one call on all
+    of them gives bit for bit what calls on parts of them give."""
+    import prime_moe
+    T, K, E, N = blocks * 128 + 1, 256, 2, 256
+    g = torch.Generator(device=device).manual_seed(blocks)
+    x = torch.randn((T, K), generator=g, device=device).to(torch.bfloat16)
+    ids = torch.randint(0, E, (T, 1), generator=g, device=device, dtype=torch.int32)
+    wts = torch.rand((T, 1), generator=g, device=device)
+    w1, w1s = prime_moe.quantize_mx((torch.randn((E, N, K), generator=g, device=device) / 16).to(torch.bfloat16))
+    w2, w2s = prime_moe.quantize_mx((torch.randn((E, K, N // 2), generator=g, device=device) / 11).to(torch.bfloat16))
+    w1s, w2s = prime_moe.pack_scales_blocked(w1s), prime_moe.pack_scales_blocked(w2s)
+    xq, xs = prime_moe.quantize_mx(x)
+
+    def forward(a, b):
+        sched = torch.ops.prime_moe.moe_align(ids[a:b].contiguous(), E, 128, 1)
+        out = torch.empty((b - a, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_mxfp8(xq[a:b].contiguous(), xs[a:b].contiguous(), w1, w1s, w2, w2s, *sched, wts[a:b].contiguous(), out, 1,
+                                  128, 64, 4, 2, split=True)
+        return out, int(sched[2][0]) // 128
+    got, live = forward(0, T)
+    assert (live <= 4160) == (blocks == 4157)
+    for a in range(0, T, 65536):
+        part, _ = forward(a, min(a + 65536, T))
+        assert torch.equal(got[a:a + 65536].view(torch.int16), part.view(torch.int16))
