@@ -562,20 +562,20 @@ __global__ __launch_bounds__(512) void moe_up_kernel_bf16(MoeArgs a) {
 
 // Few up jobs (at most kDeepJobs (block, weight tile) pairs, K >= 2048).  All of them together leave most CUs idle, so every
 // job's contraction is shared among up to kDeepParts workgroups, which store fp32 partial sums; moe_up_join_kernel adds them in
-// part order and applies SwiGLU.  There are at most 32 blocks: a wave of every workgroup works out the row tiles (a lane per
+// part order and applies SwiGLU.  There are at most 64 blocks: a wave of every workgroup works out the row tiles (a lane per
 // block) while the last workgroup writes what the kernels behind need, and no prologue runs in front.
 // What bounds a workgroup is a chain: 1.4 us until it has the last rows of the blocks, 0.9 to cut them, 1.3 to its first
 // copies, 2 - 3 until these land, 0.7 - 1 per slab of its share (an eighth of K), 1 for the sums.  So the tiles are small, one
 // pair of fragments or two: there are twice as many busy CUs as with tiles of up to six pairs, a slab takes 0.72 instead of 1.0
 // us, and half as many sums leave through each CU (a run of blocks has at most twice as many pairs as blocks, so tiles of two
-// leave every job its eight parts on 256 CUs).  The weight rows that two tiles of a run share come from one L2: part p of every
+// leave the jobs of 32 (block, weight tile) pairs their eight parts on 256 CUs, those of 128 two).  The weight rows that two tiles of a run share come from one L2: part p of every
 // job runs on XCD p.  The token rows are gathered by the ids read for the plan.  8 experts of K 4096, N 512, top 4, the layer at
 // 256 tokens 41.7 -> 39.8 us (this kernel 18.6 -> 17.4), with up to six / up to two pairs a tile.  With 12 and 16 parts the K
 // loop is shorter by what the sums are longer: 25.1 and 25.2 us with the join instead of 23.6 (six pairs a tile).
 struct DeepTiles {
-    int4 tile[kDeepJobs];  // {first fragment, pairs of fragments, expert, first fragment's number}
-    int rows[kDeepJobs];   // of every block: 1 + its last live row
-    int ids[kDeepJobs * kBlockRows];  // sorted ids: the rows of a tile are gathered by them
+    int4 tile[kDeepBlocks];  // {first fragment, pairs of fragments, expert, first fragment's number}
+    int rows[kDeepBlocks];   // of every block: 1 + its last live row
+    int ids[kDeepBlocks * kBlockRows];  // sorted ids: the rows of a tile are gathered by them
     KernelPlan plan;
 };
 __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_down, int n_cus, int plan_only) {
@@ -585,14 +585,24 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
     const unsigned n_pairs = (unsigned)(a.M * a.top_k);
     const int n_slabs = a.K * 2 / tall::kRB;
     const int ntpp = a.ntpp[0], e_all = lane < a.n_blocks ? a.expert_ids[lane] : -1;
-    // the last live row of every block, a block per wave and turn
-    for (int blk = wave; blk < a.n_blocks; blk += 8) {
-        const int64_t at = (int64_t)blk * kBlockRows + lane;
-        const int id0 = at < a.sorted_num ? a.sorted_ids[at] : -1, id1 = at + 64 < a.sorted_num ? a.sorted_ids[at + 64] : -1;
-        const uint64_t m0 = __ballot((unsigned)id0 < n_pairs), m1 = __ballot((unsigned)id1 < n_pairs);
-        s.ids[blk * kBlockRows + lane] = id0;
-        s.ids[blk * kBlockRows + 64 + lane] = id1;
-        if (lane == 0) s.rows[blk] = m1 ? 128 - __builtin_clzll(m1) : m0 ? 64 - __builtin_clzll(m0) : 0;
+    // the last live row of every block: four blocks of a wave in flight
+    for (int b0 = wave; b0 < a.n_blocks; b0 += 32) {
+        int id[4][2];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t at = (int64_t)(b0 + 8 * u) * kBlockRows + lane;
+            id[u][0] = at < a.sorted_num ? a.sorted_ids[at] : -1;
+            id[u][1] = at + 64 < a.sorted_num ? a.sorted_ids[at + 64] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int blk = b0 + 8 * u;
+            if (blk >= a.n_blocks) break;
+            const uint64_t m0 = __ballot((unsigned)id[u][0] < n_pairs), m1 = __ballot((unsigned)id[u][1] < n_pairs);
+            s.ids[blk * kBlockRows + lane] = id[u][0];
+            s.ids[blk * kBlockRows + 64 + lane] = id[u][1];
+            if (lane == 0) s.rows[blk] = m1 ? 128 - __builtin_clzll(m1) : m0 ? 64 - __builtin_clzll(m0) : 0;
+        }
     }
     __syncthreads();
     if (wave == 0) {
@@ -606,17 +616,17 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
         const int f2 = last && e >= 0 && e < a.E ? ((lane - run) * kBlockRows + s.rows[lane] + 63) >> 6 : 0;
         const int n = (f2 + 5) / 6;
         const int halves = (f2 + 1) / 2;  // tiles of two pairs
-        // tiles, runs, pairs of fragments and tiles of two pairs (at most 32, 32, 64 and 32) up to and including this lane,
+        // tiles, runs, pairs of fragments and tiles of two pairs (at most 64, 64, 128 and 64) up to and including this lane,
         // added up together
         auto up_to = [&](int v) {
 #pragma unroll
-            for (int d = 1; d < kDeepJobs; d <<= 1) {
+            for (int d = 1; d < kDeepBlocks; d <<= 1) {
                 const int t = __shfl_up(v, d, 64);
                 if (lane >= d) v += t;
             }
             return v;
         };
-        const int sums = up_to(n | (f2 > 0 ? 1 << 8 : 0) | f2 << 16 | halves << 24), all = __shfl(sums, kDeepJobs - 1, 64);
+        const int sums = up_to(n | (f2 > 0 ? 1 << 8 : 0) | f2 << 16 | halves << 24), all = __shfl(sums, kDeepBlocks - 1, 64);
         const int tiles = sums & 0xff, runs = (sums >> 8) & 0xff, pairs = (sums >> 16) & 0xff;
         const int n_tiles = all & 0xff, n_runs = (all >> 8) & 0xff, n_f2 = (all >> 16) & 0xff;
         auto cut = [&](int4 *dst, int at, int count) {  // this lane's run in `count` tiles
@@ -635,13 +645,14 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
         KernelPlan kp{};
         kp.n_tiles = n_up_tiles;
         kp.deep = 1;
-        kp.parts = max(1, min(min(kDeepParts, n_slabs / 4), (int)gridDim.x / max(n_up_tiles * a.n_wtiles, 1)));
+        kp.parts = min(min(kDeepParts, n_slabs / 4), (int)gridDim.x / max(n_up_tiles * a.n_wtiles, 1));
+        kp.parts = max(1, min(kp.parts, kDeepSums / max(2 * n_f2 * a.n_wtiles, 1)));
         if (lane == 0) s.plan = kp;
         if (blockIdx.x == gridDim.x - 1) {
             // for the kernels behind: the down kernel's tiles and queues, the plans, the sorted numbers of the fragments
             const int want = choose_tiles(n_tiles, a.n_blocks, n_f2, n_wt_down, a.H * 2 / tall::kRB, n_cus), extra = max(want - n_tiles, 0);
             const int mine = f2 > 0 ? min(f2, n + extra / n_runs + (runs <= extra % n_runs ? 1 : 0)) : 0;
-            const int at = up_to(mine), n_down = __shfl(at, kDeepJobs - 1, 64);
+            const int at = up_to(mine), n_down = __shfl(at, kDeepBlocks - 1, 64);
             cut(a.tiles_down, at - mine, mine);
             int *numbers = reinterpret_cast<int *>(a.runs);
             for (int q = 0; q < 2 * f2; ++q) numbers[2 * (pairs - f2) + q] = 4 * run + q;
@@ -921,15 +932,30 @@ static int launch_few_pipeline(const MoeArgs &a, void *out, int split, hipStream
     return check_launch("fused_moe_bf16 launch");
 }
 
+// A workgroup of moe_deep_up_kernel has one job and comes back for no other: the grid holds every job, however the blocks
+// fall into tiles, and shares it between two workgroups at least.  Prologue and resident kernel / deep mode, whole layer, us: 8
+// experts of K 4096, N 512, top 4: 63.2 / 43.7 at 280 tokens (17 blocks), 75.3 / 46.8 at 400, 78.9 / 57.9 at 600, 88.7 / 57.8 at 770, 89.0 /
+// 72.1 at 1000, 98.4 / 82.4 at 1400, 111.8 / 95.3 at 1790 (64 blocks); one of N 2048 82.9 / 62.3 at 1000 tokens; 2 of N 4096 73.7 / 62.8 at
+// 300; 4 of K 2048, N 1024, top 2 58.3 / 50.5 at 1000; 4 of K 7168, N 2048 121.3 / 86.1 at 500.
+static bool use_deep(const MoeArgs &a) { return a.deep_ok && a.n_blocks > 0 && 2 * a.n_blocks * (a.H / 128) <= resident_grid(); }
+
 // Few rows per expert on average: what the problem costs is the stream of the weights (moe_stream.h).  Whole op,
 // stream against tall tiles, us (graph replays): 8 large experts (K 4096, N 28672, top 2) 117 / 300 at 1 token, 424 /
 // 567 at 32, 487 / 570 at 128 (32 rows per expert), 576 / 573 at 192; 128 small experts (K 2048, N 1536, top 8) 24 /
 // 45 at 1 token, 163 / 232 at 64, 251 / 264 at 384, 285 / 282 at 512 (32 rows per expert), 343 / 293 at 768.
 // With few jobs of tall tiles and no deep mode to share them it pays longer (37 experts, K 4096, N 256, top 9: 74 / 121
-// at 256 tokens, 62 rows per expert).
+// at 256 tokens, 62 rows per expert).  With the deep mode for up to 32 (block, weight tile) pairs it ends at 32 rows; beyond, the
+// deep mode is the faster one where the contraction is long and the weight tiles are one or two.  Stream / deep at 34 and 62 rows
+// per expert, us: K 4096, 37 experts of N 256 51.9 / 50.5 and 60 / 51, 16 of N 512 40.4 / 41.6 and 60.3 / 45.4; K 7168, 32 of N 256
+// 62.2 / 59.9 and 96.6 / 69.2; but K 2048, 37 of N 256 35.9 / 40.4 and 47.8 / 44.3, 24 of N 512 36.1 / 38.2 and 45.4 / 42.1, 8 of N 2048
+// 33.8 / 42.9 and 44.2 / 47.6; K 4096, 8 of N 1024 33.1 / 40.1 and 48.4 / 44.2.  One expert named by all of 180 tokens, 37 of K
+// 4096, N 256: 72.2 / 54.0.
 static bool use_stream(const MoeArgs &a) {
     const int64_t tall_jobs = std::min<int64_t>(a.n_blocks, a.E) * (a.H / 128);
-    const int64_t rows = tall_jobs < resident_grid() / 2 && !a.deep_ok ? 64 : 32;
+    const int n_wt = a.H / 128;
+    const bool few_jobs = tall_jobs < resident_grid() / 2;
+    int64_t rows = few_jobs ? 64 : 32;
+    if (few_jobs && use_deep(a)) rows = a.n_blocks * n_wt <= 32 ? 32 : a.K >= 4096 && n_wt <= 2 ? 34 : 64;
     return (int64_t)a.M * a.top_k <= rows * a.E;
 }
 
@@ -991,9 +1017,9 @@ size_t bf16_workspace(MoeArgs &a, char *ws) {
     a.tiles_down = reinterpret_cast<int4 *>(take((blocks + 1) * sizeof(int4)));
     // few up jobs for the chip and a contraction long enough to share (whether the chip has room is seen at the launch: the
     // size does not depend on the device)
-    a.deep_ok = (blocks * n_wt_up <= (size_t)kDeepJobs && a.K >= 2048) ? 1 : 0;
+    a.deep_ok = (blocks <= (size_t)kDeepBlocks && blocks * n_wt_up <= (size_t)kDeepJobs && a.K >= 2048) ? 1 : 0;
     a.up_partials = reinterpret_cast<float *>(
-        take(a.deep_ok ? (size_t)kDeepParts * 4 * blocks * n_wt_up * 2048 * sizeof(float4) : 0));
+        take(a.deep_ok ? std::min<size_t>(kDeepParts * 4 * blocks * n_wt_up, kDeepSums) * 2048 * sizeof(float4) : 0));
     const size_t pairs = (size_t)a.M * (size_t)std::max(a.top_k, 1);
     a.inv = reinterpret_cast<int32_t *>(take(pairs * sizeof(int32_t)));
     a.y = take(pairs * a.K * 2);  // one row per pair id
@@ -1009,9 +1035,7 @@ int launch_bf16_pipeline(MoeArgs a, void *out, int split, hipStream_t s) {
     const int n_wt_up = a.H / 128, n_wt_down = (a.K + kWRows - 1) / kWRows;
     const int n_cus = resident_grid();
     a.n_wtiles = n_wt_up;
-    // A workgroup of moe_deep_up_kernel has one job and comes back for no other: the grid holds every job, however the blocks
-    // fall into tiles, and shares it between two workgroups at least.
-    if (a.deep_ok && a.n_blocks > 0 && 2 * a.n_blocks * n_wt_up <= n_cus) {
+    if (use_deep(a)) {
         // (the plan is part of the up kernel, and a launch of its own only where the down kernel runs without it)
         if (mask & (PMOE_PHASE_UP | PMOE_PHASE_DOWN | PMOE_PHASE_PROLOGUE))
             hipLaunchKernelGGL(moe_deep_up_kernel, dim3(n_cus), dim3(512), 0, s, a, n_wt_down, n_cus,

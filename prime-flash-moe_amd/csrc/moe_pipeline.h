@@ -53,7 +53,9 @@ struct TallJob {
     int part, parts;
 };
 constexpr int kDeepParts = 8;    // most parts of an up job in deep mode
-constexpr int kDeepJobs = 32;    // deep mode is taken up to this many (row block, weight tile) pairs
+constexpr int kDeepJobs = 128;   // deep mode is taken up to this many (row block, weight tile) pairs
+constexpr int kDeepBlocks = 64;  // and this many blocks, a lane each where they are cut
+constexpr int kDeepSums = 1024;  // (fragment, weight tile, part) sums the workspace holds at most: four per workgroup of 256
 
 // Position l of a kernel's walk -> job.
 __device__ __forceinline__ void walk_to_job(int l, int nt, int n_wt, int &tile, int &wt) {

@@ -350,6 +350,12 @@ def test_deep_up_kernel_cuts_and_plans(K, N, counts, device):
     (4096, 256, [64] * 10 + [700, 640]),       # 31 pairs x 1
     (2304, 1024, [300, 129]),                  # 8 pairs x 4: as many as there is room for; a share of 4 or 5 slabs
     (2048, 1280, [321, 63]),                   # 7 pairs x 5: one tile of two pairs and a single one
+    (2048, 512, [8065]),                       # 64 blocks, the most, x 2: two parts each, as many sums as the workspace holds
+    (2048, 512, [8066]),                       # 65: the resident kernel
+    (2304, 256, [4000, 3, 1500, 129, 64]),     # 49 blocks: five parts of 7 or 8 slabs
+    (2048, 2048, [700, 600, 200]),             # 15 blocks x 8
+    (2048, 2048, [700, 600, 367]),             # 16 blocks x 8: the most pairs
+    (2048, 2048, [700, 600, 368]),             # 17 x 8: the resident kernel
 ])
 def test_deep_up_kernel_tiles_of_one_pair_and_two(K, N, counts, device):
     """The edge between tiles of one pair of fragments and of two (256 CUs: pairs x weight tiles x 8 parts), against the oracle."""
@@ -361,7 +367,9 @@ def test_deep_up_kernel_tiles_of_one_pair_and_two(K, N, counts, device):
     g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
     wts = torch.rand((T, 1), generator=g, device=device)
     sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
-    assert T > 32 * E and sched[0].numel() // 128 * (N // 256) <= 32 and K >= 2048  # the rules of the dispatch
+    blocks = sched[0].numel() // 128
+    assert T > 64 * E and K >= 2048  # the rules of the dispatch
+    assert (blocks <= 64 and blocks * (N // 256) <= 128) == (counts not in ([8066], [700, 600, 368]))
     ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
     out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
     prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, 1, 128, 64, 4, 2, 1, 1, True)
