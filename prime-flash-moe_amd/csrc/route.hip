@@ -134,7 +134,7 @@ __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restric
     extern __shared__ int32_t smem[];
     __shared__ int32_t ids[NW * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int reach_blocks = min((reach + o.block_m - 1) / o.block_m, o.max_blocks);
+    const int reach_blocks = (int)min(((int64_t)reach + o.block_m - 1) / o.block_m, (int64_t)o.max_blocks);
     if (blockIdx.x > 0) {
         const int n = (int)(gridDim.x - 1) * NW * 64, me = (int)(blockIdx.x - 1) * NW * 64 + tid;
         pmoe::align::fill_minus_one(o.sorted_token_ids + reach, o.max_padded - reach, me, n);
@@ -184,8 +184,8 @@ int launch_topk(const T *logits, const float *bias, int32_t *topk_ids, float *to
             const int n = n_tokens * top_k;
             const int64_t rows = n + (int64_t)std::min(n, E) * (o->pad_to - 1);
             const int reach = (int)std::min<int64_t>(o->max_padded, (rows + o->block_m - 1) / o->block_m * o->block_m);
-            const int rest = std::max(o->max_padded - reach, 4 * (o->max_blocks - reach / o->block_m));
-            const int fillers = std::min((rest + NW * 256 - 1) / (NW * 256), 15);  // 16 bytes a thread and turn
+            const int64_t rest = std::max<int64_t>(o->max_padded - reach, 4 * ((int64_t)o->max_blocks - reach / o->block_m));
+            const int fillers = (int)std::min<int64_t>((rest + NW * 256 - 1) / (NW * 256), 15);  // 16 bytes a thread and turn
             hipLaunchKernelGGL((route_small_kernel<NW, EPL, T>), dim3(1 + fillers), dim3(NW * 64), sizeof(int32_t) * (size_t)pmoe::align::sort_words(NW, E),
                                s, logits, bias, topk_ids, topk_weights, *o, reach, n_tokens, E, top_k, pmoe::align::id_bits_for(E));
         });

@@ -84,6 +84,16 @@ def test_rows_that_no_pair_can_reach(T, E, k, spread, block_m, bpc, device):
     _check(logits, k, block_m=block_m, bpc=bpc)
 
 
+def test_one_token_with_a_block_beyond_half_of_31_bits(device):
+    """Rows and blocks are added in 64 bits: one block of 1.2e9 rows, all of which the pair can reach."""
+    import prime_moe
+    block_m = 1_200_000_000
+    ids, w, s, e, t = prime_moe.route(torch.zeros((1, 1), device=device), 1, block_m, 1)
+    torch.cuda.synchronize()
+    assert s.numel() == block_m and e.tolist() == [0] and t.tolist() == [block_m]
+    assert int(s[0]) == 0 and bool((s[1:] == -1).all())
+
+
 def test_route_ties_go_to_the_lower_index(device):
     # few distinct values: almost every selection is decided by the tie rule
     g = torch.Generator(device=device).manual_seed(3)
