@@ -565,12 +565,13 @@ __global__ __launch_bounds__(512) void moe_up_kernel_bf16(MoeArgs a) {
 // part order and applies SwiGLU.  There are at most 64 blocks: a wave of every workgroup works out the row tiles (a lane per
 // block) while the last workgroup writes what the kernels behind need, and no prologue runs in front.
 // What bounds a workgroup is a chain: 1.4 us until it has the last rows of the blocks, 0.9 to cut them, 1.3 to its first
-// copies, 2 - 3 until these land, 0.7 - 1 per slab of its share (an eighth of K), 1 for the sums.  So the tiles are small, one
-// pair of fragments or two: there are twice as many busy CUs as with tiles of up to six pairs, a slab takes 0.72 instead of 1.0
-// us, and half as many sums leave through each CU (a run of blocks has at most twice as many pairs as blocks, so tiles of two
-// leave the jobs of 32 (block, weight tile) pairs their eight parts on 256 CUs, those of 128 two).  The weight rows that two tiles of a run share come from one L2: part p of every
-// job runs on XCD p.  The token rows are gathered by the ids read for the plan.  8 experts of K 4096, N 512, top 4, the layer at
-// 256 tokens 41.7 -> 39.8 us (this kernel 18.6 -> 17.4), with up to six / up to two pairs a tile.  With 12 and 16 parts the K
+// copies, 2 - 3 until these land, 0.7 - 1 per slab of its share of K, 1 for the sums.  So the tiles are small, one
+// pair of fragments or two: there are more busy CUs than with tiles of up to six pairs, a slab takes 0.72 instead of 1.0
+// us, and fewer sums leave through each CU (a run of blocks has at most twice as many pairs as blocks, so tiles of two
+// leave the jobs of 32 (block, weight tile) pairs their eight parts on 256 CUs, those of 128 two).  Of eight parts, part p of every
+// job runs on XCD p, and the weight rows that two tiles of a run share come from one L2.  The token rows are gathered by the ids
+// read for the plan.  8 experts of K 4096, N 512, top 4, the layer at 256 tokens 41.7 -> 39.8 us (this kernel 18.6 -> 17.4),
+// with up to six / up to two pairs a tile.  With 12 and 16 parts the K
 // loop is shorter by what the sums are longer: 25.1 and 25.2 us with the join instead of 23.6 (six pairs a tile).
 struct DeepTiles {
     int4 tile[kDeepBlocks];  // {first fragment, pairs of fragments, expert, first fragment's number}
