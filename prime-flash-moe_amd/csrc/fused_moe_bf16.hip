@@ -93,7 +93,9 @@ __device__ __forceinline__ float estimate_kernel(int n_tiles, int f2, int n_wt, 
     const int jobs = n_tiles * n_wt, rounds = jobs / n_cus, rest = jobs % n_cus;
     float t = (float)rounds * cost(g);
     if (rest > 0) {
-        const int p = rounds >= 16 ? 1 : min(min(4, n_cus / rest), max(1, (int)g));
+        // (the walk is dealt in whole rounds of kWalkRound jobs, and a split takes all that is left behind them: only where that
+        // is what the chip has left over, too, always on as many CUs)
+        const int p = rounds >= 16 || rest != jobs % kWalkRound ? 1 : min(min(4, n_cus / rest), max(1, (int)g));
         t += p > 1 ? 1.3f * cost(g / (float)p) : cost(g);
         if (p > 1) {
             parts = p;

@@ -52,6 +52,7 @@ struct TallJob {
     int tile, wt;
     int part, parts;
 };
+constexpr int kWalkRound = 256;  // jobs of a whole round of the walk (see above): as many as CUs
 constexpr int kDeepParts = 8;    // most parts of an up job in deep mode
 constexpr int kDeepJobs = 128;   // deep mode is taken up to this many (row block, weight tile) pairs
 constexpr int kDeepBlocks = 64;  // and this many blocks, a lane each where they are cut
@@ -77,7 +78,7 @@ __device__ __forceinline__ int resolve_tall_job(int b, int n_wt, const KernelPla
         j.part = b - l * kp.parts;
         j.parts = kp.parts;
     } else {
-        const int full = n_jobs & ~255, main_end = (n_jobs + 255) & ~255;
+        const int full = n_jobs & ~(kWalkRound - 1), main_end = (n_jobs + kWalkRound - 1) & ~(kWalkRound - 1);
         if (b < full) {
             const int xcd = b & 7, pos = b >> 3;
             l = (((pos >> 5) * 8 + xcd) << 5) + (pos & 31);

@@ -445,6 +445,38 @@ def test_few_up_jobs_on_fewer_cus(cus, device):
     assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
 
 
+@pytest.mark.parametrize("counts,N,cus", [
+    ([65] * 33, 2048, 1024),   # 33 tiles of two pairs of fragments x 8 weight tiles: 264 jobs, a round of 256 and 8
+    ([65] * 33, 2048, 512),
+    ([400] * 5, 1024, 32),     # 40 jobs: 8 behind a round of 32, 40 behind no round of 256
+    ([400] * 5, 1024, 128),    # one round that is not full on either
+    ([700] * 5, 2048, 64),     # 80 jobs
+    ([700] * 5, 2048, 256),
+])
+def test_last_round_of_the_resident_kernels_on_other_numbers_of_cus(counts, N, cus, device):
+    """The part of the last round that is shared by rows is the one that the walk of the jobs leaves over, on any number of CUs."""
+    import prime_moe
+    from prime_moe import _native
+    K, E, lib = 512, len(counts), _native.load()
+    ids = torch.repeat_interleave(torch.arange(E, dtype=torch.int32, device=device), torch.tensor(counts, device=device)).view(-1, 1).contiguous()
+    T = ids.shape[0]
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=T)
+    wts = torch.rand((T, 1), generator=g, device=device)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    assert T > 64 * E and K < 2048  # the rules of the dispatch: prologue and resident kernels
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    lib.pmoe_set_compute_units(cus)
+    try:
+        prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, 1, 128, 64, 4, 2, 1, 1, True)
+    finally:
+        lib.pmoe_set_compute_units(0)
+    torch.cuda.synchronize()
+    got = out.float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
 def _prologue_workspace(x, w1, w2, sched, wts, out, top_k):
     """The workspace after the prologue of the tall-tile path: it starts with the plan, the run list and the table of row
     tiles (bf16_workspace in csrc/fused_moe_bf16.hip)."""
