@@ -641,8 +641,9 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
                 number += 2 * fg;
             }
         };
-        // The up kernel's tiles: one pair of fragments where that leaves a workgroup for every part of every job, or two.
-        const bool single = n_f2 * a.n_wtiles * kDeepParts <= (int)gridDim.x;
+        // The up kernel's tiles: one pair of fragments where that leaves a workgroup for every part of every job, or two (of
+        // which there are never more than blocks; more than 64 of one pair would take 520 CUs, and have no room in the table).
+        const bool single = n_f2 <= kDeepBlocks && n_f2 * a.n_wtiles * kDeepParts <= (int)gridDim.x;
         const int n_up = single ? f2 : halves, n_up_tiles = single ? n_f2 : all >> 24;
         cut(s.tile, (single ? pairs : sums >> 24) - n_up, n_up);
         KernelPlan kp{};

@@ -378,6 +378,36 @@ def test_deep_up_kernel_tiles_of_one_pair_and_two(K, N, counts, device):
     assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
 
 
+@pytest.mark.parametrize("counts", [
+    [8065],       # 64 blocks, 127 pairs of fragments: the table of the cut has room for 64 tiles
+    [4096],       # 64 pairs: all of one pair
+    [4097],       # 65
+    [65] * 33,    # 33 blocks, 66 pairs
+])
+def test_deep_up_kernel_on_more_cus_than_its_table_has_tiles(counts, device):
+    """From 520 CUs on there would be a workgroup for every part of more tiles of one pair of fragments than the table holds."""
+    from prime_moe import _native
+    import prime_moe
+    K, N, E, lib = 2048, 256, len(counts), _native.load()
+    ids = torch.repeat_interleave(torch.arange(E, dtype=torch.int32, device=device), torch.tensor(counts, device=device)).view(-1, 1).contiguous()
+    T = ids.shape[0]
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=T)
+    wts = torch.rand((T, 1), generator=g, device=device)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    assert 32 < sched[0].numel() // 128 <= 64 and T > 64 * E  # the rules of the dispatch
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    for cus in (512, 520, 1024):
+        lib.pmoe_set_compute_units(cus)
+        try:
+            out = torch.full((T, K), float("nan"), dtype=torch.bfloat16, device=device)
+            prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, 1, 128, 64, 4, 2, 1, 1, True)
+        finally:
+            lib.pmoe_set_compute_units(0)
+        torch.cuda.synchronize()
+        got = out.float().cpu()
+        assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE, cus
+
+
 @pytest.mark.parametrize("counts,order", [
     ([0, 700, 0, 700], None),                            # ascending, expert 0 without rows: two runs of six blocks
     ([130, 60, 40, 230], [4, 0, 1, 2, 3, 5]),            # experts 3 0 0 1 2 3: another expert in front of expert 0
