@@ -89,8 +89,8 @@ int pmoe_moe_align_static(const int32_t *topk_ids, int32_t *sorted_token_ids, in
 /*
  * Workspace (bytes) the fused calls below need for a problem of this size.  The
  * caller allocates it on the device (any 256-byte aligned buffer) and passes it in.
- * The size does not depend on `split` (both values run the same kernels); the argument
- * is kept so that the query takes what the call takes.
+ * The query takes the sizes of the call.  The size does not depend on `split` (both values
+ * run the same kernels).
  */
 size_t pmoe_fused_moe_bf16_workspace_bytes(int M, int K, int N, int num_experts, int sorted_num,
                                            int top_k, int split);

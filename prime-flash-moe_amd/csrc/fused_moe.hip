@@ -997,11 +997,10 @@ extern "C" void pmoe_set_tiles_per_workgroup(int n) { g_tiles_per_wg = n < 0 ? 0
 
 extern "C" size_t pmoe_fused_moe_bf16_workspace_bytes(int M, int K, int N, int num_experts,
                                                       int sorted_num, int top_k, int split) {
-    (void)num_experts;
     (void)split;
     if (M <= 0 || K <= 0 || N <= 0 || sorted_num < 0) return 0;
     MoeArgs a{};
-    a.M = M; a.K = K; a.N = N; a.H = N / 2; a.sorted_num = sorted_num; a.top_k = top_k;
+    a.M = M; a.K = K; a.N = N; a.H = N / 2; a.E = num_experts; a.sorted_num = sorted_num; a.top_k = top_k;
     return bf16_workspace(a, nullptr);
 }
 

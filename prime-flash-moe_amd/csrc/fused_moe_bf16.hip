@@ -954,12 +954,14 @@ static bool use_deep(const MoeArgs &a) { return a.deep_ok && a.n_blocks > 0 && 2
 // 62.2 / 59.9 and 96.6 / 69.2; but K 2048, 37 of N 256 35.9 / 40.4 and 47.8 / 44.3, 24 of N 512 36.1 / 38.2 and 45.4 / 42.1, 8 of N 2048
 // 33.8 / 42.9 and 44.2 / 47.6; K 4096, 8 of N 1024 33.1 / 40.1 and 48.4 / 44.2.  One expert named by all of 180 tokens, 37 of K
 // 4096, N 256: 72.2 / 54.0.
+constexpr int64_t kStreamRows = 32;  // the fewest rows per expert up to which any call streams
+static bool always_streams(const MoeArgs &a) { return (int64_t)a.M * a.top_k <= kStreamRows * a.E; }
 static bool use_stream(const MoeArgs &a) {
     const int64_t tall_jobs = std::min<int64_t>(a.n_blocks, a.E) * (a.H / 128);
     const int n_wt = a.H / 128;
     const bool few_jobs = tall_jobs < resident_grid() / 2;
-    int64_t rows = few_jobs ? 64 : 32;
-    if (few_jobs && use_deep(a)) rows = a.n_blocks * n_wt <= 32 ? 32 : a.K >= 4096 && n_wt <= 2 ? 34 : 64;
+    int64_t rows = few_jobs ? 64 : kStreamRows;
+    if (few_jobs && use_deep(a)) rows = a.n_blocks * n_wt <= 32 ? kStreamRows : a.K >= 4096 && n_wt <= 2 ? 34 : 64;
     return (int64_t)a.M * a.top_k <= rows * a.E;
 }
 
@@ -1020,8 +1022,8 @@ size_t bf16_workspace(MoeArgs &a, char *ws) {
     a.tiles = reinterpret_cast<int4 *>(take((blocks + 1) * sizeof(int4)));
     a.tiles_down = reinterpret_cast<int4 *>(take((blocks + 1) * sizeof(int4)));
     // few up jobs for the chip and a contraction long enough to share (whether the chip has room is seen at the launch: the
-    // size does not depend on the device)
-    a.deep_ok = (blocks <= (size_t)kDeepBlocks && blocks * n_wt_up <= (size_t)kDeepJobs && a.K >= 2048) ? 1 : 0;
+    // size does not depend on the device), and not so few rows that the streaming kernels run whatever the device
+    a.deep_ok = (blocks <= (size_t)kDeepBlocks && blocks * n_wt_up <= (size_t)kDeepJobs && a.K >= 2048 && !always_streams(a)) ? 1 : 0;
     a.up_partials = reinterpret_cast<float *>(
         take(a.deep_ok ? std::min<size_t>(kDeepParts * 4 * blocks * n_wt_up, kDeepSums) * 2048 * sizeof(float4) : 0));
     const size_t pairs = (size_t)a.M * (size_t)std::max(a.top_k, 1);

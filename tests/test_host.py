@@ -71,6 +71,20 @@ def test_workspace_query_and_c_side_validation_need_no_gpu():
     assert rc == 1 and b"smaller than 4 GiB" in lib.pmoe_last_error()
 
 
+@pytest.mark.parametrize("M,top_k,E,sums", [(8, 9, 37, False), (148, 8, 37, False), (149, 8, 37, True)])
+def test_partial_sums_are_not_reserved_for_calls_that_always_stream(M, top_k, E, sums):
+    """Up to 32 rows per expert on average the streaming kernels run on every device, and the deep contraction split never does."""
+    from prime_moe import _native
+    K, N = 4096, 256
+    rows = (M * top_k + E * 127 + 127) // 128 * 128
+    blocks, pairs = rows // 128, M * top_k
+    assert blocks <= 64 and blocks * (N // 256) <= 128 and sums == (pairs > 32 * E)  # few enough for the deep split
+    up = lambda n: (n + 255) // 256 * 256
+    assert _native.load().pmoe_fused_moe_bf16_workspace_bytes(M, K, N, E, rows, top_k, 1) == \
+        256 + up((blocks + 1) * 20) + 2 * up((blocks + 1) * 16) + (min(8 * 4 * blocks, 1024) * 32768 if sums else 0) + \
+        up(pairs * 4) + pairs * K * 2 + rows * N
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     from prime_moe import _native
     monkeypatch.setattr(_native, "_lib", None)
