@@ -949,11 +949,16 @@ static bool use_deep(const MoeArgs &a) { return a.deep_ok && a.n_blocks > 0 && 2
 // 45 at 1 token, 163 / 232 at 64, 251 / 264 at 384, 285 / 282 at 512 (32 rows per expert), 343 / 293 at 768.
 // With few jobs of tall tiles and no deep mode to share them it pays longer (37 experts, K 4096, N 256, top 9: 74 / 121
 // at 256 tokens, 62 rows per expert).  With the deep mode for up to 32 (block, weight tile) pairs it ends at 32 rows; beyond, the
-// deep mode is the faster one where the contraction is long and the weight tiles are one or two.  Stream / deep at 34 and 62 rows
-// per expert, us: K 4096, 37 experts of N 256 51.9 / 50.5 and 60 / 51, 16 of N 512 40.4 / 41.6 and 60.3 / 45.4; K 7168, 32 of N 256
-// 62.2 / 59.9 and 96.6 / 69.2; but K 2048, 37 of N 256 35.9 / 40.4 and 47.8 / 44.3, 24 of N 512 36.1 / 38.2 and 45.4 / 42.1, 8 of N 2048
-// 33.8 / 42.9 and 44.2 / 47.6; K 4096, 8 of N 1024 33.1 / 40.1 and 48.4 / 44.2.  One expert named by all of 180 tokens, 37 of K
-// 4096, N 256: 72.2 / 54.0.
+// deep mode is the faster one where the contraction is long and the weight tiles are one or two.  How early depends on the bytes of
+// the weights, which streaming reads once per 32 or 64 rows: from 34 rows per expert on with 112 MB or more, behind 48 with less.  Stream /
+// deep at 35, 44 and 58 rows, whole layer, us: K 4096, 16 experts of N 512 (101 MB) 39.4 / 41.7, 41.5 / 42.0 and 51.0 / 43.5, 28 of N 256 (88
+// MB) 43.2 / 44.7, 46.5 / 44.7 and 61.9 / 50.4, 24 of N 256 (75 MB) 40.8 / 41.8 at 44 and 53.9 / 44.3, 18 of N 512 (113 MB) 49.1 / 46.6, 54.4 /
+// 47.8 and 72.2 / 51.3, 37 of N 256 (116 MB) 53.4 / 49.2, 57.3 / 50.7 and 67.6 / 53.4; K 5120, 14 of N 512 (110 MB) 43.3 / 45.4, 48.3 / 46.0 and
+// 60.5 / 48.5; K 6144, 13 of N 512 (123 MB) 47.3 / 45.7, 52.5 / 46.8 and 67.2 / 48.9; K 16384, 37 of N 256 183 / 137, 188 / 143 and 209 / 149.
+// With a shorter contraction or more weight tiles, at 34 and 62 rows: K 2048, 37 of N 256 35.9 / 40.4 and 47.8 / 44.3, 24 of N 512 36.1 / 38.2
+// and 45.4 / 42.1, 8 of N 2048 33.8 / 42.9 and 44.2 / 47.6; K 4096, 8 of N 1024 33.1 / 40.1 and 48.4 / 44.2: these stream up to 64.
+// One expert named by all of 180 tokens, 37 of K 4096, N 256: 72.2 / 54.0.
+constexpr float kStreamBytes = 112e6f;
 constexpr int64_t kStreamRows = 32;  // the fewest rows per expert up to which any call streams
 static bool always_streams(const MoeArgs &a) { return (int64_t)a.M * a.top_k <= kStreamRows * a.E; }
 static bool use_stream(const MoeArgs &a) {
@@ -961,7 +966,10 @@ static bool use_stream(const MoeArgs &a) {
     const int n_wt = a.H / 128;
     const bool few_jobs = tall_jobs < resident_grid() / 2;
     int64_t rows = few_jobs ? 64 : kStreamRows;
-    if (few_jobs && use_deep(a)) rows = a.n_blocks * n_wt <= 32 ? kStreamRows : a.K >= 4096 && n_wt <= 2 ? 34 : 64;
+    if (few_jobs && use_deep(a)) {
+        const bool heavy = 3.f * (float)a.E * (float)a.N * (float)a.K >= kStreamBytes;
+        rows = a.n_blocks * n_wt <= 32 ? kStreamRows : a.K >= 4096 && n_wt <= 2 ? (heavy ? 34 : 48) : 64;
+    }
     return (int64_t)a.M * a.top_k <= rows * a.E;
 }
 
