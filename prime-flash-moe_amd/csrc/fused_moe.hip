@@ -542,13 +542,18 @@ __device__ __forceinline__ void emit_work(int4 *work, int grid, int n_wt, int pe
 // block-wide scans per 256 blocks, then the two walk orders).  Each of them works out all tiles, in LDS, and writes its
 // share of the lists; only of more than kLdsTiles blocks workgroup 0 writes them alone, from tiles in the workspace.  What bounds it is
 // the chain of scans; the lists of 4096 tokens on 256 experts have 22440 entries, 11264 of them jobs.
-// The re-tiling of the x scales took 28 us there for want of loads in flight (a row and its token at a time): eight rows of
-// every lane, a block per workgroup and no division in the loop.  Prologue, before / now, us: 4096 tokens on 256 experts (K 7168,
-// N 4096) 28.7 / 10.9, 24593 on 32 (K = N = 2048) 17.7 / 10.8; the layers 2474 / 2462 and 818 / 814.
+// A builder comes late to its share of the rest, so there are only as many as the lists are long (kListEntries).  Prologue with one builder /
+// one per 512 entries / a quarter of the workgroups, us: 600 tokens on 8 experts (K = N = 512) 4.2 / 4.4 / 5.3, 2000 on 8 (K 2048, N 512) 4.8 /
+// 4.9 / 6.0, 4000 on 16 (K 4096, N 2048) 7.2 / 6.0 / 8.8, 24593 on 32 (K = N = 2048) 17.5 / 10.8 / 10.4, 6000 on 128 (K 2048, N 1536) 13.4 /
+// 7.9 / 7.7, 4096 on 257 (K 7168, N 512) 15.0 / 9.9 / 9.7.
+// The re-tiling of the x scales is done with eight rows of every lane in flight, a block per workgroup and no division in the loop.  Prologue
+// with a row and its token at a time and the lists by one workgroup / as it is, us: 4096 tokens on 256 experts (K 7168, N 4096) 28.7 /
+// 10.9, 24593 on 32 16.6 / 10.8, 2000 on 8 9.7 / 4.9.  Beyond some 100 us the layer shows nothing of it.
 // All workgroups invert the sorted order: inv[pair id] = sorted row.  Entries of pairs that are not
 // in the schedule keep whatever the buffer held; the reader validates an entry against sorted_ids.
 // CROWD: only for crowded schedules (`n_cus`: see crowded_mx).
 constexpr int kLdsTiles = kBlockRows * 65 / 2;
+constexpr int kListEntries = 512;  // of both lists, a builder each
 template <bool CROWD>
 __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert_ids, const int32_t *ntpp,
                                                            int n_blocks, int2 *tiles, int *n_tiles,
@@ -560,9 +565,9 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
                                                            uint32_t *xs_tiled, int nkt, int top_k, int M, int n_cus) {
     if (CROWD && !crowded_mx(ntpp, n_blocks, n_pairs, n_wt_up, n_cus)) return;
     const int n_live = min((ntpp[0] + kBlockRows - 1) / kBlockRows, n_blocks);
-    const int builders = min(max((int)gridDim.x / 4, 1), 32);
+    const int builders = n_live <= kLdsTiles ? max(min(min((grid_up + grid_down) / kListEntries, (int)gridDim.x / 4), 32), 1) : 1;
     __shared__ uint32_t s_sc[kBlockRows][65];  // row tiles first
-    if ((int)blockIdx.x < (n_live <= kLdsTiles ? builders : 1)) {
+    if ((int)blockIdx.x < builders) {
         __shared__ int s_max[4], s_sum[4], s_carry[2];
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
         int2 *table = n_live <= kLdsTiles ? reinterpret_cast<int2 *>(&s_sc[0][0]) : tiles;
@@ -605,7 +610,7 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
         if (blockIdx.x == 0 && tid == 0) n_tiles[0] = nt;
         __threadfence_block();
         __syncthreads();  // tiles written above are read below by other threads
-        const int me = (int)blockIdx.x * 256 + tid, threads = (n_live <= kLdsTiles ? builders : 1) * 256;
+        const int me = (int)blockIdx.x * 256 + tid, threads = builders * 256;
         emit_work(work_up, grid_up, n_wt_up, per_job_up, table, nt, num_experts, me, threads);
         emit_work(work_down, grid_down, n_wt_down, per_job_down, table, nt, num_experts, me, threads);
         __syncthreads();  // (a workgroup that re-tiles, too, uses the LDS again)
