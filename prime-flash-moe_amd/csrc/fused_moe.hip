@@ -511,36 +511,64 @@ __global__ __launch_bounds__(512) void moe_down_kernel(MoeArgs a) {
 // tiles), w = 1 if the row tile is the only one of its expert.
 //
 // The work list of a kernel with n_wt weight tiles, of which a workgroup takes `per_job` consecutive ones, over `n_tiles` row
-// tiles {first block | blocks << 28, expert}: thread `me` of `threads` writes entries me, me + threads, ... of the `grid` there are,
-// -1 where the walk has ended or a block names no expert.  By position, so that neighbouring threads write neighbouring entries
+// tiles {first block | blocks << 28, expert}, has `grid` entries: -1 where the walk has ended or a block names no expert.
+struct ListShape {
+    int n_wt, per_job, n_jobs, total, per_xcd;
+    __device__ __forceinline__ ListShape(int n_wt_, int per_job_, int n_tiles) : n_wt(n_wt_), per_job(per_job_) {
+        n_jobs = (n_wt + per_job - 1) / per_job;
+        total = n_tiles * n_jobs;
+        per_xcd = (total + 7) >> 3;
+    }
+};
+__device__ __forceinline__ int4 list_entry(const ListShape &l, const int2 *tiles, int n_tiles, int num_experts, int t, int j) {
+    const int2 tl = tiles[t];
+    if (tl.y < 0 || tl.y >= num_experts) return make_int4(-1, -1, 0, 0);
+    // (the only row tile of its expert: then nobody else reads that expert's weight rows)
+    const bool shared = (t > 0 && tiles[t - 1].y == tl.y) || (t + 1 < n_tiles && tiles[t + 1].y == tl.y);
+    const int wt = j * l.per_job, cnt = min(l.per_job, l.n_wt - wt);
+    return make_int4(tl.x, wt | (tl.y << 16) | ((cnt - 1) << 26), 0, shared ? 0 : 1);
+}
+constexpr int kListGroup = 8;  // weight tiles of a group of the walk
+// Thread `me` of `threads` writes entries me, me + threads, ...: by position, so that neighbouring threads write neighbouring entries
 // and nobody has to clear the list before.
-__device__ __forceinline__ void emit_work(int4 *work, int grid, int n_wt, int per_job, const int2 *tiles, int n_tiles, int num_experts,
-                                          int me, int threads) {
-    constexpr int GW = 8;
-    const int n_jobs = (n_wt + per_job - 1) / per_job, total = n_tiles * n_jobs;
-    const int per_xcd = (total + 7) >> 3;
+__device__ __forceinline__ void emit_work(int4 *work, int grid, const ListShape &s, const int2 *tiles, int n_tiles, int num_experts, int me,
+                                          int threads) {
+    constexpr int GW = kListGroup;
     for (int w = me; w < grid; w += threads) {
-        const int pos = w >> 3, l = (w & 7) * per_xcd + pos;
+        const int pos = w >> 3, l = (w & 7) * s.per_xcd + pos;
         int4 entry = make_int4(-1, -1, 0, 0);
-        if (pos < per_xcd && l < total) {
+        if (pos < s.per_xcd && l < s.total) {
             const int wg = l / (GW * n_tiles), rem = l - wg * GW * n_tiles;
-            const int gw = min(GW, n_jobs - wg * GW), t = rem / gw, j = wg * GW + rem - t * gw;
-            const int2 tl = tiles[t];
-            if (tl.y >= 0 && tl.y < num_experts) {
-                // (the only row tile of its expert: then nobody else reads that expert's weight rows)
-                const bool shared = (t > 0 && tiles[t - 1].y == tl.y) || (t + 1 < n_tiles && tiles[t + 1].y == tl.y);
-                const int wt = j * per_job, cnt = min(per_job, n_wt - wt);
-                entry = make_int4(tl.x, wt | (tl.y << 16) | ((cnt - 1) << 26), 0, shared ? 0 : 1);
-            }
+            const int gw = min(GW, s.n_jobs - wg * GW), t = rem / gw;
+            entry = list_entry(s, tiles, n_tiles, num_experts, t, wg * GW + rem - t * gw);
         }
         work[w] = entry;
+    }
+}
+// The same list, a row tile of a thread after the other: where the tiles are in memory, an entry is too little to wait for them.
+__device__ __forceinline__ void emit_work_by_tile(int4 *work, int grid, const ListShape &s, const int2 *tiles, int n_tiles, int num_experts,
+                                                  int me, int threads) {
+    constexpr int GW = kListGroup;
+    for (int w = me; w < grid; w += threads) {
+        const int pos = w >> 3;
+        if (pos >= s.per_xcd || (w & 7) * s.per_xcd + pos >= s.total) work[w] = make_int4(-1, -1, 0, 0);
+    }
+    for (int t = me; t < n_tiles; t += threads) {
+        const int4 first = list_entry(s, tiles, n_tiles, num_experts, t, 0);
+        for (int j = 0; j < s.n_jobs; ++j) {
+            const int wg = j / GW, l = wg * GW * n_tiles + t * min(GW, s.n_jobs - wg * GW) + (j - wg * GW);
+            const int xcd = l / s.per_xcd, wt = j * s.per_job, cnt = min(s.per_job, s.n_wt - wt);
+            work[8 * (l - xcd * s.per_xcd) + xcd] =
+                first.x < 0 ? first : make_int4(first.x, (first.y & (0x3ff << 16)) | wt | ((cnt - 1) << 26), 0, first.w);
+        }
     }
 }
 
 // Prologue of an mxfp8 call.  The first workgroups build the row tiles and work lists of the two-group kernels:
 // consecutive blocks of one expert are paired, an expert's odd last block stays single (one pass of
 // block-wide scans per 256 blocks, then the two walk orders).  Each of them works out all tiles, in LDS, and writes its
-// share of the lists; only of more than kLdsTiles blocks workgroup 0 writes them alone, from tiles in the workspace.  What bounds it is
+// share of the lists; only of more than kLdsTiles blocks workgroup 0 writes them alone, from tiles in the workspace, a tile at a time
+// (140000 tokens on 32 experts, K = N = 2048, by position there 81.9, by tile 63.7 us).  What bounds it is
 // the chain of scans; the lists of 4096 tokens on 256 experts have 22440 entries, 11264 of them jobs.
 // A builder comes late to its share of the rest, so there are only as many as the lists are long (kListEntries).  Prologue with one builder /
 // one per 512 entries / a quarter of the workgroups, us: 600 tokens on 8 experts (K = N = 512) 4.2 / 4.4 / 5.3, 2000 on 8 (K 2048, N 512) 4.8 /
@@ -611,8 +639,14 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
         __threadfence_block();
         __syncthreads();  // tiles written above are read below by other threads
         const int me = (int)blockIdx.x * 256 + tid, threads = builders * 256;
-        emit_work(work_up, grid_up, n_wt_up, per_job_up, table, nt, num_experts, me, threads);
-        emit_work(work_down, grid_down, n_wt_down, per_job_down, table, nt, num_experts, me, threads);
+        const ListShape up(n_wt_up, per_job_up, nt), down(n_wt_down, per_job_down, nt);
+        if (n_live <= kLdsTiles) {
+            emit_work(work_up, grid_up, up, table, nt, num_experts, me, threads);
+            emit_work(work_down, grid_down, down, table, nt, num_experts, me, threads);
+        } else {
+            emit_work_by_tile(work_up, grid_up, up, table, nt, num_experts, me, threads);
+            emit_work_by_tile(work_down, grid_down, down, table, nt, num_experts, me, threads);
+        }
         __syncthreads();  // (a workgroup that re-tiles, too, uses the LDS again)
     }
     if (do_invert) {

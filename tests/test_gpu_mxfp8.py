@@ -381,3 +381,45 @@ def test_prologue_tables_in_lds_and_in_the_workspace(blocks, device):
     for a in range(0, T, 65536):
         part, _ = forward(a, min(a + 65536, T))
         assert torch.equal(got[a:a + 65536].view(torch.int16), part.view(torch.int16))
+
+
+@pytest.mark.parametrize("blocks", [40, 4170])  # lists from row tiles in LDS, and from the workspace
+@pytest.mark.parametrize("per", [1, 2])
+def test_work_lists_leave_out_blocks_without_an_expert(blocks, per, device):
+    """Two groups of weight tiles in the down kernel (9, one or two per job): bit for bit what calls on parts of the tokens give, and nothing
+    for the tokens of blocks whose expert does not exist."""
+    import prime_moe
+    from prime_moe import _native
+    T, K, E, N = blocks * 128, 2304, 3, 512
+    g = torch.Generator(device=device).manual_seed(blocks)
+    xq, xs = prime_moe.quantize_mx(torch.randn((T, K), generator=g, device=device, dtype=torch.bfloat16))
+    ids = torch.randint(0, E, (T, 1), generator=g, device=device, dtype=torch.int32)
+    wts = torch.ones((T, 1), device=device)
+    w1, w1s = prime_moe.quantize_mx((torch.randn((E, N, K), generator=g, device=device) / 48).to(torch.bfloat16))
+    w2, w2s = prime_moe.quantize_mx((torch.randn((E, K, N // 2), generator=g, device=device) / 16).to(torch.bfloat16))
+    w1s, w2s = prime_moe.pack_scales_blocked(w1s), prime_moe.pack_scales_blocked(w2s)
+
+    def forward(a, b, drop=()):
+        s, e, n = torch.ops.prime_moe.moe_align(ids[a:b].contiguous(), E, 128, 1)
+        for i, blk in enumerate(drop):
+            e[blk] = (-1, E + 3)[i % 2]
+        out = torch.empty((b - a, K), dtype=torch.bfloat16, device=device)
+        prime_moe.fused_moe_mxfp8(xq[a:b].contiguous(), xs[a:b].contiguous(), w1, w1s, w2, w2s, s, e, n, wts[a:b].contiguous(), out, 1,
+                                  128, 64, 4, 2, split=True)
+        return out, s, int(n[0]) // 128
+    _native.load().pmoe_set_tiles_per_workgroup(per)
+    try:
+        drop = [0, 5, 6, blocks // 2, blocks - 1]
+        got, s, live = forward(0, T, drop)
+        assert (live <= 4160) == (blocks == 40) and T > 64 * E
+        for blk in drop:
+            rows = s[128 * blk:128 * blk + 128]
+            rows = rows[rows >= 0].long()
+            assert rows.numel() > 0 and not bool(got[rows].any())
+            got[rows] = float("nan")
+        for a in range(0, T, 65536):
+            part, _, _ = forward(a, min(a + 65536, T))
+            kept = ~torch.isnan(got[a:a + 65536, :1])
+            assert torch.equal(torch.where(kept, got[a:a + 65536], 0).view(torch.int16), torch.where(kept, part, 0).view(torch.int16))
+    finally:
+        _native.load().pmoe_set_tiles_per_workgroup(0)
