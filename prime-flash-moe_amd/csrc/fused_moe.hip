@@ -594,7 +594,8 @@ __global__ __launch_bounds__(256) void moe_prologue_kernel(const int32_t *expert
     if (CROWD && !crowded_mx(ntpp, n_blocks, n_pairs, n_wt_up, n_cus)) return;
     const int n_live = min((ntpp[0] + kBlockRows - 1) / kBlockRows, n_blocks);
     const int builders = n_live <= kLdsTiles ? max(min(min((grid_up + grid_down) / kListEntries, (int)gridDim.x / 4), 32), 1) : 1;
-    __shared__ uint32_t s_sc[kBlockRows][65];  // row tiles first
+    __shared__ alignas(16) uint32_t s_sc[kBlockRows][65];  // row tiles first
+    static_assert(kLdsTiles * sizeof(int2) <= sizeof(s_sc), "the row tiles fit");
     if ((int)blockIdx.x < builders) {
         __shared__ int s_max[4], s_sum[4], s_carry[2];
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
