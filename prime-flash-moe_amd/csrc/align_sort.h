@@ -107,11 +107,11 @@ __device__ __forceinline__ void write_expert_ids(const Outputs &o, const int32_t
 __host__ __device__ constexpr int sort_words(int n_waves, int E) { return 2 * E + 1 + n_waves * E; }
 
 // The whole sort by one workgroup of NW waves whose ids are in registers (load_ids from 0; n <= NW * 64 * PER), in two steps
-// with a barrier between them.  What does not need the ids:
+// with a barrier between them.  What does not need the ids, by thread `me` of `n_threads`:
 template <int NW>
-__device__ __forceinline__ void begin_sort(const Outputs &o, int E, int32_t *smem) {
-    fill_minus_one(o.sorted_token_ids, o.max_padded, threadIdx.x, NW * 64);  // complete before any pair id lands on top of it: barriers follow
-    for (int i = threadIdx.x; i < NW * E; i += NW * 64) smem[2 * E + 1 + i] = 0;
+__device__ __forceinline__ void begin_sort(const Outputs &o, int E, int32_t *smem, int me, int n_threads) {
+    fill_minus_one(o.sorted_token_ids, o.max_padded, me, n_threads);  // complete before any pair id lands on top of it: barriers follow
+    for (int i = me; i < NW * E; i += n_threads) smem[2 * E + 1 + i] = 0;
 }
 template <int NW, int PER>
 __device__ __forceinline__ void finish_sort(const int (&id)[PER], const Outputs &o, int E, int id_bits, int32_t *smem) {
@@ -145,7 +145,7 @@ __device__ __forceinline__ void finish_sort(const int (&id)[PER], const Outputs 
 }
 template <int NW, int PER>
 __device__ __forceinline__ void sort_in_workgroup(const int (&id)[PER], const Outputs &o, int E, int id_bits, int32_t *smem) {
-    begin_sort<NW>(o, E, smem);
+    begin_sort<NW>(o, E, smem, threadIdx.x, NW * 64);
     __syncthreads();
     finish_sort<NW, PER>(id, o, E, id_bits, smem);
 }

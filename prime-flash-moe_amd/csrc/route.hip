@@ -125,16 +125,17 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const T *__restrict__ l
 // Top-k of all tokens (wave w: tokens w, w + NW, ...) and the sort of their ids: n_tokens * top_k <= NW * 64.  Workgroup 0 does
 // that for the rows that the pairs can reach (`reach`, a multiple of block_m or max_padded: every pair in an expert of its own);
 // the others write what is known of the rest, -1 and the last expert.  (A token of 128 experts has room for 16264 rows and
-// reaches 1024, five of 256 experts 32552 and 5120; one CU takes 0.5 and 1 us to fill them.  One token of 128 experts, the whole
-// layer, all rows behind the top-k / in front of it / with other workgroups 24.75 / 24.55 / 24.35 us.)
+// reaches 1024, five of 256 experts 32552 and 5120; one CU takes 0.5 and 1 us to fill them.)  Workgroup 0 fills its rows with the waves that
+// have no token, beside the top-k, or with all of them behind it: stores in front of its logits are waited for with them.  The whole
+// kernel, all rows by one workgroup behind the top-k / as it is, us: one token, top 1 of 3 3.7 / 3.6, top 8 of 64, 128, 256 and 512 5.0 / 4.7, 6.0 /
+// 5.4, 7.6 / 6.4 and 10.5 / 8.3; 16 tokens, top 1 of 3 4.0 / 4.0, top 8 of 64, 256 and 512 5.7 / 5.7, 8.6 / 7.8 and 12.2 / 10.7.
 template <int NW, int EPL, typename T>
 __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restrict__ logits, const float *__restrict__ bias,
                                                               int32_t *__restrict__ topk_ids, float *__restrict__ topk_weights,
-                                                              pmoe::align::Outputs o, int reach, int n_tokens, int E, int top_k, int id_bits) {
+                                                              pmoe::align::Outputs o, int reach, int reach_blocks, int n_tokens, int E, int top_k, int id_bits) {
     extern __shared__ int32_t smem[];
     __shared__ int32_t ids[NW * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int reach_blocks = (int)min(((int64_t)reach + o.block_m - 1) / o.block_m, (int64_t)o.max_blocks);
     if (blockIdx.x > 0) {
         const int n = (int)(gridDim.x - 1) * NW * 64, me = (int)(blockIdx.x - 1) * NW * 64 + tid;
         pmoe::align::fill_minus_one(o.sorted_token_ids + reach, o.max_padded - reach, me, n);
@@ -143,7 +144,8 @@ __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restric
     }
     o.max_padded = reach;
     o.max_blocks = reach_blocks;
-    pmoe::align::begin_sort<NW>(o, E, smem);  // (its stores are on their way while the logits are)
+    const int busy = n_tokens <= NW - 2 ? n_tokens : 0;  // (one wave alone would be the last to arrive)
+    if (busy > 0 && wave >= busy) pmoe::align::begin_sort<NW>(o, E, smem, tid - 64 * busy, 64 * (NW - busy));
     for (int t = wave; t < n_tokens; t += NW) {
         int id;
         float w;
@@ -154,6 +156,7 @@ __global__ __launch_bounds__(NW * 64) void route_small_kernel(const T *__restric
             topk_weights[t * top_k + lane] = w;
         }
     }
+    if (busy == 0) pmoe::align::begin_sort<NW>(o, E, smem, tid, 64 * NW);
     __syncthreads();
     const int id[1] = {tid < n_tokens * top_k ? ids[tid] : -1};
     pmoe::align::finish_sort<NW, 1>(id, o, E, id_bits, smem);
@@ -184,10 +187,11 @@ int launch_topk(const T *logits, const float *bias, int32_t *topk_ids, float *to
             const int n = n_tokens * top_k;
             const int64_t rows = n + (int64_t)std::min(n, E) * (o->pad_to - 1);
             const int reach = (int)std::min<int64_t>(o->max_padded, (rows + o->block_m - 1) / o->block_m * o->block_m);
+            const int reach_blocks = (int)std::min<int64_t>(((int64_t)reach + o->block_m - 1) / o->block_m, o->max_blocks);
             const int64_t rest = std::max<int64_t>(o->max_padded - reach, 4 * ((int64_t)o->max_blocks - reach / o->block_m));
             const int fillers = (int)std::min<int64_t>((rest + NW * 256 - 1) / (NW * 256), 15);  // 16 bytes a thread and turn
             hipLaunchKernelGGL((route_small_kernel<NW, EPL, T>), dim3(1 + fillers), dim3(NW * 64), sizeof(int32_t) * (size_t)pmoe::align::sort_words(NW, E),
-                               s, logits, bias, topk_ids, topk_weights, *o, reach, n_tokens, E, top_k, pmoe::align::id_bits_for(E));
+                               s, logits, bias, topk_ids, topk_weights, *o, reach, reach_blocks, n_tokens, E, top_k, pmoe::align::id_bits_for(E));
         });
         return pmoe::check_launch("route launch");
     }

@@ -26,6 +26,29 @@ def _check(logits: torch.Tensor, top_k: int, bias=None, block_m=128, bpc=1):
     return ids, w, s, e, t
 
 
+def _check_every_word(logits: torch.Tensor, top_k: int, block_m: int, bpc: int, shift: int = 0):
+    """The C entry point on outputs that hold something else: every word of the schedule is written and none beside it.  `shift`: words
+    by which the rows of the schedule start off 16-byte alignment."""
+    from prime_moe import _native
+    T, E = logits.shape
+    pad_to = block_m * bpc
+    n_rows = (T * top_k + E * (pad_to - 1) + pad_to - 1) // pad_to * pad_to
+    sizes, guard, old = (n_rows, n_rows // block_m, 1), 64, 12345
+    bufs = [torch.full((guard + shift + n + guard,), old, dtype=torch.int32, device=logits.device) for n in sizes]
+    ids = torch.empty((T, top_k), dtype=torch.int32, device=logits.device)
+    w = torch.empty((T, top_k), dtype=torch.float32, device=logits.device)
+    ptrs = [b.data_ptr() + 4 * (guard + shift) for b in bufs]
+    _native.check(_native.load().pmoe_route(logits.data_ptr(), 0, None, ids.data_ptr(), w.data_ptr(), *ptrs, T, E, top_k, block_m, pad_to, n_rows,
+                                            n_rows // block_m, None, 0, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    ref_ids, _ = O.route_topk(logits.cpu().numpy(), top_k, None)
+    for b, n, want, name in zip(bufs, sizes, O.moe_align_fast(ref_ids, E, block_m, bpc),
+                                ("sorted_token_ids", "expert_ids", "num_tokens_post_padded")):
+        got = b.cpu().numpy()
+        np.testing.assert_array_equal(got[guard + shift:guard + shift + n], want, err_msg=name)
+        assert (got[:guard + shift] == old).all() and (got[guard + shift + n:] == old).all(), name
+
+
 @pytest.mark.parametrize("name", ["c1_readme_bf16", "c2_mixtral_bf16", "c3_qwen3_bf16", "c4_dsv3_mxfp8"])
 def test_route_on_benchmark_routings(name, device):
     # the gate logits of the benchmark configurations (those that route by top-k of logits)
@@ -80,8 +103,17 @@ def test_rows_that_no_pair_can_reach(T, E, k, spread, block_m, bpc, device):
     for t in range(T):
         first = t * k if spread else 0
         logits[t, [(first + i) % E for i in range(k)]] = torch.arange(k, 0, -1, device=device, dtype=torch.float32)
-    torch.empty((1 << 22,), dtype=torch.int32, device=device).fill_(12345)  # dirty the allocator's blocks
     _check(logits, k, block_m=block_m, bpc=bpc)
+    _check_every_word(logits, k, block_m, bpc)
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 8, 2), (13, 70, 4), (14, 3, 1), (14, 256, 8), (15, 256, 8), (16, 256, 8), (32, 8, 2), (5, 600, 8), (6, 600, 8),
+                                   (7, 600, 8), (8, 600, 8)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_rows_filled_beside_the_top_k_and_behind_it(T, E, k, shift, device):
+    """By the waves without a token, where two are left of the 16 (8 beyond 512 experts), and by all of them otherwise."""
+    g = torch.Generator(device=device).manual_seed(T + E + k)
+    _check_every_word(torch.randn((T, E), generator=g, device=device), k, 128, 1, shift)
 
 
 def test_one_token_with_a_block_beyond_half_of_31_bits(device):
