@@ -666,7 +666,6 @@ __global__ __launch_bounds__(512) void moe_deep_up_kernel(MoeArgs a, int n_wt_do
                 down.n_tiles = n_down;
                 estimate_kernel(n_down, n_f2, n_wt_down, a.H * 2 / tall::kRB, n_cus, down.parts, down.tail);
                 a.plan->up = kp;
-                a.plan->up.n_tiles = n_tiles;  // (as the down kernel's choice counts them: tiles of up to six pairs)
                 a.plan->down = down;
                 a.plan->deep_frags = 2 * n_f2;
             }

@@ -343,6 +343,14 @@ def test_deep_up_kernel_cuts_and_plans(K, N, counts, device):
         assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
 
 
+def _deep_cut(f2, K, N, device):
+    """(tiles, parts) of the up kernel in deep mode, of runs with f2 pairs of fragments each."""
+    cus = torch.cuda.get_device_properties(device).multi_processor_count // 8 * 8
+    pairs, n_wt = sum(f2), N // 256
+    tiles = pairs if pairs <= 64 and pairs * n_wt * 8 <= cus else sum((f + 1) // 2 for f in f2)
+    return tiles, max(1, min(8, K // 64 // 4, cus // (tiles * n_wt), 1024 // (2 * pairs * n_wt)))
+
+
 @pytest.mark.parametrize("K,N,counts", [
     (2048, 512, [193, 512, 130, 126]),         # 4 + 8 + 3 + 2 = 17 pairs of fragments x 2 weight tiles: one more than tiles of one pair
     (2048, 512, [192, 512, 130, 126]),         # 16: the most that tiles of one pair take
@@ -371,6 +379,11 @@ def test_deep_up_kernel_tiles_of_one_pair_and_two(K, N, counts, device):
     assert T > 64 * E and K >= 2048  # the rules of the dispatch
     assert (blocks <= 64 and blocks * (N // 256) <= 128) == (counts not in ([8066], [700, 600, 368]))
     ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    plan = _prologue_workspace(x, w1, w2, sched, wts, torch.empty_like(x), 1)[:16].view(torch.int32).tolist()
+    if counts not in ([8066], [700, 600, 368]):
+        assert (plan[0], plan[1], plan[3]) == (*_deep_cut([(c + 63) // 64 for c in counts], K, N, device), 1)
+    else:
+        assert plan[3] == 0
     out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
     prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, 1, 128, 64, 4, 2, 1, 1, True)
     torch.cuda.synchronize()
@@ -439,7 +452,7 @@ def test_deep_up_kernel_takes_blocks_in_any_order(counts, order, device):
             f2.append((128 * (b - start) + rows[b] + 63) // 64)
     ws = _prologue_workspace(x, w1, w2, (s, e, n), wts, torch.empty_like(x), top_k)
     plan = ws[:36].view(torch.int32).tolist()
-    assert plan[0] == sum((f + 5) // 6 for f in f2) and plan[3] == 1  # the up kernel's tiles, deep
+    assert (plan[0], plan[1]) == _deep_cut(f2, K, N, device) and plan[3] == 1  # the up kernel's tiles and parts, deep
     assert plan[8] == 2 * sum(f2)                                     # fragments
     ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
     out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
