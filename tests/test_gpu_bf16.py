@@ -275,12 +275,25 @@ def test_block_without_expert_and_duplicate_pair(device):
         assert rel_clamp(got[keep], ref[keep], 1.0) <= BF16_GATE
 
 
+def _takes_deep(pairs, E, blocks, K, N):
+    """The rules of the dispatch, on 256 CUs."""
+    n_wt = N // 256
+    if K < 2048 or blocks > 64 or blocks * n_wt > 128:
+        return False
+    if blocks * n_wt <= 32:
+        return pairs > 32 * E
+    return pairs > (64 if K < 4096 or n_wt > 2 else 34 if 3 * E * N * K >= 112e6 else 48) * E
+
+
 @pytest.mark.parametrize("T,K,E,N,top_k,exact,deep", [
     (256, 4096, 8, 512, 4, False, True),    # the README shape: 8 - 16 row tiles x 2 weight tiles, every tile split 8 ways
     (100, 2048, 4, 256, 2, False, True),    # one weight tile, tiles of two to four fragments
     (130, 6144, 3, 512, 3, True, True),     # exact-size schedule, a second block with two live rows
     (33, 2048, 1, 256, 1, False, True),     # one weight tile, a second fragment with one live row
     (300, 2176, 2, 1024, 2, False, True),   # 17 slabs: parts of unequal length
+    (700, 4096, 8, 512, 4, False, True),    # 30 blocks x 2: tiles of two pairs of fragments
+    (180, 4096, 37, 256, 9, False, True),   # 50 blocks, a fragment or two each
+    (900, 2304, 2, 2048, 1, True, True),    # exact-size schedule, 8 weight tiles
     (40, 2048, 4, 256, 2, False, False),    # up to 32 rows per expert: the streaming kernels, no deep split
     (1, 2048, 1, 256, 1, False, False),     # one row, likewise
 ])
@@ -290,7 +303,7 @@ def test_few_jobs_deep_split_and_join_kernel(T, K, E, N, top_k, exact, deep, dev
     oracle, and bit for bit the same on a second call (the join adds the parts in part order)."""
     import prime_moe
     n_blocks = (T * top_k + E * 127 + 127) // 128
-    assert deep == (T * top_k > 32 * E) and n_blocks * (N // 256) <= 32 and K >= 2048  # the rules of the dispatch
+    assert deep == _takes_deep(T * top_k, E, n_blocks, K, N)
     for split in (True, False):
         _run_case(T, K, E, N, top_k, split, device, seed=T + K, use_op_align=not exact, exact=exact, hot_last=False)
     g, x, w1, w2 = _inputs(T, K, E, N, device, T + K)
@@ -313,6 +326,8 @@ def test_few_jobs_deep_split_and_join_kernel(T, K, E, N, top_k, exact, deep, dev
     (2048, 256, [40] * 9 + [1, 0, 63, 64, 65, 127, 128, 129, 0, 33]),  # 28 blocks: most runs a block long, some experts without rows
     (2304, 768, [385, 3]),                                            # a run of four blocks with one row in the last, two tiles
     (4096, 512, [0, 700, 0]),                                         # two runs of six blocks
+    (4096, 256, [48] * 24 + [1, 0, 63, 64, 65, 127, 128, 129, 0, 33, 200, 257]),  # 57 blocks, 41 of them live, most runs a block long
+    (2304, 512, [385, 900, 3, 2300, 700]),                            # 58 blocks x 2, runs of up to 18
 ])
 def test_deep_up_kernel_cuts_and_plans(K, N, counts, device):
     """The tiles that every workgroup of the deep up kernel works out for itself: also with tokens beyond M (holes in a block),
@@ -326,13 +341,13 @@ def test_deep_up_kernel_cuts_and_plans(K, N, counts, device):
     keep = T - T // 8
     g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
     s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
-    assert keep * top_k > 32 * E and s.numel() // 128 * (N // 256) <= 32 and K >= 2048  # the rules of the dispatch
+    last = int((s >= 0).nonzero().max()) + 1
+    assert _takes_deep(T * top_k, E, s.numel() // 128, K, N) and _takes_deep(keep * top_k, E, (last + 127) // 128, K, N)
     e_bad = e.clone()
     e_bad[1] = E + 3
     w_ref = wts.clone()
     lost = s[128:256]
     w_ref.view(-1)[lost[lost >= 0].long()] = 0.0
-    last = int((s >= 0).nonzero().max()) + 1
     for e_, w_, m, length in ((e, wts, T, s.numel()), (e_bad, w_ref, keep, last)):
         ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), w_.cpu())[:m]
         torch.empty((32 << 20,), dtype=torch.float32, device=device).fill_(float("nan"))  # dirty the allocator's blocks
@@ -426,6 +441,8 @@ def test_deep_up_kernel_on_more_cus_than_its_table_has_tiles(counts, device):
     ([130, 60, 40, 230], [4, 0, 1, 2, 3, 5]),            # experts 3 0 0 1 2 3: another expert in front of expert 0
     ([130, 60, 40, 230], [2, 0, 4, 1, 5, 3]),            # experts 1 0 3 0 3 2: no expert's blocks side by side
     ([40, 230, 60, 130], [1, 2, 0, 4, 5, 3]),            # experts 1 1 0 3 3 2
+    ([900, 1300, 1100, 700, 1300], "any"),               # 45 blocks: neighbours of one expert by chance, short blocks inside a run
+    ([60] * 30 + [900, 900], "any"),                     # 46
 ])
 def test_deep_up_kernel_takes_blocks_in_any_order(counts, order, device):
     """expert_ids says which expert a block belongs to, in whatever order the blocks come; neighbours of one expert are one run."""
@@ -436,8 +453,10 @@ def test_deep_up_kernel_takes_blocks_in_any_order(counts, order, device):
     T = ids.shape[0]
     g, x, w1, w2 = _inputs(T, K, E, N, device, seed=N)
     s, e, n = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
-    assert T * top_k > 32 * E and s.numel() // 128 * (N // 256) <= 32  # the rules of the dispatch
+    assert _takes_deep(T * top_k, E, s.numel() // 128, K, N)
     n_live = int(n[0]) // 128
+    if order == "any":
+        order = torch.randperm(n_live, generator=torch.Generator().manual_seed(E)).tolist()
     if order is not None:
         assert len(order) == n_live
         s, e = s.clone(), e.clone()
@@ -457,6 +476,30 @@ def test_deep_up_kernel_takes_blocks_in_any_order(counts, order, device):
     ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
     out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
     prime_moe.fused_moe_bf16(x, w1, w2, s, e, n, wts, out, top_k, 128, 64, 4, 2, 1, 1, True)
+    torch.cuda.synchronize()
+    got = out.float().cpu()
+    assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE
+
+
+@pytest.mark.parametrize("K,E,N,rows", [
+    (4096, 37, 256, 34),   # 116 MB of weights, more than 32 blocks
+    (4096, 16, 512, 48),   # 101 MB
+    (2048, 24, 512, 64),   # a shorter contraction
+    (4096, 8, 512, 32),    # up to 32 (block, weight tile) pairs
+])
+@pytest.mark.parametrize("more", [0, 1])
+def test_line_between_streaming_and_deep_mode(K, E, N, rows, more, device):
+    import prime_moe
+    T = rows * E + more
+    g, x, w1, w2 = _inputs(T, K, E, N, device, seed=E)
+    ids, wts = reference_routing(T, E, 1, device, g, hot_last=False)
+    sched = torch.ops.prime_moe.moe_align(ids, E, 128, 1)
+    assert _takes_deep(T, E, sched[0].numel() // 128, K, N) == bool(more)
+    plan = _prologue_workspace(x, w1, w2, sched, wts, torch.empty_like(x), 1)[:16].view(torch.int32).tolist()
+    assert plan[3] == more
+    ref = O.fused_moe_dense(x.cpu(), w1.cpu(), w2.cpu(), ids.cpu(), wts.cpu())
+    out = torch.empty((T, K), dtype=torch.bfloat16, device=device)
+    prime_moe.fused_moe_bf16(x, w1, w2, *sched, wts, out, 1, 128, 64, 4, 2, 1, 1, True)
     torch.cuda.synchronize()
     got = out.float().cpu()
     assert torch.isfinite(got).all() and rel_clamp(got, ref, 1.0) <= BF16_GATE

@@ -35,8 +35,8 @@ def test_workspace_query_and_c_side_validation_need_no_gpu():
     lib = _native.load()
     # bf16: plan (256 B) + run list with its order (20 B per block + 1) + the two tables of row tiles (16 B per block
     # + 1 each) + fp32 partial sums of
-    # the deep contraction split when the problem has at most 32 (block, up weight tile) pairs and K >= 2048
-    # (8 parts x 32 KB per fragment and weight tile) + inverse of the sorted order (4 B per pair) + y (one row of
+    # the deep contraction split (8 parts x 32 KB per fragment and weight tile, 1024 sums at most) for at most 64 blocks and 128 (block, up
+    # weight tile) pairs and K >= 2048, unless the call always streams + inverse of the sorted order (4 B per pair) + y (one row of
     # K bf16 per pair) + act (rows * H bf16), each rounded to 256 B; the same for both values of split
     assert lib.pmoe_fused_moe_bf16_workspace_bytes(256, 4096, 512, 8, 2048, 4, 1) == \
         256 + 3 * 512 + 8 * 4 * 16 * 2 * 32768 + 256 * 4 * 4 + 256 * 4 * 4096 * 2 + 2048 * 256 * 2
@@ -83,6 +83,25 @@ def test_partial_sums_are_not_reserved_for_calls_that_always_stream(M, top_k, E,
     assert _native.load().pmoe_fused_moe_bf16_workspace_bytes(M, K, N, E, rows, top_k, 1) == \
         256 + up((blocks + 1) * 20) + 2 * up((blocks + 1) * 16) + (min(8 * 4 * blocks, 1024) * 32768 if sums else 0) + \
         up(pairs * 4) + pairs * K * 2 + rows * N
+
+
+@pytest.mark.parametrize("K,N,blocks,sums", [
+    (2048, 256, 10, 320),      # 8 parts of 4 fragments of every block
+    (2048, 256, 33, 1024),     # more than the limit, which two parts of 128 pairs come to
+    (2048, 512, 64, 1024),     # the most blocks, and the most pairs
+    (2048, 512, 65, 0),
+    (2048, 256, 65, 0),        # blocks alone
+    (2048, 2048, 16, 1024),
+    (2048, 2048, 17, 0),       # 136 pairs
+    (1920, 256, 10, 0),        # a contraction too short to share
+])
+def test_partial_sums_of_the_deep_split(K, N, blocks, sums):
+    from prime_moe import _native
+    rows, E = blocks * 128, 1
+    pairs = rows - 127
+    up = lambda n: (n + 255) // 256 * 256
+    assert _native.load().pmoe_fused_moe_bf16_workspace_bytes(pairs, K, N, E, rows, 1, 1) == \
+        256 + up((blocks + 1) * 20) + 2 * up((blocks + 1) * 16) + sums * 32768 + up(pairs * 4) + up(pairs * K * 2) + rows * N
 
 
 def test_missing_library_fails_loudly(monkeypatch):
